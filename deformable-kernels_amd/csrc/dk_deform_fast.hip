@@ -30,6 +30,7 @@
 #include <algorithm>
 #include <cstdlib>
 
+#include "dk_deform.h"
 #include "dk_kernels.h"
 #include "dk_scope_table.h"
 
@@ -1027,56 +1028,6 @@ __global__ __launch_bounds__(256) void absmax_kernel(const T* __restrict__ p, lo
   if ((threadIdx.x & 63) == 0) wave_max[threadIdx.x >> 6] = m;
   __syncthreads();
   if (threadIdx.x == 0) out[blockIdx.x] = max(max(wave_max[0], wave_max[1]), max(wave_max[2], wave_max[3]));
-}
-constexpr int kAbsParts = 512;  // workgroups of absmax_kernel = words the consumers reduce
-
-// The maximum of absmax_kernel's words, for every thread of the workgroup (two barriers).
-__device__ __forceinline__ float block_absmax(const unsigned* __restrict__ parts) {
-  __shared__ unsigned s_max;
-  if (threadIdx.x == 0) s_max = 0u;
-  __syncthreads();
-  unsigned m = 0u;
-  for (int i = threadIdx.x; i < kAbsParts; i += blockDim.x) m = max(m, parts[i]);
-  for (int s = 32; s > 0; s >>= 1) m = max(m, (unsigned)__shfl_xor((int)m, s));
-  if ((threadIdx.x & 63) == 0) atomicMax(&s_max, m);
-  __syncthreads();
-  return __uint_as_float(s_max);
-}
-
-// The fixed-point sums need a finite bound gmax * wmax[c] on a term.  With an infinity or a NaN in
-// out_grad (gmax is then that value: the maximum is taken on bit patterns) or in a channel's filter
-// there is none, and the conversions to integers would turn such terms into zeros or wrapped numbers:
-// the workgroup then writes NaN to the planes it owns instead (all of grad_input for a non-finite
-// out_grad).  The reference's float atomics carry a non-finite term to the elements it touches;
-// what a caller tests -- any non-finite value in the gradient, as loss scaling does -- gives the
-// same answer.  Uniform over the workgroup; must be called by all its threads after wmax is visible.
-template <typename T>
-__device__ __forceinline__ bool write_nan_if_unbounded(float gmax, const float* wmax, int nch, T* planes0, size_t step,
-                                                       int plane) {
-  bool bounded = true;
-  for (int j = 0; j < nch; ++j) bounded = bounded && (fabsf(gmax * wmax[j]) < __builtin_inff());  // false for NaN
-  if (bounded) return false;
-  for (int j = 0; j < nch; ++j)
-    for (int e = threadIdx.x; e < plane; e += blockDim.x) dk::st(planes0 + (size_t)j * step + e, __builtin_nanf(""));
-  return true;
-}
-
-// A result element that is not read again by the operator: non-temporal for 4-byte elements (a wave writes whole
-// lines), the plain store for 2-byte ones (as partial lines they reach memory one by one).
-__device__ __forceinline__ void st_stream(float* p, float v) { __builtin_nontemporal_store(v, p); }
-template <typename T>
-__device__ __forceinline__ void st_stream(T* p, float v) { dk::st(p, v); }
-
-// Two channels share a 64-bit sum while at most 2^kPairHead samples touch one input element: a term is then
-// rounded on a grid of 2^-(31 - kPairHead) = 2^-24 of the largest possible term or finer.  (3 x 3 taps at stride 1
-// put 36 samples on an element on average and about 65 on the fullest element of a large plane.)
-constexpr int kPairHead = 7;
-
-// floor(v + 0.5) as a signed 32-bit integer, one instruction
-__device__ __forceinline__ int round_half_up(float v) {
-  int r;
-  asm("v_cvt_rpi_i32_f32 %0, %1" : "=v"(r) : "v"(v));
-  return r;
 }
 
 template <typename T, int SH, int SW>
@@ -2849,6 +2800,10 @@ bool run_deform_grad_input(const Geo& g, const T* gout, const T* off, const T* r
   if (reinterpret_cast<uintptr_t>(gout) % 16 != 0) return false;  // absmax_kernel reads 16-byte vectors
   unsigned* gmax = static_cast<unsigned*>(ws);
   const long n = (long)g.batch * g.channel * g.out_h * g.out_w;
+  if (lanes_deform_grad_input_applies(g)) {
+    absmax_kernel<T><<<kAbsParts, 256, 0, stream>>>(gout, n, gmax);
+    if (lanes_deform_grad_input<T>(g, gout, off, rot, filter, gin, gmax, stream)) return true;
+  }
   if (tiled) {
     // workspace: the maxima of |gout|, the images' sample counts, the tiles' rows
     unsigned* most_img = gmax + kAbsParts;

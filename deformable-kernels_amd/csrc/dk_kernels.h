@@ -40,6 +40,8 @@ enum TestSwitch : unsigned {
   kNoNhwcStaged = 1u << 22,     // DK_NO_NHWC_STAGED     the channels-last kernels that stage planar tiles in LDS / contract 32 channels per matrix instruction (the kernels named under DK_NO_NHWC_MFMA run instead)
   kForceNhwcGatherMfma = 1u << 23,  // DK_FORCE_NHWC_GATHER_MFMA  the channels-last matrix-core forward / grad input wherever it applies, not only where it is the faster kernel
   kNoImagePacked = 1u << 24,    // DK_NO_IMAGE_PACKED    the packed flat-copy kernels of the per-image depthwise convolution on 16-bit tensors (the flat-copy kernels that unpack to fp32 run instead)
+  kNoDeformLanes = 1u << 25,    // DK_NO_DEFORM_LANES    the deformable kernels with the lanes along the channels (dk_deform_lanes.hip; those with a pixel per lane run instead)
+  kForceDeformLanes = 1u << 26, // DK_FORCE_DEFORM_LANES ... wherever they apply, not only where they are the faster ones
   kNoOffsetPairs = 1u << 18,    // DK_NO_OFFSET_PAIRS    the offset branch's convolution on float32 tensors as bfloat16 pairs (the fp32 matrix-instruction forward runs instead, the other passes are not offered)
 };
 unsigned test_switches();  // dk_api.hip
@@ -94,6 +96,11 @@ size_t fast_deform_grad_input_workspace(const Geo& g);
 template <typename T>
 bool fast_deform_grad_input(const Geo& g, const T* gout, const T* off, const T* rot, const T* filter, T* gin,
                             void* ws, hipStream_t stream);
+// its form with the lanes along the channels (dk_deform_lanes.hip), called behind absmax_kernel: gmax = its maxima
+bool lanes_deform_grad_input_applies(const Geo& g);
+template <typename T>
+bool lanes_deform_grad_input(const Geo& g, const T* gout, const T* off, const T* rot, const T* filter, T* gin,
+                             const unsigned* gmax, hipStream_t stream);
 // rotation = false: gradient w.r.t. the image-space offsets
 size_t fast_deform_grad_coord_workspace(const Geo& g, bool rotation);
 template <typename T>
