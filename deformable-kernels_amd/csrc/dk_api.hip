@@ -8,6 +8,7 @@
 #include <cstdlib>
 #include <initializer_list>
 #include <mutex>
+#include <type_traits>
 #include <utility>
 #include <vector>
 
@@ -201,6 +202,14 @@ int static_scratch_of_current_device(void** ptr) {
   *ptr = p;
   return DK_OK;
 }
+// by_dtype without float64, which these kernels do not take
+template <typename F>
+int by_tensor_dtype(int dtype, F&& f) {
+  return by_dtype(dtype, [&]<typename T>() {
+    if constexpr (!std::is_same_v<T, double>) f.template operator()<T>();
+  });
+}
+
 }  // namespace
 
 extern "C" {
@@ -623,8 +632,9 @@ int dk_image_depthwise_forward(const dk_conv_desc* desc, const void* input, cons
   return ok ? st : DK_ERR_UNSUPPORTED;
 }
 
-int dk_image_depthwise_backward_data(const dk_conv_desc* desc, const void* out_grad, const void* weight,
-                                     const int64_t* weight_strides, void* in_grad, void* stream) {
+int dk_image_depthwise_backward_data_add(const dk_conv_desc* desc, const void* out_grad, const void* weight,
+                                         const int64_t* weight_strides, const float* plane_grad, void* in_grad,
+                                         void* stream) {
   Geo g;
   const int rc = make_geo(desc, g);
   if (rc != DK_OK) return rc;
@@ -638,9 +648,14 @@ int dk_image_depthwise_backward_data(const dk_conv_desc* desc, const void* out_g
   hipStream_t s = static_cast<hipStream_t>(stream);
   bool ok = true;
   const int st = by_dtype(desc->dtype, [&]<typename T>() {
-    ok = image_conv_grad_input<T>(g, ws, in<T>(out_grad), in<T>(weight), out<T>(in_grad), s);
+    ok = image_conv_grad_input<T>(g, ws, in<T>(out_grad), in<T>(weight), plane_grad, out<T>(in_grad), s);
   });
   return ok ? st : DK_ERR_UNSUPPORTED;
+}
+
+int dk_image_depthwise_backward_data(const dk_conv_desc* desc, const void* out_grad, const void* weight,
+                                     const int64_t* weight_strides, void* in_grad, void* stream) {
+  return dk_image_depthwise_backward_data_add(desc, out_grad, weight, weight_strides, nullptr, in_grad, stream);
 }
 
 int dk_image_depthwise_backward_weight(const dk_conv_desc* desc, const void* out_grad, const void* input,
@@ -661,6 +676,54 @@ int dk_image_depthwise_backward_weight(const dk_conv_desc* desc, const void* out
     ok = image_conv_grad_weight<T>(g, ws, in<T>(out_grad), in<T>(input), out<T>(weight_grad), s);
   });
   return ok ? st : DK_ERR_UNSUPPORTED;
+}
+
+// ---- the per-image kernels of the global layer ---------------------------------------------
+
+static int check_global_kernels(const dk_conv_desc* desc, Geo& g) {
+  const int rc = make_geo(desc, g);
+  if (rc != DK_OK) return rc;
+  return desc->layout == DK_LAYOUT_NCHW && global_kernels_supported(g, desc->dtype) ? DK_OK : DK_ERR_UNSUPPORTED;
+}
+
+int dk_global_kernels_supported(const dk_conv_desc* desc) {
+  Geo g;
+  return check_global_kernels(desc, g) == DK_OK;
+}
+
+int dk_global_kernels_forward(const dk_conv_desc* desc, const void* input, const void* fc_weight, const void* fc_bias,
+                              const void* weight, void* pooled, void* coord, void* clamped, void* kernels, void* stream) {
+  Geo g;
+  const int rc = check_global_kernels(desc, g);
+  if (rc != DK_OK) return rc;
+  if (!input || !fc_weight || !fc_bias || !weight || !pooled || !coord || !clamped || !kernels) return DK_ERR_NULL_POINTER;
+  if (g.batch == 0) return DK_OK;
+  return by_tensor_dtype(desc->dtype, [&]<typename T>() {
+    global_kernels_forward<T>(g, in<T>(input), in<T>(fc_weight), in<T>(fc_bias), in<T>(weight), out<T>(pooled), out<T>(coord),
+                              out<T>(clamped), out<T>(kernels), static_cast<hipStream_t>(stream));
+  });
+}
+
+size_t dk_global_kernels_backward_workspace(const dk_conv_desc* desc) {
+  Geo g;
+  return check_global_kernels(desc, g) == DK_OK ? global_kernels_backward_workspace(g, desc->dtype) : 0;
+}
+
+int dk_global_kernels_backward(const dk_conv_desc* desc, const void* kernels_grad, const void* pooled, const void* coord,
+                               const void* clamped, const void* weight, const void* fc_weight, void* weight_grad,
+                               void* fc_weight_grad, void* fc_bias_grad, float* pooled_grad, void* workspace,
+                               size_t workspace_bytes, void* stream) {
+  Geo g;
+  const int rc = check_global_kernels(desc, g);
+  if (rc != DK_OK) return rc;
+  if (!kernels_grad || !pooled || !coord || !clamped || !weight || !fc_weight) return DK_ERR_NULL_POINTER;
+  if (!workspace || workspace_bytes < global_kernels_backward_workspace(g, desc->dtype)) return DK_ERR_WORKSPACE;
+  if (g.batch == 0) return DK_ERR_UNSUPPORTED;  // nothing to sum: the caller's zeros
+  return by_tensor_dtype(desc->dtype, [&]<typename T>() {
+    global_kernels_backward<T>(g, desc->dtype, in<T>(kernels_grad), in<T>(pooled), in<T>(coord), in<T>(clamped), in<T>(weight),
+                               in<T>(fc_weight), out<T>(weight_grad), out<T>(fc_weight_grad), out<T>(fc_bias_grad),
+                               pooled_grad, workspace, static_cast<hipStream_t>(stream));
+  });
 }
 
 // forward: the call is (or asks about) the forward, the one pass that has a stride-2 kernel

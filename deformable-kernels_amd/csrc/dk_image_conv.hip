@@ -131,7 +131,8 @@ struct Taps<T, CT, 0> {
 // K: taps per side known at compile time (0: run-time k_h x k_w); UNIT: stride 1 and dilation 1.
 template <typename T, int K, bool UNIT>
 __global__ __launch_bounds__(kWave* kWaves) void image_conv_kernel(ImgConv a, const T* __restrict__ src,
-                                                                   const T* __restrict__ weight, T* __restrict__ dst) {
+                                                                   const T* __restrict__ weight, T* __restrict__ dst,
+                                                                   const float* __restrict__ plane_add) {
   using CT = compute_t<T>;
   extern __shared__ __align__(16) unsigned char lds_raw[];
   const int lane = threadIdx.x & (kWave - 1);
@@ -147,6 +148,7 @@ __global__ __launch_bounds__(kWave* kWaves) void image_conv_kernel(ImgConv a, co
   taps.load(weight + (plane / a.channel) * a.wl.n + (plane % a.channel) * a.wl.c, a, lds_w, lane);
   const T* sp = src + (size_t)plane * a.src_h * a.src_w;
   T* dp = dst + (size_t)plane * a.dst_h * a.dst_w;
+  const CT base = plane_add ? (CT)plane_add[plane] : CT(0);
   const int strips = (a.dst_w + kStrip - 1) / kStrip;
   const int dro = kWave / strips, dso = kWave - dro * strips;
 
@@ -163,7 +165,7 @@ __global__ __launch_bounds__(kWave* kWaves) void image_conv_kernel(ImgConv a, co
       const CT* t0 = tile + orow * sh * a.pitch + oc * sw;
       CT acc[kStrip];
 #pragma unroll
-      for (int i = 0; i < kStrip; ++i) acc[i] = CT(0);
+      for (int i = 0; i < kStrip; ++i) acc[i] = base;
       if constexpr (K > 0 && UNIT) {
 #pragma unroll
         for (int i = 0; i < K; ++i) {
@@ -201,7 +203,8 @@ template <typename T>
 __global__ __launch_bounds__(256) void image_conv_grad_input_strided_kernel(ImgConv a, int pad_h, int pad_w,
                                                                             const T* __restrict__ gout,
                                                                             const T* __restrict__ weight,
-                                                                            T* __restrict__ gin) {
+                                                                            T* __restrict__ gin,
+                                                                            const float* __restrict__ plane_add) {
   using CT = compute_t<T>;
   // here src_* is the input plane (the result) and dst_* the output plane (out_grad)
   const long total = (long)a.planes * a.src_h * a.src_w;
@@ -212,7 +215,7 @@ __global__ __launch_bounds__(256) void image_conv_grad_input_strided_kernel(ImgC
     const long plane = rest / a.src_h;
     const T* gp = gout + plane * a.dst_h * a.dst_w;
     const T* wp = weight + (plane / a.channel) * a.wl.n + (plane % a.channel) * a.wl.c;
-    CT acc = CT(0);
+    CT acc = plane_add ? (CT)plane_add[plane] : CT(0);
     for (int i = 0; i < a.k_h; ++i) {
       const int hh = h + pad_h - i * a.dil_h;
       if (hh < 0 || hh % a.stride_h != 0) continue;
@@ -523,7 +526,8 @@ __device__ __forceinline__ long tap_offset(const WLayout& wl, int t) { return (t
 template <typename T, int NCH, bool W4, int PR>
 __global__ __launch_bounds__(kWave* kWaves) void image_conv3_flat_kernel(FlatConv a, const T* __restrict__ src,
                                                                          const T* __restrict__ weight,
-                                                                         T* __restrict__ dst) {
+                                                                         T* __restrict__ dst,
+                                                                         const float* __restrict__ plane_add) {
   extern __shared__ __align__(16) unsigned char lds_raw[];
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
@@ -544,10 +548,13 @@ __global__ __launch_bounds__(kWave* kWaves) void image_conv3_flat_kernel(FlatCon
   FlatLoads<T, NCH> loads;
   loads.issue(src, total, cur, lane);
   T taps_next = taps_of(first_plane);
+  auto base_of = [&](int plane) { return plane_add ? plane_add[plane] : 0.f; };
+  float base = base_of(first_plane), base_next = base;
   for (;;) {
     loads.commit(tile, cur, lane);
     float taps_cur = ld(&taps_next);
     asm volatile("" : "+v"(taps_cur));  // converted here, before the next loads are issued, not next to its use
+    base = base_next;
     if (cur.r0 == 0) zero_row(tile + kFront + cur.shift, a.w, lane);
     if (cur.r1 == a.h) zero_row(tile + kFront + cur.shift + (cur.r1 - cur.r0 + 1) * a.w, a.w, lane);
     // the next band's loads fly while this one is computed
@@ -557,7 +564,10 @@ __global__ __launch_bounds__(kWave* kWaves) void image_conv3_flat_kernel(FlatCon
     const FlatUnit nxt = flat_unit<T>(a, more ? next_plane : cur.plane, more_bands ? cur.band + 1 : 0, true);
     if (more) {
       loads.issue(src, total, nxt, lane);
-      if (!more_bands) taps_next = taps_of(next_plane);
+      if (!more_bands) {
+        taps_next = taps_of(next_plane);
+        base_next = base_of(next_plane);
+      }
     }
     lds_sync();
     float w9[9];
@@ -573,7 +583,7 @@ __global__ __launch_bounds__(kWave* kWaves) void image_conv3_flat_kernel(FlatCon
       load_rows<W4, PR>(band + orow * PR * a.w + oc, a.w, oc, x);
 #pragma unroll
       for (int pr = 0; pr < PR; ++pr) {
-        float acc[kStrip] = {0.f, 0.f, 0.f, 0.f};
+        float acc[kStrip] = {base, base, base, base};
 #pragma unroll
         for (int i = 0; i < 3; ++i)
 #pragma unroll
@@ -740,7 +750,8 @@ __device__ __forceinline__ void load_rows16(const unsigned* top, int w, int oc, 
 template <typename T, int NCH, int PR>
 __global__ __launch_bounds__(kWave* kWaves) void image_conv3_flat16_kernel(FlatConv a, const T* __restrict__ src,
                                                                            const T* __restrict__ weight,
-                                                                           T* __restrict__ dst) {
+                                                                           T* __restrict__ dst,
+                                                                           const float* __restrict__ plane_add) {
   extern __shared__ __align__(16) unsigned char lds_raw[];
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
@@ -757,10 +768,13 @@ __global__ __launch_bounds__(kWave* kWaves) void image_conv3_flat16_kernel(FlatC
   FlatLoads16<T, NCH> loads;
   loads.issue(src, total, cur, lane);
   T taps_next = taps_of(first_plane);
+  auto base_of = [&](int plane) { return plane_add ? plane_add[plane] : 0.f; };
+  float base = base_of(first_plane), base_next = base;
   for (;;) {
     loads.commit16(tile, cur, lane);
     float taps_cur = ld(&taps_next);
     asm volatile("" : "+v"(taps_cur));
+    base = base_next;
     // the halo rows above the first and below the last row of the plane (the range starts at an even element)
     if (cur.r0 == 0) zero_row16(tile + (kFront + cur.shift) / 2, a.w, lane);
     if (cur.r1 == a.h) zero_row16(tile + (kFront + cur.shift + (cur.r1 - cur.r0 + 1) * a.w) / 2, a.w, lane);
@@ -770,7 +784,10 @@ __global__ __launch_bounds__(kWave* kWaves) void image_conv3_flat16_kernel(FlatC
     const FlatUnit nxt = flat_unit<T>(a, more ? next_plane : cur.plane, more_bands ? cur.band + 1 : 0, true);
     if (more) {
       loads.issue(src, total, nxt, lane);
-      if (!more_bands) taps_next = taps_of(next_plane);
+      if (!more_bands) {
+        taps_next = taps_of(next_plane);
+        base_next = base_of(next_plane);
+      }
     }
     lds_sync();
     float w9[9];
@@ -794,7 +811,7 @@ __global__ __launch_bounds__(kWave* kWaves) void image_conv3_flat16_kernel(FlatC
       load_rows16<PR>(band + (orow * PR * a.w + oc) / 2, a.w, oc, x);
 #pragma unroll
       for (int pr = 0; pr < PR; ++pr) {
-        float acc[kStrip] = {0.f, 0.f, 0.f, 0.f};
+        float acc[kStrip] = {base, base, base, base};
 #pragma unroll
         for (int i = 0; i < 3; ++i) {
           const unsigned* r = x[pr + i];
@@ -958,7 +975,8 @@ int flat_grid(const FlatConv& a) {
 }
 
 template <typename T>
-bool launch_flat_conv(const Geo& g, const long* ws, bool flip, const T* src, const T* weight, T* dst, hipStream_t stream) {
+bool launch_flat_conv(const Geo& g, const long* ws, bool flip, const T* src, const T* weight, T* dst, const float* plane_add,
+                      hipStream_t stream) {
   if constexpr (std::is_same<T, double>::value) {
     return false;
   } else {
@@ -977,8 +995,8 @@ bool launch_flat_conv(const Geo& g, const long* ws, bool flip, const T* src, con
       // 16-bit tensors with rows of a multiple of 4 elements: the packed kernels
       if (w4 && a.w % kStrip == 0 && a.w >= kStrip && !path_disabled(kNoImagePacked)) {
 #define DK_FLAT16(NN)                                                                                                      \
-  if (patches) hipLaunchKernelGGL((image_conv3_flat16_kernel<T, NN, 4>), grid, block, lds, stream, a, src, weight, dst);      \
-  else hipLaunchKernelGGL((image_conv3_flat16_kernel<T, NN, 1>), grid, block, lds, stream, a, src, weight, dst)
+  if (patches) hipLaunchKernelGGL((image_conv3_flat16_kernel<T, NN, 4>), grid, block, lds, stream, a, src, weight, dst, plane_add);      \
+  else hipLaunchKernelGGL((image_conv3_flat16_kernel<T, NN, 1>), grid, block, lds, stream, a, src, weight, dst, plane_add)
         if (nch == 1) { DK_FLAT16(1); }
         else if (nch == 2) { DK_FLAT16(2); }
         else if (nch == 4) { DK_FLAT16(4); }
@@ -988,9 +1006,9 @@ bool launch_flat_conv(const Geo& g, const long* ws, bool flip, const T* src, con
       }
     }
 #define DK_FLAT(NN)                                                                                                        \
-  if (patches) hipLaunchKernelGGL((image_conv3_flat_kernel<T, NN, true, 4>), grid, block, lds, stream, a, src, weight, dst);  \
-  else if (w4) hipLaunchKernelGGL((image_conv3_flat_kernel<T, NN, true, 1>), grid, block, lds, stream, a, src, weight, dst);  \
-  else hipLaunchKernelGGL((image_conv3_flat_kernel<T, NN, false, 1>), grid, block, lds, stream, a, src, weight, dst)
+  if (patches) hipLaunchKernelGGL((image_conv3_flat_kernel<T, NN, true, 4>), grid, block, lds, stream, a, src, weight, dst, plane_add);  \
+  else if (w4) hipLaunchKernelGGL((image_conv3_flat_kernel<T, NN, true, 1>), grid, block, lds, stream, a, src, weight, dst, plane_add);  \
+  else hipLaunchKernelGGL((image_conv3_flat_kernel<T, NN, false, 1>), grid, block, lds, stream, a, src, weight, dst, plane_add)
     if (nch == 1) { DK_FLAT(1); }
     else if (nch == 2) { DK_FLAT(2); }
     else if (nch == 4) { DK_FLAT(4); }
@@ -1044,14 +1062,14 @@ size_t lds_bytes(const ImgConv& a, bool run_time_taps) {
 }
 
 template <typename T>
-bool launch_conv(ImgConv a, const T* src, const T* weight, T* dst, hipStream_t stream) {
+bool launch_conv(ImgConv a, const T* src, const T* weight, T* dst, const float* plane_add, hipStream_t stream) {
   if (!plan(a, sizeof(compute_t<T>))) return false;
   a.vec_ok = aligned_rows(dst, a.dst_w, sizeof(T));
   const bool unit = a.stride_h == 1 && a.stride_w == 1 && a.dil_h == 1 && a.dil_w == 1;
   const int k = a.k_h == a.k_w ? a.k_h : 0;
   const dim3 grid((a.planes + kWaves - 1) / kWaves), block(kWave * kWaves);
 #define DK_IMG_CONV(KK, UU) \
-  hipLaunchKernelGGL((image_conv_kernel<T, KK, UU>), grid, block, lds_bytes<T>(a, KK == 0), stream, a, src, weight, dst)
+  hipLaunchKernelGGL((image_conv_kernel<T, KK, UU>), grid, block, lds_bytes<T>(a, KK == 0), stream, a, src, weight, dst, plane_add)
   if (k == 3 && unit) DK_IMG_CONV(3, true);
   else if (k == 3) DK_IMG_CONV(3, false);
   else if (k == 1) DK_IMG_CONV(1, false);
@@ -1089,26 +1107,26 @@ bool image_conv_supported(const Geo& g, int dtype) {
 
 template <typename T>
 bool image_conv_forward(const Geo& g, const long* wstrides, const T* x, const T* weight, T* out, hipStream_t stream) {
-  if (!path_disabled(kNoImageFlat) && launch_flat_conv<T>(g, wstrides, false, x, weight, out, stream)) return true;
-  return launch_conv<T>(forward_args(g, wstrides), x, weight, out, stream);
+  if (!path_disabled(kNoImageFlat) && launch_flat_conv<T>(g, wstrides, false, x, weight, out, nullptr, stream)) return true;
+  return launch_conv<T>(forward_args(g, wstrides), x, weight, out, nullptr, stream);
 }
 
 template <typename T>
-bool image_conv_grad_input(const Geo& g, const long* wstrides, const T* gout, const T* weight, T* gin,
-                           hipStream_t stream) {
-  if (!path_disabled(kNoImageFlat) && launch_flat_conv<T>(g, wstrides, true, gout, weight, gin, stream)) return true;
+bool image_conv_grad_input(const Geo& g, const long* wstrides, const T* gout, const T* weight, const float* plane_add,
+                           T* gin, hipStream_t stream) {
+  if (!path_disabled(kNoImageFlat) && launch_flat_conv<T>(g, wstrides, true, gout, weight, gin, plane_add, stream)) return true;
   ImgConv a = forward_args(g, wstrides);
   if (g.stride_h == 1 && g.stride_w == 1) {
     a.src_h = g.out_h, a.src_w = g.out_w, a.dst_h = g.in_h, a.dst_w = g.in_w;
     a.org_h = g.pad_h - (g.k_h - 1) * g.dil_h, a.org_w = g.pad_w - (g.k_w - 1) * g.dil_w;
     a.flip = 1;
-    return launch_conv<T>(a, gout, weight, gin, stream);
+    return launch_conv<T>(a, gout, weight, gin, plane_add, stream);
   }
   if ((long)g.k_h * g.k_w > kMaxTaps) return false;
   const long total = (long)a.planes * g.in_h * g.in_w;
   const int blocks = (int)std::min<long>((total + 255) / 256, 1 << 20);
   hipLaunchKernelGGL((image_conv_grad_input_strided_kernel<T>), dim3(blocks), dim3(256), 0, stream, a, g.pad_h, g.pad_w,
-                     gout, weight, gin);
+                     gout, weight, gin, plane_add);
   return true;
 }
 
@@ -1135,7 +1153,7 @@ bool image_conv_grad_weight(const Geo& g, const long* wstrides, const T* gout, c
 
 #define DK_INSTANTIATE(T)                                                                              \
   template bool image_conv_forward<T>(const Geo&, const long*, const T*, const T*, T*, hipStream_t);    \
-  template bool image_conv_grad_input<T>(const Geo&, const long*, const T*, const T*, T*, hipStream_t); \
+  template bool image_conv_grad_input<T>(const Geo&, const long*, const T*, const T*, const float*, T*, hipStream_t); \
   template bool image_conv_grad_weight<T>(const Geo&, const long*, const T*, const T*, T*, hipStream_t);
 DK_INSTANTIATE(float)
 DK_INSTANTIATE(__half)

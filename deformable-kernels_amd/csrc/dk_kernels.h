@@ -210,11 +210,23 @@ bool image_conv_supported(const Geo& g, int dtype);
 // for a contiguous [N, C, k_h, k_w] tensor
 template <typename T>
 bool image_conv_forward(const Geo& g, const long* wstrides, const T* x, const T* weight, T* out, hipStream_t stream);
+// plane_add: null, or one number per (image, channel) that every element of the plane's gradient gets on top
 template <typename T>
-bool image_conv_grad_input(const Geo& g, const long* wstrides, const T* gout, const T* weight, T* gin,
-                           hipStream_t stream);
+bool image_conv_grad_input(const Geo& g, const long* wstrides, const T* gout, const T* weight, const float* plane_add,
+                           T* gin, hipStream_t stream);
 template <typename T>
 bool image_conv_grad_weight(const Geo& g, const long* wstrides, const T* gout, const T* x, T* gweight,
                             hipStream_t stream);
+
+// dk_global.hip: the per-image kernels of GlobalDeformKernel2d from the pooled input, and their gradients (not float64)
+bool global_kernels_supported(const Geo& g, int dtype);
+template <typename T>
+void global_kernels_forward(const Geo& g, const T* x, const T* fc_w, const T* fc_b, const T* weight, T* pooled, T* coord,
+                            T* clamped, T* kernels, hipStream_t stream);
+size_t global_kernels_backward_workspace(const Geo& g, int dtype);
+template <typename T>
+void global_kernels_backward(const Geo& g, int dtype, const T* gkernels, const T* pooled, const T* coord,
+                             const T* clamped, const T* weight, const T* fc_w, T* gweight, T* gfc_w, T* gfc_b,
+                             float* gpooled, void* ws, hipStream_t stream);
 
 }  // namespace dk

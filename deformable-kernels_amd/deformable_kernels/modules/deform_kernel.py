@@ -12,7 +12,7 @@ import torch
 from torch import nn
 
 from ..ops.deform_kernel.functions import (
-    image_depthwise_conv, image_depthwise_conv_supported, nd_linear_sample, offset_conv, sample_depthwise)
+    global_deform_conv, global_deform_conv_supported, image_depthwise_conv, image_depthwise_conv_supported, nd_linear_sample, offset_conv, sample_depthwise)
 from ..ops.deform_kernel.modules import (
     SampleDepthwise,
     DeformableSampleDepthwise,
@@ -46,6 +46,12 @@ def _plain_conv(conv):
     hooks = (conv._forward_hooks, conv._forward_pre_hooks, conv._backward_hooks,
              getattr(conv, "_backward_pre_hooks", {}))
     return not any(len(h) for h in hooks) and conv.padding_mode == 'zeros' and conv.groups == 1
+
+
+def _plain_linear(fc):
+    """Whether its parameters stand for the linear layer: no hooks on it, and not replaced by something else."""
+    hooks = (fc._forward_hooks, fc._forward_pre_hooks, fc._backward_hooks, getattr(fc, "_backward_pre_hooks", {}))
+    return type(fc) is nn.Linear and not any(len(h) for h in hooks)
 
 
 class GlobalDeformKernel2d(nn.Module):
@@ -148,6 +154,17 @@ class GlobalDeformKernel2d(nn.Module):
         # library's convolution computes in the tensors' own type, so it is only taken outside such regions)
         if (self.native_conv and x.is_cuda and self.group == self.in_planes == self.out_planes
                 and not torch.is_autocast_enabled()):
+            # the whole layer in the library where its kernels cover it and nobody has put something else in
+            # the place of the pooled branch
+            if (len(self.weight_shape) == 2 and self.weight_dilate == 1 and _plain_linear(self.fc)
+                    and type(self)._dynamic_weight is GlobalDeformKernel2d._dynamic_weight
+                    and type(self).dynamic_weight is GlobalDeformKernel2d.dynamic_weight
+                    and 'dynamic_weight' not in self.__dict__ and '_dynamic_weight' not in self.__dict__
+                    and self.fc_bias == _centred_tap_grid(self.weight_shape, self.kernel_size, 1)):
+                args = (x, self.weight, self.fc.weight, self.fc.bias, self.kernel_size, self.stride, self.padding,
+                        self.dilation)
+                if global_deform_conv_supported(*args):
+                    return global_deform_conv(*args)
             kernels = self.dynamic_weight(x, self.weight, per_image=True).to(x.dtype)
             if image_depthwise_conv_supported(x, kernels, self.stride, self.padding, self.dilation):
                 return image_depthwise_conv(x, kernels, self.stride, self.padding, self.dilation)

@@ -88,6 +88,11 @@ SIGNATURES = {
     "dk_image_depthwise_supported": (ctypes.c_int, [_CD]),
     "dk_image_depthwise_forward": (ctypes.c_int, [_CD, _P, _P, _I64P, _P, _P]),
     "dk_image_depthwise_backward_data": (ctypes.c_int, [_CD, _P, _P, _I64P, _P, _P]),
+    "dk_image_depthwise_backward_data_add": (ctypes.c_int, [_CD, _P, _P, _I64P, _P, _P, _P]),
+    "dk_global_kernels_supported": (ctypes.c_int, [_CD]),
+    "dk_global_kernels_forward": (ctypes.c_int, [_CD] + [_P] * 9),
+    "dk_global_kernels_backward_workspace": (_SZ, [_CD]),
+    "dk_global_kernels_backward": (ctypes.c_int, [_CD] + [_P] * 11 + [_SZ, _P]),
     "dk_image_depthwise_backward_weight": (ctypes.c_int, [_CD, _P, _P, _P, _I64P, _P]),
     "dk_offset_conv_supported": (ctypes.c_int, [_OC]),
     "dk_offset_conv_worthwhile": (ctypes.c_int, [_OC]),

@@ -5,6 +5,7 @@ from .filter_sample_depthwise import (
 from .nd_linear_sample import nd_linear_sample
 from .offset_conv import offset_conv, offset_conv_supported
 from .image_depthwise_conv import image_depthwise_conv, image_depthwise_conv_supported
+from .global_deform_conv import global_deform_conv, global_deform_conv_supported
 
 __all__ = [
     'sample_depthwise',
@@ -14,4 +15,6 @@ __all__ = [
     'offset_conv_supported',
     'image_depthwise_conv',
     'image_depthwise_conv_supported',
+    'global_deform_conv',
+    'global_deform_conv_supported',
 ]

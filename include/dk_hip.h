@@ -375,8 +375,37 @@ int dk_image_depthwise_forward(const dk_conv_desc *desc, const void *input, cons
                                const int64_t *weight_strides, void *output, void *stream);
 int dk_image_depthwise_backward_data(const dk_conv_desc *desc, const void *out_grad, const void *weight,
                                      const int64_t *weight_strides, void *in_grad, void *stream);
+/* ... with plane_grad[batch][channel] (float, or NULL) added to every element of its plane: the share of a gradient
+ * that reaches the input through its mean. */
+int dk_image_depthwise_backward_data_add(const dk_conv_desc *desc, const void *out_grad, const void *weight,
+                                         const int64_t *weight_strides, const float *plane_grad,
+                                         void *in_grad, void *stream);
 int dk_image_depthwise_backward_weight(const dk_conv_desc *desc, const void *out_grad, const void *input,
                                        void *weight_grad, const int64_t *weight_strides, void *stream);
+
+/* ---- the per-image kernels of GlobalDeformKernel2d ---------------------------- */
+
+/* dynamic_weight of a depthwise layer with a two-dimensional scope (modules/deform_kernel.py:68-101): pooled =
+ * mean(input) over each plane; coord = pooled * fc_weight^T + fc_bias + the undeformed tap positions, every step
+ * rounded to the tensor type; clamped = coord clamped to [0, scope_h - 1] (:83); kernels = `weight` [channel, scope_h,
+ * scope_w] sampled bilinearly at clamped.
+ *   input [batch, channel, in_h, in_w], fc_weight [2 k_h k_w, channel], fc_bias [2 k_h k_w], pooled [batch, channel],
+ *   coord and clamped [batch, k_h k_w, 2], kernels [batch, k_h k_w, channel] (in dk_image_depthwise_*'s terms the
+ *   strides {k_h k_w channel, 1, k_w channel, channel}).
+ * The backward takes what the forward wrote and the gradient of `kernels`; weight_grad, fc_weight_grad, fc_bias_grad
+ * (like weight, fc_weight, fc_bias) and pooled_grad (float [batch, channel], divided by in_h in_w: plane_grad above)
+ * may each be NULL.  Any dtype but float64, groups = 1, at most 64 taps and 8192 channels, batch > 0 in the backward;
+ * sums in fp32, a fixed order for those over the images. */
+int dk_global_kernels_supported(const dk_conv_desc *desc);
+int dk_global_kernels_forward(const dk_conv_desc *desc, const void *input, const void *fc_weight,
+                              const void *fc_bias, const void *weight, void *pooled, void *coord,
+                              void *clamped, void *kernels, void *stream);
+size_t dk_global_kernels_backward_workspace(const dk_conv_desc *desc);
+int dk_global_kernels_backward(const dk_conv_desc *desc, const void *kernels_grad, const void *pooled,
+                               const void *coord, const void *clamped, const void *weight,
+                               const void *fc_weight, void *weight_grad, void *fc_weight_grad,
+                               void *fc_bias_grad, float *pooled_grad, void *workspace,
+                               size_t workspace_bytes, void *stream);
 
 /* ---- misc ------------------------------------------------------------------- */
 

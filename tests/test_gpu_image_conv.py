@@ -182,3 +182,54 @@ def test_c_abi_rejections_and_empty_batch():
     assert L.dk_image_depthwise_backward_data(empty, _lib.ptr(out), _lib.ptr(w), None, _lib.ptr(x), st) == 0
     assert L.dk_image_depthwise_backward_weight(empty, _lib.ptr(out), _lib.ptr(x), _lib.ptr(w), None, st) == 0
     torch.cuda.synchronize()
+
+
+# ---- the whole global layer as one Function --------------------------------------------------------
+
+def _global_layer(C, S, k, stride, padding, dtype, seed):
+    from deformable_kernels.modules import GlobalDeformKernel2d
+    torch.manual_seed(seed)
+    m = GlobalDeformKernel2d(S, C, C, kernel_size=k, stride=stride, padding=padding, groups=C)
+    with torch.no_grad():
+        m.fc.weight.normal_(0.0, 3.0 / C ** 0.5)
+        m.fc.bias.normal_(0.0, 1.0)          # some coordinates end up clamped on either side
+    return m.to("cuda:0").to(dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("case", [
+    (1, 1, 5, 7, (3, 3), 3, 1, 1),        # one plane of 35 elements: no wide loads, rows of the fc in one lane
+    (3, 70, 9, 10, (4, 4), 3, 2, 1),      # channels not a multiple of 64, two channel splits, stride 2
+    (2, 65, 8, 8, (5, 3), 3, 1, 1),       # scope narrower than the clamp allows in the second axis
+    (2, 8, 12, 12, (6, 6), 5, 1, 2),      # 25 taps: the weight gradient in three groups of rows
+    (19, 260, 16, 16, (5, 5), 3, 1, 1),   # planes of wide loads, four per wave; images not a multiple of the slices
+])
+def test_global_layer_as_one_function(case, dtype):
+    N, C, H, W, S, k, stride, padding = case
+    m = _global_layer(C, S, k, stride, padding, dtype, seed=11)
+    g = torch.Generator().manual_seed(12)
+    x = torch.randn(N, C, H, W, generator=g).to(dtype).to("cuda:0")
+    oh, ow = (H + 2 * padding - k) // stride + 1, (W + 2 * padding - k) // stride + 1
+    gout = torch.randn(N, C, oh, ow, generator=g).to(dtype).to("cuda:0")
+
+    def run(module, x, gout):
+        x = x.detach().requires_grad_()
+        out = module(x)
+        return [out.detach()] + list(torch.autograd.grad(out, [x] + list(module.parameters()), gout))
+
+    got = run(m, x, gout)
+    assert type(m(x.requires_grad_()).grad_fn).__name__.startswith("GlobalDeformConvFunction")
+    if dtype == torch.float32:
+        # against the layer-by-layer route in float64 (which this Function does not take): fp32 sums of up to
+        # N * H * W terms
+        want = run(m.double(), x.double(), gout.double())
+        tol = 2e-5
+    else:
+        # against the layer-by-layer route in the same type, which rounds the same tensors
+        m.dynamic_weight = m.dynamic_weight
+        want = run(m, x, gout)
+        tol = 1e-2 if dtype == torch.float16 else 3e-2   # a handful of roundings of the type
+    for a, b, what in zip(got, want, ("output", "grad input", "grad weight", "grad fc weight", "grad fc bias")):
+        assert a.dtype == dtype and a.shape == b.shape
+        err = float((a.double() - b.double()).abs().max() / b.double().abs().max().clamp_min(1e-30))
+        assert err < tol, (what, err)
