@@ -134,6 +134,26 @@ def lib():
     return _lib
 
 
+_native = None
+
+
+def native():
+    """The module of native autograd operators (``csrc/dk_torch.cpp``); raises if it has not been built."""
+    global _native
+    if _native is None:
+        lib()
+        try:
+            from . import _native as module
+        except ImportError as e:
+            raise DkError("the operator module _native.so is missing or does not load (%s) -- build it with "
+                          "`make -C deformable-kernels_amd/csrc` (there is no fallback)" % e) from e
+        if module.conv_desc_size != ctypes.sizeof(ConvDesc):
+            raise DkError("_native.so and the library are out of step: build both with `make -C deformable-kernels_amd/csrc`")
+        module.set_error_class(DkError)
+        _native = module
+    return _native
+
+
 def check(status, what):
     if status != 0:
         raise DkError("%s failed: %s (status %d)" % (what, lib().dk_status_string(status).decode(), status))

@@ -218,7 +218,7 @@ def test_global_layer_as_one_function(case, dtype):
         return [out.detach()] + list(torch.autograd.grad(out, [x] + list(module.parameters()), gout))
 
     got = run(m, x, gout)
-    assert type(m(x.requires_grad_()).grad_fn).__name__.startswith("GlobalDeformConvFunction")
+    assert m(x.requires_grad_()).grad_fn.name().startswith("GlobalDeformConvFunction")
     if dtype == torch.float32:
         # against the layer-by-layer route in float64 (which this Function does not take): fp32 sums of up to
         # N * H * W terms
