@@ -1131,10 +1131,11 @@ __global__ __launch_bounds__(kMfBlock, 4) void local_grad_filter_mfma_kernel(
   const int pix = threadIdx.x % kMfPix;                                 // pixel whose coordinates this thread stages
   const int tapq = __builtin_amdgcn_readfirstlane(threadIdx.x / kMfPix);  // ... for taps tapq + 4 k
   float r_rot[2 * kTapsT], r_x[kChW][NX], r_g[kChW][kMfPix / 64];
-  // CL: thread (pixel slot cl_p, channel quad cl_q) stages four channels of NX / 2 input pixels and of one gout pixel
-  static_assert(!CL || (!S2 && NX % 2 == 0 && kMfBlock == 4 * kMfPix), "channels-last staging: four threads per pixel");
+  // CL: thread (pixel slot cl_p, channel quad cl_q) stages four channels of NXC input pixels and of one gout pixel
+  static_assert(!CL || kMfBlock == 4 * kMfPix, "channels-last staging: four threads per pixel");
+  constexpr int NXC = (64 * NX + kMfPix - 1) / kMfPix;  // (S2: the last of them is half empty)
   const int cl_p = threadIdx.x >> 2, cl_q = threadIdx.x & 3;
-  typename std::conditional<sizeof(T) == 4, nhwc_u4, nhwc_u2>::type c_x[NX / 2], c_g;
+  typename std::conditional<sizeof(T) == 4, nhwc_u4, nhwc_u2>::type c_x[NXC], c_g;
   auto issue_loads = [&](int item, int cbi, bool with_rot) {
     const int cb = cb_lo + cbi;
     const int n = item / tiles, p0 = (item % tiles) * tile_pix;
@@ -1175,7 +1176,7 @@ __global__ __launch_bounds__(kMfBlock, 4) void local_grad_filter_mfma_kernel(
       const bool quad = c4 < C;
       const unsigned co = (unsigned)c4 * (unsigned)sizeof(T);
 #pragma unroll
-      for (int k = 0; k < NX / 2; ++k) {
+      for (int k = 0; k < NXC; ++k) {
         const int e = x0 + cl_p + kMfPix * k;
         c_x[k] = raw_ld4(rx, e < 0 || !quad ? kOutOfRange : (unsigned)(e * C) * (unsigned)sizeof(T) + co, x);
       }
@@ -1233,7 +1234,8 @@ __global__ __launch_bounds__(kMfBlock, 4) void local_grad_filter_mfma_kernel(
 #pragma unroll
       for (int i = 0; i < 4; ++i) gs[(4 * cl_q + i) * kMfPitchG + cl_p] = gv[i];
 #pragma unroll
-      for (int k = 0; k < NX / 2; ++k) {
+      for (int k = 0; k < NXC; ++k) {
+        if (64 * NX % kMfPix != 0 && cl_p + kMfPix * k >= 64 * NX) continue;  // past the row
         float xv[4];
         raw_cvt4(c_x[k], xv, x);
 #pragma unroll
@@ -1271,7 +1273,7 @@ __global__ __launch_bounds__(kMfBlock, 4) void local_grad_filter_mfma_kernel(
   // small (one channel, 3 x 3 scope: 1.1e-2 seen), so groups of fewer than 16 channels keep the
   // fp32 instructions (template parameter BF, chosen by the host).
   static_assert(!BF || sizeof(T) == 2, "bfloat16 matrix instructions are for 16-bit inputs");
-  static_assert(!SPLIT || (sizeof(T) == 4 && !BF), "the split is for float32 inputs");
+  static_assert(!SPLIT || !BF, "one or the other");
   constexpr bool kHalfIn = BF;
   float A[(kHalfIn || SPLIT) ? 1 : 4][K];
   mfb4 Ab[(kHalfIn || SPLIT) ? K : 1];  // SPLIT: the hi parts
@@ -1706,7 +1708,7 @@ FilterGrid filter_grid(const Geo& g) {
   return f;
 }
 
-// CL: channels-last tensors, matrix-core kernel at stride 1 only (false otherwise)
+// CL: channels-last tensors, matrix-core kernel only (false otherwise)
 template <typename T, int SH, int SW, bool CL = false>
 bool run_grad_filter(const Geo& g, const T* gout, const T* x, const T* rot, T* gfilter, float* ws,
                      hipStream_t stream) {
@@ -1716,13 +1718,10 @@ bool run_grad_filter(const Geo& g, const T* gout, const T* x, const T* rot, T* g
     if (f.mfma) {
 #define DK_LAUNCH_BF(CELL0, BF, SP)                                                                                 \
   if (f.th > 0) {                                                                                                \
-    if constexpr (CL) return false;                                                                              \
-    else {                                                                                                       \
-    auto kernel = local_grad_filter_mfma_kernel<T, SH, SW, CELL0, kMfXS2, true, BF, SP>;                                                           \
+    auto kernel = local_grad_filter_mfma_kernel<T, SH, SW, CELL0, kMfXS2, true, BF, SP, CL>;                     \
     if (!allow_max_dynamic_lds(reinterpret_cast<const void*>(kernel)))                                                           \
       return false;                                                                                              \
     kernel<<<grid, kMfBlock, f.lds, stream>>>(g, gout, x, rot, ws, f.tiles, f.parts, f.splits, f.pitch_x, f.th); \
-    }                                                                                                            \
   } else if (f.nx == 4)                                                                                          \
     local_grad_filter_mfma_kernel<T, SH, SW, CELL0, 4, false, BF, SP, CL><<<grid, kMfBlock, f.lds, stream>>>(g, gout, x, rot, ws, f.tiles, f.parts, f.splits, f.pitch_x, 0); \
   else                                                                                                           \
@@ -1731,8 +1730,19 @@ bool run_grad_filter(const Geo& g, const T* gout, const T* x, const T* rot, T* g
       // float32 inputs: bfloat16 pairs (three products) unless switched off, at stride 2 as well (N=64: 96 x 112^2
       // 98 -> 90 us, 144 x 56^2 46 -> 41, 192 x 28^2 25.9 -> 24.3, 576 x 14^2 32.8 -> 30.1)
       const bool split = !path_disabled(kNoFilterSplit);
+      // Channels-last at stride 2: the fp32 instructions for float32 tensors and the pairs for 16-bit ones (whose
+      // products a pair holds exactly for bfloat16): the operands' rounding stays below that of the kernel that
+      // served this geometry before (nhwc_grad_filter_mfma_kernel, fp32 instructions: us for N=64 96 x 112^2, it / this
+      // kernel: float32 149 / 126, bfloat16 142 / 88).
 #define DK_LAUNCH(CELL0)                                                    \
-  if constexpr (sizeof(T) == 2) {                                           \
+  if constexpr (CL) {                                                       \
+    if (f.th > 0) { DK_LAUNCH_BF(CELL0, false, sizeof(T) == 2) }            \
+    else if constexpr (sizeof(T) == 2) {                                    \
+      if (g.channel / g.groups >= kMfCh) { DK_LAUNCH_BF(CELL0, true, false) } \
+      else { DK_LAUNCH_BF(CELL0, false, false) }                            \
+    } else if (split) { DK_LAUNCH_BF(CELL0, false, true) }                  \
+    else { DK_LAUNCH_BF(CELL0, false, false) }                              \
+  } else if constexpr (sizeof(T) == 2) {                                    \
     if (g.channel / g.groups >= kMfCh) { DK_LAUNCH_BF(CELL0, true, false) } \
     else { DK_LAUNCH_BF(CELL0, false, false) }                              \
   } else if (split) { DK_LAUNCH_BF(CELL0, false, true) }                    \
@@ -1828,13 +1838,13 @@ bool fast_local_grad_filter(const Geo& g, const T* gout, const T* x, const T* ro
 }
 
 // Channels-last tensors on the matrix-core grad filter (its staging reads four consecutive channels per
-// thread): one group, a multiple of 4 channels, stride-1 same-width geometry, 16-byte (16-bit types: 8-byte)
+// thread): one group, a multiple of 4 channels, a same-width or stride-2 geometry, 16-byte (16-bit types: 8-byte)
 // aligned tensors, an image's tensor within 2 GB.
 bool fast_local_grad_filter_cl_shape(const Geo& g, size_t elem) {
   if (!fast_shape(g) || g.groups != 1 || g.channel % 4 != 0 || path_disabled(kNoNhwcStaged)) return false;
   if ((long)std::max(g.in_h * g.in_w, g.out_h * g.out_w) * g.channel * (long)elem >= (1L << 31)) return false;
   const FilterGrid f = filter_grid(g);
-  return f.mfma && f.th == 0;
+  return f.mfma;
 }
 
 size_t fast_local_grad_filter_cl_workspace(const Geo& g) {

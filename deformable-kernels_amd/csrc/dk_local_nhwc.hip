@@ -1077,34 +1077,70 @@ constexpr int kG16Waves = 4;  // (two: 75.9 us on benchmark configuration 2, fou
 // measured 85.8 against 81.4 us on benchmark configuration 2, four 96).
 constexpr int kG16TilesPerWave = 1;
 
-template <typename T, int SH, int SW, bool TRANSPOSED>
-__global__ __launch_bounds__(64 * kG16Waves) void nhwc_gather_mfma16_kernel(
-    Geo g, const T* __restrict__ src, const T* __restrict__ rot, const T* __restrict__ filter, T* __restrict__ dst,
-    int tiles_per_wave, int total_blocks) {
+// CPL consecutive channels of a pixel in one load: 16 bytes for float32 (CPL = 4) and, with CPL = 8, for the 16-bit types.
+template <typename T, int CPL>
+using NhwcRaw = typename std::conditional<sizeof(T) * CPL == 16, nhwc_u4, nhwc_u2>::type;
+template <int CPL, typename T>
+__device__ __forceinline__ NhwcRaw<T, CPL> raw_ld(rsrc_t r, unsigned off, const T*) {
+  if constexpr (sizeof(T) * CPL == 16) return __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, 0, 0);
+  else return __builtin_amdgcn_raw_buffer_load_b64(r, (int)off, 0, 0);
+}
+template <typename V, typename T>
+__device__ __forceinline__ void raw_cvt(V v, float (&f)[4], const T* tag) { raw_cvt4(v, f, tag); }
+template <typename T>
+__device__ __forceinline__ void raw_cvt(nhwc_u4 v, float (&f)[8], const T* tag) {
+  float lo[4], hi[4];
+  raw_cvt4(nhwc_u2{v.x, v.y}, lo, tag);
+  raw_cvt4(nhwc_u2{v.z, v.w}, hi, tag);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) f[i] = lo[i], f[4 + i] = hi[i];
+}
+template <int AUX, typename T>
+__device__ __forceinline__ void raw_st(rsrc_t r, unsigned off, const float (&v)[4], T* tag) { raw_st4<AUX>(r, off, v, tag); }
+template <int AUX, typename T>
+__device__ __forceinline__ void raw_st(rsrc_t r, unsigned off, const float (&v)[8], T*) {
+  struct { T e[8]; } pk;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) st(pk.e + i, v[i]);
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(nhwc_u4, pk), r, (int)off, 0, AUX);
+}
+
+// The operand of a scope coordinate on the pixels' side: the hat products of the lane group's four cells, their high
+// parts in front of their low ones.
+template <typename E>
+__device__ __forceinline__ typename NhwcMx<E>::v8 hat_operand(float2 c, const float (&crow)[4], const float (&ccol)[4]) {
+  typedef float f2v __attribute__((ext_vector_type(2)));
+  typedef E e2v __attribute__((ext_vector_type(2)));
+  float v[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    v[k] = nhwc_hat(c.x - crow[k]) * nhwc_hat(c.y - ccol[k]);
+    asm volatile("" : "+v"(v[k]));  // one fp32 value for both parts
+  }
+  const e2v h01 = __builtin_convertvector(f2v{v[0], v[1]}, e2v), h23 = __builtin_convertvector(f2v{v[2], v[3]}, e2v);
+  const f2v b01 = __builtin_convertvector(h01, f2v), b23 = __builtin_convertvector(h23, f2v);
+  const e2v l01 = __builtin_convertvector(f2v{v[0] - b01[0], v[1] - b01[1]}, e2v);
+  const e2v l23 = __builtin_convertvector(f2v{v[2] - b23[0], v[3] - b23[1]}, e2v);
+  return typename NhwcMx<E>::v8{h01[0], h01[1], h23[0], h23[1], l01[0], l01[1], l23[0], l23[1]};
+}
+
+// The split filter operands of every channel block, for a workgroup.  An entry is lane l of its wave, so the
+// channel's largest weight is the maximum over the four lanes l % 16 + 16 k of what each holds: one load per lane
+// instead of the channel's sixteen (a workgroup lives about as long as a dozen trips to L2, and every thread
+// waits for this table: forward 80 -> 75 us on benchmark configuration 2).  Issuing several entries' loads
+// together measured slower (83 us).
+//
+// CPL: channels a lane holds per step.  With 4, the rows of block b are its sixteen channels in order, so that the lane
+// group kg gets channels 4 kg .. 4 kg + 3; with 8, blocks 2 s and 2 s + 1 deal the channels of step s to their rows such
+// that the group gets 8 kg .. 8 kg + 3 from the one and 8 kg + 4 .. 8 kg + 7 from the other.
+template <typename T, int CELLS, int CPL>
+__device__ __forceinline__ void stage_split_filter(const T* __restrict__ filter, int C, int blk0, int blk1, uint4* wsp, float* unscale) {
   using E = typename NhwcMxOf<T>::type;
   using M = NhwcMx<E>;
-  using Raw = typename std::conditional<sizeof(T) == 4, nhwc_u4, nhwc_u2>::type;
   constexpr bool kThird = sizeof(T) == 4;  // float32 tensors: the filter has a low part
-  constexpr int TAPS = 9, CELLS = SH * SW;
-  static_assert(CELLS <= 16, "one block of sixteen cells");
-  extern __shared__ __align__(16) unsigned char nhwc_lds[];
-  const int C = g.channel, nblk = (C + 15) >> 4;
-  uint4* wsp = reinterpret_cast<uint4*>(nhwc_lds);                // [nblk][64]: Wh (2 words), Wl (2 words) of lane (channel, cells 4 kg ..)
-  float* unscale = reinterpret_cast<float*>(wsp + nblk * 64);     // [nblk][16]: 1 / s of the channel
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  float2* cw = reinterpret_cast<float2*>(unscale + nblk * 16) + wave * (TAPS * 16);             // [tap][pixel]: scope coordinates
-  unsigned* xo = reinterpret_cast<unsigned*>(reinterpret_cast<float2*>(unscale + nblk * 16) + kG16Waves * TAPS * 16) +
-                 wave * (TAPS * 16);                                                             // [tap][pixel]: source offsets
-  const int lb = logical_block(total_blocks);
-  if (lb >= total_blocks) return;
-
-  // ---- per workgroup: the split filter operands of every channel block.  An entry is lane l of its wave, so the
-  // channel's largest weight is the maximum over the four lanes l % 16 + 16 k of what each holds: one load per lane
-  // instead of the channel's sixteen (a workgroup lives about as long as a dozen trips to L2, and every thread
-  // waits for this table: forward 80 -> 75 us on benchmark configuration 2).  Issuing several entries' loads
-  // together measured slower (83 us).
-  for (int e = threadIdx.x; e < nblk * 64; e += 64 * kG16Waves) {
-    const int b = e >> 6, l = e & 63, cj = b * 16 + (l & 15), c0 = 4 * (l >> 4);
+  for (int e = blk0 * 64 + threadIdx.x; e < blk1 * 64; e += 64 * kG16Waves) {
+    const int b = e >> 6, l = e & 63, c0 = 4 * (l >> 4);
+    const int cj = CPL == 4 ? b * 16 + (l & 15) : (b >> 1) * 32 + 8 * ((l & 15) >> 2) + 4 * (b & 1) + (l & 3);
     float v[4] = {0.f, 0.f, 0.f, 0.f}, s = 1.f;
     if (cj < C) {
       const T* f = filter + (size_t)cj * CELLS;
@@ -1136,6 +1172,33 @@ __global__ __launch_bounds__(64 * kG16Waves) void nhwc_gather_mfma16_kernel(
     const uint2 hb = __builtin_bit_cast(uint2, h4), lb2 = __builtin_bit_cast(uint2, l4);
     wsp[e] = make_uint4(hb.x, hb.y, lb2.x, lb2.y);
   }
+}
+
+template <typename T, int SH, int SW, bool TRANSPOSED, int CPL>
+__global__ __launch_bounds__(64 * kG16Waves) void nhwc_gather_mfma16_kernel(
+    Geo g, const T* __restrict__ src, const T* __restrict__ rot, const T* __restrict__ filter, T* __restrict__ dst,
+    int tiles_per_wave, int total_blocks, int steps_per_split) {
+  using E = typename NhwcMxOf<T>::type;
+  using M = NhwcMx<E>;
+  using Raw = NhwcRaw<T, CPL>;
+  constexpr bool kThird = sizeof(T) == 4;  // float32 tensors: the filter has a low part
+  constexpr int TAPS = 9, CELLS = SH * SW;
+  static_assert(CELLS <= 16, "one block of sixteen cells");
+  extern __shared__ __align__(16) unsigned char nhwc_lds[];
+  constexpr int SUB = CPL / 4;  // channel blocks of a step
+  const int C = g.channel, nstep = (C + 16 * SUB - 1) / (16 * SUB), nblk = nstep * SUB;
+  uint4* wsp = reinterpret_cast<uint4*>(nhwc_lds);                // [nblk][64]: Wh (2 words), Wl (2 words) of lane (channel, cells 4 kg ..)
+  float* unscale = reinterpret_cast<float*>(wsp + nblk * 64);     // [nblk][16]: 1 / s of the channel
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  float2* cw = reinterpret_cast<float2*>(unscale + nblk * 16) + wave * (TAPS * 16);             // [tap][pixel]: scope coordinates
+  unsigned* xo = reinterpret_cast<unsigned*>(reinterpret_cast<float2*>(unscale + nblk * 16) + kG16Waves * TAPS * 16) +
+                 wave * (TAPS * 16);                                                             // [tap][pixel]: source offsets
+  const int lb = logical_block(total_blocks);
+  if (lb >= total_blocks) return;
+
+  // the channels of this workgroup (blockIdx.y: a split of them)
+  const int step0 = blockIdx.y * steps_per_split, step1 = min(nstep, step0 + steps_per_split);
+  stage_split_filter<T, CELLS, CPL>(filter, C, step0 * SUB, step1 * SUB, wsp, unscale);
   __syncthreads();
 
   const int n = lane & 15, kg = lane >> 4;
@@ -1192,69 +1255,209 @@ __global__ __launch_bounds__(64 * kG16Waves) void nhwc_gather_mfma16_kernel(
     for (int t = 0; t < TAPS; ++t) {
       const float2 c = cw[t * 16 + n];
       xoff[t] = xo[t * 16 + n];
-      typedef float f2v __attribute__((ext_vector_type(2)));
-      typedef E e2v __attribute__((ext_vector_type(2)));
-      float v[4];
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        v[k] = nhwc_hat(c.x - crow[k]) * nhwc_hat(c.y - ccol[k]);
-        asm volatile("" : "+v"(v[k]));  // one fp32 value for both parts
-      }
-      const e2v h01 = __builtin_convertvector(f2v{v[0], v[1]}, e2v), h23 = __builtin_convertvector(f2v{v[2], v[3]}, e2v);
-      const f2v b01 = __builtin_convertvector(h01, f2v), b23 = __builtin_convertvector(h23, f2v);
-      const e2v l01 = __builtin_convertvector(f2v{v[0] - b01[0], v[1] - b01[1]}, e2v);
-      const e2v l23 = __builtin_convertvector(f2v{v[2] - b23[0], v[3] - b23[1]}, e2v);
-      A[t] = typename M::v8{h01[0], h01[1], h23[0], h23[1], l01[0], l01[1], l23[0], l23[1]};
+      A[t] = hat_operand<E>(c, crow, ccol);
     }
 
     // ---- the channel blocks
     const unsigned doff = live ? (unsigned)(qc * C) * (unsigned)sizeof(T) : kOutOfRange;
-    auto chan_off = [&](int blk) {
-      const int c4 = blk * 16 + 4 * kg;
-      return c4 < C ? (unsigned)c4 * (unsigned)sizeof(T) : kNoChannels;
+    auto chan_off = [&](int step) {
+      const int c = (step * 4 + kg) * CPL;
+      return c < C ? (unsigned)c * (unsigned)sizeof(T) : kNoChannels;
     };
     Raw xr[3][3];  // [tap row][tap]: two tap rows ahead of the arithmetic
     auto issue_row = [&](Raw (&buf)[3], int r, unsigned co) {
 #pragma unroll
-      for (int tt = 0; tt < 3; ++tt) buf[tt] = raw_ld4(rs, xoff[3 * r + tt] + co, src);
+      for (int tt = 0; tt < 3; ++tt) buf[tt] = raw_ld<CPL>(rs, xoff[3 * r + tt] + co, src);
     };
-    unsigned co = chan_off(0);
+    unsigned co = chan_off(step0);
     issue_row(xr[0], 0, co);
     issue_row(xr[1], 1, co);
-    for (int blk = 0; blk < nblk; ++blk) {
-      const unsigned co_next = chan_off(blk + 1);  // past the last block: no channels, zeros
-      const uint4 wv = wsp[blk * 64 + lane];
-      const typename M::v4 wh = __builtin_bit_cast(typename M::v4, make_uint2(wv.x, wv.y));
-      const typename M::v4 wl = __builtin_bit_cast(typename M::v4, make_uint2(wv.z, wv.w));
-      const typename M::v8 whh = __builtin_shufflevector(wh, wh, 0, 1, 2, 3, 0, 1, 2, 3);
-      const typename M::v4 zero4 = {E(0), E(0), E(0), E(0)};
-      const typename M::v8 wl0 = __builtin_shufflevector(wl, zero4, 0, 1, 2, 3, 4, 5, 6, 7);
-      float acc[4] = {0.f, 0.f, 0.f, 0.f};
+    for (int step = step0; step < step1; ++step) {
+      const unsigned co_next = chan_off(step + 1);  // past the last block: no channels, zeros
+      typename M::v8 whh[SUB], wl0[SUB];
+#pragma unroll
+      for (int h = 0; h < SUB; ++h) {
+        const uint4 wv = wsp[(step * SUB + h) * 64 + lane];
+        const typename M::v4 wh = __builtin_bit_cast(typename M::v4, make_uint2(wv.x, wv.y));
+        const typename M::v4 wl = __builtin_bit_cast(typename M::v4, make_uint2(wv.z, wv.w));
+        const typename M::v4 zero4 = {E(0), E(0), E(0), E(0)};
+        whh[h] = __builtin_shufflevector(wh, wh, 0, 1, 2, 3, 0, 1, 2, 3);
+        wl0[h] = __builtin_shufflevector(wl, zero4, 0, 1, 2, 3, 4, 5, 6, 7);
+      }
+      float acc[CPL];
+#pragma unroll
+      for (int i = 0; i < CPL; ++i) acc[i] = 0.f;
 #pragma unroll
       for (int r = 0; r < 3; ++r) {
         if (r == 0) issue_row(xr[2], 2, co);
         else issue_row(xr[r - 1], r - 1, co_next);
-        nhwc_f4 d[3];
-        M::template rows3<kThird>(d[0], d[1], d[2], whh, wl0, A[3 * r], A[3 * r + 1], A[3 * r + 2]);
+        nhwc_f4 d[SUB][3];
+#pragma unroll
+        for (int h = 0; h < SUB; ++h)
+          M::template rows3<kThird>(d[h][0], d[h][1], d[h][2], whh[h], wl0[h], A[3 * r], A[3 * r + 1], A[3 * r + 2]);
 #pragma unroll
         for (int tt = 0; tt < 3; ++tt) {
-          float xv[4];
-          raw_cvt4(xr[r][tt], xv, src);
+          float xv[CPL];
+          raw_cvt(xr[r][tt], xv, src);
 #pragma unroll
-          for (int i = 0; i < 4; ++i) acc[i] = fmaf(xv[i], d[tt][i], acc[i]);
+          for (int i = 0; i < CPL; ++i) acc[i] = fmaf(xv[i], d[i / 4][tt][i % 4], acc[i]);
         }
       }
       if constexpr (kThird) {
-        const nhwc_f4 us = *reinterpret_cast<const nhwc_f4*>(unscale + blk * 16 + 4 * kg);
+        const nhwc_f4 us = *reinterpret_cast<const nhwc_f4*>(unscale + step * 16 + 4 * kg);
 #pragma unroll
         for (int i = 0; i < 4; ++i) acc[i] *= us[i];
       }
       // non-temporal: written with the default policy the result pushes the operands of the next kernel out of
       // the memory-side cache (the step of benchmark configuration 2 took 0.425 instead of 0.363 ms)
-      raw_st4<kStreamingStore>(rd, doff + co, acc, dst);
+      raw_st<kStreamingStore>(rd, doff + co, acc, dst);
       co = co_next;
     }
   }
+}
+
+// Grad input of the stride-2 layers (padding 1, no dilation).  On the transposed geometry above an input pixel is tested
+// against nine taps of which two and a quarter reach it on average.  Here a column of the matrix instruction is a QUAD of
+// input pixels, rows 2 a, 2 a + 1 and columns 2 b, 2 b + 1: the nine taps that reach its pixels come from the four
+// output pixels (a, b), (a, b + 1), (a + 1, b), (a + 1, b + 1), each tap exactly once --
+//   (0, 0): tap 4 of (a, b)                        (0, 1): taps 5 of (a, b), 3 of (a, b + 1)
+//   (1, 0): taps 7 of (a, b), 1 of (a + 1, b)      (1, 1): 8 of (a, b), 6 of (a, b + 1), 2 of (a + 1, b), 0 of (a + 1, b + 1)
+// -- so that a quad costs nine products, four loads and thirty-six multiply-adds per four channels where four columns of
+// the kernel above cost four times the products and multiply-adds and thirty-six loads.
+template <typename T, int SH, int SW, int CPL>
+__global__ __launch_bounds__(64 * kG16Waves) void nhwc_grad_input_s2_kernel(
+    Geo g, const T* __restrict__ gout, const T* __restrict__ rot, const T* __restrict__ filter, T* __restrict__ gin,
+    int total_blocks, int steps_per_split) {
+  using E = typename NhwcMxOf<T>::type;
+  using M = NhwcMx<E>;
+  using Raw = NhwcRaw<T, CPL>;
+  constexpr bool kThird = sizeof(T) == 4;
+  constexpr int TAPS = 9, CELLS = SH * SW;
+  static_assert(CELLS <= 16, "one block of sixteen cells");
+  extern __shared__ __align__(16) unsigned char nhwc_lds[];
+  constexpr int SUB = CPL / 4;  // channel blocks of a step
+  const int C = g.channel, nstep = (C + 16 * SUB - 1) / (16 * SUB), nblk = nstep * SUB;
+  uint4* wsp = reinterpret_cast<uint4*>(nhwc_lds);
+  float* unscale = reinterpret_cast<float*>(wsp + nblk * 64);
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  float2* cw = reinterpret_cast<float2*>(unscale + nblk * 16) + wave * (TAPS * 16);  // [tap][quad]: scope coordinates
+  const int lb = logical_block(total_blocks);
+  if (lb >= total_blocks) return;
+  // the channels of this workgroup (blockIdx.y: a split of them)
+  const int step0 = blockIdx.y * steps_per_split, step1 = min(nstep, step0 + steps_per_split);
+  stage_split_filter<T, CELLS, CPL>(filter, C, step0 * SUB, step1 * SUB, wsp, unscale);
+  __syncthreads();
+
+  const int n = lane & 15, kg = lane >> 4;
+  const int OH = g.out_h, OW = g.out_w, oplane = OH * OW;
+  const long quads = (long)g.batch * oplane;
+  const rsrc_t rs = plane_rsrc(gout, g.batch * oplane * C);
+  const rsrc_t rd = plane_rsrc(gin, g.batch * g.in_h * g.in_w * C);
+  float crow[4], ccol[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int c = 4 * kg + k;
+    crow[k] = c < CELLS ? (float)(c / SW) : 64.f;
+    ccol[k] = (float)(c % SW);
+  }
+  const long q0 = ((long)lb * kG16Waves + wave) * 16;
+  if (q0 >= quads) return;  // uniform over the wave, and no barrier follows
+  const bool live = q0 + n < quads;
+  const long q = live ? q0 + n : 0;
+  const int b = (int)(q / oplane), pix = (int)(q - (long)b * oplane), a = pix / OW, c = pix - a * OW;
+
+  // scope coordinates: lane group kg takes taps kg, kg + 4, kg + 8; tap t belongs to output pixel (a + (t < 3), c + (t % 3 == 0))
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    const int t = kg + 4 * k;
+    if (t < TAPS) {
+      const int oh = a + (t < 3 ? 1 : 0), ow = c + (t % 3 == 0 ? 1 : 0);
+      float2 at = make_float2(-2.f, -2.f);
+      if (live && oh < OH && ow < OW) {
+        const size_t ri = ((size_t)b * oplane + oh * OW + ow) * (TAPS * 2) + 2 * t;
+        const float h = scope_coord<float>(g, t / 3, (float)ld(rot + ri), g.centre_h);
+        const float w = scope_coord<float>(g, t % 3, (float)ld(rot + ri + 1), g.centre_w);
+        if (h > -1.f && w > -1.f && h < (float)SH && w < (float)SW) at = make_float2(h, w);
+      }
+      cw[t * 16 + n] = at;
+    }
+  }
+  lds_fence_wave();
+  typename M::v8 A[TAPS];
+#pragma unroll
+  for (int t = 0; t < TAPS; ++t) A[t] = hat_operand<E>(cw[t * 16 + n], crow, ccol);
+
+  // the four output pixels' and the four input pixels' element offsets (kOutOfRange: not there)
+  unsigned so[4], po[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int oh = a + (i >> 1), ow = c + (i & 1), ih = 2 * a + (i >> 1), iw = 2 * c + (i & 1);
+    so[i] = live && oh < OH && ow < OW ? (unsigned)((((long)b * oplane + oh * OW + ow) * C) * (long)sizeof(T)) : kOutOfRange;
+    po[i] = live && ih < g.in_h && iw < g.in_w ? (unsigned)((((long)b * g.in_h + ih) * g.in_w + iw) * C * (long)sizeof(T)) : kOutOfRange;
+  }
+  auto chan_off = [&](int step) {
+    const int ch = (step * 4 + kg) * CPL;
+    return ch < C ? (unsigned)ch * (unsigned)sizeof(T) : kNoChannels;
+  };
+  Raw xr[2][4];  // a step ahead of the arithmetic
+  unsigned co[2] = {chan_off(step0), 0};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) xr[0][i] = raw_ld<CPL>(rs, so[i] + co[0], gout);
+  auto do_step = [&](int step, Raw (&cur)[4], Raw (&nxt)[4], unsigned cur_off, unsigned& nxt_off) {
+    nxt_off = chan_off(step + 1);  // past the last block: no channels, zeros
+#pragma unroll
+    for (int i = 0; i < 4; ++i) nxt[i] = raw_ld<CPL>(rs, so[i] + nxt_off, gout);
+    float x[4][CPL], acc[4][CPL];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      raw_cvt(cur[i], x[i], gout);
+#pragma unroll
+      for (int k = 0; k < CPL; ++k) acc[i][k] = 0.f;
+    }
+#pragma unroll
+    for (int h = 0; h < SUB; ++h) {
+      const uint4 wv = wsp[(step * SUB + h) * 64 + lane];
+      const typename M::v4 wh = __builtin_bit_cast(typename M::v4, make_uint2(wv.x, wv.y));
+      const typename M::v4 wl = __builtin_bit_cast(typename M::v4, make_uint2(wv.z, wv.w));
+      const typename M::v4 zero4 = {E(0), E(0), E(0), E(0)};
+      const typename M::v8 whh = __builtin_shufflevector(wh, wh, 0, 1, 2, 3, 0, 1, 2, 3);
+      const typename M::v8 wl0 = __builtin_shufflevector(wl, zero4, 0, 1, 2, 3, 4, 5, 6, 7);
+      auto add = [&](float (&to)[CPL], const float (&from)[CPL], const nhwc_f4& w) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) to[4 * h + k] = fmaf(from[4 * h + k], w[k], to[4 * h + k]);
+      };
+      nhwc_f4 d[3];
+      M::template rows3<kThird>(d[0], d[1], d[2], whh, wl0, A[3], A[4], A[5]);
+      add(acc[1], x[1], d[0]);
+      add(acc[0], x[0], d[1]);
+      add(acc[1], x[0], d[2]);
+      M::template rows3<kThird>(d[0], d[1], d[2], whh, wl0, A[6], A[7], A[8]);
+      add(acc[3], x[1], d[0]);
+      add(acc[2], x[0], d[1]);
+      add(acc[3], x[0], d[2]);
+      M::template rows3<kThird>(d[0], d[1], d[2], whh, wl0, A[0], A[1], A[2]);
+      add(acc[3], x[3], d[0]);
+      add(acc[2], x[2], d[1]);
+      add(acc[3], x[2], d[2]);
+    }
+    nhwc_f4 us = {1.f, 1.f, 1.f, 1.f};
+    if constexpr (kThird) us = *reinterpret_cast<const nhwc_f4*>(unscale + step * 16 + 4 * kg);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if constexpr (kThird)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) acc[i][k] *= us[k];
+      // 16-bit types: the default policy, for the L2 to put a pixel's pieces together (N=64 96 x 112^2, bfloat16, four
+      // channels per lane: 163 us with non-temporal stores, which reached memory one by one, 62 with these)
+      raw_st<sizeof(T) == 4 ? kStreamingStore : kMergedStore>(rd, po[i] + cur_off, acc[i], gin);
+    }
+  };
+  int step = step0;
+  for (; step + 1 < step1; step += 2) {
+    do_step(step, xr[0], xr[1], co[0], co[1]);
+    do_step(step + 1, xr[1], xr[0], co[1], co[0]);
+  }
+  if (step < step1) do_step(step, xr[0], xr[1], co[0], co[1]);
 }
 
 // ---- host side --------------------------------------------------------------------------
@@ -1295,19 +1498,39 @@ bool nhwc_supported(const Geo& g, int dtype) {
   return true;
 }
 
+// Steps over the channels that a workgroup of the two kernels below takes.  Few tiles and many channels (grad input, N=64
+// 576 x 14^2 stride 2, float32: 49 workgroups, 33 us): the channels go over workgroups, at least four blocks each (their
+// set-up is about one block's work), for about eight waves per SIMD (12 us).
+int channel_steps_per_split(int nstep, int nblk, int blocks) {
+  return ceil_div(nstep, std::max(1, std::min(nblk / 4, 2048 / std::max(1, blocks))));
+}
+
 // The matrix-core forward / grad input; false where it does not apply.
-template <typename T, int SH, int SW>
+template <typename T, int SH, int SW, int CPL>
 bool launch_gather_mfma16(const Geo& g, bool transposed, const T* src, const T* rot, const T* filter, T* dst,
                           hipStream_t stream) {
-  const int nblk = ceil_div(g.channel, 16);
+  const int nstep = ceil_div(g.channel, 4 * CPL), nblk = nstep * (CPL / 4);
   const size_t lds = (size_t)nblk * 64 * 16 + (size_t)nblk * 16 * 4 + (size_t)kG16Waves * 9 * 16 * (8 + 4);
   const long pixels = (long)g.batch * (transposed ? g.in_h * g.in_w : g.out_h * g.out_w);
   const long tiles = ceil_div(pixels, 16L);
   const int blocks = (int)ceil_div(tiles, (long)kG16Waves * kG16TilesPerWave);
-  auto kernel = transposed ? nhwc_gather_mfma16_kernel<T, SH, SW, true> : nhwc_gather_mfma16_kernel<T, SH, SW, false>;
+  auto kernel = transposed ? nhwc_gather_mfma16_kernel<T, SH, SW, true, CPL> : nhwc_gather_mfma16_kernel<T, SH, SW, false, CPL>;
   if (lds > 64 * 1024 && !(lds <= 120 * 1024 && allow_dynamic_lds(reinterpret_cast<const void*>(kernel), 120 * 1024))) return false;
-  hipLaunchKernelGGL(kernel, dim3((unsigned)xcd_grid_size(blocks)), dim3(64 * kG16Waves), lds, stream, g, src, rot, filter, dst,
-                     kG16TilesPerWave, blocks);
+  const int per = channel_steps_per_split(nstep, nblk, blocks);
+  kernel<<<dim3((unsigned)xcd_grid_size(blocks), (unsigned)ceil_div(nstep, per)), 64 * kG16Waves, lds, stream>>>(
+      g, src, rot, filter, dst, kG16TilesPerWave, blocks, per);
+  return true;
+}
+
+template <typename T, int SH, int SW, int CPL>
+bool launch_grad_input_s2(const Geo& g, const T* gout, const T* rot, const T* filter, T* gin, hipStream_t stream) {
+  const int nstep = ceil_div(g.channel, 4 * CPL), nblk = nstep * (CPL / 4);
+  const size_t lds = (size_t)nblk * 64 * 16 + (size_t)nblk * 16 * 4 + (size_t)kG16Waves * 9 * 16 * 8;
+  const int blocks = (int)ceil_div((long)g.batch * g.out_h * g.out_w, 16L * kG16Waves);
+  auto kernel = nhwc_grad_input_s2_kernel<T, SH, SW, CPL>;
+  if (lds > 64 * 1024 && !(lds <= 120 * 1024 && allow_dynamic_lds(reinterpret_cast<const void*>(kernel), 120 * 1024))) return false;
+  const int per = channel_steps_per_split(nstep, nblk, blocks);
+  kernel<<<dim3((unsigned)xcd_grid_size(blocks), (unsigned)ceil_div(nstep, per)), 64 * kG16Waves, lds, stream>>>(g, gout, rot, filter, gin, blocks, per);
   return true;
 }
 
@@ -1322,18 +1545,37 @@ bool nhwc_gather_mfma16(const Geo& g, bool transposed, const T* src, const T* ro
         reinterpret_cast<uintptr_t>(src) % (4 * sizeof(T)) != 0 || reinterpret_cast<uintptr_t>(dst) % (4 * sizeof(T)) != 0 ||
         path_disabled(kNoNhwcMfma) || path_disabled(kNoNhwcStaged))
       return false;
-    // Where it is the faster kernel (step-level measurements on the MobileNetV2-DK layer shapes, batch 64, float32;
-    // this kernel against the table kernel): its per-tile set-up (a third of its instructions at 144 channels) and
-    // its one-tile-per-wave grid want many channels and many tiles.  Forward 144 x 56^2: 80 against 103 us, but
-    // 32 x 112^2 136 / 109, 192 x 28^2 50 / 39, 960 x 7^2 58 / 22.  Grad input at stride 2, where the table kernel
-    // tests every tap of every input pixel against the stride's grid: 96 x 112^2 166 / 262, 144 x 56^2 61 / 96,
-    // 192 x 28^2 28 / 38.  DK_FORCE_NHWC_GATHER_MFMA takes it wherever it applies (the tests).
+    // 16-bit tensors of whole, aligned 16-byte groups: eight channels per lane and load.  With four, a wave's load and
+    // store touch sixteen pieces of 32 bytes, and the kernel is bound by the pieces: forward, bfloat16, batch 64, table
+    // kernel / four / eight channels, us: 96 x 56^2 74 / 54 / 37, 192 x 28^2 41 / 50 / 29, 64 x 112^2 189 / 210 / 136,
+    // 96 x 112^2 stride 2 76 / 91 / 59; grad input of the last 144 / 62 / 40 (144: the kernel above on the transposed geometry).
+    const bool eight = sizeof(T) == 2 && g.channel % 8 == 0 && reinterpret_cast<uintptr_t>(src) % 16 == 0 &&
+                       reinterpret_cast<uintptr_t>(dst) % 16 == 0;
+#define DK_NHWC16(LAUNCH, ...)                                                             \
+  if (g.scope_h == 4 && g.scope_w == 4) {                                                  \
+    if constexpr (sizeof(T) == 2) if (eight) return LAUNCH<T, 4, 4, 8>(g, __VA_ARGS__);    \
+    return LAUNCH<T, 4, 4, 4>(g, __VA_ARGS__);                                             \
+  }                                                                                        \
+  if (g.scope_h == 3 && g.scope_w == 3) {                                                  \
+    if constexpr (sizeof(T) == 2) if (eight) return LAUNCH<T, 3, 3, 8>(g, __VA_ARGS__);    \
+    return LAUNCH<T, 3, 3, 4>(g, __VA_ARGS__);                                             \
+  }
+    if (transposed && g.stride_h == 2 && g.stride_w == 2 && g.pad_h == 1 && g.pad_w == 1 && g.dil_h == 1 && g.dil_w == 1) {
+      DK_NHWC16(launch_grad_input_s2, src, rot, filter, dst, stream)
+      return false;
+    }
     const long tiles = ((long)g.batch * (transposed ? g.in_h * g.in_w : g.out_h * g.out_w) + 15) / 16;
     const bool strided = g.stride_h > 1 || g.stride_w > 1;
-    const bool faster = (g.channel >= 128 && tiles >= 8192) || (transposed && strided && g.channel >= 64 && tiles >= 3000);
+    // Where it is the faster kernel (step-level measurements on the MobileNetV2-DK layer shapes, batch 64, float32;
+    // this kernel against the table kernel): with eight channels per lane everywhere; with four its per-tile set-up (a
+    // third of its instructions at 144 channels) and its one-tile-per-wave grid want many channels and many tiles.
+    // Forward 144 x 56^2: 80 against 103 us, but 32 x 112^2 136 / 109, 192 x 28^2 50 / 39, 960 x 7^2 58 / 22.  Grad input
+    // at other strides than 1 and 2, where the table kernel tests every tap of every input pixel against the stride's
+    // grid: from 64 channels and 3000 tiles on.  DK_FORCE_NHWC_GATHER_MFMA takes it wherever it applies (the tests).
+    const bool faster = eight || (g.channel >= 128 && tiles >= 8192) || (transposed && strided && g.channel >= 64 && tiles >= 3000);
     if (!faster && !path_disabled(kForceNhwcGatherMfma)) return false;
-    if (g.scope_h == 4 && g.scope_w == 4) return launch_gather_mfma16<T, 4, 4>(g, transposed, src, rot, filter, dst, stream);
-    if (g.scope_h == 3 && g.scope_w == 3) return launch_gather_mfma16<T, 3, 3>(g, transposed, src, rot, filter, dst, stream);
+    DK_NHWC16(launch_gather_mfma16, transposed, src, rot, filter, dst, stream)
+#undef DK_NHWC16
     return false;
   }
 }

@@ -224,3 +224,22 @@ def test_channels_last_input_of_a_geometry_the_channels_last_kernels_do_not_cove
         assert torch.equal(a, b)  # the same kernels ran on the same values
     o64 = _oracle((x, wt, rot, gout, cfg), np.float64)
     assert rel_err(res[1][0], o64[0]) < 1e-5 and rel_err(res[1][3], o64[3]) < 1e-4
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("case", [
+    (1, 16, 2, 3, 3, (4, 4), 2, 1, 1, 1, 0.7),      # one quad row, the second quad without a right column
+    (2, 20, 15, 18, 3, (3, 3), 2, 1, 1, 1, 0.7),    # odd rows, even columns; four channels per lane, the last block a quarter full
+    (3, 24, 18, 15, 3, (4, 4), 2, 1, 1, 1, 0.7),    # eight channels per lane, a step of 32 not full
+    (1, 136, 21, 22, 3, (4, 4), 2, 1, 1, 1, 0.7),   # channels split over workgroups, the last split partial
+    (2, 40, 14, 112, 3, (4, 4), 2, 1, 1, 1, 0.7),   # grad filter: tiles of two output rows, the last of one
+    (2, 40, 20, 13, 3, (4, 4), 1, 1, 1, 1, 0.7),    # stride 1: forward and grad input with eight channels per lane
+    (1, 264, 6, 9, 3, (3, 3), 1, 1, 1, 1, 0.7),     # ... and their channels split over workgroups
+])
+def test_quads_at_stride_2_and_eight_channels_per_lane(case, dtype):
+    inputs, got = _run(case, dtype, seed=3)
+    o32, o64 = _oracle(inputs, np.float32), _oracle(inputs, np.float64)
+    tol = (1e-5, 1e-5, 1e-4, 1e-4) if dtype == torch.float32 else (1e-2,) * 4   # as stated at the head of the file
+    for a, b32, b64, t in zip(got, o32, o64, tol):
+        assert a.dtype == dtype
+        assert rel_err(a.float(), b64 if t == 1e-4 else b32) < t
