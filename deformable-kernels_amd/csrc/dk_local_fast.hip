@@ -1037,8 +1037,10 @@ __device__ __forceinline__ int mf_row(int j, int pitch_x) { return j * pitch_x +
 
 __device__ __forceinline__ float hat(float d) { return __builtin_amdgcn_fmed3f(1.f - fabsf(d), 0.f, 1.f); }
 
-// CELL0: the kernel sums the scope cells CELL0 .. CELL0 + 15 (the 16 rows of one MFMA block); a
-// scope of more than 16 cells takes further launches (5 x 5: CELL0 = 16; 7 x 7: 16, 32, 48).
+// CELL0, NSL: the kernel sums the scope cells CELL0 .. CELL0 + 16 NSL - 1, NSL slices of 16 rows.  A scope of more than
+// 16 cells runs two slices per launch (5 x 5: one launch; 7 x 7: two) with 16-bit operands: the staging and the
+// products P, which are the vector work of a unit, serve both, and the second slice's matrix instructions run
+// beside other waves' vector work.  (The fp32 instructions do not; they keep a launch per slice.)
 // S2: the stride-2 geometry of local_forward_s2_kernel.  A tile is then `th` whole output rows (at
 // most 128 pixels), so that the input rows its taps read, 2 oh0 - 1 .. 2 (oh0 + th - 1) + 1, are
 // one contiguous range of the plane like the stride-1 tile with its halo rows; a lane's four
@@ -1057,20 +1059,22 @@ __device__ __forceinline__ float hat(float d) { return __builtin_amdgcn_fmed3f(1
 // one group).  Only the staging differs: a thread loads four consecutive channels of a pixel (the unit's
 // sixteen channels are 64 contiguous bytes per pixel) and stores them into the same channel-major tiles
 // in LDS, so the products run as for planar tensors.
-template <typename T, int SH, int SW, int CELL0, int NX, bool S2, bool BF = false, bool SPLIT = false, bool CL = false>
-__global__ __launch_bounds__(kMfBlock, 4) void local_grad_filter_mfma_kernel(
+template <typename T, int SH, int SW, int CELL0, int NX, bool S2, bool BF = false, bool SPLIT = false, bool CL = false,
+          int NSL = 1>
+__global__ __launch_bounds__(kMfBlock, NSL == 2 && SPLIT ? 2 : 4) void local_grad_filter_mfma_kernel(
     Geo g, const T* __restrict__ gout, const T* __restrict__ x, const T* __restrict__ rot,
     float* __restrict__ partial, int tiles, int nwg, int csplits, int pitch_x, int th) {
   constexpr int K = 9, CELLS = SH * SW;
   constexpr int kWaves = kMfBlock / 64;
   static_assert(CELL0 % 16 == 0 && CELL0 < CELLS, "the cells come in slices of 16, the rows of one MFMA block");
+  static_assert(NSL == 1 || BF || SPLIT, "more than one slice per launch: 16-bit operands");
   static_assert(kMfPix == 16 * kWaves, "one 16-pixel group per wave");
   extern __shared__ __align__(16) float lds[];
   float* xs = lds;                                                  // [kMfCh][pitch_x]
   float* gs = xs + kMfCh * pitch_x;                                 // [kMfCh][kMfPitchG]
   float2* hw = reinterpret_cast<float2*>(gs + kMfCh * kMfPitchG);   // [K][kMfPix]
-  float* red = reinterpret_cast<float*>(hw + K * kMfPix);           // [kWaves][256]
-  float* accs = red + kWaves * 256;                                 // [blocks of this split][256]
+  float* red = reinterpret_cast<float*>(hw + K * kMfPix);           // [NSL][kWaves][256]
+  float* accs = red + NSL * kWaves * 256;                           // [blocks of this split][NSL][256]
 
   const int cpg = g.channel / g.groups;
   const int nblk_all = ceil_div(cpg, kMfCh);
@@ -1091,9 +1095,14 @@ __global__ __launch_bounds__(kMfBlock, 4) void local_grad_filter_mfma_kernel(
   const int row_step = g.dil_h * W;               // elements between two tap rows
   const int lo = -g.pad_h * W - 1;                // first staged input element, relative to the tile
   // rows past the last cell (9..15 of a 3 x 3 scope, 25..31 of a 5 x 5 one) stay 0
-  const float ci = CELL0 + q < CELLS ? float((CELL0 + q) / SW) : 64.f, cj = float((CELL0 + q) % SW);
+  float ci[NSL], cj[NSL];
+#pragma unroll
+  for (int s = 0; s < NSL; ++s) {
+    const int cell = CELL0 + 16 * s + q;
+    ci[s] = cell < CELLS ? float(cell / SW) : 64.f, cj[s] = float(cell % SW);
+  }
 
-  for (int e = threadIdx.x; e < nblk * 256; e += kMfBlock) accs[e] = 0.f;
+  for (int e = threadIdx.x; e < nblk * (NSL * 256); e += kMfBlock) accs[e] = 0.f;
 
   // This workgroup's share of the (tile, channel block) units of its group and channel split, as
   // segments (tile, first block, end block).  Whole tiles are dealt out round-robin, tile t to
@@ -1276,28 +1285,42 @@ __global__ __launch_bounds__(kMfBlock, 4) void local_grad_filter_mfma_kernel(
   static_assert(!SPLIT || !BF, "one or the other");
   constexpr bool kHalfIn = BF;
   float A[(kHalfIn || SPLIT) ? 1 : 4][K];
-  mfb4 Ab[(kHalfIn || SPLIT) ? K : 1];  // SPLIT: the hi parts
-  mfb4 Al[SPLIT ? K : 1];               // ... and the lo parts
-  mf4 acc = {0.f, 0.f, 0.f, 0.f};
+  mfb4 Ab[NSL][(kHalfIn || SPLIT) ? K : 1];  // SPLIT: the hi parts
+  mfb4 Al[NSL][SPLIT ? K : 1];               // ... and the lo parts
+  mf4 acc[NSL];
+#pragma unroll
+  for (int s = 0; s < NSL; ++s) acc[s] = mf4{0.f, 0.f, 0.f, 0.f};
   int done_cb = -1;  // channel block (within the split) whose result `acc` holds
+
+  // the waves' results of the last unit to LDS; their sums, in wave order, into the block's accumulator
+  auto write_red = [&]() {
+#pragma unroll
+    for (int s = 0; s < NSL; ++s) *reinterpret_cast<mf4*>(red + ((s * kWaves + wave) * 64 + lane) * 4) = acc[s];
+  };
+  auto add_red = [&]() {
+    if (threadIdx.x >= NSL * 256) return;
+    const int sl = threadIdx.x / 256, e = threadIdx.x % 256;
+    float s = 0.f;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) s += red[(sl * kWaves + w) * 256 + e];
+    accs[(done_cb * NSL + sl) * 256 + e] += s;
+  };
+  static_assert(NSL * 256 <= kMfBlock, "an owner thread per entry");
 
   // stage the unit whose loads are in flight, hand the previous unit's result to its owner
   // threads, start the next unit's loads (n_item < 0: there is none)
   auto begin_unit = [&](int item, bool new_tile, int n_item, int n_cbi, bool n_new_tile) {
     __syncthreads();  // the previous unit's reads of the tiles (and of `red`) are done
     store_unit(item, new_tile);
-    if (done_cb >= 0) *reinterpret_cast<mf4*>(red + (wave * 64 + lane) * 4) = acc;
+    if (done_cb >= 0) write_red();
     __syncthreads();
     if (n_item >= 0) issue_loads(n_item, n_cbi, n_new_tile);
-    if (done_cb >= 0 && threadIdx.x < 256) {
-      float s = 0.f;
-#pragma unroll
-      for (int w = 0; w < kWaves; ++w) s += red[w * 256 + threadIdx.x];
-      accs[done_cb * 256 + threadIdx.x] += s;
-    }
+    if (done_cb >= 0) add_red();
   };
   auto multiply_unit = [&](int cbi) {
-    mf4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
+    // two chains of sums per launch: the odd and even taps', or the slices'
+    mf4 sums[2];
+    sums[0] = sums[1] = mf4{0.f, 0.f, 0.f, 0.f};
     const float4 gv = *reinterpret_cast<const float4*>(gs + q * kMfPitchG + px);
     const float gq[4] = {gv.x, gv.y, gv.z, gv.w};
 #pragma unroll
@@ -1341,35 +1364,37 @@ __global__ __launch_bounds__(kMfBlock, 4) void local_grad_filter_mfma_kernel(
           const unsigned l23 = pack_bf16(pr[2] - bf16_lo(h23), pr[3] - bf16_hi(h23));
           const mfb4 bh = __builtin_bit_cast(mfb4, make_uint2(h01, h23));
           const mfb4 bl = __builtin_bit_cast(mfb4, make_uint2(l01, l23));
-          if (t & 1) {
-            acc1 = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(Ab[t], bh, acc1, 0, 0, 0);
-            acc1 = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(Ab[t], bl, acc1, 0, 0, 0);
-            acc1 = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(Al[t], bh, acc1, 0, 0, 0);
-          } else {
-            acc0 = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(Ab[t], bh, acc0, 0, 0, 0);
-            acc0 = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(Ab[t], bl, acc0, 0, 0, 0);
-            acc0 = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(Al[t], bh, acc0, 0, 0, 0);
+#pragma unroll
+          for (int sl = 0; sl < NSL; ++sl) {
+            mf4& d = sums[NSL == 1 ? t & 1 : sl];
+            d = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(Ab[sl][t], bh, d, 0, 0, 0);
+            d = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(Ab[sl][t], bl, d, 0, 0, 0);
+            d = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(Al[sl][t], bh, d, 0, 0, 0);
           }
         } else if constexpr (kHalfIn) {
           const mfb4 b = __builtin_bit_cast(mfb4, make_uint2(pack_bf16(xv[0][f_w] * gq[0], xv[1][f_w] * gq[1]),
                                                              pack_bf16(xv[2][f_w] * gq[2], xv[3][f_w] * gq[3])));
-          if (t & 1)
-            acc1 = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(Ab[t], b, acc1, 0, 0, 0);
-          else
-            acc0 = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(Ab[t], b, acc0, 0, 0, 0);
+#pragma unroll
+          for (int sl = 0; sl < NSL; ++sl) {
+            mf4& d = sums[NSL == 1 ? t & 1 : sl];
+            d = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(Ab[sl][t], b, d, 0, 0, 0);
+          }
         } else {
 #pragma unroll
           for (int ii = 0; ii < 4; ++ii) {
             const float b = xv[ii][f_w] * gq[ii];
-            if ((ii + t) & 1)
-              acc1 = __builtin_amdgcn_mfma_f32_16x16x4f32(A[ii][t], b, acc1, 0, 0, 0);
-            else
-              acc0 = __builtin_amdgcn_mfma_f32_16x16x4f32(A[ii][t], b, acc0, 0, 0, 0);
+            mf4& d = sums[(ii + t) & 1];
+            d = __builtin_amdgcn_mfma_f32_16x16x4f32(A[ii][t], b, d, 0, 0, 0);
           }
         }
       }
     }
-    acc = acc0 + acc1;
+    if constexpr (NSL == 1) {
+      acc[0] = sums[0] + sums[1];
+    } else {
+#pragma unroll
+      for (int s = 0; s < NSL; ++s) acc[s] = sums[s];
+    }
     done_cb = cbi;
   };
 
@@ -1387,23 +1412,26 @@ __global__ __launch_bounds__(kMfBlock, 4) void local_grad_filter_mfma_kernel(
     for (int t = 0; t < K; ++t) {
       const float4 hw01 = *reinterpret_cast<const float4*>(hw + t * kMfPix + px);
       const float4 hw23 = *reinterpret_cast<const float4*>(hw + t * kMfPix + px + 2);
-      const float a0 = hat(hw01.x - ci) * hat(hw01.y - cj), a1 = hat(hw01.z - ci) * hat(hw01.w - cj);
-      const float a2 = hat(hw23.x - ci) * hat(hw23.y - cj), a3 = hat(hw23.z - ci) * hat(hw23.w - cj);
-      if constexpr (SPLIT) {
-        float av[4] = {a0, a1, a2, a3};
 #pragma unroll
-        for (int ii = 0; ii < 4; ++ii) asm volatile("" : "+v"(av[ii]));
-        const unsigned h01 = pack_bf16(av[0], av[1]), h23 = pack_bf16(av[2], av[3]);
-        Ab[t] = __builtin_bit_cast(mfb4, make_uint2(h01, h23));
-        Al[t] = __builtin_bit_cast(mfb4, make_uint2(pack_bf16(av[0] - bf16_lo(h01), av[1] - bf16_hi(h01)),
-                                                    pack_bf16(av[2] - bf16_lo(h23), av[3] - bf16_hi(h23))));
-      } else if constexpr (kHalfIn) {
-        Ab[t] = __builtin_bit_cast(mfb4, make_uint2(pack_bf16(a0, a1), pack_bf16(a2, a3)));
-      } else {
-        A[0][t] = a0;
-        A[1][t] = a1;
-        A[2][t] = a2;
-        A[3][t] = a3;
+      for (int s = 0; s < NSL; ++s) {
+        const float a0 = hat(hw01.x - ci[s]) * hat(hw01.y - cj[s]), a1 = hat(hw01.z - ci[s]) * hat(hw01.w - cj[s]);
+        const float a2 = hat(hw23.x - ci[s]) * hat(hw23.y - cj[s]), a3 = hat(hw23.z - ci[s]) * hat(hw23.w - cj[s]);
+        if constexpr (SPLIT) {
+          float av[4] = {a0, a1, a2, a3};
+#pragma unroll
+          for (int ii = 0; ii < 4; ++ii) asm volatile("" : "+v"(av[ii]));
+          const unsigned h01 = pack_bf16(av[0], av[1]), h23 = pack_bf16(av[2], av[3]);
+          Ab[s][t] = __builtin_bit_cast(mfb4, make_uint2(h01, h23));
+          Al[s][t] = __builtin_bit_cast(mfb4, make_uint2(pack_bf16(av[0] - bf16_lo(h01), av[1] - bf16_hi(h01)),
+                                                         pack_bf16(av[2] - bf16_lo(h23), av[3] - bf16_hi(h23))));
+        } else if constexpr (kHalfIn) {
+          Ab[s][t] = __builtin_bit_cast(mfb4, make_uint2(pack_bf16(a0, a1), pack_bf16(a2, a3)));
+        } else {
+          A[0][t] = a0;
+          A[1][t] = a1;
+          A[2][t] = a2;
+          A[3][t] = a3;
+        }
       }
     }
     multiply_unit(cb_begin);
@@ -1420,18 +1448,13 @@ __global__ __launch_bounds__(kMfBlock, 4) void local_grad_filter_mfma_kernel(
   // the last unit's result, then D[cell = 4 * (l / 16) + r][channel = l % 16] (register r of lane l,
   // entry 4 l + r of a block's accumulator) goes out as this workgroup's partial
   __syncthreads();
-  if (done_cb >= 0) *reinterpret_cast<mf4*>(red + (wave * 64 + lane) * 4) = acc;
+  if (done_cb >= 0) write_red();
   __syncthreads();
-  if (done_cb >= 0 && threadIdx.x < 256) {
-    float s = 0.f;
-#pragma unroll
-    for (int w = 0; w < kWaves; ++w) s += red[w * 256 + threadIdx.x];
-    accs[done_cb * 256 + threadIdx.x] += s;
-  }
+  if (done_cb >= 0) add_red();
   __syncthreads();
-  for (int e = threadIdx.x; e < nblk * 256; e += kMfBlock) {
-    const int b = e / 256, l = (e % 256) / 4, r = e % 4;
-    const int cell = CELL0 + 4 * (l / 16) + r, cj_ = (cb_lo + b) * kMfCh + l % 16;
+  for (int e = threadIdx.x; e < nblk * (NSL * 256); e += kMfBlock) {
+    const int b = e / (NSL * 256), sl = e / 256 % NSL, l = (e % 256) / 4, r = e % 4;
+    const int cell = CELL0 + 16 * sl + 4 * (l / 16) + r, cj_ = (cb_lo + b) * kMfCh + l % 16;
     if (cell < CELLS && cj_ < cpg)
       partial[((size_t)wg * g.channel + grp + (size_t)g.groups * cj_) * CELLS + cell] = accs[e];
   }
@@ -1636,29 +1659,34 @@ struct FilterGrid {
   int nx;          // its staged input elements per lane and channel (4 or 6; 9 for stride 2)
   int th;          // stride 2: output rows per tile
   size_t lds;      // its LDS bytes
+  size_t lds_more; // ... and for every further slice of 16 cells in one launch
 };
 
-FilterGrid filter_grid(const Geo& g) {
+// two_slices: for launches of two slices of sixteen cells on 16-bit operands -- more channel splits, so that two
+// workgroups' LDS still fit a CU (never more partials than without)
+FilterGrid filter_grid(const Geo& g, bool two_slices = false) {
   FilterGrid f;
   const int cpg = g.channel / g.groups;
   f.mfma = false;
   f.pitch_x = 0;
   f.nx = 0;
   f.th = 0;
-  f.lds = 0;
+  f.lds = f.lds_more = 0;
   if (same_width_geometry(g) && !path_disabled(kNoMfma)) {
     const long xt = kMfPix + 2 + 2L * g.dil_h * g.in_w;
     // a row holds 64 * nx staged elements (nx = 4 or 6 per lane) plus the skew of mf_row() (at most 51)
     const long pitch = (xt <= 256 ? 256 : 64 * kMfX) + 64;
     const int nblk = ceil_div(cpg, kMfCh);
-    const int csplits = ceil_div(nblk, kMfMaxBlk);
-    const long lds = ((long)kMfCh * pitch + (long)kMfCh * kMfPitchG) * 4 + 9L * kMfPix * 8 +
-                     (long)(kMfBlock / 64) * 256 * 4 + (long)ceil_div(nblk, csplits) * 256 * 4;
+    const long tiles_lds = ((long)kMfCh * pitch + (long)kMfCh * kMfPitchG) * 4 + 9L * kMfPix * 8;
+    const long room = 80 * 1024 - tiles_lds - 2L * (kMfBlock / 64) * 256 * 4;  // for two slices' accumulators
+    const int csplits = ceil_div(nblk, two_slices ? (int)std::clamp<long>(room / (2 * 256 * 4), 1, kMfMaxBlk) : kMfMaxBlk);
+    const long lds = tiles_lds + (long)(kMfBlock / 64) * 256 * 4 + (long)ceil_div(nblk, csplits) * 256 * 4;
     if (lds <= 64 * 1024 && xt <= 64 * kMfX) {
       f.mfma = true;
       f.pitch_x = (int)pitch;
       f.nx = xt <= 256 ? 4 : kMfX;
       f.lds = (size_t)lds;
+      f.lds_more = (size_t)(kMfBlock / 64 + ceil_div(nblk, csplits)) * 256 * 4;
       f.per = kMfCh;
       f.splits = csplits;
       f.tiles = ceil_div(g.out_h * g.out_w, kMfPix);
@@ -1747,6 +1775,30 @@ bool run_grad_filter(const Geo& g, const T* gout, const T* x, const T* rot, T* g
     else { DK_LAUNCH_BF(CELL0, false, false) }                              \
   } else if (split) { DK_LAUNCH_BF(CELL0, false, true) }                    \
   else { DK_LAUNCH_BF(CELL0, false, false) }
+      // A scope of more than 16 cells with 16-bit operands: two slices per launch.  16-bit tensors keep two workgroups per
+      // CU; the pairs of float32 take 168 registers, one workgroup per CU, and gain less.  (us, a launch per slice / two
+      // slices per launch: N=64 C=192 28x28 scope 5 float16 66 / 42, float32 75 / 63; scope 7 bfloat16 131 / 83.)
+      if constexpr (SH * SW > 16) {
+        constexpr bool half = sizeof(T) == 2;
+        const FilterGrid f2 = filter_grid(g, half);
+        const size_t lds = f2.lds + f2.lds_more;
+        if (f2.th == 0 && lds <= (half ? 80 : 150) * 1024 && (half ? g.channel / g.groups >= kMfCh : split)) {
+          const unsigned grid2 = (unsigned)xcd_grid_size((long)f2.parts * f2.splits * g.groups);
+          auto launch = [&](auto kernel) {
+            if (!allow_max_dynamic_lds(reinterpret_cast<const void*>(kernel))) return false;
+            kernel<<<grid2, kMfBlock, lds, stream>>>(g, gout, x, rot, ws, f2.tiles, f2.parts, f2.splits, f2.pitch_x, 0);
+            return true;
+          };
+          bool ok = launch(f2.nx == 4 ? local_grad_filter_mfma_kernel<T, SH, SW, 0, 4, false, half, !half, CL, 2>
+                                      : local_grad_filter_mfma_kernel<T, SH, SW, 0, kMfX, false, half, !half, CL, 2>);
+          if constexpr (SH * SW > 32)
+            ok = ok && launch(f2.nx == 4 ? local_grad_filter_mfma_kernel<T, SH, SW, 32, 4, false, half, !half, CL, 2>
+                                         : local_grad_filter_mfma_kernel<T, SH, SW, 32, kMfX, false, half, !half, CL, 2>);
+          if (!ok) return false;
+          launch_reduce_partials<float, T>(ws, f2.parts, g.channel * SH * SW, gfilter, stream);
+          return true;
+        }
+      }
       DK_LAUNCH(0)
       // the further 16-cell slices of a larger scope, into the same partials
       if constexpr (SH * SW > 16) DK_LAUNCH(16)

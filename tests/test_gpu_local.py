@@ -99,6 +99,20 @@ def test_fp32_matches_oracle(case):
     assert elem_err(got[3], o64[3], 0.1) < 1e-4, "grad filter, element-wise"
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("case", [
+    (1, 16, 5, 7, 3, (5, 5), 1, 1, 1, 1, 1.5),      # one tile that is not full, one channel block
+    (2, 33, 16, 33, 3, (5, 5), 1, 1, 1, 1, 1.5),    # five tiles of 128 pixels, the last of 16; three blocks, the last of one channel
+    (1, 272, 9, 40, 3, (5, 5), 1, 1, 1, 1, 1.5),    # 17 channel blocks: several channel splits, more of them on 16-bit tensors
+    (1, 36, 8, 100, 3, (7, 7), 1, 1, 1, 2, 2.0),    # 49 cells: the last slice holds one; two groups; the wide staged tile
+])
+def test_filter_gradient_with_two_slices_of_cells_per_launch(case, dtype):
+    inputs, got = _run(case, dtype, seed=11)
+    want = _oracle(inputs, np.float64)[3]
+    # float32: pairs of bfloat16 leave about 2^-16 per product; 16-bit: operands rounded to 2^-9, sums over >= 35 pixels
+    assert rel_err(got[3].float(), want) < (1e-4 if dtype == torch.float32 else 1e-2)
+
+
 @pytest.mark.parametrize("case", [c for c in TUNED if c[6] == 1 and c[7] == 1 and c[8] == 1 and c[5] in ((4, 4), (3, 3))])
 def test_matrix_core_forward_and_grad_input_on_every_same_width_shape(case, switch_off):
     """The dispatch takes the matrix-core forward / grad input only on large planes with many channels,
