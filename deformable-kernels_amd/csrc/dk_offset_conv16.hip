@@ -112,6 +112,78 @@ __device__ __forceinline__ uint4 load_octet(rsrc_t rs, bool live, unsigned elem,
   }
 }
 
+// The register stage of a chunk: operand octets of a zero-padded tile on their way to LDS, asked for in front of the
+// previous chunk's products.  WIDE (even widths, tensors aligned to two elements): an item is two neighbouring
+// pixels, loaded as two elements per channel; else one pixel.
+template <typename T, int W, int ITEMS, bool WIDE>
+struct Stage16 {
+  static constexpr int PIX = WIDE ? 2 : 1;
+  static_assert(!WIDE || W % 2 == 0, "pairs of pixels stay within a row");
+  static constexpr int REGS = kOctOf<T> * PIX * (int)sizeof(T) < 4 * kOctOf<T> ? kOctOf<T> : kOctOf<T> * PIX * (int)sizeof(T) / 4;
+  unsigned off[ITEMS];  // byte offset of the item's first element in the chunk's planes; outside the image: out of range
+  int dst[ITEMS];       // word of its octet in the tile; -1: no item
+  int items;            // (planes lower than the tile fill the first few only)
+  unsigned raw[ITEMS][REGS];
+
+  __device__ __forceinline__ bool none(int v) const { return W <= 14 && v >= items; }
+  __device__ __forceinline__ void place(int rows, int r0, int h, int plane) {
+    items = ((rows + 2) * 4 * (W / PIX) + kC16Block - 1) / kC16Block;
+#pragma unroll
+    for (int v = 0; v < ITEMS; ++v) {
+      const int e = threadIdx.x + v * kC16Block;
+      const int col = e % (W / PIX) * PIX, ry = e / (W / PIX) % (rows + 2), oct = e / (W / PIX) / (rows + 2);
+      const int row = r0 - 1 + ry;
+      dst[v] = oct < 4 ? (ry * (W + 2) + col + 1) * kC16Pitch + oct * 4 : -1;
+      off[v] = oct < 4 && row >= 0 && row < h ? (unsigned)(oct * kOctOf<T> * plane + row * W + col) * (unsigned)sizeof(T) : kOutOfRange;
+    }
+  }
+  // channels past the buffer's last one and rows outside the image fail the range check and read zero
+  __device__ __forceinline__ void load(rsrc_t rs, unsigned plane_bytes) {
+#pragma unroll
+    for (int v = 0; v < ITEMS; ++v) {
+      if (none(v)) break;
+#pragma unroll
+      for (int j = 0; j < kOctOf<T>; ++j) {
+        const int at = (int)(off[v] + j * plane_bytes);
+        if constexpr (sizeof(T) * PIX == 8) {
+          const nhwc_u2 two = __builtin_amdgcn_raw_buffer_load_b64(rs, at, 0, 0);
+          raw[v][2 * j] = two.x, raw[v][2 * j + 1] = two.y;
+        } else if constexpr (sizeof(T) * PIX == 4) {
+          raw[v][j] = __builtin_amdgcn_raw_buffer_load_b32(rs, at, 0, 0);
+        } else {
+          raw[v][j] = __builtin_amdgcn_raw_buffer_load_b16(rs, at, 0, 0);
+        }
+      }
+    }
+  }
+  __device__ __forceinline__ void store(unsigned* tile) const {
+#pragma unroll
+    for (int v = 0; v < ITEMS; ++v) {
+      if (none(v)) break;
+      if (dst[v] < 0) continue;
+#pragma unroll
+      for (int p = 0; p < PIX; ++p) {
+        uint4 o;
+        if constexpr (kPairs<T>) {
+          float f[4];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) f[j] = __uint_as_float(raw[v][j * PIX + p]);
+          const unsigned h01 = pack_bf16(f[0], f[1]), h23 = pack_bf16(f[2], f[3]);
+          o = make_uint4(h01, h23, pack_bf16(f[0] - bf16_lo(h01), f[1] - bf16_hi(h01)),
+                         pack_bf16(f[2] - bf16_lo(h23), f[3] - bf16_hi(h23)));
+        } else {
+          // the p-th halves of two words side by side
+          constexpr unsigned kLow = 0x05040100u, kHigh = 0x07060302u;
+          const unsigned sel = p == 0 ? kLow : kHigh;
+          o = make_uint4(__builtin_amdgcn_perm(raw[v][1], raw[v][0], sel), __builtin_amdgcn_perm(raw[v][3], raw[v][2], sel),
+                         __builtin_amdgcn_perm(raw[v][5], raw[v][4], sel), __builtin_amdgcn_perm(raw[v][7], raw[v][6], sel));
+        }
+        *reinterpret_cast<uint4*>(tile + dst[v] + p * kC16Pitch) = o;
+      }
+    }
+  }
+};
+
 // wp[t][chunk][block][part][lane] = the lane's eight operand elements of A_t, rows 16 block + lane % 16, zeros past
 // the tensor.  16-bit tensors (one part): k = 32 chunk + 8 (lane / 16) .. + 7.  float32 (parts hi, lo): the part
 // of k = 16 chunk + 4 (lane / 16) .. + 3, twice.  weight is [O][C][3][3]; forward: rows = O, k = C; transposed:
@@ -137,7 +209,10 @@ __global__ void conv16_pack_kernel(const T* __restrict__ weight, int O, int C, i
 // in [batch][kin][h][W] -> out [batch][mout][h][W]; wp as packed above with `chunks` = ceil(kin / 32) and
 // `blocks` = ceil(mout / 16); bias [mout] or null.
 // grid = (image, row tile, walk of MTB row blocks)
-template <typename T, int W, int MTB>
+// The chunks' loads are a chunk ahead of the products: without that a workgroup waited for them in every chunk, and on
+// 28 x 28 planes there is one workgroup per CU or less to hide it.  (Forward, us, without / with: bfloat16 N=128 C=192
+// 28x28 52 / 37, N=64 C=144 56x56 52 / 38, float32 of that shape 99 / 89.)
+template <typename T, int W, int MTB, bool WIDE>
 __global__ __launch_bounds__(kC16Block, 2) void conv16_kernel(int batch, int kin, int mout, int h, int tiles, int chunks,
                                                               int blocks, const T* __restrict__ in,
                                                               const uint4* __restrict__ wp, const T* __restrict__ bias,
@@ -168,6 +243,14 @@ __global__ __launch_bounds__(kC16Block, 2) void conv16_kernel(int batch, int kin
   const int live_groups = (rows * W + 15) / 16;
   for (int e = threadIdx.x; e < (rows + 2) * RS * kC16Pitch; e += kC16Block) tile[e] = 0u;  // the padding stays zero
 
+  // Three row blocks -- the input gradient, one chunk or two -- on small planes: octet by octet, which takes the fewest
+  // registers (14 x 14 bfloat16, N=128 C=576: 32 us, through the register stage 39); on wide rows the stage without the
+  // chunk ahead, as with a pixel per item, whose registers would not hold it.
+  constexpr bool DIRECT = MTB >= 3 && W <= 14, AHEAD = MTB < 3 && (WIDE || W == 7);
+  constexpr int kItems = DIRECT ? 1 : ((TH + 2) * 4 * (W / (WIDE ? 2 : 1)) + kC16Block - 1) / kC16Block;
+  Stage16<T, W, kItems, WIDE> stage;
+  if (!DIRECT) stage.place(rows, r0, h, plane);
+
   // word index of the lane's B operand for each of its pixel groups (tap shifts are immediates)
   int bword[kC16Gpw];
 #pragma unroll
@@ -183,11 +266,16 @@ __global__ __launch_bounds__(kC16Block, 2) void conv16_kernel(int batch, int kin
 #pragma unroll
       for (int m = 0; m < MTB; ++m) acc[i][m] = c16f4{0.f, 0.f, 0.f, 0.f};
 
+    // one buffer over the chunk's planes
+    auto load = [&](int ch) {
+      const int kc = min(kChunkOf<T>, kin - ch * kChunkOf<T>);
+      stage.load(plane_rsrc(in + ((size_t)n * kin + (size_t)ch * kChunkOf<T>) * plane, kc * plane), (unsigned)plane * (unsigned)sizeof(T));
+    };
+    if (AHEAD && ch_lo < ch_hi) load(ch_lo);
     for (int ch = ch_lo; ch < ch_hi; ++ch) {
-      {
-        __syncthreads();  // the previous chunk's reads are done
-        // one buffer over the chunk's planes: channels past the tensor and rows outside the image fail
-        // the range check and read zero
+      if (!AHEAD && !DIRECT) load(ch);
+      __syncthreads();  // the previous chunk's reads are done
+      if constexpr (DIRECT) {
         const int kc = min(kChunkOf<T>, kin - ch * kChunkOf<T>);
         const rsrc_t rs = plane_rsrc(in + ((size_t)n * kin + (size_t)ch * kChunkOf<T>) * plane, kc * plane);
         for (int e = threadIdx.x; e < (rows + 2) * 4 * W; e += kC16Block) {
@@ -196,8 +284,11 @@ __global__ __launch_bounds__(kC16Block, 2) void conv16_kernel(int batch, int kin
           *reinterpret_cast<uint4*>(tile + (ry * RS + col + 1) * kC16Pitch + oct * 4) = load_octet<T>(
               rs, row >= 0 && row < h, (unsigned)(oct * kOctOf<T> * plane + row * W + col), (unsigned)plane);
         }
-        __syncthreads();
+      } else {
+        stage.store(tile);
       }
+      __syncthreads();
+      if (AHEAD && ch + 1 < ch_hi) load(ch + 1);
 #pragma unroll
       for (int t = 0; t < 9; ++t) {
         const int shift = ((t / 3 - 1) * RS + (t % 3 - 1)) * kC16Pitch;
@@ -519,11 +610,12 @@ size_t pack_bytes(int kin, int mout, bool pairs) {
   return (size_t)9 * ceil_div(kin, pairs ? kC16Chunk / 2 : kC16Chunk) * ceil_div(mout, 16) * (pairs ? 2 : 1) * 64 * sizeof(uint4);
 }
 
-// Chunk splits of a pass: enough for about two workgroups per CU, at least four chunks per split
+// Chunk splits of a pass: enough for about two workgroups per CU, at least two chunks per split (float16 N=64 C=192
+// 28x28, 128 (image, tile) items: in one part 34 us, in three 27)
 int conv16_splits(int batch, int kin, int mout, int h, int w, int mtb, bool pairs) {
   const long base = std::max(1L, (long)batch * ceil_div(h, kC16Pix / w) * ceil_div(ceil_div(mout, 16), mtb));
   if (base >= 256) return 1;
-  return (int)std::max<long>(1, std::min<long>((512 + base - 1) / base, ceil_div(kin, pairs ? kC16Chunk / 2 : kC16Chunk) / 4));
+  return (int)std::max<long>(1, std::min<long>((512 + base - 1) / base, ceil_div(kin, pairs ? kC16Chunk / 2 : kC16Chunk) / 2));
 }
 
 template <typename T, int MTB>
@@ -531,13 +623,15 @@ bool launch_conv16(int batch, int kin, int mout, int h, int w, const T* in, cons
                    float* partial, hipStream_t stream) {
   const int chunks = ceil_div(kin, kChunkOf<T>), blocks = ceil_div(mout, 16);
   const int ksplit = conv16_splits(batch, kin, mout, h, w, MTB, kPairs<T>);
+  const bool wide = reinterpret_cast<uintptr_t>(in) % (2 * sizeof(T)) == 0;  // (even widths: every row then is)
 #define DK_C16(WW)                                                                                                     \
   {                                                                                                                    \
     const int tiles = ceil_div(h, Tile16<WW>::TH);                                                                     \
-    const size_t lds = (size_t)Tile16<WW>::POS * kC16Pitch * sizeof(unsigned);                                         \
+    const size_t lds = (size_t)(std::min(Tile16<WW>::TH, h) + 2) * Tile16<WW>::RS * kC16Pitch * sizeof(unsigned);      \
     const long wgs = (long)batch * tiles * ceil_div(blocks, MTB) * ksplit;                                             \
-    conv16_kernel<T, WW, MTB><<<(unsigned)xcd_grid_size(wgs), kC16Block, lds, stream>>>(                               \
-        batch, kin, mout, h, tiles, chunks, blocks, in, wp, bias, out, partial, ksplit);                               \
+    auto kernel = WW % 2 == 0 && wide ? conv16_kernel<T, WW, MTB, WW % 2 == 0> : conv16_kernel<T, WW, MTB, false>;     \
+    kernel<<<(unsigned)xcd_grid_size(wgs), kC16Block, lds, stream>>>(batch, kin, mout, h, tiles, chunks, blocks, in,   \
+                                                                     wp, bias, out, partial, ksplit);                  \
   }
   switch (w) {
     case 7: DK_C16(7) break;

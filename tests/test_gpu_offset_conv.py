@@ -57,6 +57,34 @@ def test_forward_matches_float64_convolution(shape, pairs):
     assert rel_err(got.cpu(), want) < 1e-5
 
 
+@pytest.mark.parametrize("dtype,tol", [(torch.float32, 1e-5), (torch.float16, 2e-3), (torch.bfloat16, 1e-2)])
+@pytest.mark.parametrize("shape", [
+    (2, 80, 5, 7, 18),      # a pixel per staged item, three chunks of 16-bit channels, the last half full
+    (2, 48, 17, 14, 18),    # a plane lower than the tile
+    (1, 96, 33, 28, 18),    # a third tile of one row
+    (2, 48, 9, 56, 16),     # one block of outputs
+    (1, 144, 5, 112, 18),   # five chunks, split between workgroups
+])
+@pytest.mark.parametrize("offset", [0, 1])  # 1: tensors that start between two aligned pairs of elements
+def test_staged_pairs_of_pixels_and_tensors_off_their_alignment(shape, dtype, tol, offset):
+    from deformable_kernels.ops.deform_kernel.functions import offset_conv
+    N, C, H, W, O = shape
+    g = torch.Generator().manual_seed(37)
+    dev = torch.device("cuda:0")
+
+    def tensor(*size, std=1.0):
+        n = torch.Size(size).numel()
+        return (torch.randn(n + offset, generator=g) * std).to(dtype).to(dev)[offset:].view(size)
+
+    x, w, b, gout = tensor(N, C, H, W), tensor(O, C, 3, 3, std=0.05), tensor(O), tensor(N, O, H, W)
+    x.requires_grad_()
+    out = offset_conv(x, w, b, force=True)
+    gx, = torch.autograd.grad(out, x, gout)
+    want, want_gx, _, _ = reference(x, w, b, gout)
+    assert rel_err(out.detach().float().cpu(), want) < tol
+    assert rel_err(gx.float().cpu(), want_gx) < tol
+
+
 @pytest.mark.parametrize("shape", [
     (2, 16, 5, 7, 18), (3, 32, 14, 14, 18), (2, 48, 28, 28, 18), (2, 144, 56, 56, 18), (1, 32, 9, 112, 18),
     (2, 32, 56, 56, 16), (1, 16, 13, 28, 20), (40, 32, 56, 56, 18),   # the last: several items per workgroup
