@@ -3035,6 +3035,7 @@ bool run_deform_grad_filter(const Geo& g, const T* gout, const T* x, const T* of
 template <typename T>
 bool fast_deform_forward(const Geo& g, const T* x, const T* off, const T* rot, const T* filter, T* out,
                          hipStream_t stream) {
+  if (!rot && plain_deform_forward<T>(g, x, off, filter, out, stream)) return true;
 #define CALL(SH, SW) run_deform_forward<T, SH, SW>(g, x, off, rot, filter, out, stream)
   DK_DISPATCH_SCOPE(g, CALL)
 #undef CALL
@@ -3044,6 +3045,7 @@ bool fast_deform_forward(const Geo& g, const T* x, const T* off, const T* rot, c
 template <typename T>
 bool fast_deform_grad_coord(const Geo& g, bool rotation, const T* gout, const T* x, const T* off, const T* rot,
                             const T* filter, T* result, void* ws, hipStream_t stream) {
+  if (!rotation && !rot && plain_deform_grad_offset<T>(g, gout, x, off, filter, result, static_cast<float*>(ws), stream)) return true;
 #define CALL(SH, SW) \
   run_deform_grad_coord<T, SH, SW>(g, rotation, gout, x, off, rot, filter, result, static_cast<float*>(ws), stream)
   DK_DISPATCH_SCOPE(g, CALL)
@@ -3058,7 +3060,8 @@ size_t fast_deform_grad_coord_workspace(const Geo& g, bool rotation) {
   if (!d.ok) d = deform_plan_wide(g, table);
   if (!d.ok) return 0;
   // both lay out chunks * groups * batch planes of 18 * out pixels
-  return (size_t)d.chunks * g.groups * g.batch * 18 * g.out_h * g.out_w * sizeof(float);
+  const size_t bytes = (size_t)d.chunks * g.groups * g.batch * 18 * g.out_h * g.out_w * sizeof(float);
+  return rotation ? bytes : std::max(bytes, plain_deform_grad_offset_workspace(g));  // (the call may come without a rotation tensor)
 }
 
 size_t fast_deform_grad_coords_workspace(const Geo& g) {

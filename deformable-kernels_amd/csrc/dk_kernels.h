@@ -42,6 +42,7 @@ enum TestSwitch : unsigned {
   kNoImagePacked = 1u << 24,    // DK_NO_IMAGE_PACKED    the packed flat-copy kernels of the per-image depthwise convolution on 16-bit tensors (the flat-copy kernels that unpack to fp32 run instead)
   kNoDeformLanes = 1u << 25,    // DK_NO_DEFORM_LANES    the deformable kernels with the lanes along the channels (dk_deform_lanes.hip; those with a pixel per lane run instead)
   kForceDeformLanes = 1u << 26, // DK_FORCE_DEFORM_LANES ... wherever they apply, not only where they are the faster ones
+  kNoDeformPlain = 1u << 27,    // DK_NO_DEFORM_PLAIN    the deformable kernels for calls without a rotation tensor (those that take one run instead)
   kNoOffsetPairs = 1u << 18,    // DK_NO_OFFSET_PAIRS    the offset branch's convolution on float32 tensors as bfloat16 pairs (the fp32 matrix-instruction forward runs instead, the other passes are not offered)
 };
 unsigned test_switches();  // dk_api.hip
@@ -92,6 +93,13 @@ bool fast_local_grad_filter(const Geo& g, const T* gout, const T* x, const T* ro
 template <typename T>
 bool fast_deform_forward(const Geo& g, const T* x, const T* off, const T* rot, const T* filter, T* out,
                          hipStream_t stream);
+// without a rotation tensor (dk_deform_plain.hip); false where those kernels do not apply
+template <typename T>
+bool plain_deform_forward(const Geo& g, const T* x, const T* off, const T* filter, T* out, hipStream_t stream);
+size_t plain_deform_grad_offset_workspace(const Geo& g);
+template <typename T>
+bool plain_deform_grad_offset(const Geo& g, const T* gout, const T* x, const T* off, const T* filter, T* goff, float* ws,
+                              hipStream_t stream);
 size_t fast_deform_grad_input_workspace(const Geo& g);
 template <typename T>
 bool fast_deform_grad_input(const Geo& g, const T* gout, const T* off, const T* rot, const T* filter, T* gin,

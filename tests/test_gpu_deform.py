@@ -404,3 +404,47 @@ def test_grad_input_with_the_lanes_along_the_channels(case, dtype):
         assert mixed_err(gin.cpu(), want) < 1e-5
     else:
         assert rel_err(gin.float().cpu(), want) < 1e-2
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("case", [
+    (1, 1, 3, 4, 3, (4, 4), 1, 1, 1, 1, 0.0, 1.0),       # one channel, one wave that is not full
+    (3, 9, 7, 7, 3, (3, 3), 1, 1, 1, 1, 0.0, 2.0),       # one channel past a step of eight; whole scope coordinates
+    (2, 35, 21, 24, 3, (5, 5), 1, 1, 1, 1, 0.0, 2.0),    # 504 pixels: eight waves, the last 56 lanes; several chunks
+    (1, 34, 23, 23, 3, (4, 4), 1, 2, 2, 2, 0.0, 3.0),    # 529 pixels: two tiles; two groups of 17 channels, dilation
+    (1, 20, 31, 40, 3, (4, 4), 2, 1, 1, 1, 0.0, 9.0),    # stride 2, most samples outside the image
+    (1, 6, 8, 120, 3, (4, 4), 4, 1, 1, 1, 0.0, 2.0),     # sixteen inputs per output: threads that only stage
+    (1, 10, 57, 60, 3, (4, 4), 1, 1, 1, 1, 0.0, 2.0),    # one workgroup of 14 waves per CU, four staging passes
+])
+def test_without_a_rotation_tensor_on_the_kernels_of_nine_weights(case, dtype):
+    from deformable_kernels.ops.deform_kernel.functions import deform_sample_depthwise
+    N, C, H, W, k, S, s, p, d, G, rs, os_ = case
+    x, wt, rot, off, gout, cfg = make_deform(N, C, H, W, k, S, s, p, d, G, rs, os_, seed=8, dtype=dtype)
+    rot.zero_()
+    dev = torch.device("cuda:0")
+    xg, og, wg = [t.to(dev).requires_grad_() for t in (x, off, wt)]
+    out = deform_sample_depthwise(xg, og, None, wg, cfg["kernel_size"], cfg["stride"], cfg["padding"], cfg["dilation"], G)
+    got = [out.detach()] + list(torch.autograd.grad(out, [xg, og, wg], gout.to(dev)))
+    inputs = (x, wt, rot, off, gout, cfg)
+    o32, o64 = _oracle(inputs, np.float32), _oracle(inputs, np.float64)
+    if dtype == torch.float32:
+        got.insert(3, torch.from_numpy(o64[3]))  # no rotation gradient here
+        assert_fp32_parity([t.cpu() for t in got], o32, o64)
+    else:
+        for g, want in zip(got, (o32[0], o32[1], o32[2], o32[4])):
+            assert rel_err(g.float().cpu(), want) < 1e-2
+
+
+@pytest.mark.parametrize("poison", [float("inf"), float("nan")])
+def test_without_a_rotation_tensor_a_tap_outside_the_image_meets_no_weight(poison):
+    """A channel's weights that are not finite reach the pixels whose taps sample the image, and no others."""
+    from deformable_kernels.ops.deform_kernel.functions import deform_sample_depthwise
+    g = torch.Generator().manual_seed(3)
+    x, wt, off = torch.randn(1, 12, 9, 9, generator=g), torch.randn(12, 1, 4, 4, generator=g), torch.zeros(1, 18, 9, 9)
+    wt[5] = poison
+    off[..., :4, :] = 100.0  # the pixels of the first rows sample nothing
+    xg, og, wg = [t.cuda().requires_grad_() for t in (x, off, wt)]
+    out = deform_sample_depthwise(xg, og, None, wg, (3, 3), (1, 1), (1, 1), (1, 1), 1)
+    goff, = torch.autograd.grad(out, og, torch.ones_like(out))
+    assert (out[:, :, :4] == 0).all() and (goff[:, :, :4] == 0).all()
+    assert not torch.isfinite(out[:, 5, 4:]).any() and torch.isfinite(out[:, 6:, 4:]).all()
