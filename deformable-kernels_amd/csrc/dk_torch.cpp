@@ -103,8 +103,12 @@ struct OpNode : Node {
 };
 
 // Runs `forward` without recording and hooks the node that `save` fills to its result if an input requires grad.
+// An input with a forward-mode tangent is refused: the kernels have no such derivative, and the result would lose it.
 template <typename N, typename Forward, typename Save>
 Tensor record(std::initializer_list<const Tensor*> inputs, Forward&& forward, Save&& save) {
+  for (const Tensor* t : inputs)
+    TORCH_CHECK_NOT_IMPLEMENTED(!t->defined() || !t->_fw_grad(0).defined(),
+                                "deformable-kernel operators have no forward-mode derivative (no jvp)");
   bool tracked = false;
   if (at::GradMode::is_enabled())
     for (const Tensor* t : inputs) tracked = tracked || (t->defined() && t->requires_grad());

@@ -385,3 +385,24 @@ def test_c_abi_filter_gradient_of_an_empty_batch_is_written_as_zeros(deform, sha
     torch.cuda.synchronize()
     assert rc == 0
     assert torch.count_nonzero(gw).item() == 0 and torch.isfinite(gw).all()
+
+
+def test_forward_mode_and_second_derivatives_are_refused():
+    """The operators have neither: asking raises, instead of a result without its tangent."""
+    from torch.autograd import forward_ad
+    from deformable_kernels.ops.deform_kernel.functions import nd_linear_sample, sample_depthwise
+    x, wt, rot, gout, cfg = make_local(1, 16, 9, 9, 3, (4, 4), 1, 1, 1, 1, 0.5, seed=0)
+    x, wt, rot, gout = [t.cuda() for t in (x, wt, rot, gout)]
+    args = (cfg["kernel_size"], cfg["stride"], cfg["padding"], cfg["dilation"], cfg["groups"])
+    with forward_ad.dual_level():
+        for i in range(3):
+            given = [x, rot, wt]
+            given[i] = forward_ad.make_dual(given[i], torch.ones_like(given[i]))
+            with pytest.raises(NotImplementedError):
+                sample_depthwise(*given, *args)
+        with pytest.raises(NotImplementedError):
+            nd_linear_sample(forward_ad.make_dual(wt[:, 0], torch.ones_like(wt[:, 0])), torch.zeros(5, 2, device="cuda"))
+    xg = x.clone().requires_grad_()
+    gin, = torch.autograd.grad(sample_depthwise(xg, rot, wt, *args), xg, gout.requires_grad_(), create_graph=True)
+    with pytest.raises(RuntimeError, match="once_differentiable"):
+        gin.sum().backward()
