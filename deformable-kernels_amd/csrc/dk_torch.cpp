@@ -13,6 +13,7 @@
 #include <torch/extension.h>
 
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/hip/HIPStream.h>
 
 #include <array>
@@ -104,8 +105,12 @@ struct OpNode : Node {
 
 // Runs `forward` without recording and hooks the node that `save` fills to its result if an input requires grad.
 // An input with a forward-mode tangent is refused: the kernels have no such derivative, and the result would lose it.
+// So is a call inside a functorch transform (vmap, grad, jvp, functionalize): the node would hang on the transform's
+// wrapper of the result, and what the transform hands back has lost it.
 template <typename N, typename Forward, typename Save>
 Tensor record(std::initializer_list<const Tensor*> inputs, Forward&& forward, Save&& save) {
+  TORCH_CHECK_NOT_IMPLEMENTED(!c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode),
+                              "deformable-kernel operators do not run inside functorch transforms (torch.func, torch.vmap)");
   for (const Tensor* t : inputs)
     TORCH_CHECK_NOT_IMPLEMENTED(!t->defined() || !t->_fw_grad(0).defined(),
                                 "deformable-kernel operators have no forward-mode derivative (no jvp)");
