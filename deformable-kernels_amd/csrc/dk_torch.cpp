@@ -669,13 +669,16 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
       }
     });
   });
-  m.def("sample_depthwise", &sample_depthwise);
-  m.def("deform_sample_depthwise", &deform_sample_depthwise);
-  m.def("nd_linear_sample", &nd_linear_sample);
-  m.def("offset_conv", &offset_conv);
+  // The operators run without the interpreter lock, as the framework's own do: a call may wait in the allocator, load a
+  // code object or search for a convolution.  (Saved-tensor hooks and Python dispatch take the lock themselves.)
+  const py::call_guard<py::gil_scoped_release> unlocked;
+  m.def("sample_depthwise", &sample_depthwise, unlocked);
+  m.def("deform_sample_depthwise", &deform_sample_depthwise, unlocked);
+  m.def("nd_linear_sample", &nd_linear_sample, unlocked);
+  m.def("offset_conv", &offset_conv, unlocked);
   m.def("offset_conv_supported", &offset_conv_supported);
-  m.def("image_depthwise_conv", &image_depthwise_conv);
-  m.def("global_deform_conv", &global_deform_conv);
+  m.def("image_depthwise_conv", &image_depthwise_conv, unlocked);
+  m.def("global_deform_conv", &global_deform_conv, unlocked);
   m.def("global_deform_conv_supported", &global_deform_conv_supported);
   m.attr("conv_desc_size") = sizeof(dk_conv_desc);
 }

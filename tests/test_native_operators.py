@@ -1,8 +1,12 @@
 """The native operators' host path (csrc/dk_torch.cpp) where it meets the framework: transforms, threads, errors, saved
 tensors.  What can be shown without a GPU runs on fake tensors or CPU tensors."""
+import threading
+import time
+
 import pytest
 import torch
 
+from deformable_kernels.ops.deform_kernel import _lib
 from deformable_kernels.ops.deform_kernel.functions import offset_conv
 
 
@@ -20,3 +24,32 @@ def test_offset_conv_inside_vmap_is_refused_not_returned_without_its_graph(wrapp
         with pytest.raises(NotImplementedError, match="functorch"):
             calls[wrapped]()
         assert offset_conv(x[0], w).requires_grad
+
+
+def test_other_python_threads_run_during_an_operator_call():
+    # CPU tensors: the native entry hands them to the framework's convolution, here some 100 ms of it and more
+    x, w = torch.randn(1, 64, 64, 64), torch.randn(18, 64, 3, 3)
+    call = lambda: _lib.native().offset_conv(x, w, None, (1, 1), (1, 1), (1, 1), False)
+    call()
+    t0 = time.perf_counter()
+    call()
+    copies = max(1, int(0.3 / (time.perf_counter() - t0)))
+    x = x.expand(copies, -1, -1, -1)
+    ticks, stop = [0], threading.Event()
+
+    def tick():
+        while not stop.is_set():
+            ticks[0] += 1
+            time.sleep(0.001)
+
+    thread = threading.Thread(target=tick)
+    thread.start()
+    try:
+        before = ticks[0]
+        call()
+        during = ticks[0] - before
+    finally:
+        stop.set()
+        thread.join()
+    # a call that held the interpreter lock would let through a tick or two around its edges
+    assert during >= 10, during
