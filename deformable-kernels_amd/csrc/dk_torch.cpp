@@ -6,6 +6,7 @@
 // Counterparts of the reference's functions/filter_sample_depthwise.py:19-206 and functions/nd_linear_sample.py:18-62
 // (the two extension modules' pybind functions are the C ABI's); the Python files of the same names keep the signatures.
 // Saved tensors go through SavedVariable (version checks, saved-tensor hooks); nothing else is kept from a forward call.
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/function.h>
 #include <torch/csrc/autograd/functions/basic_ops.h>
 #include <torch/csrc/autograd/functions/utils.h>
@@ -32,9 +33,13 @@ using torch::autograd::variable_list;
 using Pair = std::array<int64_t, 2>;
 using OptTensor = std::optional<Tensor>;
 
+// A failing native call; the user gets it as the package's DkError (a RuntimeError, handed in by _lib.py): from a forward
+// call by the module's exception translator, from a backward node by OpNode::apply.
 struct DkFailure : std::runtime_error {
   using std::runtime_error::runtime_error;
 };
+PyObject* g_error_class = nullptr;  // read with the interpreter lock held
+void set_python_error(const DkFailure& e) { PyErr_SetString(g_error_class ? g_error_class : PyExc_RuntimeError, e.what()); }
 
 void check(int status, const char* what) {
   if (status != DK_OK)
@@ -91,7 +96,16 @@ struct OpNode : Node {
       at::AutoGradMode no_grad(false);
       c10::OptionalDeviceGuard device;
       if (grads[0].defined()) device.reset_device(grads[0].device());
-      results = grads[0].defined() ? backward(grads) : variable_list(num_outputs());
+      try {
+        results = grads[0].defined() ? backward(grads) : variable_list(num_outputs());
+      } catch (const DkFailure& e) {
+        // the engine hands a Python error through as it is, and anything else as a RuntimeError
+        py::gil_scoped_acquire gil;
+        set_python_error(e);
+        python_error error;
+        error.persist();
+        throw error;
+      }
     }
     if (!at::GradMode::is_enabled() || !grads[0].defined() || !grads[0].requires_grad()) return results;
     for (Tensor& t : results)
@@ -656,18 +670,13 @@ Tensor global_deform_conv(const Tensor& input, const Tensor& weight, const Tenso
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
-  // a failing native call raises the package's DkError (a RuntimeError; the class is handed in by _lib.py)
-  m.def("set_error_class", [](py::object cls) {
-    static py::object error;
-    error = std::move(cls);
-    error.inc_ref();  // outlives the interpreter's shutdown order
-    py::register_exception_translator([](std::exception_ptr p) {
-      try {
-        if (p) std::rethrow_exception(p);
-      } catch (const DkFailure& e) {
-        PyErr_SetString(error.ptr(), e.what());
-      }
-    });
+  m.def("set_error_class", [](py::object cls) { g_error_class = cls.release().ptr(); });  // (never given back: outlives the shutdown order)
+  py::register_exception_translator([](std::exception_ptr p) {
+    try {
+      if (p) std::rethrow_exception(p);
+    } catch (const DkFailure& e) {
+      set_python_error(e);
+    }
   });
   // The operators run without the interpreter lock, as the framework's own do: a call may wait in the allocator, load a
   // code object or search for a convolution.  (Saved-tensor hooks and Python dispatch take the lock themselves.)

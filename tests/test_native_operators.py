@@ -7,7 +7,7 @@ import pytest
 import torch
 
 from deformable_kernels.ops.deform_kernel import _lib
-from deformable_kernels.ops.deform_kernel.functions import offset_conv
+from deformable_kernels.ops.deform_kernel.functions import image_depthwise_conv, offset_conv
 
 
 @pytest.mark.parametrize("wrapped", ["input", "weight", "neither"])
@@ -53,3 +53,19 @@ def test_other_python_threads_run_during_an_operator_call():
         thread.join()
     # a call that held the interpreter lock would let through a tick or two around its edges
     assert during >= 10, during
+
+
+@pytest.mark.gpu
+def test_failing_native_calls_raise_the_packages_error_forward_and_backward():
+    # a kernel tensor whose (unused) batch stride is past what the library's 32-bit offsets take: refused on the host
+    bad = torch.empty_strided((1, 8, 3, 3), (1 << 31, 1, 24, 8), device="cuda").fill_(0.5)
+    x = torch.randn(1, 8, 12, 12, device="cuda", requires_grad=True)
+    with pytest.raises(_lib.DkError, match="forward failed"):
+        image_depthwise_conv(x, bad, 1, 1)
+    good = bad.contiguous()
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: bad if t.shape == bad.shape else t):
+        out = image_depthwise_conv(x, good, 1, 1)
+    with pytest.raises(_lib.DkError, match="grad input failed"):
+        out.sum().backward()
+    image_depthwise_conv(x, good, 1, 1).sum().backward()  # and the engine goes on
+    assert x.grad is not None
