@@ -86,7 +86,8 @@ bool channels_last(const Tensor& t) {  // stored channels-last and not also in t
   return t.dim() == 4 && !t.is_contiguous() && t.is_contiguous(at::MemoryFormat::ChannelsLast);
 }
 
-// Base of the backward nodes.  Their results are not differentiable a second time: asking for it raises.
+// Base of the backward nodes.  Their results are not differentiable a second time: asking for it raises.  An undefined
+// upstream gradient stands for zeros, as in a Python Function: the inputs get gradients of zeros.
 struct OpNode : Node {
   virtual variable_list backward(const variable_list& grads) = 0;
   variable_list apply(variable_list&& grads) override {
@@ -94,10 +95,10 @@ struct OpNode : Node {
     variable_list results;
     {
       at::AutoGradMode no_grad(false);
-      c10::OptionalDeviceGuard device;
-      if (grads[0].defined()) device.reset_device(grads[0].device());
+      if (!grads[0].defined()) grads[0] = input_metadata(0).zeros_like();
+      const c10::DeviceGuard device(grads[0].device());
       try {
-        results = grads[0].defined() ? backward(grads) : variable_list(num_outputs());
+        results = backward(grads);
       } catch (const DkFailure& e) {
         // the engine hands a Python error through as it is, and anything else as a RuntimeError
         py::gil_scoped_acquire gil;
@@ -107,7 +108,7 @@ struct OpNode : Node {
         throw error;
       }
     }
-    if (!at::GradMode::is_enabled() || !grads[0].defined() || !grads[0].requires_grad()) return results;
+    if (!at::GradMode::is_enabled() || !grads[0].requires_grad()) return results;
     for (Tensor& t : results)
       if (t.defined()) t = t.detach().requires_grad_();
     return torch::autograd::DelayedError("trying to differentiate twice a function that was marked with @once_differentiable",

@@ -7,7 +7,7 @@ import pytest
 import torch
 
 from deformable_kernels.ops.deform_kernel import _lib
-from deformable_kernels.ops.deform_kernel.functions import image_depthwise_conv, offset_conv
+from deformable_kernels.ops.deform_kernel.functions import image_depthwise_conv, nd_linear_sample, offset_conv
 
 
 @pytest.mark.parametrize("wrapped", ["input", "weight", "neither"])
@@ -69,3 +69,23 @@ def test_failing_native_calls_raise_the_packages_error_forward_and_backward():
         out.sum().backward()
     image_depthwise_conv(x, good, 1, 1).sum().backward()  # and the engine goes on
     assert x.grad is not None
+
+
+class _Dropped(torch.autograd.Function):
+    """Passes its input on, and no gradient back."""
+
+    @staticmethod
+    def forward(ctx, x):
+        return x.clone()
+
+    @staticmethod
+    def backward(ctx, grad):
+        return None
+
+
+@pytest.mark.gpu
+def test_no_gradient_from_above_counts_as_zeros():
+    data = torch.randn(6, 5, 5, device="cuda", requires_grad=True)
+    coord = torch.rand(40, 2, device="cuda").mul_(4).requires_grad_()
+    _Dropped.apply(nd_linear_sample(data, coord)).sum().backward()
+    assert torch.equal(data.grad, torch.zeros_like(data)) and torch.equal(coord.grad, torch.zeros_like(coord))
