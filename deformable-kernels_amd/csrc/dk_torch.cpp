@@ -5,7 +5,8 @@
 //
 // Counterparts of the reference's functions/filter_sample_depthwise.py:19-206 and functions/nd_linear_sample.py:18-62
 // (the two extension modules' pybind functions are the C ABI's); the Python files of the same names keep the signatures.
-// Saved tensors go through SavedVariable (version checks, saved-tensor hooks); nothing else is kept from a forward call.
+// What a forward call keeps for its backward pass goes through SavedVariable (version checks; saved-tensor hooks, which
+// may offload or pack it), except the sampler's order of the points: bytes of the library's own layout.
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/function.h>
 #include <torch/csrc/autograd/functions/basic_ops.h>
@@ -336,7 +337,7 @@ Tensor deform_sample_depthwise(const Tensor& input, const Tensor& offset, const 
 
 struct NdLinearSampleFunctionBackward : OpNode {
   SavedVariable input, coord;
-  Tensor order;  // the points' order by cell, not a differentiable quantity
+  Tensor order;  // the points' order by cell
   dk_nd_desc desc;
   std::string name() const override { return "NdLinearSampleFunctionBackward"; }
   void release_variables() override {
@@ -586,15 +587,16 @@ Tensor image_depthwise_conv(const Tensor& input, const Tensor& weight, const Pai
 
 struct GlobalDeformConvFunctionBackward : OpNode {
   SavedVariable input, weight, fc_weight;
-  Tensor pooled, coord, kernels;  // made by the forward call, reachable from here only
+  SavedVariable saved_pooled, saved_coord, saved_kernels;  // made by the forward call
   dk_conv_desc desc;
   std::string name() const override { return "GlobalDeformConvFunctionBackward"; }
   void release_variables() override {
     input.reset_data(), weight.reset_data(), fc_weight.reset_data();
-    pooled.reset(), coord.reset(), kernels.reset();
+    saved_pooled.reset_data(), saved_coord.reset_data(), saved_kernels.reset_data();
   }
   variable_list backward(const variable_list& grads) override {
     const Tensor x = input.unpack(), w = weight.unpack(), fw = fc_weight.unpack(), g = grads[0].contiguous();
+    const Tensor pooled = saved_pooled.unpack(), coord = saved_coord.unpack(), kernels = saved_kernels.unpack();
     const int64_t c = x.size(1), k = desc.k_h;
     const Strides strides{k * k * c, 1, k * c, c};
     void* const s = stream_of(x);
@@ -663,7 +665,8 @@ Tensor global_deform_conv(const Tensor& input, const Tensor& weight, const Tenso
       },
       [&](GlobalDeformConvFunctionBackward& n) {
         n.input = SavedVariable(x, false), n.weight = SavedVariable(w, false), n.fc_weight = SavedVariable(fw, false);
-        n.pooled = pooled, n.coord = coord, n.kernels = kernels;
+        n.saved_pooled = SavedVariable(pooled, false), n.saved_coord = SavedVariable(coord, false);
+        n.saved_kernels = SavedVariable(kernels, false);
         n.desc = desc;
       });
 }

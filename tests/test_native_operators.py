@@ -6,6 +6,7 @@ import time
 import pytest
 import torch
 
+from deformable_kernels.modules import GlobalDeformKernel2d
 from deformable_kernels.ops.deform_kernel import _lib
 from deformable_kernels.ops.deform_kernel.functions import image_depthwise_conv, nd_linear_sample, offset_conv
 
@@ -89,3 +90,24 @@ def test_no_gradient_from_above_counts_as_zeros():
     coord = torch.rand(40, 2, device="cuda").mul_(4).requires_grad_()
     _Dropped.apply(nd_linear_sample(data, coord)).sum().backward()
     assert torch.equal(data.grad, torch.zeros_like(data)) and torch.equal(coord.grad, torch.zeros_like(coord))
+
+
+@pytest.mark.gpu
+def test_saved_tensor_hooks_see_everything_the_global_layer_keeps():
+    torch.manual_seed(0)
+    layer = GlobalDeformKernel2d((4, 4), 16, 16, 3, padding=1, groups=16).cuda()
+    x = torch.randn(3, 16, 14, 14, device="cuda", requires_grad=True)
+    leaves = [x] + list(layer.parameters())
+    want = torch.autograd.grad(layer(x).square().sum(), leaves)
+    kept = []
+
+    def pack(t):
+        kept.append(tuple(t.shape))
+        return t.cpu()
+
+    with torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t.cuda()):
+        out = layer(x)
+    # the sampled kernels [image, tap, channel], the coordinates before and behind the clamp, the pooled input
+    assert {(3, 9, 16), (2, 3, 9, 2), (3, 16), (3, 16, 14, 14)} <= set(kept), kept
+    for a, b in zip(torch.autograd.grad(out.square().sum(), leaves), want):
+        assert torch.equal(a, b)
