@@ -91,6 +91,12 @@ bool channels_last(const Tensor& t) {  // stored channels-last and not also in t
 // upstream gradient stands for zeros, as in a Python Function: the inputs get gradients of zeros.
 struct OpNode : Node {
   virtual variable_list backward(const variable_list& grads) = 0;
+  virtual void release() = 0;  // gives back what the forward call kept
+  // (one thread's backward pass may end while another's is inside apply on the same graph)
+  void release_variables() override {
+    std::lock_guard<std::mutex> lock(mutex_);
+    release();
+  }
   variable_list apply(variable_list&& grads) override {
     std::lock_guard<std::mutex> lock(mutex_);
     variable_list results;
@@ -209,7 +215,7 @@ struct SampleDepthwiseFunctionBackward : OpNode {
   SavedVariable input, rotation, weight;
   dk_conv_desc desc;
   std::string name() const override { return "SampleDepthwiseFunctionBackward"; }
-  void release_variables() override {
+  void release() override {
     input.reset_data(), rotation.reset_data(), weight.reset_data();
   }
   variable_list backward(const variable_list& grads) override {
@@ -261,7 +267,7 @@ struct DeformableSampleDepthwiseFunctionBackward : OpNode {
   bool has_rotation = false;
   dk_conv_desc desc;
   std::string name() const override { return "DeformableSampleDepthwiseFunctionBackward"; }
-  void release_variables() override {
+  void release() override {
     input.reset_data(), offset.reset_data(), rotation.reset_data(), weight.reset_data();
   }
   variable_list backward(const variable_list& grads) override {
@@ -340,7 +346,7 @@ struct NdLinearSampleFunctionBackward : OpNode {
   Tensor order;  // the points' order by cell
   dk_nd_desc desc;
   std::string name() const override { return "NdLinearSampleFunctionBackward"; }
-  void release_variables() override {
+  void release() override {
     input.reset_data(), coord.reset_data();
     order.reset();
   }
@@ -433,7 +439,7 @@ struct OffsetConvFunctionBackward : OpNode {
   Pair stride, padding, dilation;
   bool native = false, forced = false, has_bias = false;
   std::string name() const override { return "OffsetConvFunctionBackward"; }
-  void release_variables() override {
+  void release() override {
     input.reset_data(), weight.reset_data();
   }
   variable_list backward(const variable_list& grads) override {
@@ -536,7 +542,7 @@ struct ImageDepthwiseConvFunctionBackward : OpNode {
   SavedVariable input, weight;
   dk_conv_desc desc;
   std::string name() const override { return "ImageDepthwiseConvFunctionBackward"; }
-  void release_variables() override {
+  void release() override {
     input.reset_data(), weight.reset_data();
   }
   variable_list backward(const variable_list& grads) override {
@@ -590,7 +596,7 @@ struct GlobalDeformConvFunctionBackward : OpNode {
   SavedVariable saved_pooled, saved_coord, saved_kernels;  // made by the forward call
   dk_conv_desc desc;
   std::string name() const override { return "GlobalDeformConvFunctionBackward"; }
-  void release_variables() override {
+  void release() override {
     input.reset_data(), weight.reset_data(), fc_weight.reset_data();
     saved_pooled.reset_data(), saved_coord.reset_data(), saved_kernels.reset_data();
   }
