@@ -28,8 +28,14 @@ from .. import _lib
 __all__ = ['offset_conv', 'offset_conv_supported']
 
 
+_NATIVE_DTYPES = (torch.float32, torch.float16, torch.bfloat16)
+
+
 def _pair(v):
-    return tuple(int(e) for e in v) if isinstance(v, (tuple, list)) else (int(v), int(v))
+    """Both dimensions' value of a convolution argument: a number, a pair, or (as F.conv2d takes) one number in a list."""
+    if isinstance(v, (tuple, list)):
+        return tuple(int(e) for e in v) if len(v) != 1 else (int(v[0]), int(v[0]))
+    return int(v), int(v)
 
 
 def offset_conv_supported(input, weight, bias, stride, padding, dilation, worthwhile=False):
@@ -44,6 +50,7 @@ def offset_conv_supported(input, weight, bias, stride, padding, dilation, worthw
 def offset_conv(input, weight, bias=None, stride=1, padding=1, dilation=1, force=False):
     """``F.conv2d(input, weight, bias, stride, padding, dilation)`` for the offset branch (see the
     module docstring for what runs where)."""
-    if not input.is_cuda or torch.is_autocast_enabled():
+    if (not input.is_cuda or torch.is_autocast_enabled()
+            or isinstance(padding, str) and input.dtype not in _NATIVE_DTYPES):
         return F.conv2d(input, weight, bias, stride, padding, dilation)
     return _lib.native().offset_conv(input, weight, bias, _pair(stride), _pair(padding), _pair(dilation), bool(force))

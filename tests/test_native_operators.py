@@ -27,6 +27,15 @@ def test_offset_conv_inside_vmap_is_refused_not_returned_without_its_graph(wrapp
         assert offset_conv(x[0], w).requires_grad
 
 
+def test_offset_conv_takes_the_argument_forms_of_the_frameworks_convolution():
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    with FakeTensorMode():
+        x, w = torch.empty(2, 8, 29, 29, device="cuda"), torch.empty(18, 8, 3, 3, device="cuda")
+        assert offset_conv(x, w, None, (1,), [1], (1,)).shape == (2, 18, 29, 29)  # one number in a list
+        assert offset_conv(x.double(), w.double(), None, (2,), (1,), 1).shape == (2, 18, 15, 15)
+        assert offset_conv(x.double(), w.double(), None, 1, "same", 1).shape == (2, 18, 29, 29)  # a named padding: float64
+
+
 def test_other_python_threads_run_during_an_operator_call():
     # CPU tensors: the native entry hands them to the framework's convolution, here some 100 ms of it and more
     x, w = torch.randn(1, 64, 64, 64), torch.randn(18, 64, 3, 3)
