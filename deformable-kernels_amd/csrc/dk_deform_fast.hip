@@ -43,7 +43,8 @@ constexpr int K9 = 9;
 
 // Where tap t of the lane's pixel samples the padded image plane: index of the top-left corner
 // and the fractional position.  A sample outside (-1, H) x (-1, W) (K.cu:500), or a lane without
-// a pixel, points at the padding corner with lh = lw = 0 and so reads 0.
+// a pixel, points at the last column of the top padding row (RS - 1, rows of W + 2) with lh = lw = 0: its four
+// corners are padding, so that it reads 0 also where the plane holds an infinity or a NaN.
 struct ImgTap {
   int pidx;
   float lh, lw;
@@ -75,7 +76,7 @@ __device__ __forceinline__ void deform_taps(const Geo& g, const T* off, const T*
     const float w = float(ow * g.stride_w - g.pad_w + f_w * g.dil_w) + buf_ld(ro, o + step, off);
     const bool hit = live && (h > -1.f) && (w > -1.f) && (h < float(g.in_h)) && (w < float(g.in_w));
     const float hf = floorf(h), wf = floorf(w);
-    it[t].pidx = hit ? (static_cast<int>(hf) + 1) * RS + static_cast<int>(wf) + 1 : 0;
+    it[t].pidx = hit ? (static_cast<int>(hf) + 1) * RS + static_cast<int>(wf) + 1 : RS - 1;
     it[t].lh = hit ? h - hf : 0.f;
     it[t].lw = hit ? w - wf : 0.f;
     const float sh = scope_coord<float>(g, f_h, buf_ld(rr, o, rot), g.centre_h);
@@ -1802,7 +1803,7 @@ __global__ __launch_bounds__(kGfBlock, 1) void deform_grad_filter_mfma_kernel(
         const float w = float(ow * g.stride_w - g.pad_w + f_w * g.dil_w) + buf_ld(ro, o + step, off);
         const bool hit = live && (h > -1.f) && (w > -1.f) && (h < float(H)) && (w < float(W));
         const float hf = floorf(h), wf = floorf(w);
-        const int pidx = hit ? (static_cast<int>(hf) + 1) * RS + static_cast<int>(wf) + 1 : 0;
+        const int pidx = hit ? (static_cast<int>(hf) + 1) * RS + static_cast<int>(wf) + 1 : RS - 1;
         const float sh = scope_coord<float>(g, f_h, buf_ld(rr, o, rot), g.centre_h);
         const float sw = scope_coord<float>(g, f_w, buf_ld(rr, o + step, rot), g.centre_w);
         const bool in = hit && (sh > -1.f) && (sw > -1.f) && (sh < float(SH)) && (sw < float(SW));

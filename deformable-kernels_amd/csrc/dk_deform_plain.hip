@@ -150,7 +150,9 @@ __global__ __launch_bounds__(kPlThreads) void deform_plain_kernel(
     w = float(ow * g.stride_w - g.pad_w + t % 3 * g.dil_w) + buf_ld(roff, o + (unsigned)out_plane * (unsigned)sizeof(T), off);
     return live && (h > -1.f) && (w > -1.f) && (h < float(H)) && (w < float(W));
   };
-  int at[K9];  // byte offset of the sample's top-left corner; a tap outside the image: the padding corner, four zeros
+  // byte offset of the sample's top-left corner; a tap outside the image: the last column of the top padding row, whose
+  // four corners -- that position, the next row's first and last, the one after's first -- are all padding
+  int at[K9];
   float lh[GRAD ? 1 : K9], lw[GRAD ? 1 : K9];
   unsigned hits = 0u;
 #pragma unroll
@@ -158,7 +160,7 @@ __global__ __launch_bounds__(kPlThreads) void deform_plain_kernel(
     float h, w;
     const bool hit = sample(t, h, w);
     const float hf = floorf(h), wf = floorf(w);
-    at[t] = hit ? ((static_cast<int>(hf) + 1) * RS + static_cast<int>(wf) + 1) * kPlPos : 0;
+    at[t] = hit ? ((static_cast<int>(hf) + 1) * RS + static_cast<int>(wf) + 1) * kPlPos : (W + 1) * kPlPos;
     if constexpr (!GRAD) lh[t] = hit ? h - hf : 0.f, lw[t] = hit ? w - wf : 0.f;
     hits |= hit ? 1u << t : 0u;
   }

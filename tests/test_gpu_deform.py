@@ -448,3 +448,27 @@ def test_without_a_rotation_tensor_a_tap_outside_the_image_meets_no_weight(poiso
     goff, = torch.autograd.grad(out, og, torch.ones_like(out))
     assert (out[:, :, :4] == 0).all() and (goff[:, :, :4] == 0).all()
     assert not torch.isfinite(out[:, 5, 4:]).any() and torch.isfinite(out[:, 6:, 4:]).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rotation", [True, False])
+@pytest.mark.parametrize("shape,stride,off_std", [
+    ((2, 10, 9, 11), 1, 4.0),    # whole planes, interleaved
+    ((1, 6, 30, 33), 2, 12.0),   # most samples outside the image
+    ((1, 5, 70, 66), 1, 4.0),    # wider than 64 columns: windows of rows
+])
+@pytest.mark.parametrize("poison", [float("inf"), float("nan")])
+def test_a_tap_outside_the_image_does_not_read_the_first_pixel(shape, stride, off_std, rotation, dtype, poison):
+    """Taps that sample nothing are skipped (K.cu:500): a non-finite first pixel of a plane reaches the outputs whose
+    samples touch it, and no others."""
+    from deformable_kernels.ops.deform_kernel.functions import deform_sample_depthwise
+    N, C, H, W = shape
+    x, wt, rot, off, gout, cfg = make_deform(N, C, H, W, 3, (4, 4), stride, 1, 1, 1, 0.5, off_std, seed=9, dtype=dtype)
+    rot = rot.clamp(-1, 1) if rotation else torch.zeros_like(rot)  # (inside the scope band)
+    x[:, 1::2, 0, 0] = poison
+    want = orc.deform_sample_depthwise_forward(*[t.float().numpy() for t in (x, off, rot, wt)], **cfg)
+    got = deform_sample_depthwise(*[t.cuda() if t is not None else None for t in (x, off, rot if rotation else None, wt)],
+                                  cfg["kernel_size"], cfg["stride"], cfg["padding"], cfg["dilation"], 1)
+    touched = ~np.isfinite(want)
+    assert touched.any() and not touched.all()
+    assert np.array_equal(~torch.isfinite(got).cpu().numpy(), touched)
