@@ -371,16 +371,17 @@ def test_both_coordinate_gradients_from_one_call_equal_the_separate_entry_points
     assert torch.equal(goff, goff2) and torch.equal(grot, grot2)
 
 
-@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("case", [
+LANES_CASES = [
     (1, 1, 2, 3, 3, (4, 4), 1, 1, 1, 1, 0.5, 1.0),       # one channel, one unit of 16 pixels that is not full
     (2, 33, 9, 11, 3, (3, 3), 1, 1, 1, 1, 0.7, 2.0),     # 99 pixels: no group of four is aligned; a second chunk of one channel
     (1, 66, 16, 12, 3, (5, 5), 1, 1, 1, 2, 1.0, 3.0),    # two groups of 33 channels, aligned groups of four
     (1, 20, 28, 28, 3, (4, 4), 2, 1, 1, 1, 0.5, 6.0),    # stride 2, many samples outside the image
     (1, 40, 30, 31, 3, (4, 4), 1, 2, 2, 1, 0.7, 2.0),    # dilation; the largest plane whose sums fit LDS
     (1, 34, 14, 14, 3, (4, 4), 1, 1, 1, 1, 0.5, None),   # every sample in one input cell: one channel per 64-bit sum
-])
-def test_grad_input_with_the_lanes_along_the_channels(case, dtype):
+]
+
+
+def _grad_input_with_the_lanes_along_the_channels(case, dtype, rotation=True, clip=None):
     from deformable_kernels.ops.deform_kernel import _lib
     pile = case[-1] is None
     N, C, H, W, k, S, s, p, d, G, rs, os_ = case[:-1] + (0.0,) if pile else case
@@ -389,21 +390,43 @@ def test_grad_input_with_the_lanes_along_the_channels(case, dtype):
         oh, ow = torch.meshgrid(torch.arange(H), torch.arange(W), indexing="ij")
         for t in range(9):
             off[:, 2 * t], off[:, 2 * t + 1] = 6.25 - (oh - 1 + t // 3), 7.5 - (ow - 1 + t % 3)
+    if not rotation:
+        rot.zero_()
     dev = torch.device("cuda:0")
     wg, rg, og, gg = [t.to(dev) for t in (wt, rot, off, gout)]
+    if clip is not None:
+        rot = clipped_rotation(rot, clip, cfg["kernel_size"], S, G)[0]
     gin = torch.full((N, C, H, W), float("nan"), device=dev, dtype=dtype)
     L, P = _lib.lib(), _lib.ptr
-    desc = _lib.conv_desc(gin, wg, cfg["kernel_size"], cfg["stride"], cfg["padding"], cfg["dilation"], G)
+    desc = _lib.conv_desc(gin, wg, cfg["kernel_size"], cfg["stride"], cfg["padding"], cfg["dilation"], G,
+                          clip)
     ws, nbytes = _lib.workspace(L.dk_deformable_sample_depthwise_backward_data_workspace(desc), dev)
     with _lib.test_switches("DK_FORCE_DEFORM_LANES"):
         _lib.check(L.dk_deformable_sample_depthwise_backward_data(
-            desc, P(gg), P(og), P(rg), P(wg), P(gin), P(ws), nbytes, _lib.stream_ptr(gin)), "grad input")
+            desc, P(gg), P(og), P(rg if rotation else None), P(wg), P(gin), P(ws), nbytes, _lib.stream_ptr(gin)), "grad input")
     want = _oracle((x, wt, rot, off, gout, cfg), np.float64)[1]
     if dtype == torch.float32:
         # rounding of each term on a grid of 2^-24 of the largest possible one, and of the positions
         assert mixed_err(gin.cpu(), want) < 1e-5
     else:
         assert rel_err(gin.float().cpu(), want) < 1e-2
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("case", LANES_CASES)
+def test_grad_input_with_the_lanes_along_the_channels(case, dtype):
+    _grad_input_with_the_lanes_along_the_channels(case, dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("case", LANES_CASES)
+def test_grad_input_with_the_lanes_along_the_channels_without_a_rotation_tensor(case, dtype):
+    _grad_input_with_the_lanes_along_the_channels(case, dtype, rotation=False)
+
+
+@pytest.mark.parametrize("clip", [(0.25, 0.75), (-1.5, -0.75)])
+def test_grad_input_with_the_lanes_along_the_channels_at_a_clipped_zero_rotation(clip):
+    _grad_input_with_the_lanes_along_the_channels(LANES_CASES[2], torch.float32, rotation=False, clip=clip)
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
