@@ -49,9 +49,11 @@ def _plain_conv(conv):
 
 
 def _plain_linear(fc):
-    """Whether its parameters stand for the linear layer: no hooks on it, and not replaced by something else."""
+    """Whether its parameters stand for the linear layer: no hooks on it or on all modules, and neither the layer nor its
+    ``forward`` replaced by something else."""
     hooks = (fc._forward_hooks, fc._forward_pre_hooks, fc._backward_hooks, getattr(fc, "_backward_pre_hooks", {}))
-    return type(fc) is nn.Linear and not any(len(h) for h in hooks)
+    return (type(fc) is nn.Linear and not any(len(h) for h in hooks) and "forward" not in fc.__dict__
+            and not nn.modules.module._has_any_global_hook())
 
 
 class GlobalDeformKernel2d(nn.Module):

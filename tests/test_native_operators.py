@@ -120,3 +120,22 @@ def test_saved_tensor_hooks_see_everything_the_global_layer_keeps():
     assert {(3, 9, 16), (2, 3, 9, 2), (3, 16), (3, 16, 14, 14)} <= set(kept), kept
     for a, b in zip(torch.autograd.grad(out.square().sum(), leaves), want):
         assert torch.equal(a, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("how", ["forward replaced", "hook on every module"])
+def test_the_global_layer_calls_a_linear_layer_that_is_more_than_its_parameters(how):
+    torch.manual_seed(0)
+    layer = GlobalDeformKernel2d((4, 4), 16, 16, 3, padding=1, groups=16).cuda()
+    x, seen = torch.randn(3, 16, 14, 14, device="cuda"), []
+    if how == "forward replaced":
+        plain = layer.fc.forward
+        layer.fc.forward = lambda v: (seen.append(layer.fc), plain(v))[1]
+        layer(x)
+    else:
+        handle = torch.nn.modules.module.register_module_forward_hook(lambda mod, args, out: seen.append(mod))
+        try:
+            layer(x)
+        finally:
+            handle.remove()
+    assert any(mod is layer.fc for mod in seen)
