@@ -1010,51 +1010,52 @@ template <typename E> struct NhwcMx;
 template <> struct NhwcMx<_Float16> {
   typedef _Float16 v4 __attribute__((ext_vector_type(4)));
   typedef _Float16 v8 __attribute__((ext_vector_type(8)));
-  // d_i = w0 * h_i (+ w1 * h_i): rows = 16 channels, columns = 16 pixels.  From inline assembly with
+  // d_i = w0 * h_i + w1 * h_i (float32 tensors): rows = 16 channels, columns = 16 pixels.  From inline assembly with
   // early-clobber results: a result of these instructions must not share registers with an operand,
   // which the compiler otherwise arranges at an operand's last use.  The second product on a result
   // follows two independent instructions; s_nop 7 covers the wait states before the vector ALU may read.
-  template <bool SECOND>
   static __device__ __forceinline__ void rows3(nhwc_f4& d0, nhwc_f4& d1, nhwc_f4& d2, v8 w0, v8 w1, v8 h0, v8 h1, v8 h2) {
-    if constexpr (SECOND)
-      asm volatile(
-          "s_nop 1\n\t"
-          "v_mfma_f32_16x16x32_f16 %0, %3, %5, 0\n\t"
-          "v_mfma_f32_16x16x32_f16 %1, %3, %6, 0\n\t"
-          "v_mfma_f32_16x16x32_f16 %2, %3, %7, 0\n\t"
-          "v_mfma_f32_16x16x32_f16 %0, %4, %5, %0\n\t"
-          "v_mfma_f32_16x16x32_f16 %1, %4, %6, %1\n\t"
-          "v_mfma_f32_16x16x32_f16 %2, %4, %7, %2\n\t"
-          "s_nop 7"
-          : "=&v"(d0), "=&v"(d1), "=&v"(d2)
-          : "v"(w0), "v"(w1), "v"(h0), "v"(h1), "v"(h2));
-    else
-      asm volatile(
-          "s_nop 1\n\t"
-          "v_mfma_f32_16x16x32_f16 %0, %3, %4, 0\n\t"
-          "v_mfma_f32_16x16x32_f16 %1, %3, %5, 0\n\t"
-          "v_mfma_f32_16x16x32_f16 %2, %3, %6, 0\n\t"
-          "s_nop 7"
-          : "=&v"(d0), "=&v"(d1), "=&v"(d2)
-          : "v"(w0), "v"(h0), "v"(h1), "v"(h2));
+    asm volatile(
+        "s_nop 1\n\t"
+        "v_mfma_f32_16x16x32_f16 %0, %3, %5, 0\n\t"
+        "v_mfma_f32_16x16x32_f16 %1, %3, %6, 0\n\t"
+        "v_mfma_f32_16x16x32_f16 %2, %3, %7, 0\n\t"
+        "v_mfma_f32_16x16x32_f16 %0, %4, %5, %0\n\t"
+        "v_mfma_f32_16x16x32_f16 %1, %4, %6, %1\n\t"
+        "v_mfma_f32_16x16x32_f16 %2, %4, %7, %2\n\t"
+        "s_nop 7"
+        : "=&v"(d0), "=&v"(d1), "=&v"(d2)
+        : "v"(w0), "v"(w1), "v"(h0), "v"(h1), "v"(h2));
   }
 };
 template <> struct NhwcMx<__bf16> {
   typedef __bf16 v4 __attribute__((ext_vector_type(4)));
   typedef __bf16 v8 __attribute__((ext_vector_type(8)));
-  template <bool SECOND>
-  static __device__ __forceinline__ void rows3(nhwc_f4& d0, nhwc_f4& d1, nhwc_f4& d2, v8 w0, v8 w1, v8 h0, v8 h1, v8 h2) {
-    static_assert(!SECOND, "bfloat16 tensors need no second product");
-    asm volatile(
-        "s_nop 1\n\t"
-        "v_mfma_f32_16x16x32_bf16 %0, %3, %4, 0\n\t"
-        "v_mfma_f32_16x16x32_bf16 %1, %3, %5, 0\n\t"
-        "v_mfma_f32_16x16x32_bf16 %2, %3, %6, 0\n\t"
-        "s_nop 7"
-        : "=&v"(d0), "=&v"(d1), "=&v"(d2)
-        : "v"(w0), "v"(h0), "v"(h1), "v"(h2));
-  }
 };
+// 16-bit tensors: the filter is one part, and the float32 hats are three (bfloat16: 8 + 8 + 8 bits; two parts, 16 bits,
+// show where the cells of a channel cancel: relative error against 64 bits of such sums 5.4e-3, 1.7e-3 with the third;
+// float16 4.2e-4 and 3.6e-4).  The third part, m_i, goes through the product of sixteen, half the registers.  The s_nop
+// between the two shapes covers an accumulator's way from the one to the other.
+#define DK_ROWS3(TYPE)                             \
+  asm volatile(                                    \
+      "s_nop 1\n\t"                                \
+      "v_mfma_f32_16x16x32_" TYPE " %0, %3, %5, 0\n\t"  \
+      "v_mfma_f32_16x16x32_" TYPE " %1, %3, %6, 0\n\t"  \
+      "v_mfma_f32_16x16x32_" TYPE " %2, %3, %7, 0\n\t"  \
+      "s_nop 7\n\t"                                \
+      "v_mfma_f32_16x16x16_" TYPE " %0, %4, %8, %0\n\t" \
+      "v_mfma_f32_16x16x16_" TYPE " %1, %4, %9, %1\n\t" \
+      "v_mfma_f32_16x16x16_" TYPE " %2, %4, %10, %2\n\t" \
+      "s_nop 7\n\t"                                \
+      "s_nop 2"                                    \
+      : "=&v"(d0), "=&v"(d1), "=&v"(d2)            \
+      : "v"(w0), "v"(w), "v"(h0), "v"(h1), "v"(h2), "v"(m0), "v"(m1), "v"(m2))
+template <typename E, typename V4 = typename NhwcMx<E>::v4, typename V8 = typename NhwcMx<E>::v8>
+__device__ __forceinline__ void rows3_hats3(nhwc_f4& d0, nhwc_f4& d1, nhwc_f4& d2, V8 w0, V4 w, V8 h0, V8 h1, V8 h2, V4 m0, V4 m1, V4 m2) {
+  if constexpr (std::is_same<E, __bf16>::value) DK_ROWS3("bf16");
+  else DK_ROWS3("f16");
+}
+#undef DK_ROWS3
 template <typename T> struct NhwcMxOf { using type = _Float16; };  // float, __half
 template <> struct NhwcMxOf<bf16_t> { using type = __bf16; };
 
@@ -1106,23 +1107,61 @@ __device__ __forceinline__ void raw_st(rsrc_t r, unsigned off, const float (&v)[
 }
 
 // The operand of a scope coordinate on the pixels' side: the hat products of the lane group's four cells, their high
-// parts in front of their low ones.
-template <typename E>
-__device__ __forceinline__ typename NhwcMx<E>::v8 hat_operand(float2 c, const float (&crow)[4], const float (&ccol)[4]) {
+// parts in front of their low ones; 16-bit tensors: the third parts beside them.
+template <typename T>
+struct HatParts {
+  using M = NhwcMx<typename NhwcMxOf<T>::type>;
+  typename M::v8 hl;
+  typename M::v4 m;  // (float32 tensors: not used)
+};
+// float16: hats times 2^14, or their lower parts would be subnormal numbers
+template <typename T>
+constexpr float kHatScale = std::is_same<T, __half>::value ? 16384.f : 1.f;
+template <typename T>
+__device__ __forceinline__ HatParts<T> hat_operand(float2 c, const float (&crow)[4], const float (&ccol)[4]) {
+  using E = typename NhwcMxOf<T>::type;
+  using M = NhwcMx<E>;
   typedef float f2v __attribute__((ext_vector_type(2)));
   typedef E e2v __attribute__((ext_vector_type(2)));
   float v[4];
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
-    v[k] = nhwc_hat(c.x - crow[k]) * nhwc_hat(c.y - ccol[k]);
+    v[k] = nhwc_hat(c.x - crow[k]) * nhwc_hat(c.y - ccol[k]) * kHatScale<T>;
     asm volatile("" : "+v"(v[k]));  // one fp32 value for both parts
   }
   const e2v h01 = __builtin_convertvector(f2v{v[0], v[1]}, e2v), h23 = __builtin_convertvector(f2v{v[2], v[3]}, e2v);
   const f2v b01 = __builtin_convertvector(h01, f2v), b23 = __builtin_convertvector(h23, f2v);
-  const e2v l01 = __builtin_convertvector(f2v{v[0] - b01[0], v[1] - b01[1]}, e2v);
-  const e2v l23 = __builtin_convertvector(f2v{v[2] - b23[0], v[3] - b23[1]}, e2v);
-  return typename NhwcMx<E>::v8{h01[0], h01[1], h23[0], h23[1], l01[0], l01[1], l23[0], l23[1]};
+  const f2v r01 = f2v{v[0] - b01[0], v[1] - b01[1]}, r23 = f2v{v[2] - b23[0], v[3] - b23[1]};
+  const e2v l01 = __builtin_convertvector(r01, e2v), l23 = __builtin_convertvector(r23, e2v);
+  HatParts<T> p;
+  p.hl = typename M::v8{h01[0], h01[1], h23[0], h23[1], l01[0], l01[1], l23[0], l23[1]};
+  if constexpr (sizeof(T) == 2) {
+    const f2v c01 = __builtin_convertvector(l01, f2v), c23 = __builtin_convertvector(l23, f2v);
+    const e2v m01 = __builtin_convertvector(f2v{r01[0] - c01[0], r01[1] - c01[1]}, e2v);
+    const e2v m23 = __builtin_convertvector(f2v{r23[0] - c23[0], r23[1] - c23[1]}, e2v);
+    p.m = typename M::v4{m01[0], m01[1], m23[0], m23[1]};
+  }
+  return p;
 }
+
+// The weights of three taps for a block of channels from the block's staged filter operands
+template <typename T>
+struct FilterParts {
+  using E = typename NhwcMxOf<T>::type;
+  using M = NhwcMx<E>;
+  typename M::v4 wh;
+  typename M::v8 whh, wl0;
+  __device__ __forceinline__ explicit FilterParts(const uint4& wv) {
+    wh = __builtin_bit_cast(typename M::v4, make_uint2(wv.x, wv.y));
+    const typename M::v4 wl = __builtin_bit_cast(typename M::v4, make_uint2(wv.z, wv.w)), zero4 = {E(0), E(0), E(0), E(0)};
+    whh = __builtin_shufflevector(wh, wh, 0, 1, 2, 3, 0, 1, 2, 3);
+    wl0 = __builtin_shufflevector(wl, zero4, 0, 1, 2, 3, 4, 5, 6, 7);
+  }
+  __device__ __forceinline__ void rows3(nhwc_f4 (&d)[3], const HatParts<T>& a0, const HatParts<T>& a1, const HatParts<T>& a2) const {
+    if constexpr (sizeof(T) == 2) rows3_hats3<E>(d[0], d[1], d[2], whh, wh, a0.hl, a1.hl, a2.hl, a0.m, a1.m, a2.m);
+    else M::rows3(d[0], d[1], d[2], whh, wl0, a0.hl, a1.hl, a2.hl);
+  }
+};
 
 // The split filter operands of every channel block, for a workgroup.  An entry is lane l of its wave, so the
 // channel's largest weight is the maximum over the four lanes l % 16 + 16 k of what each holds: one load per lane
@@ -1175,11 +1214,9 @@ __device__ __forceinline__ void stage_split_filter(const T* __restrict__ filter,
 }
 
 template <typename T, int SH, int SW, bool TRANSPOSED, int CPL>
-__global__ __launch_bounds__(64 * kG16Waves) void nhwc_gather_mfma16_kernel(
+__global__ __launch_bounds__(64 * kG16Waves, 3) void nhwc_gather_mfma16_kernel(
     Geo g, const T* __restrict__ src, const T* __restrict__ rot, const T* __restrict__ filter, T* __restrict__ dst,
     int tiles_per_wave, int total_blocks, int steps_per_split) {
-  using E = typename NhwcMxOf<T>::type;
-  using M = NhwcMx<E>;
   using Raw = NhwcRaw<T, CPL>;
   constexpr bool kThird = sizeof(T) == 4;  // float32 tensors: the filter has a low part
   constexpr int TAPS = 9, CELLS = SH * SW;
@@ -1249,13 +1286,13 @@ __global__ __launch_bounds__(64 * kG16Waves) void nhwc_gather_mfma16_kernel(
       }
     }
     lds_fence_wave();
-    typename M::v8 A[TAPS];
+    HatParts<T> A[TAPS];
     unsigned xoff[TAPS];
 #pragma unroll
     for (int t = 0; t < TAPS; ++t) {
       const float2 c = cw[t * 16 + n];
       xoff[t] = xo[t * 16 + n];
-      A[t] = hat_operand<E>(c, crow, ccol);
+      A[t] = hat_operand<T>(c, crow, ccol);
     }
 
     // ---- the channel blocks
@@ -1264,37 +1301,32 @@ __global__ __launch_bounds__(64 * kG16Waves) void nhwc_gather_mfma16_kernel(
       const int c = (step * 4 + kg) * CPL;
       return c < C ? (unsigned)c * (unsigned)sizeof(T) : kNoChannels;
     };
-    Raw xr[3][3];  // [tap row][tap]: two tap rows ahead of the arithmetic
+    // [tap row][tap]: two tap rows ahead of the arithmetic; with eight channels, one, for the registers
+    constexpr bool kTwoAhead = CPL == 4;
+    Raw xr[3][3];
     auto issue_row = [&](Raw (&buf)[3], int r, unsigned co) {
 #pragma unroll
       for (int tt = 0; tt < 3; ++tt) buf[tt] = raw_ld<CPL>(rs, xoff[3 * r + tt] + co, src);
     };
     unsigned co = chan_off(step0);
     issue_row(xr[0], 0, co);
-    issue_row(xr[1], 1, co);
+    if constexpr (kTwoAhead) issue_row(xr[1], 1, co);
     for (int step = step0; step < step1; ++step) {
       const unsigned co_next = chan_off(step + 1);  // past the last block: no channels, zeros
-      typename M::v8 whh[SUB], wl0[SUB];
+      uint4 wv[SUB];
 #pragma unroll
-      for (int h = 0; h < SUB; ++h) {
-        const uint4 wv = wsp[(step * SUB + h) * 64 + lane];
-        const typename M::v4 wh = __builtin_bit_cast(typename M::v4, make_uint2(wv.x, wv.y));
-        const typename M::v4 wl = __builtin_bit_cast(typename M::v4, make_uint2(wv.z, wv.w));
-        const typename M::v4 zero4 = {E(0), E(0), E(0), E(0)};
-        whh[h] = __builtin_shufflevector(wh, wh, 0, 1, 2, 3, 0, 1, 2, 3);
-        wl0[h] = __builtin_shufflevector(wl, zero4, 0, 1, 2, 3, 4, 5, 6, 7);
-      }
+      for (int h = 0; h < SUB; ++h) wv[h] = wsp[(step * SUB + h) * 64 + lane];
       float acc[CPL];
 #pragma unroll
       for (int i = 0; i < CPL; ++i) acc[i] = 0.f;
 #pragma unroll
       for (int r = 0; r < 3; ++r) {
-        if (r == 0) issue_row(xr[2], 2, co);
-        else issue_row(xr[r - 1], r - 1, co_next);
+        constexpr int kAhead = kTwoAhead ? 2 : 1;
+        if (r + kAhead < 3) issue_row(xr[r + kAhead], r + kAhead, co);
+        else issue_row(xr[r + kAhead - 3], r + kAhead - 3, co_next);
         nhwc_f4 d[SUB][3];
 #pragma unroll
-        for (int h = 0; h < SUB; ++h)
-          M::template rows3<kThird>(d[h][0], d[h][1], d[h][2], whh[h], wl0[h], A[3 * r], A[3 * r + 1], A[3 * r + 2]);
+        for (int h = 0; h < SUB; ++h) FilterParts<T>(wv[h]).rows3(d[h], A[3 * r], A[3 * r + 1], A[3 * r + 2]);
 #pragma unroll
         for (int tt = 0; tt < 3; ++tt) {
           float xv[CPL];
@@ -1307,6 +1339,9 @@ __global__ __launch_bounds__(64 * kG16Waves) void nhwc_gather_mfma16_kernel(
         const nhwc_f4 us = *reinterpret_cast<const nhwc_f4*>(unscale + step * 16 + 4 * kg);
 #pragma unroll
         for (int i = 0; i < 4; ++i) acc[i] *= us[i];
+      } else {
+#pragma unroll
+        for (int i = 0; i < CPL; ++i) acc[i] *= 1.f / kHatScale<T>;
       }
       // non-temporal: written with the default policy the result pushes the operands of the next kernel out of
       // the memory-side cache (the step of benchmark configuration 2 took 0.425 instead of 0.363 ms)
@@ -1325,11 +1360,9 @@ __global__ __launch_bounds__(64 * kG16Waves) void nhwc_gather_mfma16_kernel(
 // -- so that a quad costs nine products, four loads and thirty-six multiply-adds per four channels where four columns of
 // the kernel above cost four times the products and multiply-adds and thirty-six loads.
 template <typename T, int SH, int SW, int CPL>
-__global__ __launch_bounds__(64 * kG16Waves) void nhwc_grad_input_s2_kernel(
+__global__ __launch_bounds__(64 * kG16Waves, 3) void nhwc_grad_input_s2_kernel(
     Geo g, const T* __restrict__ gout, const T* __restrict__ rot, const T* __restrict__ filter, T* __restrict__ gin,
     int total_blocks, int steps_per_split) {
-  using E = typename NhwcMxOf<T>::type;
-  using M = NhwcMx<E>;
   using Raw = NhwcRaw<T, CPL>;
   constexpr bool kThird = sizeof(T) == 4;
   constexpr int TAPS = 9, CELLS = SH * SW;
@@ -1383,9 +1416,9 @@ __global__ __launch_bounds__(64 * kG16Waves) void nhwc_grad_input_s2_kernel(
     }
   }
   lds_fence_wave();
-  typename M::v8 A[TAPS];
+  HatParts<T> A[TAPS];
 #pragma unroll
-  for (int t = 0; t < TAPS; ++t) A[t] = hat_operand<E>(cw[t * 16 + n], crow, ccol);
+  for (int t = 0; t < TAPS; ++t) A[t] = hat_operand<T>(cw[t * 16 + n], crow, ccol);
 
   // the four output pixels' and the four input pixels' element offsets (kOutOfRange: not there)
   unsigned so[4], po[4];
@@ -1416,37 +1449,32 @@ __global__ __launch_bounds__(64 * kG16Waves) void nhwc_grad_input_s2_kernel(
     }
 #pragma unroll
     for (int h = 0; h < SUB; ++h) {
-      const uint4 wv = wsp[(step * SUB + h) * 64 + lane];
-      const typename M::v4 wh = __builtin_bit_cast(typename M::v4, make_uint2(wv.x, wv.y));
-      const typename M::v4 wl = __builtin_bit_cast(typename M::v4, make_uint2(wv.z, wv.w));
-      const typename M::v4 zero4 = {E(0), E(0), E(0), E(0)};
-      const typename M::v8 whh = __builtin_shufflevector(wh, wh, 0, 1, 2, 3, 0, 1, 2, 3);
-      const typename M::v8 wl0 = __builtin_shufflevector(wl, zero4, 0, 1, 2, 3, 4, 5, 6, 7);
-      auto add = [&](float (&to)[CPL], const float (&from)[CPL], const nhwc_f4& w) {
+      const FilterParts<T> w(wsp[(step * SUB + h) * 64 + lane]);
+      auto add = [&](float (&to)[CPL], const float (&from)[CPL], const nhwc_f4& wt) {
 #pragma unroll
-        for (int k = 0; k < 4; ++k) to[4 * h + k] = fmaf(from[4 * h + k], w[k], to[4 * h + k]);
+        for (int k = 0; k < 4; ++k) to[4 * h + k] = fmaf(from[4 * h + k], wt[k], to[4 * h + k]);
       };
       nhwc_f4 d[3];
-      M::template rows3<kThird>(d[0], d[1], d[2], whh, wl0, A[3], A[4], A[5]);
+      w.rows3(d, A[3], A[4], A[5]);
       add(acc[1], x[1], d[0]);
       add(acc[0], x[0], d[1]);
       add(acc[1], x[0], d[2]);
-      M::template rows3<kThird>(d[0], d[1], d[2], whh, wl0, A[6], A[7], A[8]);
+      w.rows3(d, A[6], A[7], A[8]);
       add(acc[3], x[1], d[0]);
       add(acc[2], x[0], d[1]);
       add(acc[3], x[0], d[2]);
-      M::template rows3<kThird>(d[0], d[1], d[2], whh, wl0, A[0], A[1], A[2]);
+      w.rows3(d, A[0], A[1], A[2]);
       add(acc[3], x[3], d[0]);
       add(acc[2], x[2], d[1]);
       add(acc[3], x[2], d[2]);
     }
-    nhwc_f4 us = {1.f, 1.f, 1.f, 1.f};
+    constexpr float kUnscale = 1.f / kHatScale<T>;
+    nhwc_f4 us = {kUnscale, kUnscale, kUnscale, kUnscale};
     if constexpr (kThird) us = *reinterpret_cast<const nhwc_f4*>(unscale + step * 16 + 4 * kg);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      if constexpr (kThird)
 #pragma unroll
-        for (int k = 0; k < 4; ++k) acc[i][k] *= us[k];
+      for (int k = 0; k < CPL; ++k) acc[i][k] *= us[k & 3];
       // 16-bit types: the default policy, for the L2 to put a pixel's pieces together (N=64 96 x 112^2, bfloat16, four
       // channels per lane: 163 us with non-temporal stores, which reached memory one by one, 62 with these)
       raw_st<sizeof(T) == 4 ? kStreamingStore : kMergedStore>(rd, po[i] + cur_off, acc[i], gin);
@@ -1547,8 +1575,8 @@ bool nhwc_gather_mfma16(const Geo& g, bool transposed, const T* src, const T* ro
       return false;
     // 16-bit tensors of whole, aligned 16-byte groups: eight channels per lane and load.  With four, a wave's load and
     // store touch sixteen pieces of 32 bytes, and the kernel is bound by the pieces: forward, bfloat16, batch 64, table
-    // kernel / four / eight channels, us: 96 x 56^2 74 / 54 / 37, 192 x 28^2 41 / 50 / 29, 64 x 112^2 189 / 210 / 136,
-    // 96 x 112^2 stride 2 76 / 91 / 59; grad input of the last 144 / 62 / 40 (144: the kernel above on the transposed geometry).
+    // kernel / eight channels, us: 96 x 56^2 82 / 44, 192 x 28^2 43 / 30, 64 x 112^2 188 / 139, 96 x 112^2 stride 2
+    // 75 / 54; grad input of the last 146 / 45 (146: the kernel above on the transposed geometry).
     const bool eight = sizeof(T) == 2 && g.channel % 8 == 0 && reinterpret_cast<uintptr_t>(src) % 16 == 0 &&
                        reinterpret_cast<uintptr_t>(dst) % 16 == 0;
 #define DK_NHWC16(LAUNCH, ...)                                                             \

@@ -37,9 +37,14 @@ CASES = [
 
 
 def _run(case, dtype, seed=0, clip=None):
-    from deformable_kernels.ops.deform_kernel.functions import sample_depthwise
     N, C, H, W, k, S, s, p, d, G, rs = case
-    x, wt, rot, gout, cfg = make_local(N, C, H, W, k, S, s, p, d, G, rs, seed=seed, dtype=dtype)
+    inputs = make_local(N, C, H, W, k, S, s, p, d, G, rs, seed=seed, dtype=dtype)
+    return inputs, _run_on(inputs, clip)
+
+
+def _run_on(inputs, clip=None):
+    from deformable_kernels.ops.deform_kernel.functions import sample_depthwise
+    x, wt, rot, gout, cfg = inputs
     cl = torch.channels_last
     xg = x.to(DEV).contiguous(memory_format=cl).requires_grad_()
     rg = rot.to(DEV).contiguous(memory_format=cl).requires_grad_()
@@ -49,9 +54,9 @@ def _run(case, dtype, seed=0, clip=None):
     assert out.is_contiguous(memory_format=cl)
     out.backward(gout.to(DEV).contiguous(memory_format=cl))
     torch.cuda.synchronize()
-    if C > 1 and H * W > 1:
+    if x.size(1) > 1 and x.size(2) * x.size(3) > 1:
         assert xg.grad.is_contiguous(memory_format=cl) and rg.grad.is_contiguous(memory_format=cl)
-    return (x, wt, rot, gout, cfg), [t.detach().cpu().contiguous() for t in (out, xg.grad, rg.grad, wg.grad)]
+    return [t.detach().cpu().contiguous() for t in (out, xg.grad, rg.grad, wg.grad)]
 
 
 def _oracle(inputs, np_dtype):
@@ -243,3 +248,32 @@ def test_quads_at_stride_2_and_eight_channels_per_lane(case, dtype):
     for a, b32, b64, t in zip(got, o32, o64, tol):
         assert a.dtype == dtype
         assert rel_err(a.float(), b64 if t == 1e-4 else b32) < t
+
+
+def _cancelling(C, H, S, stride, dtype, seed=5):
+    """Inputs whose weights nearly cancel: the columns of every scope filter are +a, -a, +a, -a and the samples lie 2^-13 to
+    2^-12 off the middle between two columns, so a weight is a difference of halves, about 2^-12 of them.  What such a
+    weight has lost of its 24 bits shows in 16-bit results: float32 coordinates and hats leave 2^-24 / 2^-12 = 2.4e-4 of
+    it; hats of 16 bits, 2^-18 / 2^-12 = 1.5e-2 at worst and 5e-3 in the mean."""
+    x, wt, rot, gout, cfg = make_local(2, C, H, H, 3, (S, S), stride, 1, 1, 1, 0.5, seed=seed)
+    x = x.abs() + 0.1
+    rot[:, 1::2] = 2.0 ** -13 * (1 + torch.rand(rot[:, 1::2].shape, generator=torch.Generator().manual_seed(seed)))
+    wt = wt[..., :1] * torch.tensor([1.0, -1.0] * 2)[:S]
+    return (x.to(dtype), wt.to(dtype), rot.to(dtype), gout.to(dtype), cfg)
+
+
+def _rel_l2(a, b):
+    a, b = torch.as_tensor(a).double(), torch.as_tensor(b).double()
+    return float((a - b).norm() / b.norm())
+
+
+@pytest.mark.parametrize("dtype, tol", [(torch.float16, 4e-4), (torch.bfloat16, 2.4e-3)])  # 16-bit results (rms 2.1e-4, 1.7e-3) and 3e-4 for the weights
+@pytest.mark.parametrize("C", [36, 40])   # four and eight channels per lane
+@pytest.mark.parametrize("stride", [1, 2])
+def test_half_precision_weights_keep_float32_where_the_cells_cancel(stride, C, dtype, tol, switch_off):
+    switch_off("DK_FORCE_NHWC_GATHER_MFMA")
+    inputs = _cancelling(C, 20, 4, stride, dtype)
+    got = _run_on(inputs)
+    want = _oracle(inputs, np.float64)
+    assert _rel_l2(got[0], want[0]) < tol
+    assert _rel_l2(got[1], want[1]) < tol
