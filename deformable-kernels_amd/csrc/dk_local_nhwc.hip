@@ -1588,20 +1588,24 @@ bool nhwc_gather_mfma16(const Geo& g, bool transposed, const T* src, const T* ro
     if constexpr (sizeof(T) == 2) if (eight) return LAUNCH<T, 3, 3, 8>(g, __VA_ARGS__);    \
     return LAUNCH<T, 3, 3, 4>(g, __VA_ARGS__);                                             \
   }
-    if (transposed && g.stride_h == 2 && g.stride_w == 2 && g.pad_h == 1 && g.pad_w == 1 && g.dil_h == 1 && g.dil_w == 1) {
-      DK_NHWC16(launch_grad_input_s2, src, rot, filter, dst, stream)
-      return false;
-    }
     const long tiles = ((long)g.batch * (transposed ? g.in_h * g.in_w : g.out_h * g.out_w) + 15) / 16;
     const bool strided = g.stride_h > 1 || g.stride_w > 1;
+    const bool quads = transposed && g.stride_h == 2 && g.stride_w == 2 && g.pad_h == 1 && g.pad_w == 1 && g.dil_h == 1 && g.dil_w == 1;
     // Where it is the faster kernel (step-level measurements on the MobileNetV2-DK layer shapes, batch 64, float32;
     // this kernel against the table kernel): with eight channels per lane everywhere; with four its per-tile set-up (a
     // third of its instructions at 144 channels) and its one-tile-per-wave grid want many channels and many tiles.
-    // Forward 144 x 56^2: 80 against 103 us, but 32 x 112^2 136 / 109, 192 x 28^2 50 / 39, 960 x 7^2 58 / 22.  Grad input
-    // at other strides than 1 and 2, where the table kernel tests every tap of every input pixel against the stride's
-    // grid: from 64 channels and 3000 tiles on.  DK_FORCE_NHWC_GATHER_MFMA takes it wherever it applies (the tests).
-    const bool faster = eight || (g.channel >= 128 && tiles >= 8192) || (transposed && strided && g.channel >= 64 && tiles >= 3000);
+    // Forward 144 x 56^2: 80 against 103 us, but 32 x 112^2 136 / 109, 192 x 28^2 50 / 39, 960 x 7^2 58 / 22.  Strided grad
+    // input, where the table kernel tests every tap of every input pixel against the stride's grid: from 64 channels and
+    // 3000 tiles on; 16-bit tensors' quads everywhere.  (The quads would be faster for float32 everywhere too, but there
+    // the pairs of fp16 hold 22 of the 24 bits of the table kernel's weights.)  DK_FORCE_NHWC_GATHER_MFMA takes it wherever it
+    // applies (the tests).
+    const bool faster = eight || (quads && sizeof(T) == 2) || (g.channel >= 128 && tiles >= 8192) ||
+                        (transposed && strided && g.channel >= 64 && tiles >= 3000);
     if (!faster && !path_disabled(kForceNhwcGatherMfma)) return false;
+    if (quads) {
+      DK_NHWC16(launch_grad_input_s2, src, rot, filter, dst, stream)
+      return false;
+    }
     DK_NHWC16(launch_gather_mfma16, transposed, src, rot, filter, dst, stream)
 #undef DK_NHWC16
     return false;

@@ -277,3 +277,25 @@ def test_half_precision_weights_keep_float32_where_the_cells_cancel(stride, C, d
     want = _oracle(inputs, np.float64)
     assert _rel_l2(got[0], want[0]) < tol
     assert _rel_l2(got[1], want[1]) < tol
+
+
+@pytest.mark.parametrize("case", [
+    (2, 40, 20, 20, 3, (4, 4), 2, 1, 1, 1, 0.5),     # fewer than 64 channels
+    (2, 96, 15, 18, 3, (3, 3), 2, 1, 1, 1, 0.5),     # fewer than 3000 tiles of sixteen input pixels
+])
+def test_float32_grad_input_of_few_channels_or_pixels_at_stride_2_is_the_table_kernels(case, switch_off):
+    """The matrix-core kernel holds float32 weights as pairs of fp16 (22 of 24 bits); it is left to the shapes it pays on."""
+    inputs, got = _run(case, torch.float32, seed=4)
+    switch_off("DK_NO_NHWC_MFMA")
+    assert torch.equal(got[1], _run_on(inputs)[1])
+
+
+@pytest.mark.parametrize("case", [
+    (1, 16, 2, 3, 3, (4, 4), 2, 1, 1, 1, 0.7),      # as above, float32 where the dispatch takes the table kernel
+    (2, 20, 15, 18, 3, (3, 3), 2, 1, 1, 1, 0.7),
+    (1, 136, 21, 22, 3, (4, 4), 2, 1, 1, 1, 0.7),
+])
+def test_fp32_quads_at_stride_2(case, switch_off):
+    switch_off("DK_FORCE_NHWC_GATHER_MFMA")
+    inputs, got = _run(case, torch.float32, seed=3)
+    assert rel_err(got[1], _oracle(inputs, np.float32)[1]) < 1e-5
