@@ -1287,7 +1287,7 @@ __global__ __launch_bounds__(kMfBlock, NSL == 2 && SPLIT ? 2 : 4) void local_gra
   // small (one channel, 3 x 3 scope: 1.1e-2 seen), so groups of fewer than 16 channels keep the
   // fp32 instructions (template parameter BF, chosen by the host).
   static_assert(!BF || sizeof(T) == 2, "bfloat16 matrix instructions are for 16-bit inputs");
-  static_assert(!SPLIT || !BF, "one or the other");
+  static_assert(!SPLIT || (sizeof(T) == 4 && !BF), "the split is for float32 inputs");
   constexpr bool kHalfIn = BF;
   float A[(kHalfIn || SPLIT) ? 1 : 4][K];
   mfb4 Ab[NSL][(kHalfIn || SPLIT) ? K : 1];  // SPLIT: the hi parts
@@ -1763,13 +1763,14 @@ bool run_grad_filter(const Geo& g, const T* gout, const T* x, const T* rot, T* g
       // float32 inputs: bfloat16 pairs (three products) unless switched off, at stride 2 as well (N=64: 96 x 112^2
       // 98 -> 90 us, 144 x 56^2 46 -> 41, 192 x 28^2 25.9 -> 24.3, 576 x 14^2 32.8 -> 30.1)
       const bool split = !path_disabled(kNoFilterSplit);
-      // Channels-last at stride 2: the fp32 instructions for float32 tensors and the pairs for 16-bit ones (whose
-      // products a pair holds exactly for bfloat16): the operands' rounding stays below that of the kernel that
-      // served this geometry before (nhwc_grad_filter_mfma_kernel, fp32 instructions: us for N=64 96 x 112^2, it / this
-      // kernel: float32 149 / 126, bfloat16 142 / 88).
+      // Channels-last at stride 2: the fp32 instructions for every type, as in the kernel that serves the shapes this one does
+      // not (nhwc_grad_filter_mfma_kernel: us for N=64 96 x 112^2, it / this kernel: float32 149 / 126, bfloat16 142 / 99).
+      // bfloat16 pairs are faster (bfloat16 88), but hold 16 of the 24 bits of a hat and of the 22 of a product of two
+      // float16: relative error against 64 bits where neighbouring pixels' shares cancel 2.9e-2 (float16) and 3.9e-2
+      // (bfloat16), 1.6e-3 and 2.2e-3 with the fp32 instructions.
 #define DK_LAUNCH(CELL0)                                                    \
   if constexpr (CL) {                                                       \
-    if (f.th > 0) { DK_LAUNCH_BF(CELL0, false, sizeof(T) == 2) }            \
+    if (f.th > 0) { DK_LAUNCH_BF(CELL0, false, false) }                     \
     else if constexpr (sizeof(T) == 2) {                                    \
       if (g.channel / g.groups >= kMfCh) { DK_LAUNCH_BF(CELL0, true, false) } \
       else { DK_LAUNCH_BF(CELL0, false, false) }                            \

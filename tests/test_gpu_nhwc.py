@@ -279,6 +279,25 @@ def test_half_precision_weights_keep_float32_where_the_cells_cancel(stride, C, d
     assert _rel_l2(got[1], want[1]) < tol
 
 
+@pytest.mark.parametrize("dtype, tol", [(torch.float16, 1e-2), (torch.bfloat16, 1e-2)])
+@pytest.mark.parametrize("C", [40, 24])
+def test_half_precision_filter_gradient_at_stride_2_keeps_float32_where_the_pixels_cancel(C, dtype, tol):
+    """Upstream gradients +a, -a on neighbouring pixels whose samples lie 2^-13 to 2^-12 off the middle between two columns
+    and a third of a cell off a row: a cell's gradient is a sum of differences of two hat products of 0.16 to 0.41, some
+    2^-13 * 0.2 per pair.  float32 hats and sums leave about 2^-25 per term, 1e-3 of that (and the result's rounding is
+    1.7e-3 at most in the mean); hats of 16 bits leave 2^-20 to 2^-19, 4e-2 to 8e-2."""
+    x, wt, rot, gout, cfg = make_local(2, C, 20, 20, 3, (4, 4), 2, 1, 1, 1, 0.0, seed=6)
+    rot[:, 0::2] = 0.3137
+    rot[:, 1::2] = 2.0 ** -13 * (1 + torch.rand(rot[:, 1::2].shape, generator=torch.Generator().manual_seed(6)))
+    x = (x[:1, :, :1, :1].abs() + 0.5).expand_as(x).contiguous()
+    gout = (gout[:1, :, :1, :1].abs() + 0.5) * torch.tensor([1.0, -1.0] * 5) * torch.ones_like(gout)
+    gout[:, :, 0] = 0      # taps on the padding would leave pixels without their partners
+    gout[:, :, :, :2] = 0
+    inputs = (x.to(dtype), wt.to(dtype), rot.to(dtype), gout.to(dtype), cfg)
+    got, want = _run_on(inputs)[3], _oracle(inputs, np.float64)[3]
+    assert _rel_l2(got, want) < tol
+
+
 @pytest.mark.parametrize("case", [
     (2, 40, 20, 20, 3, (4, 4), 2, 1, 1, 1, 0.5),     # fewer than 64 channels
     (2, 96, 15, 18, 3, (3, 3), 2, 1, 1, 1, 0.5),     # fewer than 3000 tiles of sixteen input pixels
