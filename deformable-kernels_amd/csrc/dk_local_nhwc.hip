@@ -1172,6 +1172,10 @@ struct FilterParts {
 // CPL: channels a lane holds per step.  With 4, the rows of block b are its sixteen channels in order, so that the lane
 // group kg gets channels 4 kg .. 4 kg + 3; with 8, blocks 2 s and 2 s + 1 deal the channels of step s to their rows such
 // that the group gets 8 kg .. 8 kg + 3 from the one and 8 kg + 4 .. 8 kg + 7 from the other.
+//
+// unscale[block][16]: what a channel's sums are multiplied by at the end (float32 tensors), or -1 throughout a block that holds
+// a weight that is not finite.  The products spread such a weight over every pixel of its channel (0 * inf), so that the
+// kernels below write those blocks a second time, from scope_weight().
 template <typename T, int CELLS, int CPL>
 __device__ __forceinline__ void stage_split_filter(const T* __restrict__ filter, int C, int blk0, int blk1, uint4* wsp, float* unscale) {
   using E = typename NhwcMxOf<T>::type;
@@ -1180,13 +1184,18 @@ __device__ __forceinline__ void stage_split_filter(const T* __restrict__ filter,
   for (int e = blk0 * 64 + threadIdx.x; e < blk1 * 64; e += 64 * kG16Waves) {
     const int b = e >> 6, l = e & 63, c0 = 4 * (l >> 4);
     const int cj = CPL == 4 ? b * 16 + (l & 15) : (b >> 1) * 32 + 8 * ((l & 15) >> 2) + 4 * (b & 1) + (l & 3);
-    float v[4] = {0.f, 0.f, 0.f, 0.f}, s = 1.f;
+    float v[4] = {0.f, 0.f, 0.f, 0.f};
     if (cj < C) {
       const T* f = filter + (size_t)cj * CELLS;
 #pragma unroll
       for (int k = 0; k < 4; ++k)
         if (c0 + k < CELLS) v[k] = (float)ld(f + c0 + k);
     }
+    bool finite = true;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) finite = finite && fabsf(v[k]) < __builtin_inff();
+    const bool block_finite = __ballot(!finite) == 0;  // (the wave's 64 entries are the block's)
+    float back = 1.f;
     if constexpr (kThird) {
       float mx = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
       mx = fmaxf(mx, __shfl_xor(mx, 16));
@@ -1194,11 +1203,12 @@ __device__ __forceinline__ void stage_split_filter(const T* __restrict__ filter,
       int ex = 0;
       if (mx > 0.f && mx < __builtin_inff()) (void)frexpf(mx, &ex);
       ex = min(max(ex, -100), 100);
-      s = ldexpf(1.f, -ex);
-      if ((l >> 4) == 0) unscale[b * 16 + (l & 15)] = cj < C ? ldexpf(1.f, ex) : 0.f;
+      const float s = ldexpf(1.f, -ex);
+      back = ldexpf(1.f, ex);
 #pragma unroll
       for (int k = 0; k < 4; ++k) v[k] *= s;
     }
+    if ((l >> 4) == 0) unscale[b * 16 + (l & 15)] = block_finite ? back : -1.f;
     typename M::v4 h4, l4;
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
@@ -1211,6 +1221,27 @@ __device__ __forceinline__ void stage_split_filter(const T* __restrict__ filter,
     const uint2 hb = __builtin_bit_cast(uint2, h4), lb2 = __builtin_bit_cast(uint2, l4);
     wsp[e] = make_uint4(hb.x, hb.y, lb2.x, lb2.y);
   }
+}
+
+// Whether blocks blk0 .. blk1 - 1 hold finite weights only (the same for every lane).
+__device__ __forceinline__ bool filter_finite(const float* unscale, int blk0, int blk1, int lane) {
+  bool bad = false;
+  for (int b = blk0 + lane; b < blk1; b += 64) bad = bad || unscale[b * 16] < 0.f;
+  return __ballot(bad) == 0;
+}
+
+// A channel's weight at a scope coordinate, from the corners inside the scope alone (K.cu:59-84); (-2, -2): no sample.
+template <typename T, int SH, int SW>
+__device__ __forceinline__ float scope_weight(const T* f, float2 c) {
+  const float hf = floorf(c.x), wf = floorf(c.y), lh = c.x - hf, lw = c.y - wf;
+  const int h = (int)hf, w = (int)wf;
+  float sum = 0.f;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int i = h + (k >> 1), j = w + (k & 1);
+    if (i >= 0 && i < SH && j >= 0 && j < SW) sum = fmaf((k >> 1 ? lh : 1.f - lh) * (k & 1 ? lw : 1.f - lw), (float)ld(f + i * SW + j), sum);
+  }
+  return sum;
 }
 
 template <typename T, int SH, int SW, bool TRANSPOSED, int CPL>
@@ -1237,6 +1268,7 @@ __global__ __launch_bounds__(64 * kG16Waves, 3) void nhwc_gather_mfma16_kernel(
   const int step0 = blockIdx.y * steps_per_split, step1 = min(nstep, step0 + steps_per_split);
   stage_split_filter<T, CELLS, CPL>(filter, C, step0 * SUB, step1 * SUB, wsp, unscale);
   __syncthreads();
+  const bool finite = filter_finite(unscale, step0 * SUB, step1 * SUB, lane);
 
   const int n = lane & 15, kg = lane >> 4;
   const int oplane = g.out_h * g.out_w, iplane = g.in_h * g.in_w;
@@ -1348,6 +1380,28 @@ __global__ __launch_bounds__(64 * kG16Waves, 3) void nhwc_gather_mfma16_kernel(
       raw_st<kStreamingStore>(rd, doff + co, acc, dst);
       co = co_next;
     }
+
+    // ---- blocks with a weight that is not finite, a second time
+    if (!finite) {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // behind the stores above
+#pragma unroll 1
+      for (int step = step0; step < step1; ++step) {
+        const int ch = (step * 4 + kg) * CPL;
+        if (filter_finite(unscale, step * SUB, (step + 1) * SUB, lane) || ch >= C) continue;
+        float acc[CPL];
+#pragma unroll
+        for (int i = 0; i < CPL; ++i) acc[i] = 0.f;
+#pragma unroll 1
+        for (int t = 0; t < TAPS; ++t) {
+          const float2 at = cw[t * 16 + n];
+          float xv[CPL];
+          raw_cvt(raw_ld<CPL>(rs, xo[t * 16 + n] + chan_off(step), src), xv, src);
+#pragma unroll
+          for (int i = 0; i < CPL; ++i) acc[i] = fmaf(xv[i], scope_weight<T, SH, SW>(filter + (size_t)(ch + i) * CELLS, at), acc[i]);
+        }
+        raw_st<kStreamingStore>(rd, doff + chan_off(step), acc, dst);
+      }
+    }
   }
 }
 
@@ -1380,6 +1434,7 @@ __global__ __launch_bounds__(64 * kG16Waves, 3) void nhwc_grad_input_s2_kernel(
   const int step0 = blockIdx.y * steps_per_split, step1 = min(nstep, step0 + steps_per_split);
   stage_split_filter<T, CELLS, CPL>(filter, C, step0 * SUB, step1 * SUB, wsp, unscale);
   __syncthreads();
+  const bool finite = filter_finite(unscale, step0 * SUB, step1 * SUB, lane);
 
   const int n = lane & 15, kg = lane >> 4;
   const int OH = g.out_h, OW = g.out_w, oplane = OH * OW;
@@ -1486,6 +1541,33 @@ __global__ __launch_bounds__(64 * kG16Waves, 3) void nhwc_grad_input_s2_kernel(
     do_step(step + 1, xr[1], xr[0], co[1], co[0]);
   }
   if (step < step1) do_step(step, xr[0], xr[1], co[0], co[1]);
+
+  // ---- blocks with a weight that is not finite, a second time
+  if (!finite) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // behind the stores above
+#pragma unroll 1
+    for (step = step0; step < step1; ++step) {
+      const int ch = (step * 4 + kg) * CPL;
+      if (filter_finite(unscale, step * SUB, (step + 1) * SUB, lane) || ch >= C) continue;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float acc[CPL];
+#pragma unroll
+        for (int k = 0; k < CPL; ++k) acc[k] = 0.f;
+#pragma unroll 1
+        for (int t = 0; t < TAPS; ++t) {  // from output pixel (a + (t / 3 == 0), c + (t % 3 == 0)) to one of the quad's
+          if (i != (t / 3 != 1 ? 2 : 0) + (t % 3 != 1 ? 1 : 0)) continue;
+          const unsigned from = t / 3 == 0 ? t % 3 == 0 ? so[3] : so[2] : t % 3 == 0 ? so[1] : so[0];
+          const float2 at = cw[t * 16 + n];
+          float xv[CPL];
+          raw_cvt(raw_ld<CPL>(rs, from + chan_off(step), gout), xv, gout);
+#pragma unroll
+          for (int k = 0; k < CPL; ++k) acc[k] = fmaf(xv[k], scope_weight<T, SH, SW>(filter + (size_t)(ch + k) * CELLS, at), acc[k]);
+        }
+        raw_st<sizeof(T) == 4 ? kStreamingStore : kMergedStore>(rd, po[i] + chan_off(step), acc, gin);
+      }
+    }
+  }
 }
 
 // ---- host side --------------------------------------------------------------------------

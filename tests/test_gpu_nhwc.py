@@ -309,6 +309,23 @@ def test_float32_grad_input_of_few_channels_or_pixels_at_stride_2_is_the_table_k
     assert torch.equal(got[1], _run_on(inputs)[1])
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("C", [36, 40])   # four and eight channels per lane for the 16-bit types
+@pytest.mark.parametrize("stride", [1, 2])
+@pytest.mark.parametrize("poison", [float("inf"), float("nan")])
+def test_a_non_finite_weight_reaches_the_pixels_that_read_it_and_no_others(poison, stride, C, dtype, switch_off):
+    switch_off("DK_FORCE_NHWC_GATHER_MFMA")
+    x, wt, rot, gout, cfg = make_local(2, C, 11, 13, 3, (4, 4), stride, 1, 1, 1, 0.7, seed=8, dtype=dtype)
+    wt[5, 0, 0, 3] = wt[C - 1, 0, 3, 1] = poison
+    inputs = (x, wt, rot, gout, cfg)
+    got, want = _run_on(inputs), _oracle(inputs, np.float64)
+    for a, b in zip(got[:2], want[:2]):
+        read = ~np.isfinite(b)
+        assert read[:, [5, C - 1]].any() and not read[:, [5, C - 1]].all()
+        assert np.array_equal(~torch.isfinite(a).numpy(), read)
+        assert rel_err(a.float()[torch.from_numpy(~read)], b[~read]) < (1e-5 if dtype == torch.float32 else 1e-2)
+
+
 @pytest.mark.parametrize("case", [
     (1, 16, 2, 3, 3, (4, 4), 2, 1, 1, 1, 0.7),      # as above, float32 where the dispatch takes the table kernel
     (2, 20, 15, 18, 3, (3, 3), 2, 1, 1, 1, 0.7),
