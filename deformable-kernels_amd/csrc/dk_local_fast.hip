@@ -707,10 +707,7 @@ __global__ __launch_bounds__(kBlock, OCC) void local_grad_rotation_kernel(
       // v_dot2c_f32_bf16 against the pair table's {b, c, d} (fp32 sums) -- six vector instructions and one
       // table read per tap and channel pair where the fp32 form takes eight and two.  The second channel
       // of an odd count's last pair is the last channel again, against a table of zeros.
-      // Stages of pairs: three on their way instead of one (122 registers, four waves per SIMD as before).  N=128 C=576
-      // 14x14, forward and backward, 178.5 -> 175 us; C=192 28x28 unchanged.  The 96-register variant has no room for it.
-      constexpr int AHEAD = OCC < 5 ? 4 : 2;
-      float xw[AHEAD][2][KH], gw[AHEAD][2];
+      float xw[2][2][KH], gw[2][2];
       auto load_pair = [&](int s, int jp) {
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
@@ -740,14 +737,12 @@ __global__ __launch_bounds__(kBlock, OCC) void local_grad_rotation_kernel(
         }
       };
       const int npair = (nch + 1) / 2;
-#pragma unroll
-      for (int u = 0; u < AHEAD - 1; ++u) load_pair(u, u);
-      for (int jp = 0; jp < npair; jp += AHEAD) {
-#pragma unroll
-        for (int u = 0; u < AHEAD; ++u) {
-          load_pair((u + AHEAD - 1) % AHEAD, jp + u + AHEAD - 1);
-          if (jp + u < npair) accumulate_pair(u, jp + u);
-        }
+      load_pair(0, 0);
+      for (int jp = 0; jp < npair; jp += 2) {
+        load_pair(1, jp + 1);
+        accumulate_pair(0, jp);
+        load_pair(0, jp + 2);
+        if (jp + 1 < npair) accumulate_pair(1, jp + 1);
       }
     } else {
 #pragma unroll
