@@ -178,7 +178,7 @@ def traffic_table(a):
     import glob
     lines = ["HBM traffic counters of the local deformable-kernel operator, MI355X, one GPU: FETCH_SIZE and WRITE_SIZE per call of each",
              "entry point, from the tables profiles/hbm_traffic_<workload>_<dtype>.json (which bench.py reads for roofline.traffic).", "",
-             "Commands (from the repository root, on the GPU box; one counter per run, then the summaries, which need no GPU):",
+             "Commands (from the repository root, on a machine with the GPU; one counter per run, then the summaries, which need no GPU):",
              "  rocprofv3 --pmc FETCH_SIZE -d /tmp/dk_prof/F -o pmc -- python3 bench.py --workload W --dtype D --steps 3 --warmup 1 --no-cpu-baseline --no-network-pass",
              "  rocprofv3 --pmc WRITE_SIZE -d /tmp/dk_prof/W -o pmc -- python3 bench.py --workload W --dtype D --steps 3 --warmup 1 --no-cpu-baseline --no-network-pass",
              "  python3 bench.py --workload W --dtype D --traffic-from /tmp/dk_prof/F/*/pmc_results.db /tmp/dk_prof/W/*/pmc_results.db",
@@ -203,8 +203,8 @@ def traffic_table(a):
             lines.append("  %-14s %12.1f %10.1f %12.1f %10.1f %10.1f %14.1f" % (key, e["fetch_kib"], fm, e["write_kib"], wm, fm + wm, per[key] / 1e6))
         lines.append("  kernels: " + "; ".join(d["kernels"]))
         lines.append("")
-    lines += ["(MB = 1e6 bytes; algorithmic = every operand touched once.)  The per-pixel operator with a 5 x 5 scope runs its",
-              "grad filter as two launches of 16 scope cells each, so it reads its operands twice; forward / grad input of the 16-bit",
+    lines += ["(MB = 1e6 bytes; algorithmic = every operand touched once.)  The grad filter of the 5 x 5 scope sums its 25 cells, two",
+              "slices of 16, in one launch and reads its 28 x 28 tiles' halo rows again; forward / grad input of the 16-bit",
               "types write with the default cache policy since the non-temporal 2-byte stores reached memory as partial lines (WRITE_SIZE",
               "47 % above the tensor's size).  Reads are within a few per cent of the compulsory amount everywhere else: the XCD-aware",
               "block order keeps halo rows and rotation planes in one L2, and the matrix-core grad filter deals its tiles round-robin",
@@ -342,8 +342,8 @@ def main():
     if a.profile_from:
         return summarise_profile(a)
     if a.gpus != 1:
-        sys.exit("bench.py measures one GPU only: every box of this build has one GPU and no "
-                 "multi-GPU path exists (the operator shards over the batch with no exchange); "
+        sys.exit("bench.py measures one GPU only: no multi-GPU path "
+                 "exists (the operator shards over the batch with no exchange); "
                  "run with --gpus 1")
 
     import torch

@@ -103,6 +103,9 @@ struct PlainStage {
 // at a time.  GRAD: grad offset, partial[group][chunk][image][18][pixel] in fp32; else the forward.
 // A weight that is not finite must not meet the zeros that stand for a tap outside the image (the reference skips such
 // taps): a chunk that holds one masks the weights of those taps.
+// Registers: 1024 threads leave 128 of them.  Instances that spill, bytes per lane for two, three and four staging passes (they
+// hold the next channels' planes): grad offset bfloat16 36, 100, 144; float16 0, 12, 80; float32 0, 0, 16; forward bfloat16
+// in four passes 8.
 template <typename T, int PASSES, bool GRAD>
 __global__ __launch_bounds__(kPlThreads) void deform_plain_kernel(
     Geo g, const T* __restrict__ gout, const T* __restrict__ x, const T* __restrict__ off, const T* __restrict__ filter,
@@ -352,7 +355,7 @@ template <typename T>
 bool plain_deform_grad_offset(const Geo& g, const T* gout, const T* x, const T* off, const T* filter, T* goff, float* ws,
                               hipStream_t stream) {
   const PlainPlan m = plain_plan<T>(g);
-  // (eight 16-bit channels in four passes take registers that the sums need: at stride 2 slower than the kernel with the
+  // (eight 16-bit channels in four passes take registers that the sums need, and spill: at stride 2 slower than the kernel with the
   // tables, bfloat16 N=64 C=512 28x28 57 against 53 us; at stride 1, 56x56, still 140 against 209)
   if (sizeof(T) == 2 && m.passes == 4 && 2L * g.out_h * g.out_w < (long)g.in_h * g.in_w) return false;
   if (!m.ok || !launch_plain<T, true>(g, m, gout, x, off, filter, static_cast<T*>(nullptr), ws, stream)) return false;

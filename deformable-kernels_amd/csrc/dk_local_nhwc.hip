@@ -1609,8 +1609,8 @@ bool nhwc_supported(const Geo& g, int dtype) {
 }
 
 // Steps over the channels that a workgroup of the two kernels below takes.  Few tiles and many channels (grad input, N=64
-// 576 x 14^2 stride 2, float32: 49 workgroups, 33 us): the channels go over workgroups, at least four blocks each (their
-// set-up is about one block's work), for about eight waves per SIMD (12 us).
+// 576 x 14^2 stride 2: 49 workgroups; 33 us with four channels per lane): the channels go over workgroups, at least four
+// blocks each (their set-up is about one block's work), for about eight waves per SIMD (12 us).
 int channel_steps_per_split(int nstep, int nblk, int blocks) {
   return ceil_div(nstep, std::max(1, std::min(nblk / 4, 2048 / std::max(1, blocks))));
 }
@@ -1657,8 +1657,8 @@ bool nhwc_gather_mfma16(const Geo& g, bool transposed, const T* src, const T* ro
       return false;
     // 16-bit tensors of whole, aligned 16-byte groups: eight channels per lane and load.  With four, a wave's load and
     // store touch sixteen pieces of 32 bytes, and the kernel is bound by the pieces: forward, bfloat16, batch 64, table
-    // kernel / eight channels, us: 96 x 56^2 82 / 44, 192 x 28^2 43 / 30, 64 x 112^2 188 / 139, 96 x 112^2 stride 2
-    // 75 / 54; grad input of the last 146 / 45 (146: the kernel above on the transposed geometry).
+    // kernel / eight channels, us: 96 x 56^2 78 / 43, 192 x 28^2 41 / 30, 64 x 112^2 182 / 135, 96 x 112^2 stride 2
+    // 79 / 57; grad input of the last 146 / 50 (146: the kernel above on the transposed geometry).
     const bool eight = sizeof(T) == 2 && g.channel % 8 == 0 && reinterpret_cast<uintptr_t>(src) % 16 == 0 &&
                        reinterpret_cast<uintptr_t>(dst) % 16 == 0;
 #define DK_NHWC16(LAUNCH, ...)                                                             \

@@ -12,7 +12,7 @@ for p in (ROOT, os.path.join(ROOT, "deformable-kernels_amd"), os.path.dirname(os
 
 
 def pytest_configure(config):
-    config.addinivalue_line("markers", "gpu: needs a real MI355X (run with -m gpu on the GPU box)")
+    config.addinivalue_line("markers", "gpu: needs a real MI355X (run with -m gpu)")
 
 
 def _have_gpu():
