@@ -495,3 +495,26 @@ def test_a_tap_outside_the_image_does_not_read_the_first_pixel(shape, stride, of
     touched = ~np.isfinite(want)
     assert touched.any() and not touched.all()
     assert np.array_equal(~torch.isfinite(got).cpu().numpy(), touched)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rotation", [True, False])
+@pytest.mark.parametrize("shape,stride,off_std", [
+    ((2, 10, 9, 11), 1, 4.0),
+    ((1, 6, 30, 33), 2, 12.0),
+    ((1, 16, 20, 130), 1, 5.0),  # wider than 128 columns
+])
+def test_a_tap_outside_the_image_takes_no_coordinate_gradient_from_the_first_pixel(shape, stride, off_std, rotation, dtype):
+    from deformable_kernels.ops.deform_kernel.functions import deform_sample_depthwise
+    N, C, H, W = shape
+    x, wt, rot, off, gout, cfg = make_deform(N, C, H, W, 3, (4, 4), stride, 1, 1, 1, 0.5, off_std, seed=9, dtype=dtype)
+    rot = rot.clamp(-1, 1) if rotation else torch.zeros_like(rot)  # (inside the scope band)
+    x[:, 1::2, 0, 0] = float("nan")
+    want = orc.deform_sample_depthwise_backward(*[t.double().numpy() for t in (gout, x, off, rot, wt)], **cfg)[1:3]
+    coords = [off.cuda().requires_grad_()] + ([rot.cuda().requires_grad_()] if rotation else [])
+    out = deform_sample_depthwise(x.cuda(), coords[0], coords[1] if rotation else None, wt.cuda(),
+                                  cfg["kernel_size"], cfg["stride"], cfg["padding"], cfg["dilation"], 1)
+    for got, w in zip(torch.autograd.grad(out, coords, gout.cuda()), want):
+        touched = ~np.isfinite(w)
+        assert touched.any() and not touched.all()
+        assert np.array_equal(~torch.isfinite(got).cpu().numpy(), touched)
