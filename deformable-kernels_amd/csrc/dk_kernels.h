@@ -192,6 +192,18 @@ template <typename T>
 bool offset_wgrad16(int batch, int cin, int cout, int h, int w, int stride, const T* x, const T* gout, T* gweight,
                     void* ws, hipStream_t stream);
 
+// dk_offset_direct.hip: the 3 x 3 offset convolution and its two large gradients on few images, on the vector unit
+bool offset_conv_direct_supported(int batch, int cin, int cout, int h, int w);
+template <typename T>
+void offset_conv_direct_forward(int batch, int cin, int cout, int h, int w, int stride, const T* x, const T* weight,
+                                const T* bias, T* out, hipStream_t stream);
+template <typename T>
+void offset_conv_direct_backward_input(int batch, int cin, int cout, int h, int w, int stride, const T* gout,
+                                       const T* weight, T* gin, hipStream_t stream);
+template <typename T>
+void offset_conv_direct_backward_weight(int batch, int cin, int cout, int h, int w, int stride, const T* gout, const T* x,
+                                        T* gweight, hipStream_t stream);
+
 // dk_local_fast.hip: the matrix-core grad filter on channels-last tensors (false / workspace 0: not covered)
 size_t fast_local_grad_filter_cl_workspace(const Geo& g);
 template <typename T>

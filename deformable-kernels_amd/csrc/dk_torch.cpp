@@ -427,17 +427,17 @@ bool offset_conv_native_tensors(const Tensor& input, const Tensor& weight, const
 }
 
 bool offset_conv_covered(const Tensor& input, const Tensor& weight, const Pair& stride, const Pair& padding, const Pair& dilation,
-                         bool worthwhile) {
+                         int (*query)(const dk_offset_conv_desc*)) {
   if (weight.size(2) != 3 || weight.size(3) != 3 || weight.size(1) != input.size(1)) return false;
   if (!(stride == Pair{1, 1} || stride == Pair{2, 2}) || padding != Pair{1, 1} || dilation != Pair{1, 1}) return false;
   const dk_offset_conv_desc d = offset_desc(input, weight, input, stride[0]);
-  return (worthwhile ? dk_offset_conv_worthwhile(&d) : dk_offset_conv_supported(&d)) != 0;
+  return query(&d) != 0;
 }
 
 struct OffsetConvFunctionBackward : OpNode {
   SavedVariable input, weight;
   Pair stride, padding, dilation;
-  bool native = false, forced = false, has_bias = false;
+  bool native = false, direct = false, forced = false, has_bias = false;
   std::string name() const override { return "OffsetConvFunctionBackward"; }
   void release() override {
     input.reset_data(), weight.reset_data();
@@ -452,7 +452,15 @@ struct OffsetConvFunctionBackward : OpNode {
     const bool native_weight = need(1) && native && dk_offset_conv_backward_weight_workspace(&d) > 0;
     const bool native_input = need(0) && native && dk_offset_conv_backward_input_workspace(&d) > 0 &&
                               (forced || dk_offset_conv_backward_input_worthwhile(&d));
-    const bool lib_input = need(0) && !native_input, lib_weight = need(1) && !native_weight;
+    const bool lib_input = need(0) && !native_input && !direct, lib_weight = need(1) && !native_weight && !direct;
+    if (direct && need(0)) {
+      res[0] = at::empty_like(x);
+      check(dk_offset_conv_direct_backward_input(&d, in(g), in(w), out(res[0]), s), "offset_conv input gradient");
+    }
+    if (direct && need(1)) {
+      res[1] = at::empty_like(w);
+      check(dk_offset_conv_direct_backward_weight(&d, in(g), in(x), out(res[1]), s), "offset_conv weight gradient");
+    }
     if (lib_input || lib_weight) {  // the framework's routine, without its bias gradient
       auto r = at::convolution_backward(g, x, w, std::nullopt, stride, padding, dilation, false, at::IntArrayRef({0, 0}), 1,
                                         {lib_input, lib_weight, false});
@@ -483,17 +491,23 @@ Tensor offset_conv(const Tensor& input, const Tensor& weight, const OptTensor& b
                    const Pair& dilation, bool force) {
   const Tensor bias = bias_arg ? *bias_arg : Tensor();
   if (!offset_conv_native_tensors(input, weight, bias)) return at::conv2d(input, weight, bias_arg, stride, padding, dilation);
-  const bool native = offset_conv_covered(input, weight, stride, padding, dilation, !force);
+  const bool native = offset_conv_covered(input, weight, stride, padding, dilation, force ? dk_offset_conv_supported : dk_offset_conv_worthwhile);
+  // few images: one launch per pass on the vector unit
+  const bool direct = !native && offset_conv_covered(input, weight, stride, padding, dilation, dk_offset_conv_direct_worthwhile);
   Tensor x, w;
   return record<OffsetConvFunctionBackward>(
       {&input, &weight, &bias},
       [&] {
         x = input.contiguous(), w = weight.contiguous();
-        if (!native) return at::conv2d(x, w, bias_arg, stride, padding, dilation);
+        if (!native && !direct) return at::conv2d(x, w, bias_arg, stride, padding, dilation);
         const Tensor b = bias.defined() ? bias.contiguous() : at::zeros({w.size(0)}, x.options());
         const int64_t st = stride[0];
         Tensor res = at::empty({x.size(0), w.size(0), (x.size(2) - 1) / st + 1, (x.size(3) - 1) / st + 1}, x.options());
         const dk_offset_conv_desc d = offset_desc(x, w, x, st);
+        if (direct) {
+          check(dk_offset_conv_direct_forward(&d, in(x), in(w), in(b), out(res), stream_of(x)), "offset_conv forward");
+          return res;
+        }
         const Workspace ws(dk_offset_conv_forward_workspace(&d), x);
         check(dk_offset_conv_forward(&d, in(x), in(w), in(b), out(res), ws.ptr(), ws.bytes, stream_of(x)), "offset_conv forward");
         return res;
@@ -501,14 +515,14 @@ Tensor offset_conv(const Tensor& input, const Tensor& weight, const OptTensor& b
       [&](OffsetConvFunctionBackward& n) {
         n.input = SavedVariable(x, false), n.weight = SavedVariable(w, false);
         n.stride = stride, n.padding = padding, n.dilation = dilation;
-        n.native = native, n.forced = force, n.has_bias = bias.defined();
+        n.native = native, n.direct = direct, n.forced = force, n.has_bias = bias.defined();
       });
 }
 
 bool offset_conv_supported(const Tensor& input, const Tensor& weight, const OptTensor& bias, const Pair& stride, const Pair& padding,
                            const Pair& dilation, bool worthwhile) {
   return offset_conv_native_tensors(input, weight, bias ? *bias : Tensor()) &&
-         offset_conv_covered(input, weight, stride, padding, dilation, worthwhile);
+         offset_conv_covered(input, weight, stride, padding, dilation, worthwhile ? dk_offset_conv_worthwhile : dk_offset_conv_supported);
 }
 
 // ---- depthwise convolution with one kernel per image and channel; the global layer ----------------

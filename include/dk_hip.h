@@ -351,6 +351,19 @@ size_t dk_offset_conv_backward_input_workspace(const dk_offset_conv_desc *desc);
 int dk_offset_conv_backward_input(const dk_offset_conv_desc *desc, const void *out_grad, const void *weight,
                                   void *input_grad, void *workspace, size_t workspace_bytes, void *stream);
 
+/* The same convolution and its input and weight gradients on few images: up to 18 output channels, any other size whose
+ * tensors hold less than 2^28 elements, stride 1 or 2 (output ((h - 1) / s + 1) x ((w - 1) / s + 1)), fp32 products and
+ * sums for every dtype, no workspace, one launch each.  dk_offset_conv_direct_worthwhile(): 1 where these are expected to
+ * beat both the kernels above and the library convolution (covered by dk_offset_conv_supported(), too few images for
+ * dk_offset_conv_worthwhile()). */
+int dk_offset_conv_direct_worthwhile(const dk_offset_conv_desc *desc);
+int dk_offset_conv_direct_forward(const dk_offset_conv_desc *desc, const void *input, const void *weight,
+                                  const void *bias, void *output, void *stream);
+int dk_offset_conv_direct_backward_input(const dk_offset_conv_desc *desc, const void *out_grad, const void *weight,
+                                         void *input_grad, void *stream);
+int dk_offset_conv_direct_backward_weight(const dk_offset_conv_desc *desc, const void *out_grad, const void *input,
+                                          void *weight_grad, void *stream);
+
 /* ---- depthwise convolution with one kernel per image and channel ------------- */
 
 /* The convolution GlobalDeformKernel2d applies with the kernels it has sampled for every image:

@@ -273,3 +273,38 @@ def test_gradients_and_module_switch():
     assert rel_err(results[2][0], results[0][0]) < 1e-5
     for got, ref in zip(results[2][1:], results[0][1:]):
         assert rel_err(got, ref) < 1e-4
+
+
+@pytest.mark.parametrize("case", [
+    # one image, three groups of six outputs; fewer channels than waves; a partial last group of four channels
+    (1, 192, 28, 28, 18, 1, "float32"), (1, 16, 7, 7, 18, 1, "float32"), (2, 80, 14, 14, 18, 1, "bfloat16"),
+    # 128 tiles of 64 pixels and more: all outputs in one workgroup; pixels no multiple of 64
+    (2, 32, 112, 112, 18, 1, "float32"), (3, 48, 53, 56, 18, 1, "float16"),
+    # the weight gradient's form for 256 channels and more, one row of pixels
+    (5, 256, 14, 14, 18, 1, "float32"), (1, 272, 1, 7, 7, 1, "float16"),
+    # stride 2: odd heights, fewer outputs than a workgroup's
+    (2, 32, 5, 14, 18, 2, "float32"), (15, 192, 28, 28, 18, 2, "bfloat16"), (1, 16, 56, 56, 1, 2, "float32"),
+])
+def test_few_images_run_on_the_vector_unit_kernels(case):
+    """Forward, input and weight gradient of batches too small for the matrix-instruction kernels against the float64
+    convolution: every sum is float32 over at most 9 * 272 (forward) or 25088 / 64 pixel groups (weight gradient) terms in
+    parts of at most 162, so 2e-6 of the largest element; 16-bit results are rounded once (2^-11, 2^-8)."""
+    from deformable_kernels.ops.deform_kernel import _lib
+    from deformable_kernels.ops.deform_kernel.functions import offset_conv
+    N, C, H, W, O, stride, dtype_name = case
+    dtype = getattr(torch, dtype_name)
+    tol = {"float32": 2e-6, "float16": 5e-4 + 2e-6, "bfloat16": 4e-3 + 2e-6}[dtype_name]
+    desc = _lib.OffsetConvDesc(N, C, O, H, W, {"float32": 0, "float16": 1, "bfloat16": 2}[dtype_name], stride)
+    assert _lib.lib().dk_offset_conv_direct_worthwhile(desc) == 1
+    g = torch.Generator().manual_seed(71)
+    dev = torch.device("cuda:0")
+    x = torch.randn(N, C, H, W, generator=g).to(dtype).to(dev).requires_grad_()
+    w = (torch.randn(O, C, 3, 3, generator=g) * 0.05).to(dtype).to(dev).requires_grad_()
+    b = torch.randn(O, generator=g).to(dtype).to(dev).requires_grad_()
+    out = offset_conv(x, w, b, stride)
+    gout = torch.randn(out.shape, generator=g).to(dtype).to(dev)
+    want, gx, gw, gb = reference(x, w, b, gout, stride=stride)
+    out.backward(gout)
+    assert rel_err(out.detach().double().cpu(), want) < tol, "forward"
+    assert rel_err(x.grad.double().cpu(), gx) < tol, "input gradient"
+    assert rel_err(w.grad.double().cpu(), gw) < tol, "weight gradient"
