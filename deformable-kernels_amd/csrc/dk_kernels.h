@@ -43,6 +43,7 @@ enum TestSwitch : unsigned {
   kNoDeformLanes = 1u << 25,    // DK_NO_DEFORM_LANES    the deformable kernels with the lanes along the channels (dk_deform_lanes.hip; those with a pixel per lane run instead)
   kForceDeformLanes = 1u << 26, // DK_FORCE_DEFORM_LANES ... wherever they apply, not only where they are the faster ones
   kNoDeformPlain = 1u << 27,    // DK_NO_DEFORM_PLAIN    the deformable kernels for calls without a rotation tensor (those that take one run instead)
+  kNoSmallBackward = 1u << 28,  // DK_NO_SMALL_BACKWARD  the one-launch gradients of small layers (dk_local_small.hip; every other switch takes them away as well)
   kNoOffsetPairs = 1u << 18,    // DK_NO_OFFSET_PAIRS    the offset branch's convolution on float32 tensors as bfloat16 pairs (the fp32 matrix-instruction forward runs instead, the other passes are not offered)
 };
 unsigned test_switches();  // dk_api.hip
@@ -191,6 +192,13 @@ size_t offset_wgrad16_workspace(int batch, int cin, int cout, int h, int w, int 
 template <typename T>
 bool offset_wgrad16(int batch, int cin, int cout, int h, int w, int stride, const T* x, const T* gout, T* gweight,
                     void* ws, hipStream_t stream);
+
+// dk_local_small.hip: the gradients of the local operator on small layers in one launch (not float64; never while a test
+// switch is set: the switches are about the kernels of the larger layers).  A null result is not computed.
+bool local_small_backward_supported(const Geo& g);
+template <typename T>
+void local_small_backward(const Geo& g, bool channels_last, const T* gout, const T* x, const T* rot, const T* filter, T* gin,
+                          T* grot, T* gfilter, hipStream_t stream);
 
 // dk_offset_direct.hip: the 3 x 3 offset convolution and its two large gradients on few images, on the vector unit
 bool offset_conv_direct_supported(int batch, int cin, int cout, int h, int w);

@@ -1,0 +1,81 @@
+"""The gradients of small layers, computed in one launch (dk_local_small.hip), against the float64 oracle: every sum is
+float32 over at most 256 channels or 2048 pixels x 9 taps in parts of at most 18 terms per lane, so the parity bars of the
+larger kernels hold (1e-5 grad input, 1e-4 the reductions, 1e-2 for 16-bit tensors)."""
+import pytest
+import torch
+
+from _cases import make_local, rel_err
+from oracle import dk_oracle as orc
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _supported(cfg, shape, scope, dtype_name, layout):
+    from deformable_kernels.ops.deform_kernel import _lib
+    N, C, H, W = shape
+    k, s, p, d = (cfg[n] for n in ("kernel_size", "stride", "padding", "dilation"))
+    desc = _lib.ConvDesc(N, C, H, W, *k, *s, *p, *d, *scope, cfg["groups"], {"float32": 0, "float16": 1, "bfloat16": 2}[dtype_name])
+    desc.layout = layout
+    return _lib.lib().dk_sample_depthwise_backward_workspace(desc) == 0
+
+
+# N, C, H, W, scope, stride, padding, dilation, groups
+CASES = [
+    (2, 32, 28, 28, 4, 1, 1, 1, 1),     # the benchmark's small layer
+    (1, 1, 1, 1, 3, 1, 1, 1, 1),        # one pixel, one channel: 63 lanes and 15 waves without work
+    (1, 17, 8, 8, 4, 1, 1, 1, 1),       # exactly one tile of 64 pixels; one channel more than waves
+    (5, 66, 5, 13, 5, 1, 1, 1, 2),      # 325 pixels, two groups of 33 channels (two shares of the channels, one short)
+    (2, 256, 32, 32, 4, 1, 1, 1, 1),    # the largest: 2048 pixels, 256 channels
+    (2, 48, 48, 8, 3, 1, 1, 1, 1),
+    (3, 40, 9, 11, 7, 1, 1, 1, 1),      # 64 table blocks: all lanes stage
+    (1, 17, 56, 56, 5, 2, 1, 1, 1),     # stride 2, even and ...
+    (2, 24, 15, 17, 4, 2, 1, 1, 3),     # ... odd planes, three groups
+    (2, 16, 12, 20, 4, 1, 0, 2, 1),     # no padding, dilation 2
+    (2, 16, 12, 20, 4, 3, 2, 1, 16),    # stride 3, padding 2, a group per channel
+]
+
+
+@pytest.mark.parametrize("layout", ["planar", "channels_last"])
+@pytest.mark.parametrize("dtype_name", ["float32", "float16", "bfloat16"])
+@pytest.mark.parametrize("case", CASES)
+def test_gradients_of_small_layers_in_one_launch(case, dtype_name, layout):
+    from deformable_kernels.ops.deform_kernel.functions import sample_depthwise
+    N, C, H, W, S, s, p, d, G = case
+    dtype = getattr(torch, dtype_name)
+    x, wt, rot, gout, cfg = make_local(N, C, H, W, 3, (S, S), s, p, d, G, 1.0, seed=5)
+    x, wt, rot, gout = [t.to(dtype) for t in (x, wt, rot, gout)]
+    if layout == "planar":
+        assert _supported(cfg, (N, C, H, W), (S, S), dtype_name, 0)
+    fmt = torch.contiguous_format if layout == "planar" else torch.channels_last
+    xg, rg, wg = [t.to(DEV).requires_grad_() for t in (x.contiguous(memory_format=fmt), rot.contiguous(memory_format=fmt), wt)]
+    out = sample_depthwise(xg, rg, wg, *(cfg[k] for k in ("kernel_size", "stride", "padding", "dilation", "groups")))
+    out.backward(gout.to(DEV).contiguous(memory_format=fmt))
+    want = orc.sample_depthwise_backward(*[t.double().numpy() for t in (gout, x, rot, wt)], **cfg)
+    again = torch.autograd.grad(sample_depthwise(xg, rg, wg, *(cfg[k] for k in ("kernel_size", "stride", "padding", "dilation", "groups"))),
+                                (xg, rg, wg), gout.to(DEV).contiguous(memory_format=fmt))
+    for got, rep, ref, tol in zip((xg.grad, rg.grad, wg.grad), again, want, (1e-5, 1e-4, 1e-4)):
+        assert rel_err(got.double().cpu(), ref) < (tol if dtype_name == "float32" else 1e-2)
+        assert torch.equal(got, rep)   # fixed order of every sum
+
+
+@pytest.mark.parametrize("clip", ["scope", (-0.4, 0.3)])
+def test_clipped_offsets_and_single_gradients(clip):
+    """The operator's own clamp, and each gradient asked for by itself: the same numbers as the larger kernels' (a test
+    switch takes the one-launch form away) within 1e-5."""
+    from deformable_kernels.ops.deform_kernel import _lib
+    from deformable_kernels.ops.deform_kernel.modules import SampleDepthwise
+    torch.manual_seed(3)
+    m = SampleDepthwise((4, 4), 24, 24, kernel_size=3, stride=1, padding=1, groups=24).to(DEV)
+    x = torch.randn(2, 24, 13, 9, device=DEV, requires_grad=True)
+    r = torch.randn(2, 18, 13, 9, device=DEV, requires_grad=True)
+    g = torch.randn(2, 24, 13, 9, device=DEV)
+    leaves = (x, r, m.weight)
+    res = torch.autograd.grad(m(x, r, clip), leaves, g)
+    for k, leaf in enumerate(leaves):
+        assert torch.equal(torch.autograd.grad(m(x, r, clip), (leaf,), g)[0], res[k])
+    with _lib.test_switches("DK_NO_IMAGE_FLAT"):
+        ref = torch.autograd.grad(m(x, r, clip), leaves, g)
+    for a, b in zip(res, ref):
+        assert rel_err(a.cpu(), b.cpu()) < 1e-5
+    assert torch.equal(res[1] == 0, ref[1] == 0)   # where the clamp is active
