@@ -2803,7 +2803,7 @@ bool run_deform_grad_input(const Geo& g, const T* gout, const T* off, const T* r
   const long n = (long)g.batch * g.channel * g.out_h * g.out_w;
   if (lanes_deform_grad_input_applies(g)) {
     absmax_kernel<T><<<kAbsParts, 256, 0, stream>>>(gout, n, gmax);
-    if (lanes_deform_grad_input<T>(g, gout, off, rot, filter, gin, gmax, stream)) return true;
+    if (lanes_deform_grad_input<T>(g, gout, off, rot, filter, gin, gmax, gmax + kAbsParts, stream)) return true;
   }
   if (tiled) {
     // workspace: the maxima of |gout|, the images' sample counts, the tiles' rows
@@ -3091,10 +3091,10 @@ bool fast_deform_grad_input(const Geo& g, const T* gout, const T* off, const T* 
 }
 
 size_t fast_deform_grad_input_workspace(const Geo& g) {
-  // absmax_kernel's per-workgroup maxima of |gout|, then the tiled form's sample count per image and its table of
-  // two rows per (image, tile)
+  // absmax_kernel's per-workgroup maxima of |gout|; then the tiled form's sample count per image and its table of two rows
+  // per (image, tile), or the lanes form's of two rows per image and 64 pixels
   return (size_t)kAbsParts * sizeof(unsigned) + (size_t)g.batch * sizeof(unsigned) +
-         (size_t)g.batch * ceil_div(g.out_h * g.out_w, 1024) * 2 * sizeof(int);
+         (size_t)g.batch * ceil_div(g.out_h * g.out_w, 64) * 2 * sizeof(int);
 }
 
 template <typename T>

@@ -81,6 +81,38 @@ __device__ __forceinline__ auto load4(rsrc_t r, unsigned off, bool wide, const T
     return V{e[0] | (e[1] << 16), e[2] | (e[3] << 16)};
 }
 
+// LDS positions: the zero-padded plane; of a band: its rows, one more (the last row's right padding), the two spare ones
+__host__ __device__ __forceinline__ int lanes_positions(int rows, int w, bool band) {
+  return band ? rows * (w + 1) + 3 : (rows + 2) * (w + 1) + 1;
+}
+
+// unit_rows of the band form: per 64 consecutive output pixels of an image the least and largest image row that their samples
+// read (K.cu:486-500); none: an empty range.  A wave per 64 pixels.
+template <typename T>
+__global__ __launch_bounds__(256) void deform_unit_rows_kernel(Geo g, const T* __restrict__ off, int2* __restrict__ unit_rows) {
+  const int out_plane = g.out_h * g.out_w, tiles = ceil_div(out_plane, 64);
+  const int id = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (id >= g.batch * tiles) return;
+  const int n = id / tiles, p = (id - n * tiles) * 64 + lane;
+  const bool live = p < out_plane;
+  const int oh = live ? p / g.out_w : 0, ow = live ? p - oh * g.out_w : 0;
+  const rsrc_t ro = plane_rsrc(off + (size_t)n * 18 * out_plane, 18 * out_plane);
+  const unsigned step = (unsigned)out_plane * (unsigned)sizeof(T);
+  int lo = 1 << 29, hi = -(1 << 29);
+#pragma unroll
+  for (int t = 0; t < 9; ++t) {
+    const unsigned o = live ? (unsigned)(2 * t * out_plane + p) * (unsigned)sizeof(T) : kOutOfRange;
+    const float h = float(oh * g.stride_h - g.pad_h + t / 3 * g.dil_h) + buf_ld(ro, o, off);
+    const float w = float(ow * g.stride_w - g.pad_w + t % 3 * g.dil_w) + buf_ld(ro, o + step, off);
+    const bool hit = live && h > -1.f && w > -1.f && h < float(g.in_h) && w < float(g.in_w);
+    const int top = (int)floorf(h);
+    lo = hit ? min(lo, top) : lo;
+    hi = hit ? max(hi, top + 1) : hi;
+  }
+  lo = wave_min(lo), hi = wave_max(hi);
+  if (lane == 0) unit_rows[id] = make_int2(lo, hi);
+}
+
 // ---------------------------------------------------------------------------
 // One workgroup per (image, group, 32 channels); its LDS holds the whole zero-padded plane.  A unit of work is 16 output pixels x one row of
 // three taps: 12 samples for each of the wave's four rows of lanes, the waves take units in turn and load the next
@@ -91,15 +123,22 @@ __device__ __forceinline__ auto load4(rsrc_t r, unsigned off, bool wide, const T
 // PLAIN: no kernel-space offsets (rot is null).  A tap then reads the scope tile at one place for all pixels: nine weights
 // per channel, a lane's two of each tap of its unit in registers, instead of two table reads and six multiply-adds per
 // sample (N=64 C=192 28x28 float16: 99 -> 82 us).
-template <typename T, int SH, int SW, bool PLAIN>
+// BAND: planes whose sums do not fit LDS for 32 channels.  A workgroup owns `band_rows` image rows of its 32 channels and
+// walks the units whose samples touch them (unit_rows: per 64 output pixels the least and largest image row that their
+// samples read); a corner pair in another band's row is added to two spare positions instead, uncounted.  A band of 19
+// rows of a 56 x 56 plane meets 61 % of the samples of the 31 - 36 rows it walks; N=64 C=144 56x56 float32, all kernels of
+// the gradient: 428 us with eight channels per workgroup and a pixel per lane (deform_grad_input_tiled_kernel, whose
+// descriptors alone take 100 vector instructions per sample and eight channels), 342 here; without a rotation tensor 417 and
+// 276, bfloat16 N=32 262 and 185.
+template <typename T, int SH, int SW, bool PLAIN, bool BAND>
 __global__ __launch_bounds__(kLnBlock) void deform_grad_input_lanes_kernel(
     Geo g, const T* __restrict__ gout, const T* __restrict__ off, const T* __restrict__ rot,
     const T* __restrict__ filter, T* __restrict__ gin, const unsigned* __restrict__ gmax_bits, unsigned inv_out_w,
-    unsigned inv_in_w, int wide) {
+    unsigned inv_in_w, int wide, int band_rows, const int2* __restrict__ unit_rows) {
   constexpr int CELLS = (SH + 1) * (SW + 1);
   extern __shared__ __align__(16) unsigned long long sums[];  // [positions][kLnPitch], then the tables
   const int H = g.in_h, W = g.in_w, RS = W + 1;               // one padding column between two rows serves both
-  const int npos = (H + 2) * RS + 1;
+  const int npos = lanes_positions(BAND ? band_rows : H, W, BAND);
   float4* tbl = reinterpret_cast<float4*>(sums + ((npos * kLnPitch + 1) & ~1));  // [CELLS][2][kLnPairs]
   __shared__ float wmax[kLnCh];
   __shared__ unsigned wave_most[kLnWaves];
@@ -107,14 +146,19 @@ __global__ __launch_bounds__(kLnBlock) void deform_grad_input_lanes_kernel(
 
   const int cpg = g.channel / g.groups;
   const int out_plane = g.out_h * g.out_w, in_plane = H * W;
-  const int chunks = ceil_div(cpg, kLnCh), total = chunks * g.batch * g.groups;
+  const int bands = BAND ? ceil_div(H, band_rows) : 1;
+  const int chunks = ceil_div(cpg, kLnCh), total = bands * chunks * g.batch * g.groups;
   const int lb = logical_block(total);
   if (lb >= total) return;
-  const int chunk = lb % chunks, z = lb / chunks;
+  const int chunk = lb % chunks, band = lb / chunks % bands, z = lb / chunks / bands;
+  // image rows r_lo .. r_hi - 1 are this workgroup's; image row r sits in LDS row r + row0
+  const int r_lo = band * band_rows, r_hi = BAND ? min(H, r_lo + band_rows) : H;
+  const int row0 = BAND ? -r_lo : 1;
+  const int spare = BAND ? band_rows * RS + 1 : 0;  // position of what is no sample of these rows (not BAND: the padding row on top)
   const int n = z / g.groups, grp = z % g.groups;
   const int j0 = chunk * kLnCh, nch = min(kLnCh, cpg - j0);
 
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int pair = lane & 15, kg = lane >> 4;  // channel pair and row of lanes
   const int si = lane & 3, sc = (lane & 15) >> 2;  // the sample a lane describes: pixel kg * 4 + si, tap column sc (< 3)
 
@@ -150,7 +194,7 @@ __global__ __launch_bounds__(kLnBlock) void deform_grad_input_lanes_kernel(
   const T* gp = gout + chan0 * out_plane;
   T* ip = gin + chan0 * in_plane;
   const size_t i_step = (size_t)g.groups * in_plane;
-  if (write_nan_if_unbounded(gmax, wmax, nch, ip, i_step, in_plane)) return;
+  if (write_nan_if_unbounded(gmax, wmax, nch, ip, i_step, in_plane)) return;  // (BAND: every band writes the same)
 
   const rsrc_t ro = plane_rsrc(off + (size_t)n * 18 * out_plane, 18 * out_plane);
   const rsrc_t rr = rot ? plane_rsrc(rot + (size_t)(n * g.groups + grp) * 18 * out_plane, 18 * out_plane) : plane_rsrc(rot, 0);
@@ -165,12 +209,18 @@ __global__ __launch_bounds__(kLnBlock) void deform_grad_input_lanes_kernel(
     return p < out_plane && h > -1.f && w > -1.f && h < fH && w < fW;
   };
 
+  auto touches = [&](int p) {  // whether samples of the 64 output pixels that p is one of read rows of this band
+    const int2 rows = unit_rows[(size_t)n * ceil_div(out_plane, 64) + (p >> 6)];
+    return rows.x < r_hi && rows.y >= r_lo;
+  };
+
   // The number of samples added to each position, kept beside its sums, and the largest, M.
   unsigned most = 1u;
   {
     unsigned* count = reinterpret_cast<unsigned*>(sums + kLnPairs);
     constexpr int CP = 2 * kLnPitch;  // words between two positions' counts
     for (int p0 = wave * 64; p0 < out_plane; p0 += kLnBlock) {
+      if (BAND && !touches(p0)) continue;
       const int p = p0 + lane;
       float dh[9], dw[9];
 #pragma unroll
@@ -183,11 +233,15 @@ __global__ __launch_bounds__(kLnBlock) void deform_grad_input_lanes_kernel(
       for (int t = 0; t < 9; ++t) {
         float h, w;
         if (!image_pos(p, t / 3, t % 3, dh[t], dw[t], h, w)) continue;
-        const int at = (((int)floorf(h) + 1) * RS + (int)floorf(w) + 1) * CP;
-        atomicAdd(count + at, 1u);
-        atomicAdd(count + at + CP, 1u);
-        atomicAdd(count + at + RS * CP, 1u);
-        atomicAdd(count + at + RS * CP + CP, 1u);
+        const int top = (int)floorf(h), at = ((top + row0) * RS + (int)floorf(w) + 1) * CP;
+        if (!BAND || (top >= r_lo && top < r_hi)) {
+          atomicAdd(count + at, 1u);
+          atomicAdd(count + at + CP, 1u);
+        }
+        if (!BAND || (top + 1 >= r_lo && top + 1 < r_hi)) {
+          atomicAdd(count + at + RS * CP, 1u);
+          atomicAdd(count + at + RS * CP + CP, 1u);
+        }
       }
     }
     __syncthreads();
@@ -246,10 +300,18 @@ __global__ __launch_bounds__(kLnBlock) void deform_grad_input_lanes_kernel(
       scale[k] = 2 * pair + k < nch ? ldexpf(1.f, min(max(30 - head - expo[k], -100), 100)) : 0.f;
     const double dscale = ldexp(1.0, 44 - (c ? expo[1] : expo[0]));
     const int lane8 = pair * 8, lane16 = pair * 16;
-    Raw nxt = load_unit(wave);
-    for (int u = wave; u < units; u += kLnWaves) {
+    auto next_unit = [&](int u) {
+      if constexpr (BAND)
+        while (u < units && !touches(u / 3 * kLnPix)) u += kLnWaves;
+      return u;
+    };
+    int next = next_unit(wave);
+    Raw nxt = load_unit(next);
+    while (next < units) {
+      const int u = next;
       const Raw cur = nxt;
-      nxt = load_unit(u + kLnWaves);
+      next = next_unit(u + kLnWaves);
+      nxt = load_unit(next);
       const int p0 = u / 3 * kLnPix, f_h = u % 3;
       // the sample this lane describes
       float h, w;
@@ -257,8 +319,11 @@ __global__ __launch_bounds__(kLnBlock) void deform_grad_input_lanes_kernel(
       const float sh = PLAIN ? 0.f : scope_coord<float>(g, f_h, cur.rh, g.centre_h);
       const float sw = PLAIN ? 0.f : scope_coord<float>(g, sc, cur.rw, g.centre_w);
       // a sample outside the scope band is added with weight zero: it is counted
-      const bool on = sc < 3 && hit, in = on && sh > -1.f && sw > -1.f && sh < float(SH) && sw < float(SW);
-      const float hf = floorf(h), wf = floorf(w), shf = floorf(sh), swf = floorf(sw);
+      const float hf = floorf(h), wf = floorf(w);
+      const int itop = (int)hf;
+      const bool in_top = !BAND || (itop >= r_lo && itop < r_hi), in_bot = !BAND || (itop + 1 >= r_lo && itop + 1 < r_hi);
+      const bool on = sc < 3 && hit && (in_top || in_bot), in = on && sh > -1.f && sw > -1.f && sh < float(SH) && sw < float(SW);
+      const float shf = floorf(sh), swf = floorf(sw);
       const float lh = on ? h - hf : 0.f, lw = on ? w - wf : 0.f;
       const float hh = on ? 1.f - lh : 0.f, hw = 1.f - lw;
       const float d00 = hh * hw, d01 = hh * lw, d10 = lh * hw, d11 = lh * lw;  // K.cu:776-789
@@ -266,8 +331,8 @@ __global__ __launch_bounds__(kLnBlock) void deform_grad_input_lanes_kernel(
       asm volatile("s_nop 1" : "+v"(e00), "+v"(e01), "+v"(e10), "+v"(e11));  // (see fma_row_lane)
       const float slh = in ? sh - shf : 0.f, slw = in ? sw - swf : 0.f;
       const int cell = in ? (((int)shf + 1) * (SW + 1) + (int)swf + 1) * (kLnCh * 16) : 0;
-      // (what is not a sample adds to the padding row on top)
-      const int top = on ? (((int)hf + 1) * RS + (int)wf + 1) * (kLnPitch * 8) : 0, bot = on ? top + RS * (kLnPitch * 8) : 0;
+      const int at = ((itop + row0) * RS + (int)wf + 1) * (kLnPitch * 8);
+      const int top = on && in_top ? at : spare * (kLnPitch * 8), bot = on && in_bot ? at + RS * (kLnPitch * 8) : spare * (kLnPitch * 8);
       const unsigned long long any = __ballot(on);
       if (any == 0ull) continue;
       float2 wt[3];  // PLAIN: the weights of the unit's taps
@@ -331,13 +396,14 @@ __global__ __launch_bounds__(kLnBlock) void deform_grad_input_lanes_kernel(
   // another.
   auto read_back = [&](auto pair_tag, int c, bool clear) {
     constexpr bool PAIR = decltype(pair_tag)::value;
-    for (int e0 = wave * 64; e0 < in_plane; e0 += kLnBlock) {
+    const int own = (r_hi - r_lo) * W;
+    for (int e0 = wave * 64; e0 < own; e0 += kLnBlock) {
       const int e = e0 + lane;
-      if (e >= in_plane) continue;
+      if (e >= own) continue;
       const int r = (int)__umulhi((unsigned)e, inv_in_w);
-      unsigned long long* cell = sums + ((r + 1) * RS + (e - r * W) + 1) * kLnPitch;
+      unsigned long long* cell = sums + ((r + (BAND ? 0 : 1)) * RS + (e - r * W) + 1) * kLnPitch;
       const unsigned long long bias = cell[kLnPairs] * kBias;
-      T* dst = ip + e;
+      T* dst = ip + r_lo * W + e;
       for (int q = 0; 2 * q < nch; ++q) {
         const unsigned long long v = cell[q];
         if constexpr (PAIR) {
@@ -370,8 +436,11 @@ __global__ __launch_bounds__(kLnBlock) void deform_grad_input_lanes_kernel(
   }
 }
 
+constexpr int kLnBandRows = 12;
+
 struct LanesPlan {
-  bool ok;
+  bool ok, band;
+  int rows;  // image rows of a workgroup
   size_t lds;
   long blocks;
 };
@@ -387,28 +456,49 @@ LanesPlan lanes_plan(const Geo& g) {
   m.ok = false;
   if (path_disabled(kNoDeformFast) || path_disabled(kNoDeformLanes)) return m;
   const long plane = (long)g.out_h * g.out_w, in_plane = (long)g.in_h * g.in_w, cpg = g.channel / g.groups;
-  // 32-bit byte offsets inside a chunk's planes (a position's LDS bounds both planes' width and height)
-  if (plane > 4096 || plane * g.groups * kLnCh * 4 >= (1L << 31) || g.in_w < 2 || g.out_w < 2) return m;
-  m.lds = (size_t)(((g.in_h + 2L) * (g.in_w + 1) + 1) * kLnPitch * 8 + (SH + 1) * (SW + 1) * kLnCh * 16 + 16);
-  if (m.lds > (size_t)kLnLds) return m;
-  m.blocks = (cpg + kLnCh - 1) / kLnCh * g.batch * g.groups;
+  // 32-bit byte offsets inside a chunk's planes, and products of a pixel and a width below 2^32 (the divisions)
+  if (plane > 16384 || in_plane > 16384 || plane * g.groups * kLnCh * 4 >= (1L << 31) || g.in_w < 2 || g.out_w < 2) return m;
+  const long tables = (long)(SH + 1) * (SW + 1) * kLnCh * 16 + 16;
+  const long fit = (kLnLds - tables) / (kLnPitch * 8);  // positions
+  m.rows = g.in_h;
+  if (lanes_positions(g.in_h, g.in_w, false) > fit) {
+    // bands of equal height.  Every band walks the rows its samples can come from: with fewer than kLnBandRows rows the
+    // walk is mostly over samples of other bands (us here / with a pixel per lane, offsets ~ N(0, 2^2): N=64 C=96 40 x 40
+    // 130 / 149, N=24 C=64 64 x 64 101 / 113, N=16 80 x 80 (12 rows) 106 / 113; 75 x 101 float16 (10 rows) 135 / 118.  Offsets
+    // ~ N(0, 5^2) widen the walk: 56 x 56 402 / 387)
+    const int most = (int)std::max(0L, (fit - 3) / (g.in_w + 1));
+    if (most < 1) return m;
+    m.rows = ceil_div(g.in_h, ceil_div(g.in_h, most));
+    m.band = true;
+    if (path_disabled(kNoDeformWindow)) return m;
+  }
+  const int bands = m.band ? ceil_div(g.in_h, m.rows) : 1;
+  m.lds = (size_t)((long)lanes_positions(m.rows, g.in_w, m.band) * kLnPitch * 8 + tables);
+  m.blocks = (cpg + kLnCh - 1) / kLnCh * g.batch * g.groups * bands;
   if (m.blocks >= (1L << 31) - 8) return m;
-  m.ok = path_disabled(kForceDeformLanes) || (plane >= 192 && in_plane <= 2 * plane && m.blocks >= 128 && cpg > kLnCh / 2);
+  m.ok = path_disabled(kForceDeformLanes) || (plane >= 192 && in_plane <= 2 * plane && m.blocks >= 128 && cpg > kLnCh / 2 &&
+                                              (!m.band || m.rows >= kLnBandRows));
   return m;
 }
 
 template <typename T, int SH, int SW>
 bool run_lanes_grad_input(const Geo& g, const T* gout, const T* off, const T* rot, const T* filter, T* gin,
-                          const unsigned* gmax, hipStream_t stream) {
+                          const unsigned* gmax, void* table, hipStream_t stream) {
   const LanesPlan m = lanes_plan<SH, SW>(g);
   if (!m.ok) return false;
   const int wide = g.out_h * g.out_w % 4 == 0 && reinterpret_cast<uintptr_t>(gout) % (4 * sizeof(T)) == 0;
   auto inverse = [](int w) { return (unsigned)(((1ull << 32) + w - 1) / w); };
   const bool plain = !rot && !path_disabled(kNoDeformPlain);
-  auto kernel = plain ? deform_grad_input_lanes_kernel<T, SH, SW, true> : deform_grad_input_lanes_kernel<T, SH, SW, false>;
+  auto kernel = m.band ? plain ? deform_grad_input_lanes_kernel<T, SH, SW, true, true> : deform_grad_input_lanes_kernel<T, SH, SW, false, true>
+                       : plain ? deform_grad_input_lanes_kernel<T, SH, SW, true, false> : deform_grad_input_lanes_kernel<T, SH, SW, false, false>;
   if (!allow_dynamic_lds(reinterpret_cast<const void*>(kernel), kLnLds)) return false;
+  int2* unit_rows = static_cast<int2*>(table);
+  if (m.band) {
+    const int tiles = g.batch * ceil_div(g.out_h * g.out_w, 64);
+    deform_unit_rows_kernel<T><<<ceil_div(tiles, 4), 256, 0, stream>>>(g, off, unit_rows);
+  }
   kernel<<<(unsigned)xcd_grid_size(m.blocks), kLnBlock, m.lds, stream>>>(g, gout, off, rot, filter, gin, gmax,
-                                                                         inverse(g.out_w), inverse(g.in_w), wide);
+                                                                         inverse(g.out_w), inverse(g.in_w), wide, m.rows, unit_rows);
   return true;
 }
 
@@ -429,8 +519,8 @@ bool lanes_deform_grad_input_applies(const Geo& g) {
 
 template <typename T>
 bool lanes_deform_grad_input(const Geo& g, const T* gout, const T* off, const T* rot, const T* filter, T* gin,
-                             const unsigned* gmax, hipStream_t stream) {
-#define CALL(SH, SW) run_lanes_grad_input<T, SH, SW>(g, gout, off, rot, filter, gin, gmax, stream)
+                             const unsigned* gmax, void* table, hipStream_t stream) {
+#define CALL(SH, SW) run_lanes_grad_input<T, SH, SW>(g, gout, off, rot, filter, gin, gmax, table, stream)
   DK_LANES_SCOPE(g, CALL)
 #undef CALL
   return false;
@@ -438,7 +528,7 @@ bool lanes_deform_grad_input(const Geo& g, const T* gout, const T* off, const T*
 
 #define DK_INSTANTIATE(T)                                                                                         \
   template bool lanes_deform_grad_input<T>(const Geo&, const T*, const T*, const T*, const T*, T*, const unsigned*, \
-                                           hipStream_t);
+                                           void*, hipStream_t);
 DK_INSTANTIATE(float)
 DK_INSTANTIATE(__half)
 DK_INSTANTIATE(bf16_t)

@@ -105,11 +105,12 @@ size_t fast_deform_grad_input_workspace(const Geo& g);
 template <typename T>
 bool fast_deform_grad_input(const Geo& g, const T* gout, const T* off, const T* rot, const T* filter, T* gin,
                             void* ws, hipStream_t stream);
-// its form with the lanes along the channels (dk_deform_lanes.hip), called behind absmax_kernel: gmax = its maxima
+// its form with the lanes along the channels (dk_deform_lanes.hip), called behind absmax_kernel: gmax = its maxima;
+// table: 8-byte aligned, two words per image and 64 output pixels
 bool lanes_deform_grad_input_applies(const Geo& g);
 template <typename T>
 bool lanes_deform_grad_input(const Geo& g, const T* gout, const T* off, const T* rot, const T* filter, T* gin,
-                             const unsigned* gmax, hipStream_t stream);
+                             const unsigned* gmax, void* table, hipStream_t stream);
 // rotation = false: gradient w.r.t. the image-space offsets
 size_t fast_deform_grad_coord_workspace(const Geo& g, bool rotation);
 template <typename T>

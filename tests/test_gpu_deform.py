@@ -424,6 +424,22 @@ def test_grad_input_with_the_lanes_along_the_channels_without_a_rotation_tensor(
     _grad_input_with_the_lanes_along_the_channels(case, dtype, rotation=False)
 
 
+LANES_BAND_CASES = [
+    (1, 34, 56, 56, 3, (4, 4), 1, 1, 1, 1, 0.7, 2.0),    # three bands of 19, 19 and 18 rows; a second chunk of two channels
+    (2, 40, 33, 33, 3, (5, 5), 1, 1, 1, 2, 1.0, 9.0),    # the first height that needs a second band; offsets of nine rows; two groups
+    (1, 18, 41, 100, 3, (4, 4), 2, 1, 1, 1, 0.5, 6.0),   # bands of ten rows and fewer at stride 2
+    (1, 20, 25, 115, 3, (3, 3), 1, 2, 2, 1, 0.7, 2.0),   # bands of a few rows, dilation, rows that no group of 64 pixels ends with
+    (1, 34, 56, 56, 3, (4, 4), 1, 1, 1, 1, 0.5, None),   # every sample in one cell of the first band: one channel per 64-bit sum; bands without samples
+]
+
+
+@pytest.mark.parametrize("rotation", [True, False])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("case", LANES_BAND_CASES)
+def test_grad_input_with_the_lanes_along_the_channels_in_bands(case, dtype, rotation):
+    _grad_input_with_the_lanes_along_the_channels(case, dtype, rotation)
+
+
 @pytest.mark.parametrize("clip", [(0.25, 0.75), (-1.5, -0.75)])
 def test_grad_input_with_the_lanes_along_the_channels_at_a_clipped_zero_rotation(clip):
     _grad_input_with_the_lanes_along_the_channels(LANES_CASES[2], torch.float32, rotation=False, clip=clip)
