@@ -47,6 +47,8 @@ int main() {
   EXPECT(dk_deformable_sample_depthwise_backward_rotation(&ok, one, one, one, one, one, nullptr, one, 1 << 20, nullptr) == DK_ERR_NULL_POINTER);
   EXPECT(dk_deformable_sample_depthwise_backward_offset_rotation(&ok, one, one, one, nullptr, one, one, one, one, 1 << 20, nullptr) == DK_ERR_NULL_POINTER);
   EXPECT(dk_deformable_sample_depthwise_backward_offset_rotation(&ok, one, one, one, one, one, one, nullptr, one, 1 << 20, nullptr) == DK_ERR_NULL_POINTER);
+  EXPECT(dk_deformable_sample_depthwise_backward_offset_filter(&ok, one, one, one, nullptr, one, one, nullptr, one, 1 << 20, nullptr) == DK_ERR_NULL_POINTER);
+  EXPECT(dk_deformable_sample_depthwise_backward_offset_filter(&ok, one, one, one, nullptr, one, one, one, one, 1, nullptr) == DK_ERR_WORKSPACE);
 
   // shapes
   dk_conv_desc bad = ok;

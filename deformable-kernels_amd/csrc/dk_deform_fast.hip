@@ -3100,6 +3100,7 @@ size_t fast_deform_grad_input_workspace(const Geo& g) {
 template <typename T>
 bool fast_deform_grad_filter(const Geo& g, const T* gout, const T* x, const T* off, const T* rot, T* gfilter,
                              void* ws, hipStream_t stream) {
+  if (!rot && plain_deform_grad_filter<T>(g, gout, x, off, gfilter, static_cast<float*>(ws), stream)) return true;
 #define CALL(SH, SW) run_deform_grad_filter<T, SH, SW>(g, gout, x, off, rot, gfilter, static_cast<float*>(ws), stream)
   DK_DISPATCH_SCOPE(g, CALL)
 #undef CALL
@@ -3107,7 +3108,8 @@ bool fast_deform_grad_filter(const Geo& g, const T* gout, const T* x, const T* o
 
 size_t fast_deform_grad_filter_workspace(const Geo& g) {  // one partial per (image, tile); the form with the most tiles
   const long tiles = std::max<long>(ceil_div(g.out_h * g.out_w, kGwPix), (long)ceil_div(g.out_w, kG2Tw) * ceil_div(g.out_h, kG2Th));
-  return (size_t)g.batch * tiles * g.channel * g.scope_h * g.scope_w * sizeof(float);
+  const size_t bytes = (size_t)g.batch * tiles * g.channel * g.scope_h * g.scope_w * sizeof(float);
+  return std::max(bytes, plain_deform_grad_filter_workspace(g));  // (the call may come without a rotation tensor)
 }
 
 #define DK_INSTANTIATE(T)                                                                              \

@@ -101,6 +101,14 @@ size_t plain_deform_grad_offset_workspace(const Geo& g);
 template <typename T>
 bool plain_deform_grad_offset(const Geo& g, const T* gout, const T* x, const T* off, const T* filter, T* goff, float* ws,
                               hipStream_t stream);
+size_t plain_deform_grad_filter_workspace(const Geo& g);
+template <typename T>
+bool plain_deform_grad_filter(const Geo& g, const T* gout, const T* x, const T* off, T* gfilter, float* ws, hipStream_t stream);
+// both from one pass over the samples
+size_t plain_deform_grad_offset_filter_workspace(const Geo& g);
+template <typename T>
+bool plain_deform_grad_offset_filter(const Geo& g, const T* gout, const T* x, const T* off, const T* filter, T* goff,
+                                     T* gfilter, float* ws, hipStream_t stream);
 size_t fast_deform_grad_input_workspace(const Geo& g);
 template <typename T>
 bool fast_deform_grad_input(const Geo& g, const T* gout, const T* off, const T* rot, const T* filter, T* gin,

@@ -276,7 +276,7 @@ struct DeformableSampleDepthwiseFunctionBackward : OpNode {
     const Tensor g = grads[0].contiguous();
     void* const s = stream_of(x);
     variable_list res(4);
-    const bool need_offset = need(1), need_rotation = has_rotation && need(2);
+    const bool need_offset = need(1), need_rotation = has_rotation && need(2), need_filter = need(3);
     if (need(0)) {
       res[0] = at::empty_like(x);
       const Workspace ws(dk_deformable_sample_depthwise_backward_data_workspace(&desc), x);
@@ -285,6 +285,15 @@ struct DeformableSampleDepthwiseFunctionBackward : OpNode {
     }
     if (need_offset) res[1] = at::empty_like(f);
     if (need_rotation) res[2] = at::empty_like(r);
+    if (need_filter) res[3] = at::empty_like(w);
+    if (need_offset && need_filter && !has_rotation) {
+      // one call for both (one pass over the samples where the library has that kernel)
+      const Workspace ws(dk_deformable_sample_depthwise_backward_offset_filter_workspace(&desc), x);
+      check(dk_deformable_sample_depthwise_backward_offset_filter(&desc, in(g), in(x), in(f), nullptr, in(w), out(res[1]), out(res[3]),
+                                                                  ws.ptr(), ws.bytes, s),
+            "deform_sample_depthwise backward_offset_filter");
+      return res;
+    }
     if (need_offset && need_rotation) {
       // one call for both coordinate gradients (one pass over the input where the library has that kernel)
       const Workspace ws(dk_deformable_sample_depthwise_backward_offset_rotation_workspace(&desc), x);
@@ -300,8 +309,7 @@ struct DeformableSampleDepthwiseFunctionBackward : OpNode {
       check(dk_deformable_sample_depthwise_backward_rotation(&desc, in(g), in(x), in(f), in(r), in(w), out(res[2]), ws.ptr(), ws.bytes, s),
             "deform_sample_depthwise backward_rotation");
     }
-    if (need(3)) {
-      res[3] = at::empty_like(w);
+    if (need_filter) {
       const Workspace ws(dk_deformable_sample_depthwise_backward_filter_workspace(&desc), x);
       check(dk_deformable_sample_depthwise_backward_filter(&desc, in(g), in(x), in(f), in(r), out(res[3]), ws.ptr(), ws.bytes, s),
             "deform_sample_depthwise backward_filter");

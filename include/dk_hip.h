@@ -235,6 +235,17 @@ int dk_deformable_sample_depthwise_backward_offset_rotation(const dk_conv_desc *
                                                             void *workspace, size_t workspace_bytes,
                                                             void *stream);
 
+/* Offset and filter gradient in one call: deformable_sample_depthwise_backward_offset_cuda and ..._backward_filter_cuda.
+ * Without a rotation tensor (NULL) one pass over the samples gives both (planes of up to about 64 x 64 pixels); otherwise
+ * the two entry points run one after the other on the stream. */
+size_t dk_deformable_sample_depthwise_backward_offset_filter_workspace(const dk_conv_desc *desc);
+int dk_deformable_sample_depthwise_backward_offset_filter(const dk_conv_desc *desc, const void *out_grad,
+                                                          const void *input, const void *offset,
+                                                          const void *rotation, const void *filter,
+                                                          void *offset_grad, void *filter_grad,
+                                                          void *workspace, size_t workspace_bytes,
+                                                          void *stream);
+
 /* ---- N-d linear sample -------------------------------------------------------
  * data [channel, shape[0..dims-1]], coord [batch, dims] in absolute index units,
  * output [batch, channel].  The reference passes `shape` as a device tensor of the

@@ -534,3 +534,61 @@ def test_a_tap_outside_the_image_takes_no_coordinate_gradient_from_the_first_pix
         touched = ~np.isfinite(w)
         assert touched.any() and not touched.all()
         assert np.array_equal(~torch.isfinite(got).cpu().numpy(), touched)
+
+
+# ---- no rotation tensor: filter gradient from the taps' sums, alone and with the offsets' gradient ----
+
+PLAIN_FILTER_CASES = [
+    (2, 1, 7, 7, 3, (3, 3), 1, 1, 1, 1, 0.0, 2.0),       # one wave, one channel
+    (1, 19, 8, 8, 3, (4, 4), 1, 1, 1, 1, 0.0, 2.0),      # a full wave; channels past the last group of eight
+    (2, 18, 9, 23, 3, (5, 5), 1, 1, 1, 2, 0.0, 3.0),     # two offset groups' channels interleaved, a ragged last wave
+    (1, 24, 33, 31, 3, (4, 4), 2, 1, 1, 1, 0.0, 2.0),    # stride 2: the input plane in four passes of the workgroup
+    (3, 12, 40, 44, 3, (3, 3), 1, 1, 1, 1, 0.0, 2.0),    # several pixel tiles
+    (2, 8, 16, 12, 3, (4, 4), 1, 2, 2, 1, 0.0, 2.0),     # dilation
+    (1, 48, 5, 5, 3, (3, 3), 1, 1, 1, 1, 0.0, 30.0),     # most taps outside the image
+]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("case", PLAIN_FILTER_CASES)
+def test_filter_gradient_without_a_rotation_tensor(case, dtype):
+    """The two ways to the filter's gradient (with the offsets' gradient in one pass, and alone) against the float64 oracle;
+    the offsets' gradient against the one formed alone.  float32: a sum of P products of rounding error 2^-24 each, relative
+    to a result of about the square root of P of them; 16 bit: the rounding of the result, 2^-11 and 2^-8."""
+    from deformable_kernels.ops.deform_kernel.functions import deform_sample_depthwise
+    N, C, H, W, k, S, s, p, d, G, rs, os_ = case
+    x, wt, rot, off, gout, cfg = make_deform(N, C, H, W, k, S, s, p, d, G, 0.0, os_, seed=9, dtype=dtype)
+    args = (cfg["kernel_size"], cfg["stride"], cfg["padding"], cfg["dilation"], cfg["groups"])
+    og, wg = off.cuda().requires_grad_(), wt.cuda().requires_grad_()
+    out = deform_sample_depthwise(x.cuda(), og, None, wg, *args)
+    both = torch.autograd.grad(out, [og, wg], gout.cuda(), retain_graph=True)
+    alone = [torch.autograd.grad(out, [t], gout.cuda(), retain_graph=True)[0] for t in (og, wg)]
+    want = _oracle((x, wt, rot, off, gout, cfg), np.float64)[4]
+    tol = {torch.float32: 1e-5, torch.float16: 2e-3, torch.bfloat16: 1.6e-2}[dtype]
+    assert rel_err(both[1].float().cpu(), want) < tol and rel_err(alone[1].float().cpu(), want) < tol
+    assert rel_err(both[0].float().cpu(), alone[0].double().cpu().numpy()) < tol
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_an_infinite_output_gradient_of_taps_outside_the_image_reaches_no_filter(dtype):
+    """The reference skips a tap outside the image (K.cu:978-984), so the output gradient of a pixel whose taps all are
+    outside is multiplied with nothing."""
+    from deformable_kernels.ops.deform_kernel.functions import deform_sample_depthwise
+    x, wt, rot, off, gout, cfg = make_deform(2, 11, 12, 10, 3, (4, 4), 1, 1, 1, 1, 0.0, 2.0, seed=3, dtype=dtype)
+    args = (cfg["kernel_size"], cfg["stride"], cfg["padding"], cfg["dilation"], cfg["groups"])
+    off[1, :, 5, 7] = 1000.0
+
+    def grads(value, wanted):
+        gout[1, :, 5, 7] = value
+        og, wg = off.cuda().requires_grad_(), wt.cuda().requires_grad_()
+        out = deform_sample_depthwise(x.cuda(), og, None, wg, *args)
+        return torch.autograd.grad(out, [t for t, on in zip((og, wg), wanted) if on], gout.cuda())
+
+    for wanted in ((True, True), (False, True)):
+        for a, b in zip(grads(float("inf"), wanted), grads(0.0, wanted)):
+            assert torch.equal(a, b)
+    gout[1, 4, 5, 7] = 0.0
+    gout[0, 4, 3, 3] = float("nan")  # ... and one that is used reaches its channel's filter only
+    og, wg = off.cuda().requires_grad_(), wt.cuda().requires_grad_()
+    got = torch.autograd.grad(deform_sample_depthwise(x.cuda(), og, None, wg, *args), [wg], gout.cuda())[0]
+    assert bool(got[4].isnan().any()) and bool(got[:4].isfinite().all()) and bool(got[5:].isfinite().all())
