@@ -116,9 +116,10 @@ int main() {
     nd.batch = b;
     total += dk_nd_linear_sample_forward_workspace(&nd) + dk_nd_linear_sample_order_bytes(&nd) +
              dk_nd_linear_sample_order_workspace(&nd) + dk_nd_linear_sample_backward_data_workspace(&nd) +
-             dk_nd_linear_sample_backward_coord_workspace(&nd);
+             dk_nd_linear_sample_backward_coord_workspace(&nd) + dk_nd_linear_sample_backward_workspace(&nd);
   }
   nd.batch = 4;
+  EXPECT(dk_nd_linear_sample_backward(&nd, one, one, one, nullptr, one, nullptr, nullptr, 0, nullptr) == DK_ERR_NULL_POINTER);
   EXPECT(dk_nd_linear_sample_forward(&nd, nullptr, one, nullptr, one, nullptr, 0, nullptr) == DK_ERR_NULL_POINTER);
 
   // offset branch

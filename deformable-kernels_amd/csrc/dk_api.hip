@@ -1130,4 +1130,24 @@ int dk_nd_linear_sample_backward_coord(const dk_nd_desc* desc, const void* out_g
   });
 }
 
+size_t dk_nd_linear_sample_backward_workspace(const dk_nd_desc* desc) {
+  if (check_nd(desc) != DK_OK) return 0;
+  return nd_backward_workspace(*desc);
+}
+
+int dk_nd_linear_sample_backward(const dk_nd_desc* desc, const void* out_grad, const void* data, const void* coord,
+                                 const void* order, void* in_grad, void* coord_grad, void* workspace, size_t workspace_bytes,
+                                 void* stream) {
+  const int rc = check_nd(desc);
+  if (rc != DK_OK) return rc;
+  if (!out_grad || !data || !coord || !in_grad || !coord_grad) return DK_ERR_NULL_POINTER;
+  const size_t need = nd_backward_workspace(*desc);
+  if (need && (!workspace || workspace_bytes < need)) return DK_ERR_WORKSPACE;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  return by_dtype(desc->dtype, [&]<typename T>() {
+    nd_backward<T>(*desc, in<T>(out_grad), in<T>(data), in<T>(coord), out<T>(in_grad), out<T>(coord_grad), workspace,
+                   static_cast<const int*>(order), s);
+  });
+}
+
 }  // extern "C"

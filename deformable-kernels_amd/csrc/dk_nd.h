@@ -17,6 +17,11 @@ void nd_grad_data(const dk_nd_desc& d, const T* gout, const T* coord, T* gdata, 
 template <typename T>
 void nd_grad_coord(const dk_nd_desc& d, const T* gout, const T* data, const T* coord, T* gcoord,
                    void* ws, const int* order, hipStream_t stream);
+// both gradients; from one read of gout where the points are sorted and the sums run on the matrix cores
+size_t nd_backward_workspace(const dk_nd_desc& d);
+template <typename T>
+void nd_backward(const dk_nd_desc& d, const T* gout, const T* data, const T* coord, T* gdata, T* gcoord, void* ws,
+                 const int* order, hipStream_t stream);
 // the points' order by cell (0 bytes when the call's kernels do not sort), to be computed once and
 // handed to the three calls above
 size_t nd_order_bytes(const dk_nd_desc& d);

@@ -831,6 +831,18 @@ __device__ __forceinline__ void wave_lds_sync() {
 
 typedef float nd4 __attribute__((ext_vector_type(4)));
 
+// Sum over the 16 lanes of a row, in each of them
+__device__ __forceinline__ float row_sum(float v) {
+  auto add = [&](auto ctrl) {
+    v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), decltype(ctrl)::value, 0xf, 0xf, true));
+  };
+  add(std::integral_constant<int, 0xB1>{});   // quad_perm [1,0,3,2]
+  add(std::integral_constant<int, 0x4E>{});   // quad_perm [2,3,0,1]
+  add(std::integral_constant<int, 0x141>{});  // row_half_mirror
+  add(std::integral_constant<int, 0x140>{});  // row_mirror
+  return v;
+}
+
 // grad coord on the sorted points with the sums over the channels on the matrix cores (fp32,
 // channel count a multiple of 64).  With the polynomial coefficients k1 .. k7 of a cell (see
 // nd_grad_coord_binned_kernel) a point's derivatives are
@@ -1058,6 +1070,166 @@ __global__ __launch_bounds__(kBlock) void nd_grad_data_mfma_kernel(NdGeo g, cons
     }
     DK_FLUSH();
 #undef DK_FLUSH
+  }
+}
+
+// Both gradients on the sorted points from one read of gout, whose 256-byte rows in the points' original order are most
+// of what either kernel above moves (fp32, channel count a multiple of 64).  Grad data as in nd_grad_data_mfma_kernel; grad
+// coord takes the operand that the products need, four channels of a point per lane: the lane multiplies them with its
+// channels' seven coefficients (28 multiply-adds), forms the three derivatives of its share and a DPP sum over the 16
+// lanes of the point completes them.  Steps of four points, the next 16 points' rows in flight; a cell's corner rows are
+// asked for before the previous cell's sums leave, so that no wait on rows is one on atomics.  A point outside the grid
+// takes part in nothing.
+template <typename T>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3, 4))) void nd_backward_mfma_kernel(
+    NdGeo g, const float* __restrict__ gout, const float* __restrict__ data_cl, const float* __restrict__ coord,
+    const int* __restrict__ order, int nbins, float* __restrict__ gdata_cl, float* __restrict__ gcoord, int per_wave) {
+  __shared__ __align__(16) float s_w[kBlock / 64][64][kClCorners];  // [wave][point][corner]
+  __shared__ float4 s_p[kBlock / 64][64];                           // [wave][point]: fractions, then derivatives; the point's row
+  __shared__ __align__(16) float s_d[kBlock / 64][kClCorners][64];  // [wave][corner][channel]
+  __shared__ int s_o[kBlock / 64][kClCorners][64];                  // [wave][corner][point]: the corner's row of data_cl
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int pr = lane & 15, kg = lane >> 4;
+  float(*wl)[kClCorners] = s_w[wave];
+  float4* pl = s_p[wave];
+  int(*ol)[64] = s_o[wave];
+  float(*dl)[64] = s_d[wave];
+  for (int c0 = 0; c0 < g.channel; c0 += 64) {
+    nd4 acc[4], k[8];  // the cell's sums (corner 4 kg + r of channel 4 pr + cb in acc[cb][r]) and coefficients (k[1 .. 7])
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[i] = nd4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < 8; ++i) k[i] = nd4{0.f, 0.f, 0.f, 0.f};
+    int at[kClCorners];
+    unsigned present = 0u;  // corners of the cell that lie on the grid
+#pragma unroll
+    for (int i = 0; i < kClCorners; ++i) at[i] = 0;
+    int cur = -2;
+    auto flush = [&] {
+      if (!present) return;
+      wave_lds_sync();
+      if (kg < 2) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          *reinterpret_cast<float4*>(&dl[4 * kg + r][4 * pr]) = make_float4(acc[0][r], acc[1][r], acc[2][r], acc[3][r]);
+      }
+      wave_lds_sync();
+#pragma unroll
+      for (int i = 0; i < kClCorners; ++i) {
+        if (present >> i & 1u) {
+          const float v = dl[i][lane];
+          if (v != 0.f) atomicAdd(gdata_cl + (size_t)at[i] * g.channel + c0 + lane, v);
+        }
+      }
+    };
+    for (int sub = 0; sub < per_wave; ++sub) {
+      BinnedWave<float> wv;
+      if (!wv.init(g, coord, order, nbins, per_wave, sub)) break;
+      const bool valid = lane < wv.npts;
+      NdPoint<float> p;
+      p.inside = false;
+#pragma unroll
+      for (int d = 0; d < DK_ND_MAX_DIMS; ++d) p.frac[d] = 0.f, p.low[d] = 0;
+      if (valid) p = load_point<float, float>(g, coord + (long)wv.id * g.dims);
+      wave_lds_sync();  // the previous chunk's reads are done
+      *reinterpret_cast<float4*>(&wl[lane][0]) = make_float4(wv.cc.w[0], wv.cc.w[1], wv.cc.w[2], wv.cc.w[3]);
+      *reinterpret_cast<float4*>(&wl[lane][4]) = make_float4(wv.cc.w[4], wv.cc.w[5], wv.cc.w[6], wv.cc.w[7]);
+      pl[lane] = make_float4(p.frac[0], p.frac[1], p.frac[2], __int_as_float(wv.id));
+#pragma unroll
+      for (int i = 0; i < kClCorners; ++i) ol[i][lane] = wv.cc.off[i];
+      wave_lds_sync();
+      auto run_end = [&](int q) {  // the keys are sorted
+        return q < wv.npts ? q + (int)__popcll(__ballot(wv.key == wv.key_of(q))) : q;
+      };
+      // a lane's channels of the points q0 + kg, + 4, + 8, + 12 of the run that ends in front of qe
+      auto load = [&](int q0, int qe, float4 (&t)[4]) {
+        if (q0 >= wv.npts || wv.key_of(q0) == nbins - 1) return;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          if (q0 + 4 * s < qe) {  // wave-uniform
+            const int q = q0 + 4 * s + kg;
+            const long id = __float_as_int(pl[q < qe ? q : q0].w);
+            t[s] = *reinterpret_cast<const float4*>(gout + id * g.channel + c0 + 4 * pr);
+          }
+        }
+      };
+      int q0 = 0, qe = run_end(0);
+      float4 nxt[4];
+#pragma unroll
+      for (int s = 0; s < 4; ++s) nxt[s] = make_float4(0.f, 0.f, 0.f, 0.f);
+      load(q0, qe, nxt);
+      while (q0 < wv.npts) {
+        const int key = wv.key_of(q0);
+        float4 now[4];
+#pragma unroll
+        for (int s = 0; s < 4; ++s) now[s] = nxt[s];
+        const int n0 = q0 + 16 < qe ? q0 + 16 : qe, ne = n0 < qe ? qe : run_end(n0);
+        if (key != cur) {
+          const unsigned on_grid = key == nbins - 1 ? 0u : (unsigned)__builtin_amdgcn_readlane((int)wv.cc.present, q0);
+          nd4 v[kClCorners];
+          int row[kClCorners];
+#pragma unroll
+          for (int i = 0; i < kClCorners; ++i) row[i] = __builtin_amdgcn_readfirstlane(ol[i][q0]);
+#pragma unroll
+          for (int i = 0; i < kClCorners; ++i) {
+            v[i] = nd4{0.f, 0.f, 0.f, 0.f};
+            if (on_grid >> i & 1u) v[i] = *reinterpret_cast<const nd4*>(data_cl + (size_t)row[i] * g.channel + c0 + 4 * pr);
+          }
+          flush();
+          load(n0, ne, nxt);
+          cur = key;
+          present = on_grid;
+#pragma unroll
+          for (int i = 0; i < kClCorners; ++i) at[i] = row[i];
+#pragma unroll
+          for (int cb = 0; cb < 4; ++cb) acc[cb] = nd4{0.f, 0.f, 0.f, 0.f};
+          // corner index: bit d = high side of dimension d (the coefficients of nd_grad_coord_binned_kernel)
+          k[1] = v[1] - v[0], k[2] = v[2] - v[0], k[3] = v[4] - v[0];
+          k[4] = (v[3] - v[2]) - k[1], k[5] = (v[5] - v[4]) - k[1], k[6] = (v[6] - v[4]) - k[2];
+          k[7] = ((v[7] - v[6]) - (v[5] - v[4])) - k[4];
+        } else {
+          load(n0, ne, nxt);
+        }
+        if (present) {
+#pragma unroll
+          for (int s = 0; s < 4; ++s) {
+            if (q0 + 4 * s < qe) {  // wave-uniform
+              const int q = q0 + 4 * s + kg;
+              const bool on = q < qe;
+              const float4 t = now[s], f = pl[on ? q : q0];
+              const float a = (on && pr < kClCorners) ? wl[q & 63][pr & (kClCorners - 1)] : 0.f;
+              float S[8];
+#pragma unroll
+              for (int m = 1; m < 8; ++m) S[m] = fmaf(t.w, k[m][3], fmaf(t.z, k[m][2], fmaf(t.y, k[m][1], t.x * k[m][0])));
+              acc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, t.x, acc[0], 0, 0, 0);
+              acc[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, t.y, acc[1], 0, 0, 0);
+              acc[2] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, t.z, acc[2], 0, 0, 0);
+              acc[3] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, t.w, acc[3], 0, 0, 0);
+              float d[3] = {fmaf(f.y * f.z, S[7], fmaf(f.z, S[5], fmaf(f.y, S[4], S[1]))),
+                            fmaf(f.x * f.z, S[7], fmaf(f.z, S[6], fmaf(f.x, S[4], S[2]))),
+                            fmaf(f.x * f.y, S[7], fmaf(f.y, S[6], fmaf(f.x, S[5], S[3])))};
+#pragma unroll
+              for (int i = 0; i < 3; ++i) d[i] = row_sum(d[i]);
+              if (on && pr == 0) *reinterpret_cast<float3*>(&pl[q]) = make_float3(d[0], d[1], d[2]);
+            }
+          }
+        }
+        q0 = n0, qe = ne;
+      }
+      wave_lds_sync();
+      if (valid) {
+        const float4 r = pl[lane];
+        const float d[3] = {r.x, r.y, r.z};
+#pragma unroll
+        for (int i = 0; i < kClMaxDims; ++i) {
+          if (i < g.dims) {
+            float* to = gcoord + (long)wv.id * g.dims + i;
+            *to = (c0 ? *to : 0.f) + (p.inside ? d[i] : 0.f);
+          }
+        }
+      }
+    }
+    flush();
   }
 }
 
@@ -1322,6 +1494,14 @@ int points_per_wave(const NdGeo& g) {
   return ppw;
 }
 
+// chunks of 64 sorted points per wave of the kernels that add to grad data: as many as keep about 16 waves per CU in the
+// grid (a cell's sums stay with the wave over its chunks)
+int chunks_per_wave(const NdGeo& g) {
+  int per_wave = 1;
+  while (per_wave < 8 && g.batch / (64L * per_wave * 2) >= 4096) per_wave *= 2;
+  return per_wave;
+}
+
 template <typename A, typename B>
 void transpose(const A* in, B* out, long rows, long cols, hipStream_t stream) {
   const dim3 grid((unsigned)((cols + 31) / 32), (unsigned)((rows + 31) / 32));
@@ -1507,9 +1687,7 @@ void nd_grad_data(const dk_nd_desc& d, const T* gout, const T* coord, T* gdata, 
       nd_fill_zero_kernel<float><<<grid_for(n_data), kBlock, 0, stream>>>(acc, n_data);
       if (const int bins = nd_bins(d)) {
         if (!order) order = sort_points<T>(g, coord, bins, static_cast<char*>(ws) + round256((size_t)n_data * sizeof(float)), stream);
-        // chunks of 64 points per wave: as many as keep about 16 waves per CU in the grid
-        int per_wave = 1;
-        while (per_wave < 8 && g.batch / (64L * per_wave * 2) >= 4096) per_wave *= 2;
+        const int per_wave = chunks_per_wave(g);
         const long waves = (g.batch + 64L * per_wave - 1) / (64L * per_wave);
         bool on_matrix_cores = false;
         if constexpr (std::is_same<T, float>::value)
@@ -1576,6 +1754,43 @@ void nd_grad_coord(const dk_nd_desc& d, const T* gout, const T* data, const T* c
   nd_grad_coord_kernel<T><<<(int)blocks, kBlock, 0, stream>>>(g, gout, data, coord, gcoord);
 }
 
+namespace {
+// Whether nd_backward_mfma_kernel serves the call (the rule of the two kernels that it takes the place of).
+bool nd_one_pass(const dk_nd_desc& d) {
+  return d.dtype == DK_F32 && d.channel % 64 == 0 && nd_bins(d) && !path_disabled(kNoNdMfma);
+}
+}  // namespace
+
+size_t nd_backward_workspace(const dk_nd_desc& d) {
+  const size_t apart = std::max(nd_grad_data_workspace(d), nd_data_cl_workspace(d));
+  return nd_one_pass(d) ? std::max(apart, 2 * round256(data_bytes(d) * sizeof(float)) + nd_sort_workspace(d)) : apart;
+}
+
+template <typename T>
+void nd_backward(const dk_nd_desc& d, const T* gout, const T* data, const T* coord, T* gdata, T* gcoord, void* ws,
+                 const int* order, hipStream_t stream) {
+  if constexpr (std::is_same<T, float>::value) {
+    // rows of gout are read as 16-byte vectors at multiples of 4 channels
+    if (nd_one_pass(d) && reinterpret_cast<uintptr_t>(gout) % 16 == 0) {
+      const NdGeo g = make_geo(d);
+      const long n_data = (long)g.channel * g.prod_shape;
+      const size_t image = round256((size_t)n_data * sizeof(float));
+      float *acc = static_cast<float*>(ws), *data_cl = reinterpret_cast<float*>(static_cast<char*>(ws) + image);
+      const int bins = nd_bins(d), per_wave = chunks_per_wave(g);
+      if (!order) order = sort_points<T>(g, coord, bins, static_cast<char*>(ws) + 2 * image, stream);
+      nd_fill_zero_kernel<float><<<grid_for(n_data), kBlock, 0, stream>>>(acc, n_data);
+      transpose<T, T>(data, data_cl, g.channel, g.prod_shape, stream);
+      const long waves = (g.batch + 64L * per_wave - 1) / (64L * per_wave);
+      nd_backward_mfma_kernel<T><<<(unsigned)((waves + 3) / 4), kBlock, 0, stream>>>(g, gout, data_cl, coord, order, bins, acc, gcoord, per_wave);
+      transpose<float, T>(acc, gdata, g.prod_shape, g.channel, stream);
+      return;
+    }
+  }
+  // one after the other, sharing the workspace (stream order)
+  nd_grad_data<T>(d, gout, coord, gdata, ws, order, stream);
+  if (d.batch > 0) nd_grad_coord<T>(d, gout, data, coord, gcoord, ws, order, stream);
+}
+
 // The sorted order of the points alone, for a caller that issues several of the three calls on
 // the same coordinates: `order` receives batch ints; ws as nd_sort_workspace() sizes it.
 size_t nd_order_bytes(const dk_nd_desc& d) { return nd_bins(d) ? (size_t)d.batch * sizeof(int) : 0; }
@@ -1596,6 +1811,7 @@ void nd_order(const dk_nd_desc& d, const T* coord, int* order, void* ws, hipStre
   template void nd_grad_data<T>(const dk_nd_desc&, const T*, const T*, T*, void*, const int*, hipStream_t); \
   template void nd_grad_coord<T>(const dk_nd_desc&, const T*, const T*, const T*, T*, void*, const int*,    \
                                  hipStream_t);                                                         \
+  template void nd_backward<T>(const dk_nd_desc&, const T*, const T*, const T*, T*, T*, void*, const int*, hipStream_t); \
   template void nd_order<T>(const dk_nd_desc&, const T*, int*, void*, hipStream_t);
 DK_INSTANTIATE(float)
 DK_INSTANTIATE(double)

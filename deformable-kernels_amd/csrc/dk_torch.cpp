@@ -364,6 +364,13 @@ struct NdLinearSampleFunctionBackward : OpNode {
     const Tensor g = grads[0].contiguous();
     void* const s = stream_of(x);
     variable_list res(2);
+    if (need(0) && need(1)) {
+      res[0] = at::empty_like(x), res[1] = at::empty_like(p);
+      const Workspace ws(dk_nd_linear_sample_backward_workspace(&desc), x);
+      check(dk_nd_linear_sample_backward(&desc, in(g), in(x), in(p), in(order), out(res[0]), out(res[1]), ws.ptr(), ws.bytes, s),
+            "nd_linear_sample backward");
+      return res;
+    }
     if (need(0)) {
       res[0] = at::empty_like(x);
       const Workspace ws(dk_nd_linear_sample_backward_data_workspace(&desc), x);

@@ -86,6 +86,8 @@ SIGNATURES = {
     "dk_nd_linear_sample_backward_data_workspace": (_SZ, [_ND]),
     "dk_nd_linear_sample_backward_data": (ctypes.c_int, [_ND, _P, _P, _P, _P, _P, _SZ, _P]),
     "dk_nd_linear_sample_backward_coord_workspace": (_SZ, [_ND]),
+    "dk_nd_linear_sample_backward_workspace": (_SZ, [_ND]),
+    "dk_nd_linear_sample_backward": (ctypes.c_int, [_ND, _P, _P, _P, _P, _P, _P, _P, _SZ, _P]),
     "dk_nd_linear_sample_backward_coord": (ctypes.c_int, [_ND, _P, _P, _P, _P, _P, _P, _SZ, _P]),
     "dk_image_depthwise_supported": (ctypes.c_int, [_CD]),
     "dk_image_depthwise_forward": (ctypes.c_int, [_CD, _P, _P, _I64P, _P, _P]),

@@ -298,6 +298,14 @@ int dk_nd_linear_sample_backward_coord(const dk_nd_desc *desc, const void *out_g
                                        void *coord_grad, void *workspace, size_t workspace_bytes,
                                        void *stream);
 
+/* Both gradients in one call; where the points are sorted and the channels are a multiple of 64 fp32 ones, from one
+ * read of out_grad.  Otherwise the two entry points above run one after the other on the stream. */
+size_t dk_nd_linear_sample_backward_workspace(const dk_nd_desc *desc);
+int dk_nd_linear_sample_backward(const dk_nd_desc *desc, const void *out_grad, const void *data,
+                                 const void *coord, const void *order, void *in_grad,
+                                 void *coord_grad, void *workspace, size_t workspace_bytes,
+                                 void *stream);
+
 /* ---- offset branch ---------------------------------------------------------- */
 
 /* The 3x3 convolution that predicts the kernel-space offsets of a LocalDeformKernel2d layer
