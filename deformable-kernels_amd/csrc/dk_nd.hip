@@ -29,7 +29,8 @@ constexpr int kClCorners = 1 << kClMaxDims;
 
 struct NdGeo {
   long batch;
-  int channel, dims;
+  int channel;
+  int dims;  // kernels with a template parameter ND > 0 set it to that, see DK_ND_BY_ANY_DIMS
   long prod_shape;
   int shape[DK_ND_MAX_DIMS];
 };
@@ -96,10 +97,11 @@ __device__ __forceinline__ bool corner(const NdGeo& g, const NdPoint<CT>& p, uns
 // ---------------------------------------------------------------------------
 // direct path
 // ---------------------------------------------------------------------------
-template <typename T>
+template <typename T, int ND>
 __global__ __launch_bounds__(kBlock) void nd_forward_kernel(NdGeo g, const T* __restrict__ data,
                                                             const T* __restrict__ coord,
                                                             T* __restrict__ out, long total) {
+  if constexpr (ND > 0) g.dims = ND;
   using CT = compute_t<T>;
   for (long id = (long)blockIdx.x * kBlock + threadIdx.x; id < total; id += (long)gridDim.x * kBlock) {
     const int c = (int)(id % g.channel);
@@ -120,10 +122,11 @@ __global__ __launch_bounds__(kBlock) void nd_forward_kernel(NdGeo g, const T* __
 
 // scatter with hardware float atomics into a zeroed buffer laid out [C][P] (cl = false) or
 // [P][C] (cl = true)
-template <typename T, typename CT, bool CL>
+template <typename T, typename CT, bool CL, int ND>
 __global__ __launch_bounds__(kBlock) void nd_grad_data_kernel(NdGeo g, const T* __restrict__ gout,
                                                               const T* __restrict__ coord,
                                                               CT* __restrict__ gdata, long total) {
+  if constexpr (ND > 0) g.dims = ND;
   for (long id = (long)blockIdx.x * kBlock + threadIdx.x; id < total; id += (long)gridDim.x * kBlock) {
     const int c = (int)(id % g.channel);
     const long b = id / g.channel;
@@ -140,11 +143,12 @@ __global__ __launch_bounds__(kBlock) void nd_grad_data_kernel(NdGeo g, const T* 
 }
 
 // one wave per point, lanes over channels, shuffle reduction
-template <typename T>
+template <typename T, int ND>
 __global__ __launch_bounds__(kBlock) void nd_grad_coord_kernel(NdGeo g, const T* __restrict__ gout,
                                                                const T* __restrict__ data,
                                                                const T* __restrict__ coord,
                                                                T* __restrict__ gcoord) {
+  if constexpr (ND > 0) g.dims = ND;
   using CT = compute_t<T>;
   const int lane = threadIdx.x & 63;
   const long waves = (long)gridDim.x * (kBlock / 64);
@@ -239,10 +243,11 @@ __device__ __forceinline__ ClCorners cl_corners(const NdGeo& g, const T* coord, 
 
 // forward: a wave owns `ppw` (a power of two <= 64) consecutive points and walks them four at a
 // time so that the corner reads of four points are in flight together
-template <typename T>
+template <typename T, int ND>
 __global__ __launch_bounds__(kBlock) void nd_forward_cl_kernel(NdGeo g, const T* __restrict__ data_cl,
                                                                const T* __restrict__ coord,
                                                                T* __restrict__ out, int ppw) {
+  g.dims = ND;
   const int lane = threadIdx.x & 63;
   const long wave0 = ((long)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6)) * ppw;
   if (wave0 >= g.batch) return;
@@ -281,11 +286,12 @@ __global__ __launch_bounds__(kBlock) void nd_forward_cl_kernel(NdGeo g, const T*
 }
 
 // grad coord: same walk; per point the lanes' partial gradients are reduced by shuffles
-template <typename T>
+template <typename T, int ND>
 __global__ __launch_bounds__(kBlock) void nd_grad_coord_cl_kernel(NdGeo g, const T* __restrict__ gout,
                                                                   const T* __restrict__ data_cl,
                                                                   const T* __restrict__ coord,
                                                                   T* __restrict__ gcoord, int ppw) {
+  g.dims = ND;
   const int lane = threadIdx.x & 63;
   const long wave0 = ((long)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6)) * ppw;
   if (wave0 >= g.batch) return;
@@ -340,10 +346,11 @@ __global__ __launch_bounds__(kBlock) void nd_grad_coord_cl_kernel(NdGeo g, const
 }
 
 // grad data: scatter into the zeroed channel-last fp32 image; one 64-channel run per atomic
-template <typename T>
+template <typename T, int ND>
 __global__ __launch_bounds__(kBlock) void nd_grad_data_cl_kernel(NdGeo g, const T* __restrict__ gout,
                                                                  const T* __restrict__ coord,
                                                                  float* __restrict__ gdata_cl, int ppw) {
+  g.dims = ND;
   const int lane = threadIdx.x & 63;
   const long wave0 = ((long)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6)) * ppw;
   if (wave0 >= g.batch) return;
@@ -587,9 +594,10 @@ __device__ __forceinline__ int point_bin(const NdGeo& g, const T* coord_b, int n
   return key;
 }
 
-template <typename T>
+template <typename T, int ND>
 __global__ __launch_bounds__(kBlock) void nd_bin_keys_kernel(NdGeo g, const T* __restrict__ coord, int nbins,
                                                              unsigned* __restrict__ keys) {
+  g.dims = ND;
   const long b = (long)blockIdx.x * kBlock + threadIdx.x;
   if (b < g.batch) keys[b] = (unsigned)point_bin<T>(g, coord + b * g.dims, nbins);
 }
@@ -627,11 +635,12 @@ __device__ __forceinline__ void settle(float (&v)[kClCorners]) {
   asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), "+v"(v[7]));
 }
 
-template <typename T>
+template <typename T, int ND>
 __global__ __launch_bounds__(kBlock) void nd_forward_binned_kernel(NdGeo g, const T* __restrict__ data_cl,
                                                                    const T* __restrict__ coord,
                                                                    const int* __restrict__ order, int nbins,
                                                                    T* __restrict__ out) {
+  g.dims = ND;
   BinnedWave<T> wv;
   if (!wv.init(g, coord, order, nbins)) return;
   const int lane = threadIdx.x & 63, ncorner = 1 << g.dims;
@@ -659,11 +668,12 @@ __global__ __launch_bounds__(kBlock) void nd_forward_binned_kernel(NdGeo g, cons
   }
 }
 
-template <typename T>
+template <typename T, int ND>
 __global__ __launch_bounds__(kBlock) void nd_grad_data_binned_kernel(NdGeo g, const T* __restrict__ gout,
                                                                      const T* __restrict__ coord,
                                                                      const int* __restrict__ order, int nbins,
                                                                      float* __restrict__ gdata_cl, int per_wave) {
+  g.dims = ND;
   const int lane = threadIdx.x & 63, ncorner = 1 << g.dims;
   constexpr int PU = 8;  // output-gradient rows in flight
   for (int c0 = 0; c0 < g.channel; c0 += 64) {
@@ -741,12 +751,13 @@ __global__ __launch_bounds__(kBlock) void nd_grad_data_binned_kernel(NdGeo g, co
 // skipping them amounts to), so that a point's three partial derivatives cost nine fused
 // multiply-adds per channel instead of eight corner products, and three wave reductions
 // instead of eight.
-template <typename T>
+template <typename T, int ND>
 __global__ __launch_bounds__(kBlock) void nd_grad_coord_binned_kernel(NdGeo g, const T* __restrict__ gout,
                                                                       const T* __restrict__ data_cl,
                                                                       const T* __restrict__ coord,
                                                                       const int* __restrict__ order, int nbins,
                                                                       T* __restrict__ gcoord) {
+  g.dims = ND;
   BinnedWave<T> wv;
   if (!wv.init(g, coord, order, nbins)) return;
   const int lane = threadIdx.x & 63;
@@ -854,12 +865,13 @@ __device__ __forceinline__ float row_sum(float v) {
 // the four lanes of a point read 64 contiguous bytes of its row with each of their four 16-byte loads; the
 // coefficients go through the wave's LDS slice).  The three wave reductions per point and channel
 // block of the VALU kernel (75 VALU instructions per point) become one MFMA per point.
-template <typename T>
+template <typename T, int ND>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 4))) void nd_grad_coord_mfma_kernel(NdGeo g, const float* __restrict__ gout,
                                                                     const float* __restrict__ data_cl,
                                                                     const float* __restrict__ coord,
                                                                     const int* __restrict__ order, int nbins,
                                                                     float* __restrict__ gcoord) {
+  g.dims = ND;
   __shared__ __align__(16) float s_coef[kBlock / 64][8][64];  // [wave][m][channel of the block]
   __shared__ __align__(16) float s_sum[kBlock / 64][16][16];  // [wave][point of the batch][m]
   BinnedWave<float> wv;
@@ -990,11 +1002,12 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 4))) 
 // channels 4 (l % 16) .. + 3 of that point's gout row (one 16-byte load; the 16 lanes of a point read
 // its 256-byte row), one MFMA per channel of the quad.  The VALU kernel spends its time on the
 // per-point broadcasts (v_readlane of eight weights, key and row index per point).
-template <typename T>
+template <typename T, int ND>
 __global__ __launch_bounds__(kBlock) void nd_grad_data_mfma_kernel(NdGeo g, const float* __restrict__ gout,
                                                                    const float* __restrict__ coord,
                                                                    const int* __restrict__ order, int nbins,
                                                                    float* __restrict__ gdata_cl, int per_wave) {
+  g.dims = ND;
   __shared__ __align__(16) float s_w[kBlock / 64][64][kClCorners];  // [wave][point][corner]
   __shared__ __align__(16) float s_d[kBlock / 64][kClCorners][64];  // [wave][corner][channel]
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1080,10 +1093,11 @@ __global__ __launch_bounds__(kBlock) void nd_grad_data_mfma_kernel(NdGeo g, cons
 // lanes of the point completes them.  Steps of four points, the next 16 points' rows in flight; a cell's corner rows are
 // asked for before the previous cell's sums leave, so that no wait on rows is one on atomics.  A point outside the grid
 // takes part in nothing.
-template <typename T>
+template <typename T, int ND>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3, 4))) void nd_backward_mfma_kernel(
     NdGeo g, const float* __restrict__ gout, const float* __restrict__ data_cl, const float* __restrict__ coord,
     const int* __restrict__ order, int nbins, float* __restrict__ gdata_cl, float* __restrict__ gcoord, int per_wave) {
+  g.dims = ND;
   __shared__ __align__(16) float s_w[kBlock / 64][64][kClCorners];  // [wave][point][corner]
   __shared__ float4 s_p[kBlock / 64][64];                           // [wave][point]: fractions, then derivatives; the point's row
   __shared__ __align__(16) float s_d[kBlock / 64][kClCorners][64];  // [wave][corner][channel]
@@ -1240,11 +1254,12 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3, 4))) 
 // its points' corner weights) and the channels 4 (l % 16) .. + 3 of corner row 4 step + l / 16 (one
 // 16-byte load per run), two steps of v_mfma_f32_16x16x4_f32 per channel of the quad; the results
 // leave as 16-byte stores, the 16 lanes of a point writing its 256-byte row.
-template <typename T>
+template <typename T, int ND>
 __global__ __launch_bounds__(kBlock) void nd_forward_mfma_kernel(NdGeo g, const float* __restrict__ data_cl,
                                                                  const float* __restrict__ coord,
                                                                  const int* __restrict__ order, int nbins,
                                                                  float* __restrict__ out) {
+  g.dims = ND;
   __shared__ __align__(16) float s_w[kBlock / 64][64][kClCorners];  // [wave][point][corner]
   BinnedWave<float> wv;
   if (!wv.init(g, coord, order, nbins)) return;
@@ -1465,6 +1480,23 @@ __global__ __launch_bounds__(kBlock) void radix_scatter_kernel(const unsigned* _
   }
 }
 
+// Launches with the number of sampling dimensions as the constant ND (DK_ND_BY_ANY_DIMS: 0 above three, g.dims says).  With
+// the loops over the dimensions of a point's cell, corners and key unrolled over DK_ND_MAX_DIMS and a test in each, the
+// corners alone are eight times eight of them per point.  us a call with g.dims / with the constant: 2^20 points x 64 channels
+// of a 32^3 volume forward 151 / 137, grad coord 149 / 112, both gradients 228 / 199 (the kernel); 3 * 10^5 x 7 of 40^3, unsorted, grad
+// coord 956 / 144; 20000 x 100 of 96 x 80 forward 26 / 16.
+#define DK_ND_BY_DIMS(dims, ...)                        \
+  do {                                                  \
+    if ((dims) == 1) { constexpr int ND = 1; __VA_ARGS__; }      \
+    else if ((dims) == 2) { constexpr int ND = 2; __VA_ARGS__; } \
+    else { constexpr int ND = 3; __VA_ARGS__; }                  \
+  } while (0)
+#define DK_ND_BY_ANY_DIMS(dims, ...)                       \
+  do {                                                     \
+    if ((dims) <= 3) { DK_ND_BY_DIMS(dims, __VA_ARGS__); } \
+    else { constexpr int ND = 0; __VA_ARGS__; }            \
+  } while (0)
+
 inline int grid_for(long total) {
   long b = (total + kBlock - 1) / kBlock;
   if (b > 1048576) b = 1048576;
@@ -1578,7 +1610,7 @@ const int* sort_points(const NdGeo& g, const T* coord, int bins, void* sort_ws, 
   unsigned* keys = reinterpret_cast<unsigned*>(base);
   unsigned* keys_sorted = reinterpret_cast<unsigned*>(base + n4);
   int* order = reinterpret_cast<int*>(base + 2 * n4);
-  nd_bin_keys_kernel<T><<<(unsigned)((g.batch + kBlock - 1) / kBlock), kBlock, 0, stream>>>(g, coord, bins, keys);
+  DK_ND_BY_DIMS(g.dims, nd_bin_keys_kernel<T, ND><<<(unsigned)((g.batch + kBlock - 1) / kBlock), kBlock, 0, stream>>>(g, coord, bins, keys));
   {
     // two radix passes of half the key bits each (one pass for keys of up to 9 bits)
     const int bits = key_bits(bins);
@@ -1625,21 +1657,21 @@ void nd_forward(const dk_nd_desc& d, const T* data, const T* coord, T* out, void
         if constexpr (std::is_same<T, float>::value) {
           // rows of out are written as 16-byte vectors at multiples of 4 channels
           if (g.channel % 64 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0 && !path_disabled(kNoNdMfma)) {
-            nd_forward_mfma_kernel<T><<<(unsigned)((g.batch + 255) / 256), kBlock, 0, stream>>>(g, data_cl, coord, order, bins, out);
+            DK_ND_BY_DIMS(g.dims, nd_forward_mfma_kernel<T, ND><<<(unsigned)((g.batch + 255) / 256), kBlock, 0, stream>>>(g, data_cl, coord, order, bins, out));
             return;
           }
         }
-        nd_forward_binned_kernel<T><<<(unsigned)((g.batch + 255) / 256), kBlock, 0, stream>>>(g, data_cl, coord, order, bins, out);
+        DK_ND_BY_DIMS(g.dims, nd_forward_binned_kernel<T, ND><<<(unsigned)((g.batch + 255) / 256), kBlock, 0, stream>>>(g, data_cl, coord, order, bins, out));
         return;
       }
       const int ppw = points_per_wave(g);
       const long waves = (g.batch + ppw - 1) / ppw;
-      nd_forward_cl_kernel<T><<<(unsigned)((waves + 3) / 4), kBlock, 0, stream>>>(g, data_cl, coord, out, ppw);
+      DK_ND_BY_DIMS(g.dims, nd_forward_cl_kernel<T, ND><<<(unsigned)((waves + 3) / 4), kBlock, 0, stream>>>(g, data_cl, coord, out, ppw));
       return;
     }
   }
   const long total = g.batch * g.channel;
-  nd_forward_kernel<T><<<grid_for(total), kBlock, 0, stream>>>(g, data, coord, out, total);
+  DK_ND_BY_ANY_DIMS(g.dims, nd_forward_kernel<T, ND><<<grid_for(total), kBlock, 0, stream>>>(g, data, coord, out, total));
 }
 
 size_t nd_grad_data_workspace(const dk_nd_desc& d) {
@@ -1695,14 +1727,14 @@ void nd_grad_data(const dk_nd_desc& d, const T* gout, const T* coord, T* gdata, 
           on_matrix_cores = g.channel % 64 == 0 && reinterpret_cast<uintptr_t>(gout) % 16 == 0 && !path_disabled(kNoNdMfma);
         if (on_matrix_cores) {
           if constexpr (std::is_same<T, float>::value)
-            nd_grad_data_mfma_kernel<T><<<(unsigned)((waves + 3) / 4), kBlock, 0, stream>>>(g, gout, coord, order, bins, acc, per_wave);
+            DK_ND_BY_DIMS(g.dims, nd_grad_data_mfma_kernel<T, ND><<<(unsigned)((waves + 3) / 4), kBlock, 0, stream>>>(g, gout, coord, order, bins, acc, per_wave));
         } else {
-          nd_grad_data_binned_kernel<T><<<(unsigned)((waves + 3) / 4), kBlock, 0, stream>>>(g, gout, coord, order, bins, acc, per_wave);
+          DK_ND_BY_DIMS(g.dims, nd_grad_data_binned_kernel<T, ND><<<(unsigned)((waves + 3) / 4), kBlock, 0, stream>>>(g, gout, coord, order, bins, acc, per_wave));
         }
       } else {
         const int ppw = points_per_wave(g);
         const long waves = (g.batch + ppw - 1) / ppw;
-        nd_grad_data_cl_kernel<T><<<(unsigned)((waves + 3) / 4), kBlock, 0, stream>>>(g, gout, coord, acc, ppw);
+        DK_ND_BY_DIMS(g.dims, nd_grad_data_cl_kernel<T, ND><<<(unsigned)((waves + 3) / 4), kBlock, 0, stream>>>(g, gout, coord, acc, ppw));
       }
       transpose<float, T>(acc, gdata, g.prod_shape, g.channel, stream);
       return;
@@ -1712,7 +1744,7 @@ void nd_grad_data(const dk_nd_desc& d, const T* gout, const T* coord, T* gdata, 
   CT* acc = direct ? reinterpret_cast<CT*>(gdata) : static_cast<CT*>(ws);
   nd_fill_zero_kernel<CT><<<grid_for(n_data), kBlock, 0, stream>>>(acc, n_data);
   if (total > 0)
-    nd_grad_data_kernel<T, CT, false><<<grid_for(total), kBlock, 0, stream>>>(g, gout, coord, acc, total);
+    DK_ND_BY_ANY_DIMS(g.dims, nd_grad_data_kernel<T, CT, false, ND><<<grid_for(total), kBlock, 0, stream>>>(g, gout, coord, acc, total));
   if (!direct) nd_convert_kernel<CT, T><<<grid_for(n_data), kBlock, 0, stream>>>(acc, gdata, n_data);
 }
 
@@ -1736,22 +1768,22 @@ void nd_grad_coord(const dk_nd_desc& d, const T* gout, const T* data, const T* c
         if constexpr (std::is_same<T, float>::value) {
           // rows of gout are read as 16-byte vectors at multiples of 16 channels
           if (g.channel % 64 == 0 && reinterpret_cast<uintptr_t>(gout) % 16 == 0 && !path_disabled(kNoNdMfma)) {
-            nd_grad_coord_mfma_kernel<T><<<(unsigned)((g.batch + 255) / 256), kBlock, 0, stream>>>(g, gout, data_cl, coord, order, bins, gcoord);
+            DK_ND_BY_DIMS(g.dims, nd_grad_coord_mfma_kernel<T, ND><<<(unsigned)((g.batch + 255) / 256), kBlock, 0, stream>>>(g, gout, data_cl, coord, order, bins, gcoord));
             return;
           }
         }
-        nd_grad_coord_binned_kernel<T><<<(unsigned)((g.batch + 255) / 256), kBlock, 0, stream>>>(g, gout, data_cl, coord, order, bins, gcoord);
+        DK_ND_BY_DIMS(g.dims, nd_grad_coord_binned_kernel<T, ND><<<(unsigned)((g.batch + 255) / 256), kBlock, 0, stream>>>(g, gout, data_cl, coord, order, bins, gcoord));
         return;
       }
       const int ppw = points_per_wave(g);
       const long waves = (g.batch + ppw - 1) / ppw;
-      nd_grad_coord_cl_kernel<T><<<(unsigned)((waves + 3) / 4), kBlock, 0, stream>>>(g, gout, data_cl, coord, gcoord, ppw);
+      DK_ND_BY_DIMS(g.dims, nd_grad_coord_cl_kernel<T, ND><<<(unsigned)((waves + 3) / 4), kBlock, 0, stream>>>(g, gout, data_cl, coord, gcoord, ppw));
       return;
     }
   }
   long blocks = (g.batch + 3) / 4;
   if (blocks > 65536) blocks = 65536;
-  nd_grad_coord_kernel<T><<<(int)blocks, kBlock, 0, stream>>>(g, gout, data, coord, gcoord);
+  DK_ND_BY_ANY_DIMS(g.dims, nd_grad_coord_kernel<T, ND><<<(int)blocks, kBlock, 0, stream>>>(g, gout, data, coord, gcoord));
 }
 
 namespace {
@@ -1781,7 +1813,7 @@ void nd_backward(const dk_nd_desc& d, const T* gout, const T* data, const T* coo
       nd_fill_zero_kernel<float><<<grid_for(n_data), kBlock, 0, stream>>>(acc, n_data);
       transpose<T, T>(data, data_cl, g.channel, g.prod_shape, stream);
       const long waves = (g.batch + 64L * per_wave - 1) / (64L * per_wave);
-      nd_backward_mfma_kernel<T><<<(unsigned)((waves + 3) / 4), kBlock, 0, stream>>>(g, gout, data_cl, coord, order, bins, acc, gcoord, per_wave);
+      DK_ND_BY_DIMS(g.dims, nd_backward_mfma_kernel<T, ND><<<(unsigned)((waves + 3) / 4), kBlock, 0, stream>>>(g, gout, data_cl, coord, order, bins, acc, gcoord, per_wave));
       transpose<float, T>(acc, gdata, g.prod_shape, g.channel, stream);
       return;
     }
