@@ -249,7 +249,7 @@ __global__ __launch_bounds__(kBlock) void nd_forward_cl_kernel(NdGeo g, const T*
                                                                T* __restrict__ out, int ppw) {
   g.dims = ND;
   const int lane = threadIdx.x & 63;
-  const long wave0 = ((long)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6)) * ppw;
+  const long wave0 = ((long)blockIdx.x * (kBlock / 64) + __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6)) * ppw;
   if (wave0 >= g.batch) return;
   const int npts = (int)min((long)ppw, g.batch - wave0);
   const ClCorners mine = cl_corners<T>(g, coord, wave0 + lane, lane < npts);
@@ -293,7 +293,7 @@ __global__ __launch_bounds__(kBlock) void nd_grad_coord_cl_kernel(NdGeo g, const
                                                                   T* __restrict__ gcoord, int ppw) {
   g.dims = ND;
   const int lane = threadIdx.x & 63;
-  const long wave0 = ((long)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6)) * ppw;
+  const long wave0 = ((long)blockIdx.x * (kBlock / 64) + __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6)) * ppw;
   if (wave0 >= g.batch) return;
   const int npts = (int)min((long)ppw, g.batch - wave0);
   const bool valid = lane < npts;
@@ -352,7 +352,7 @@ __global__ __launch_bounds__(kBlock) void nd_grad_data_cl_kernel(NdGeo g, const 
                                                                  float* __restrict__ gdata_cl, int ppw) {
   g.dims = ND;
   const int lane = threadIdx.x & 63;
-  const long wave0 = ((long)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6)) * ppw;
+  const long wave0 = ((long)blockIdx.x * (kBlock / 64) + __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6)) * ppw;
   if (wave0 >= g.batch) return;
   const int npts = (int)min((long)ppw, g.batch - wave0);
   const ClCorners mine = cl_corners<T>(g, coord, wave0 + lane, lane < npts);
@@ -602,7 +602,9 @@ __global__ __launch_bounds__(kBlock) void nd_bin_keys_kernel(NdGeo g, const T* _
   if (b < g.batch) keys[b] = (unsigned)point_bin<T>(g, coord + b * g.dims, nbins);
 }
 
-// What a wave of the binned kernels knows about its 64 sorted points: lane q holds point q.
+// What a wave of the binned kernels knows about its 64 sorted points: lane q holds point q.  An XCD walks one contiguous
+// eighth of the sorted points, so that the corner rows of neighbouring cells are read into one L2 (2^20 points of a 32^3 volume of 64
+// channels, 8 MB: forward 137 -> 131 us a call).
 template <typename T>
 struct BinnedWave {
   int npts, id, key;
@@ -611,7 +613,9 @@ struct BinnedWave {
   __device__ __forceinline__ bool init(const NdGeo& g, const T* coord, const int* order, int nbins,
                                        int per_wave = 1, int sub = 0) {
     const int lane = threadIdx.x & 63;
-    const long wave0 = (((long)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6)) * per_wave + sub) * 64;
+    // (the same for the wave's lanes, which the compiler does not see: loops and row addresses would be per lane)
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const long wave0 = (((long)logical_block((int)gridDim.x) * (kBlock / 64) + wave) * per_wave + sub) * 64;
     if (wave0 >= g.batch) return false;
     npts = (int)min(64L, g.batch - wave0);
     const bool valid = lane < npts;
@@ -1090,46 +1094,49 @@ __global__ __launch_bounds__(kBlock) void nd_grad_data_mfma_kernel(NdGeo g, cons
 // of what either kernel above moves (fp32, channel count a multiple of 64).  Grad data as in nd_grad_data_mfma_kernel; grad
 // coord takes the operand that the products need, four channels of a point per lane: the lane multiplies them with its
 // channels' seven coefficients (28 multiply-adds), forms the three derivatives of its share and a DPP sum over the 16
-// lanes of the point completes them.  Steps of four points, the next 16 points' rows in flight; a cell's corner rows are
-// asked for before the previous cell's sums leave, so that no wait on rows is one on atomics.  A point outside the grid
-// takes part in nothing.
+// lanes of the point completes them.  What bounds it is the chain of a wave from one cell to the next: the rows of the next 16
+// points and the corner rows of the next cell (a channel per lane; the coefficients take their four-channel form through
+// LDS) are asked for before the present ones are worked off, always the same number of loads, so that a wait counts
+// down to the older ones: 2^20 points x 64 channels of a 32^3 volume 161 us, 195 with loads by need and a cell's rows when
+// it begins (the two kernels above: 114 + 95).  Four waves per SIMD hold the grid of one round; 76 bytes per lane of set-up spill
+// for that.  A point outside the grid takes part in nothing.
 template <typename T, int ND>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3, 4))) void nd_backward_mfma_kernel(
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 4))) void nd_backward_mfma_kernel(
     NdGeo g, const float* __restrict__ gout, const float* __restrict__ data_cl, const float* __restrict__ coord,
     const int* __restrict__ order, int nbins, float* __restrict__ gdata_cl, float* __restrict__ gcoord, int per_wave) {
   g.dims = ND;
+  constexpr int NC = 1 << ND;
+  constexpr int KS = ND == 3 ? 7 : ND == 2 ? 3 : 1;                 // coefficients besides the constant one
   __shared__ __align__(16) float s_w[kBlock / 64][64][kClCorners];  // [wave][point][corner]
   __shared__ float4 s_p[kBlock / 64][64];                           // [wave][point]: fractions, then derivatives; the point's row
-  __shared__ __align__(16) float s_d[kBlock / 64][kClCorners][64];  // [wave][corner][channel]
-  __shared__ int s_o[kBlock / 64][kClCorners][64];                  // [wave][corner][point]: the corner's row of data_cl
+  __shared__ __align__(16) float s_d[kBlock / 64][kClCorners][64];  // [wave][corner][channel], or the coefficients [m][channel]
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int pr = lane & 15, kg = lane >> 4;
   float(*wl)[kClCorners] = s_w[wave];
   float4* pl = s_p[wave];
-  int(*ol)[64] = s_o[wave];
   float(*dl)[64] = s_d[wave];
   for (int c0 = 0; c0 < g.channel; c0 += 64) {
-    nd4 acc[4], k[8];  // the cell's sums (corner 4 kg + r of channel 4 pr + cb in acc[cb][r]) and coefficients (k[1 .. 7])
+    nd4 acc[4], k[KS];  // the cell's sums (corner 4 kg + r of channel 4 pr + cb in acc[cb][r]) and coefficients
 #pragma unroll
     for (int i = 0; i < 4; ++i) acc[i] = nd4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int i = 0; i < 8; ++i) k[i] = nd4{0.f, 0.f, 0.f, 0.f};
-    int at[kClCorners];
+    for (int i = 0; i < KS; ++i) k[i] = nd4{0.f, 0.f, 0.f, 0.f};
+    int at[NC];
     unsigned present = 0u;  // corners of the cell that lie on the grid
 #pragma unroll
-    for (int i = 0; i < kClCorners; ++i) at[i] = 0;
+    for (int i = 0; i < NC; ++i) at[i] = 0;
     int cur = -2;
     auto flush = [&] {
       if (!present) return;
       wave_lds_sync();
-      if (kg < 2) {
+      if (4 * kg < NC) {
 #pragma unroll
         for (int r = 0; r < 4; ++r)
           *reinterpret_cast<float4*>(&dl[4 * kg + r][4 * pr]) = make_float4(acc[0][r], acc[1][r], acc[2][r], acc[3][r]);
       }
       wave_lds_sync();
 #pragma unroll
-      for (int i = 0; i < kClCorners; ++i) {
+      for (int i = 0; i < NC; ++i) {
         if (present >> i & 1u) {
           const float v = dl[i][lane];
           if (v != 0.f) atomicAdd(gdata_cl + (size_t)at[i] * g.channel + c0 + lane, v);
@@ -1149,61 +1156,74 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3, 4))) 
       *reinterpret_cast<float4*>(&wl[lane][0]) = make_float4(wv.cc.w[0], wv.cc.w[1], wv.cc.w[2], wv.cc.w[3]);
       *reinterpret_cast<float4*>(&wl[lane][4]) = make_float4(wv.cc.w[4], wv.cc.w[5], wv.cc.w[6], wv.cc.w[7]);
       pl[lane] = make_float4(p.frac[0], p.frac[1], p.frac[2], __int_as_float(wv.id));
-#pragma unroll
-      for (int i = 0; i < kClCorners; ++i) ol[i][lane] = wv.cc.off[i];
       wave_lds_sync();
       auto run_end = [&](int q) {  // the keys are sorted
         return q < wv.npts ? q + (int)__popcll(__ballot(wv.key == wv.key_of(q))) : q;
       };
       // a lane's channels of the points q0 + kg, + 4, + 8, + 12 of the run that ends in front of qe
-      auto load = [&](int q0, int qe, float4 (&t)[4]) {
-        if (q0 >= wv.npts || wv.key_of(q0) == nbins - 1) return;
+      float4 nxt[4];
+      auto load = [&](int q0, int qe) {
+        const int last = min(q0, wv.npts - 1);
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
-          if (q0 + 4 * s < qe) {  // wave-uniform
-            const int q = q0 + 4 * s + kg;
-            const long id = __float_as_int(pl[q < qe ? q : q0].w);
-            t[s] = *reinterpret_cast<const float4*>(gout + id * g.channel + c0 + 4 * pr);
-          }
+          const int q = q0 + 4 * s + kg;
+          const long id = __float_as_int(pl[q < qe ? q : last].w);
+          nxt[s] = *reinterpret_cast<const float4*>(gout + id * g.channel + c0 + 4 * pr);
         }
       };
-      int q0 = 0, qe = run_end(0);
-      float4 nxt[4];
+      // the corner rows of point q's cell, channel c0 + lane (row 0 for a corner off the grid)
+      float v[NC];
+      int row[NC];
+      unsigned on_grid = 0u;
+      auto load_cell = [&](int q) {
+        const int from = min(q, wv.npts - 1);
+        on_grid = (unsigned)__builtin_amdgcn_readlane((int)wv.cc.present, from);
 #pragma unroll
-      for (int s = 0; s < 4; ++s) nxt[s] = make_float4(0.f, 0.f, 0.f, 0.f);
-      load(q0, qe, nxt);
+        for (int i = 0; i < NC; ++i) row[i] = wv.off_of(i, from);
+#pragma unroll
+        for (int i = 0; i < NC; ++i) v[i] = data_cl[(size_t)row[i] * g.channel + c0 + lane];
+      };
+      int q0 = 0, qe = run_end(0);
+      bool start = true;  // of a run
+      load_cell(q0);
+      load(q0, qe);
       while (q0 < wv.npts) {
-        const int key = wv.key_of(q0);
         float4 now[4];
 #pragma unroll
         for (int s = 0; s < 4; ++s) now[s] = nxt[s];
-        const int n0 = q0 + 16 < qe ? q0 + 16 : qe, ne = n0 < qe ? qe : run_end(n0);
-        if (key != cur) {
-          const unsigned on_grid = key == nbins - 1 ? 0u : (unsigned)__builtin_amdgcn_readlane((int)wv.cc.present, q0);
-          nd4 v[kClCorners];
-          int row[kClCorners];
+        if (start) {
+          const int key = wv.key_of(q0);
+          if (key != cur) {
+            flush();
+            cur = key;
+            present = on_grid;
 #pragma unroll
-          for (int i = 0; i < kClCorners; ++i) row[i] = __builtin_amdgcn_readfirstlane(ol[i][q0]);
+            for (int i = 0; i < NC; ++i) at[i] = row[i], v[i] = on_grid >> i & 1u ? v[i] : 0.f;
 #pragma unroll
-          for (int i = 0; i < kClCorners; ++i) {
-            v[i] = nd4{0.f, 0.f, 0.f, 0.f};
-            if (on_grid >> i & 1u) v[i] = *reinterpret_cast<const nd4*>(data_cl + (size_t)row[i] * g.channel + c0 + 4 * pr);
+            for (int cb = 0; cb < 4; ++cb) acc[cb] = nd4{0.f, 0.f, 0.f, 0.f};
+            // corner index: bit d = high side of dimension d (the coefficients of nd_grad_coord_binned_kernel)
+            wave_lds_sync();
+            const float k1 = v[1] - v[0];
+            dl[0][lane] = k1;
+            if constexpr (ND > 1) {
+              const float k2 = v[2] - v[0], k4 = (v[3] - v[2]) - k1;
+              dl[1][lane] = k2;
+              dl[2][lane] = k4;
+              if constexpr (ND > 2) {
+                dl[3][lane] = v[4] - v[0];
+                dl[4][lane] = (v[5] - v[4]) - k1;
+                dl[5][lane] = (v[6] - v[4]) - k2;
+                dl[6][lane] = ((v[7] - v[6]) - (v[5] - v[4])) - k4;
+              }
+            }
+            wave_lds_sync();
+#pragma unroll
+            for (int i = 0; i < KS; ++i) k[i] = *reinterpret_cast<const nd4*>(&dl[i][4 * pr]);
           }
-          flush();
-          load(n0, ne, nxt);
-          cur = key;
-          present = on_grid;
-#pragma unroll
-          for (int i = 0; i < kClCorners; ++i) at[i] = row[i];
-#pragma unroll
-          for (int cb = 0; cb < 4; ++cb) acc[cb] = nd4{0.f, 0.f, 0.f, 0.f};
-          // corner index: bit d = high side of dimension d (the coefficients of nd_grad_coord_binned_kernel)
-          k[1] = v[1] - v[0], k[2] = v[2] - v[0], k[3] = v[4] - v[0];
-          k[4] = (v[3] - v[2]) - k[1], k[5] = (v[5] - v[4]) - k[1], k[6] = (v[6] - v[4]) - k[2];
-          k[7] = ((v[7] - v[6]) - (v[5] - v[4])) - k[4];
-        } else {
-          load(n0, ne, nxt);
+          load_cell(qe);
         }
+        const int n0 = q0 + 16 < qe ? q0 + 16 : qe, ne = n0 < qe ? qe : run_end(n0);
+        load(n0, ne);
         if (present) {
 #pragma unroll
           for (int s = 0; s < 4; ++s) {
@@ -1212,22 +1232,27 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3, 4))) 
               const bool on = q < qe;
               const float4 t = now[s], f = pl[on ? q : q0];
               const float a = (on && pr < kClCorners) ? wl[q & 63][pr & (kClCorners - 1)] : 0.f;
-              float S[8];
-#pragma unroll
-              for (int m = 1; m < 8; ++m) S[m] = fmaf(t.w, k[m][3], fmaf(t.z, k[m][2], fmaf(t.y, k[m][1], t.x * k[m][0])));
               acc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, t.x, acc[0], 0, 0, 0);
               acc[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, t.y, acc[1], 0, 0, 0);
               acc[2] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, t.z, acc[2], 0, 0, 0);
               acc[3] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, t.w, acc[3], 0, 0, 0);
-              float d[3] = {fmaf(f.y * f.z, S[7], fmaf(f.z, S[5], fmaf(f.y, S[4], S[1]))),
-                            fmaf(f.x * f.z, S[7], fmaf(f.z, S[6], fmaf(f.x, S[4], S[2]))),
-                            fmaf(f.x * f.y, S[7], fmaf(f.y, S[6], fmaf(f.x, S[5], S[3])))};
+              float S[KS];  // of k1, k2, k4, k3, k5, k6, k7
 #pragma unroll
-              for (int i = 0; i < 3; ++i) d[i] = row_sum(d[i]);
+              for (int m = 0; m < KS; ++m) S[m] = fmaf(t.w, k[m][3], fmaf(t.z, k[m][2], fmaf(t.y, k[m][1], t.x * k[m][0])));
+              float d[3] = {S[0], 0.f, 0.f};
+              if constexpr (ND == 2) d[0] = fmaf(f.y, S[2], S[0]), d[1] = fmaf(f.x, S[2], S[1]);
+              if constexpr (ND == 3) {
+                d[0] = fmaf(f.y * f.z, S[6], fmaf(f.z, S[4], fmaf(f.y, S[2], S[0])));
+                d[1] = fmaf(f.x * f.z, S[6], fmaf(f.z, S[5], fmaf(f.x, S[2], S[1])));
+                d[2] = fmaf(f.x * f.y, S[6], fmaf(f.y, S[5], fmaf(f.x, S[4], S[3])));
+              }
+#pragma unroll
+              for (int i = 0; i < ND; ++i) d[i] = row_sum(d[i]);
               if (on && pr == 0) *reinterpret_cast<float3*>(&pl[q]) = make_float3(d[0], d[1], d[2]);
             }
           }
         }
+        start = n0 == qe;
         q0 = n0, qe = ne;
       }
       wave_lds_sync();
@@ -1235,11 +1260,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3, 4))) 
         const float4 r = pl[lane];
         const float d[3] = {r.x, r.y, r.z};
 #pragma unroll
-        for (int i = 0; i < kClMaxDims; ++i) {
-          if (i < g.dims) {
-            float* to = gcoord + (long)wv.id * g.dims + i;
-            *to = (c0 ? *to : 0.f) + (p.inside ? d[i] : 0.f);
-          }
+        for (int i = 0; i < ND; ++i) {
+          float* to = gcoord + (long)wv.id * ND + i;
+          *to = (c0 ? *to : 0.f) + (p.inside ? d[i] : 0.f);
         }
       }
     }
@@ -1602,14 +1625,15 @@ size_t nd_data_cl_workspace(const dk_nd_desc& d) {
 
 namespace {
 
-// Sorts the points by cell into `order` (at `sort_ws`, laid out as nd_sort_workspace says).
+// Sorts the points by cell into `order`, or, if that is null, into its place in `sort_ws` (laid out as nd_sort_workspace
+// says).
 template <typename T>
-const int* sort_points(const NdGeo& g, const T* coord, int bins, void* sort_ws, hipStream_t stream) {
+const int* sort_points(const NdGeo& g, const T* coord, int bins, void* sort_ws, hipStream_t stream, int* order = nullptr) {
   const size_t n4 = round256((size_t)g.batch * sizeof(int));
   char* base = static_cast<char*>(sort_ws);
   unsigned* keys = reinterpret_cast<unsigned*>(base);
   unsigned* keys_sorted = reinterpret_cast<unsigned*>(base + n4);
-  int* order = reinterpret_cast<int*>(base + 2 * n4);
+  if (!order) order = reinterpret_cast<int*>(base + 2 * n4);
   DK_ND_BY_DIMS(g.dims, nd_bin_keys_kernel<T, ND><<<(unsigned)((g.batch + kBlock - 1) / kBlock), kBlock, 0, stream>>>(g, coord, bins, keys));
   {
     // two radix passes of half the key bits each (one pass for keys of up to 9 bits)
@@ -1657,11 +1681,11 @@ void nd_forward(const dk_nd_desc& d, const T* data, const T* coord, T* out, void
         if constexpr (std::is_same<T, float>::value) {
           // rows of out are written as 16-byte vectors at multiples of 4 channels
           if (g.channel % 64 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0 && !path_disabled(kNoNdMfma)) {
-            DK_ND_BY_DIMS(g.dims, nd_forward_mfma_kernel<T, ND><<<(unsigned)((g.batch + 255) / 256), kBlock, 0, stream>>>(g, data_cl, coord, order, bins, out));
+            DK_ND_BY_DIMS(g.dims, nd_forward_mfma_kernel<T, ND><<<(unsigned)xcd_grid_size((g.batch + 255) / 256), kBlock, 0, stream>>>(g, data_cl, coord, order, bins, out));
             return;
           }
         }
-        DK_ND_BY_DIMS(g.dims, nd_forward_binned_kernel<T, ND><<<(unsigned)((g.batch + 255) / 256), kBlock, 0, stream>>>(g, data_cl, coord, order, bins, out));
+        DK_ND_BY_DIMS(g.dims, nd_forward_binned_kernel<T, ND><<<(unsigned)xcd_grid_size((g.batch + 255) / 256), kBlock, 0, stream>>>(g, data_cl, coord, order, bins, out));
         return;
       }
       const int ppw = points_per_wave(g);
@@ -1727,9 +1751,9 @@ void nd_grad_data(const dk_nd_desc& d, const T* gout, const T* coord, T* gdata, 
           on_matrix_cores = g.channel % 64 == 0 && reinterpret_cast<uintptr_t>(gout) % 16 == 0 && !path_disabled(kNoNdMfma);
         if (on_matrix_cores) {
           if constexpr (std::is_same<T, float>::value)
-            DK_ND_BY_DIMS(g.dims, nd_grad_data_mfma_kernel<T, ND><<<(unsigned)((waves + 3) / 4), kBlock, 0, stream>>>(g, gout, coord, order, bins, acc, per_wave));
+            DK_ND_BY_DIMS(g.dims, nd_grad_data_mfma_kernel<T, ND><<<(unsigned)xcd_grid_size((waves + 3) / 4), kBlock, 0, stream>>>(g, gout, coord, order, bins, acc, per_wave));
         } else {
-          DK_ND_BY_DIMS(g.dims, nd_grad_data_binned_kernel<T, ND><<<(unsigned)((waves + 3) / 4), kBlock, 0, stream>>>(g, gout, coord, order, bins, acc, per_wave));
+          DK_ND_BY_DIMS(g.dims, nd_grad_data_binned_kernel<T, ND><<<(unsigned)xcd_grid_size((waves + 3) / 4), kBlock, 0, stream>>>(g, gout, coord, order, bins, acc, per_wave));
         }
       } else {
         const int ppw = points_per_wave(g);
@@ -1768,11 +1792,11 @@ void nd_grad_coord(const dk_nd_desc& d, const T* gout, const T* data, const T* c
         if constexpr (std::is_same<T, float>::value) {
           // rows of gout are read as 16-byte vectors at multiples of 16 channels
           if (g.channel % 64 == 0 && reinterpret_cast<uintptr_t>(gout) % 16 == 0 && !path_disabled(kNoNdMfma)) {
-            DK_ND_BY_DIMS(g.dims, nd_grad_coord_mfma_kernel<T, ND><<<(unsigned)((g.batch + 255) / 256), kBlock, 0, stream>>>(g, gout, data_cl, coord, order, bins, gcoord));
+            DK_ND_BY_DIMS(g.dims, nd_grad_coord_mfma_kernel<T, ND><<<(unsigned)xcd_grid_size((g.batch + 255) / 256), kBlock, 0, stream>>>(g, gout, data_cl, coord, order, bins, gcoord));
             return;
           }
         }
-        DK_ND_BY_DIMS(g.dims, nd_grad_coord_binned_kernel<T, ND><<<(unsigned)((g.batch + 255) / 256), kBlock, 0, stream>>>(g, gout, data_cl, coord, order, bins, gcoord));
+        DK_ND_BY_DIMS(g.dims, nd_grad_coord_binned_kernel<T, ND><<<(unsigned)xcd_grid_size((g.batch + 255) / 256), kBlock, 0, stream>>>(g, gout, data_cl, coord, order, bins, gcoord));
         return;
       }
       const int ppw = points_per_wave(g);
@@ -1813,7 +1837,7 @@ void nd_backward(const dk_nd_desc& d, const T* gout, const T* data, const T* coo
       nd_fill_zero_kernel<float><<<grid_for(n_data), kBlock, 0, stream>>>(acc, n_data);
       transpose<T, T>(data, data_cl, g.channel, g.prod_shape, stream);
       const long waves = (g.batch + 64L * per_wave - 1) / (64L * per_wave);
-      DK_ND_BY_DIMS(g.dims, nd_backward_mfma_kernel<T, ND><<<(unsigned)((waves + 3) / 4), kBlock, 0, stream>>>(g, gout, data_cl, coord, order, bins, acc, gcoord, per_wave));
+      DK_ND_BY_DIMS(g.dims, nd_backward_mfma_kernel<T, ND><<<(unsigned)xcd_grid_size((waves + 3) / 4), kBlock, 0, stream>>>(g, gout, data_cl, coord, order, bins, acc, gcoord, per_wave));
       transpose<float, T>(acc, gdata, g.prod_shape, g.channel, stream);
       return;
     }
@@ -1832,8 +1856,7 @@ void nd_order(const dk_nd_desc& d, const T* coord, int* order, void* ws, hipStre
   const NdGeo g = make_geo(d);
   if constexpr (!std::is_same<T, double>::value) {
     if (const int bins = nd_bins(d)) {
-      const int* sorted = sort_points<T>(g, coord, bins, ws, stream);
-      (void)hipMemcpyAsync(order, sorted, (size_t)d.batch * sizeof(int), hipMemcpyDeviceToDevice, stream);
+      sort_points<T>(g, coord, bins, ws, stream, order);
     }
   }
 }

@@ -172,3 +172,26 @@ def test_trilinear_volume_slice_of_config5():
         assert rel_err(got[0], o32[0]) < 1e-5
         assert rel_err(got[1], o64[1]) < 1e-4
         assert rel_err(got[2], o64[2]) < 1e-4
+
+
+@pytest.mark.parametrize("shape,C,B", [
+    ((6, 5, 4), 64, 65536),      # a cell holds several waves' points
+    ((12, 11, 10), 128, 65537),  # two channel blocks: the coordinates' gradient is added up over them; one point in the last wave
+    ((33, 40), 64, 65599),       # two dimensions, runs of about 45 points
+    ((900,), 64, 65600),         # one dimension
+])
+def test_both_gradients_of_sorted_points_equal_those_formed_alone(shape, C, B):
+    """One kernel forms both from one read of the output gradient; with a single input to differentiate each has its own.  The
+    same products in another order: a few units of 2^-24 of the sums' size."""
+    from deformable_kernels.ops.deform_kernel.functions import nd_linear_sample
+    data, coord, gout = _inputs(shape, C, B, seed=48, dtype=torch.float32)
+    outside = (coord <= -1).any(1) | (coord >= torch.tensor(shape, dtype=torch.float32)).any(1)
+    gout[outside.nonzero()[0, 0]] = float("inf")  # an output gradient that a point outside the grid multiplies with nothing
+    dg, cg = data.cuda().requires_grad_(), coord.cuda().requires_grad_()
+    out = nd_linear_sample(dg, cg)
+    both = torch.autograd.grad(out, [dg, cg], gout.cuda(), retain_graph=True)
+    alone = torch.autograd.grad(out, [cg], gout.cuda(), retain_graph=True)[0]
+    gout[outside] = 0.0
+    want = _oracle(data, coord, gout, np.float64)
+    assert rel_err(both[0].cpu(), want[1]) < 1e-5 and rel_err(both[1].cpu(), want[2]) < 1e-5
+    assert rel_err(both[1].cpu(), alone.double().cpu().numpy()) < 1e-6
