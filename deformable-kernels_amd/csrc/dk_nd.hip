@@ -194,9 +194,10 @@ __global__ __launch_bounds__(kBlock) void nd_grad_coord_kernel(NdGeo g, const T*
 // channel-last path
 // ---------------------------------------------------------------------------
 
-// in [rows][cols] -> out [cols][rows], converting A -> B; 32 x 32 tiles through LDS
+// in [rows][cols] -> out [cols][rows], converting A -> B; 32 x 32 tiles through LDS.  zero != nullptr: as many floats, cleared
+// beside it (a launch less)
 template <typename A, typename B>
-__global__ __launch_bounds__(256) void nd_transpose_kernel(const A* __restrict__ in, B* __restrict__ out,
+__global__ __launch_bounds__(256) void nd_transpose_kernel(const A* __restrict__ in, B* __restrict__ out, float* __restrict__ zero,
                                                            long rows, long cols) {
   __shared__ float tile[32][33];
   const long r0 = (long)blockIdx.y * 32, c0 = (long)blockIdx.x * 32;
@@ -210,7 +211,10 @@ __global__ __launch_bounds__(256) void nd_transpose_kernel(const A* __restrict__
 #pragma unroll
   for (int k = 0; k < 32; k += 8) {
     const long c = c0 + ty + k, r = r0 + tx;
-    if (r < rows && c < cols) st(out + c * rows + r, tile[tx][ty + k]);
+    if (r < rows && c < cols) {
+      st(out + c * rows + r, tile[tx][ty + k]);
+      if (zero) zero[c * rows + r] = 0.f;
+    }
   }
 }
 
@@ -592,14 +596,6 @@ __device__ __forceinline__ int point_bin(const NdGeo& g, const T* coord_b, int n
   for (int d = 0; d < kClMaxDims; ++d)
     if (d < g.dims) key = key * (g.shape[d] + 1) + p.low[d] + 1;
   return key;
-}
-
-template <typename T, int ND>
-__global__ __launch_bounds__(kBlock) void nd_bin_keys_kernel(NdGeo g, const T* __restrict__ coord, int nbins,
-                                                             unsigned* __restrict__ keys) {
-  g.dims = ND;
-  const long b = (long)blockIdx.x * kBlock + threadIdx.x;
-  if (b < g.batch) keys[b] = (unsigned)point_bin<T>(g, coord + b * g.dims, nbins);
 }
 
 // What a wave of the binned kernels knows about its 64 sorted points: lane q holds point q.  An XCD walks one contiguous
@@ -1357,12 +1353,14 @@ __global__ void nd_convert_kernel(const CT* __restrict__ a, T* __restrict__ out,
 // ---------------------------------------------------------------------------
 // Sort of the (cell key, point) pairs: a least-significant-digit radix sort in two passes of at
 // most 9 bits (the keys have at most 18), each pass three kernels that launch nothing but
-// themselves (so the sorted path can be captured into a graph):
-//   radix_count_kernel    a workgroup counts the digits of its tile of 4096 keys (LDS atomics) into
+// themselves (so the sorted path can be captured into a graph).  What bounds it is the launches, 4 - 13 us each: the keys are formed
+// with the first count, the tile sums added up in the scatter, grad data's image cleared by the transpose beside it (2^20 points
+// of 64 x 32^3, forward and gradients: 306 us a pass with launches of their own, 297 without):
+//   radix_keys_kernel (first pass), radix_count_kernel    a workgroup counts the digits of its tile of 4096 keys (LDS atomics) into
 //                         table[digit][workgroup];
 //   radix_scan_*_kernel   exclusive prefix sum of the table in (digit, workgroup) order (per tile of
-//                         4096 entries, then over the tile sums): where each workgroup's keys of each
-//                         digit start in the output;
+//                         4096 entries, then over the tile sums -- those of up to 64 tiles in the scatter):
+//                         where each workgroup's keys of each digit start in the output;
 //   radix_scatter_kernel  stable scatter.  A wave owns 1024 consecutive keys of the tile, 16 rounds
 //                         of 64; the four waves' starts per digit follow from their counts; within
 //                         a round a lane's rank among the lanes with its digit comes from nine
@@ -1371,19 +1369,32 @@ __global__ void nd_convert_kernel(const CT* __restrict__ a, T* __restrict__ out,
 constexpr int kSortTile = 4096, kSortWaveKeys = kSortTile / (kBlock / 64), kSortRounds = kSortWaveKeys / 64;
 constexpr int kSortMaxDigits = 512;
 
-__global__ __launch_bounds__(kBlock) void radix_count_kernel(const unsigned* __restrict__ keys, long n, int shift,
-                                                             int digits, int nblocks, unsigned* __restrict__ table) {
+template <typename KeyOf>
+__device__ __forceinline__ void count_digits(KeyOf key_of, long n, int shift, int digits, int nblocks, unsigned* __restrict__ table) {
   __shared__ unsigned h[kSortMaxDigits];
   for (int d = threadIdx.x; d < digits; d += kBlock) h[d] = 0u;
   __syncthreads();
-  const long base = (long)blockIdx.x * kSortTile;
-#pragma unroll 4
-  for (int r = 0; r < kSortTile / kBlock; ++r) {
-    const long i = base + r * kBlock + threadIdx.x;
-    if (i < n) atomicAdd(&h[(keys[i] >> shift) & (unsigned)(digits - 1)], 1u);
-  }
+  const long base = (long)blockIdx.x * kSortTile + threadIdx.x;
+  unsigned key[kSortTile / kBlock];
+#pragma unroll
+  for (int r = 0; r < kSortTile / kBlock; ++r) key[r] = key_of(min(base + r * kBlock, n - 1));
+#pragma unroll
+  for (int r = 0; r < kSortTile / kBlock; ++r)
+    if (base + r * kBlock < n) atomicAdd(&h[(key[r] >> shift) & (unsigned)(digits - 1)], 1u);
   __syncthreads();
   for (int d = threadIdx.x; d < digits; d += kBlock) table[(size_t)d * nblocks + blockIdx.x] = h[d];
+}
+__global__ __launch_bounds__(kBlock) void radix_count_kernel(const unsigned* __restrict__ keys, long n, int shift,
+                                                             int digits, int nblocks, unsigned* __restrict__ table) {
+  count_digits([&](long i) { return keys[i]; }, n, shift, digits, nblocks, table);
+}
+// The first pass's, which forms the keys from the coordinates and leaves them for the scatter (a thread past the end writes
+// the last point's key once more).
+template <typename T, int ND>
+__global__ __launch_bounds__(kBlock) void radix_keys_kernel(NdGeo g, const T* __restrict__ coord, int nbins, unsigned* __restrict__ keys,
+                                                            int digits, int nblocks, unsigned* __restrict__ table) {
+  g.dims = ND;
+  count_digits([&](long i) { return keys[i] = (unsigned)point_bin<T>(g, coord + i * ND, nbins); }, g.batch, 0, digits, nblocks, table);
 }
 
 // Exclusive prefix sum of 1024 values, one per thread of the workgroup; `total` receives their sum.
@@ -1427,7 +1438,7 @@ __global__ __launch_bounds__(1024) void radix_scan_tiles_kernel(unsigned* __rest
   }
   if (threadIdx.x == 0) sums[blockIdx.x] = all;
 }
-// exclusive prefix sum of the tile sums, in place: one workgroup walks them 1024 at a time
+// exclusive prefix sum of the tile sums, in place: one workgroup walks them 1024 at a time (more than kScanInScatter tiles)
 __global__ __launch_bounds__(1024) void radix_scan_sums_kernel(unsigned* __restrict__ sums, int count) {
   __shared__ unsigned wave_sum[16];
   unsigned carry = 0u;
@@ -1443,16 +1454,30 @@ __global__ __launch_bounds__(1024) void radix_scan_sums_kernel(unsigned* __restr
 
 // idx_in == nullptr: the points are still in their own order (index = position);
 // keys_out == nullptr: the keys are not needed after this pass
+// raw_tiles != 0: tile_start holds that many sums, not yet their prefix sums, which every workgroup's first wave then forms
+// for itself (a lane per tile): a launch of one workgroup less
+constexpr int kScanInScatter = 64;
 __global__ __launch_bounds__(kBlock) void radix_scatter_kernel(const unsigned* __restrict__ keys,
                                                                const int* __restrict__ idx_in, long n, int shift,
                                                                int digits, int nblocks,
                                                                const unsigned* __restrict__ table,
-                                                               const unsigned* __restrict__ tile_start,
+                                                               const unsigned* __restrict__ tile_start, int raw_tiles,
                                                                unsigned* __restrict__ keys_out,
                                                                int* __restrict__ idx_out) {
   constexpr int kWaves = kBlock / 64;
   __shared__ unsigned h[kWaves][kSortMaxDigits];
+  __shared__ unsigned starts[kScanInScatter];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  if (raw_tiles && wave == 0) {
+    const unsigned own = lane < raw_tiles ? tile_start[lane] : 0u;
+    unsigned incl = own;
+#pragma unroll
+    for (int step = 1; step < 64; step <<= 1) {
+      const unsigned up = (unsigned)__shfl_up((int)incl, step);
+      if (lane >= step) incl += up;
+    }
+    starts[lane] = incl - own;
+  }
   for (int e = threadIdx.x; e < kWaves * kSortMaxDigits; e += kBlock) (&h[0][0])[e] = 0u;
   __syncthreads();
   const long base = (long)blockIdx.x * kSortTile + (long)wave * kSortWaveKeys;
@@ -1472,7 +1497,7 @@ __global__ __launch_bounds__(kBlock) void radix_scatter_kernel(const unsigned* _
   // counts -> where each wave's keys of each digit start
   for (int d = threadIdx.x; d < digits; d += kBlock) {
     const size_t j = (size_t)d * nblocks + blockIdx.x;
-    unsigned run = table[j] + tile_start[j / kScanTile];
+    unsigned run = table[j] + (raw_tiles ? starts[j / kScanTile] : tile_start[j / kScanTile]);
 #pragma unroll
     for (int w = 0; w < kWaves; ++w) {
       const unsigned c = h[w][d];
@@ -1558,9 +1583,9 @@ int chunks_per_wave(const NdGeo& g) {
 }
 
 template <typename A, typename B>
-void transpose(const A* in, B* out, long rows, long cols, hipStream_t stream) {
+void transpose(const A* in, B* out, long rows, long cols, hipStream_t stream, float* zero = nullptr) {
   const dim3 grid((unsigned)((cols + 31) / 32), (unsigned)((rows + 31) / 32));
-  nd_transpose_kernel<A, B><<<grid, 256, 0, stream>>>(in, out, rows, cols);
+  nd_transpose_kernel<A, B><<<grid, 256, 0, stream>>>(in, out, zero, rows, cols);
 }
 
 }  // namespace
@@ -1634,7 +1659,6 @@ const int* sort_points(const NdGeo& g, const T* coord, int bins, void* sort_ws, 
   unsigned* keys = reinterpret_cast<unsigned*>(base);
   unsigned* keys_sorted = reinterpret_cast<unsigned*>(base + n4);
   if (!order) order = reinterpret_cast<int*>(base + 2 * n4);
-  DK_ND_BY_DIMS(g.dims, nd_bin_keys_kernel<T, ND><<<(unsigned)((g.batch + kBlock - 1) / kBlock), kBlock, 0, stream>>>(g, coord, bins, keys));
   {
     // two radix passes of half the key bits each (one pass for keys of up to 9 bits)
     const int bits = key_bits(bins);
@@ -1645,10 +1669,14 @@ const int* sort_points(const NdGeo& g, const T* coord, int bins, void* sort_ws, 
     unsigned* sums = table + (size_t)kSortMaxDigits * nblocks;
     auto pass = [&](const unsigned* k_in, const int* i_in, int shift, int nbits, unsigned* k_out, int* i_out) {
       const int digits = 1 << nbits, total = digits * nblocks, tiles = (total + kScanTile - 1) / kScanTile;
-      radix_count_kernel<<<nblocks, kBlock, 0, stream>>>(k_in, g.batch, shift, digits, nblocks, table);
+      if (shift == 0)
+        DK_ND_BY_DIMS(g.dims, radix_keys_kernel<T, ND><<<nblocks, kBlock, 0, stream>>>(g, coord, bins, keys, digits, nblocks, table));
+      else
+        radix_count_kernel<<<nblocks, kBlock, 0, stream>>>(k_in, g.batch, shift, digits, nblocks, table);
       radix_scan_tiles_kernel<<<tiles, 1024, 0, stream>>>(table, total, sums);
-      radix_scan_sums_kernel<<<1, 1024, 0, stream>>>(sums, tiles);
-      radix_scatter_kernel<<<nblocks, kBlock, 0, stream>>>(k_in, i_in, g.batch, shift, digits, nblocks, table, sums, k_out, i_out);
+      const bool raw = tiles <= kScanInScatter;
+      if (!raw) radix_scan_sums_kernel<<<1, 1024, 0, stream>>>(sums, tiles);
+      radix_scatter_kernel<<<nblocks, kBlock, 0, stream>>>(k_in, i_in, g.batch, shift, digits, nblocks, table, sums, raw ? tiles : 0, k_out, i_out);
     };
     if (hi_bits == 0) {
       pass(keys, nullptr, 0, lo_bits, nullptr, order);
@@ -1834,8 +1862,7 @@ void nd_backward(const dk_nd_desc& d, const T* gout, const T* data, const T* coo
       float *acc = static_cast<float*>(ws), *data_cl = reinterpret_cast<float*>(static_cast<char*>(ws) + image);
       const int bins = nd_bins(d), per_wave = chunks_per_wave(g);
       if (!order) order = sort_points<T>(g, coord, bins, static_cast<char*>(ws) + 2 * image, stream);
-      nd_fill_zero_kernel<float><<<grid_for(n_data), kBlock, 0, stream>>>(acc, n_data);
-      transpose<T, T>(data, data_cl, g.channel, g.prod_shape, stream);
+      transpose<T, T>(data, data_cl, g.channel, g.prod_shape, stream, acc);
       const long waves = (g.batch + 64L * per_wave - 1) / (64L * per_wave);
       DK_ND_BY_DIMS(g.dims, nd_backward_mfma_kernel<T, ND><<<(unsigned)xcd_grid_size((waves + 3) / 4), kBlock, 0, stream>>>(g, gout, data_cl, coord, order, bins, acc, gcoord, per_wave));
       transpose<float, T>(acc, gdata, g.prod_shape, g.channel, stream);

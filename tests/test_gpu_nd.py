@@ -195,3 +195,24 @@ def test_both_gradients_of_sorted_points_equal_those_formed_alone(shape, C, B):
     want = _oracle(data, coord, gout, np.float64)
     assert rel_err(both[0].cpu(), want[1]) < 1e-5 and rel_err(both[1].cpu(), want[2]) < 1e-5
     assert rel_err(both[1].cpu(), alone.double().cpu().numpy()) < 1e-6
+
+
+@pytest.mark.parametrize("B", [1 << 21, (1 << 21) + 1])
+def test_sort_on_either_side_of_the_most_tiles_that_the_scatter_sums_itself(B):
+    """18 key bits, 512 or 513 workgroups: 64 tiles of the digit table, whose sums the scatter adds up itself, and 65, which have a
+    kernel for that.  An output is two products and a sum: 3 * 2^-24 of its operands' size; a gradient sums some ten."""
+    S, C = 200000, 16
+    data, coord, gout = _inputs((S,), C, B, seed=49, dtype=torch.float32, lo=0.0, extra=-2.0)
+    data, coord, gout = (t.cuda() for t in (data, coord, gout))
+    dg = data.requires_grad_()
+    from deformable_kernels.ops.deform_kernel.functions import nd_linear_sample
+    out = nd_linear_sample(dg, coord)
+    grad = torch.autograd.grad(out, dg, gout)[0]
+    low = coord[:, 0].floor().long()
+    frac = (coord[:, 0] - low).double()
+    rows = data.detach().double().t().contiguous()
+    want = rows[low] * (1 - frac)[:, None] + rows[low + 1] * frac[:, None]
+    assert float((out.detach() - want).abs().max()) < 3 * 2.0 ** -24 * 2 * float(data.detach().abs().max())
+    want = torch.zeros_like(rows).index_add_(0, low, gout.double() * (1 - frac)[:, None])
+    want.index_add_(0, low + 1, gout.double() * frac[:, None])
+    assert rel_err(grad.cpu(), want.t().cpu().numpy()) < 1e-5
