@@ -1355,18 +1355,19 @@ __global__ void nd_convert_kernel(const CT* __restrict__ a, T* __restrict__ out,
 // most 9 bits (the keys have at most 18), each pass three kernels that launch nothing but
 // themselves (so the sorted path can be captured into a graph).  What bounds it is the launches, 4 - 13 us each: the keys are formed
 // with the first count, the tile sums added up in the scatter, grad data's image cleared by the transpose beside it (2^20 points
-// of 64 x 32^3, forward and gradients: 306 us a pass with launches of their own, 297 without):
-//   radix_keys_kernel (first pass), radix_count_kernel    a workgroup counts the digits of its tile of 4096 keys (LDS atomics) into
+// of 64 x 32^3, forward and gradients: 306 us a pass with launches of their own, 297 without; tiles of 2048 keys instead of 4096, two
+// waves per SIMD of 2^20 points, 293):
+//   radix_keys_kernel (first pass), radix_count_kernel    a workgroup counts the digits of its tile of 2048 keys (LDS atomics) into
 //                         table[digit][workgroup];
 //   radix_scan_*_kernel   exclusive prefix sum of the table in (digit, workgroup) order (per tile of
 //                         4096 entries, then over the tile sums -- those of up to 64 tiles in the scatter):
 //                         where each workgroup's keys of each digit start in the output;
-//   radix_scatter_kernel  stable scatter.  A wave owns 1024 consecutive keys of the tile, 16 rounds
+//   radix_scatter_kernel  stable scatter.  A wave owns 512 consecutive keys of the tile, 8 rounds
 //                         of 64; the four waves' starts per digit follow from their counts; within
 //                         a round a lane's rank among the lanes with its digit comes from nine
 //                         ballots, and the first of them advances the wave's LDS counter.
 // ---------------------------------------------------------------------------
-constexpr int kSortTile = 4096, kSortWaveKeys = kSortTile / (kBlock / 64), kSortRounds = kSortWaveKeys / 64;
+constexpr int kSortTile = 2048, kSortWaveKeys = kSortTile / (kBlock / 64), kSortRounds = kSortWaveKeys / 64;
 constexpr int kSortMaxDigits = 512;
 
 template <typename KeyOf>

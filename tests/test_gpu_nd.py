@@ -197,7 +197,7 @@ def test_both_gradients_of_sorted_points_equal_those_formed_alone(shape, C, B):
     assert rel_err(both[1].cpu(), alone.double().cpu().numpy()) < 1e-6
 
 
-@pytest.mark.parametrize("B", [1 << 21, (1 << 21) + 1])
+@pytest.mark.parametrize("B", [1 << 20, (1 << 20) + 1])
 def test_sort_on_either_side_of_the_most_tiles_that_the_scatter_sums_itself(B):
     """18 key bits, 512 or 513 workgroups: 64 tiles of the digit table, whose sums the scatter adds up itself, and 65, which have a
     kernel for that.  An output is two products and a sum: 3 * 2^-24 of its operands' size; a gradient sums some ten."""
