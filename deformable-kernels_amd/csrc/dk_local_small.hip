@@ -8,7 +8,9 @@
 //   grad input     64 input pixels, a share of the channels: a wave walks channels, a lane gathers its pixel's taps
 //   grad rotation  64 output pixels: 16 waves share the channels, their sums are added in wave order
 //   grad filter    one channel: 16 waves share the pixels; a lane keeps a sum per scope cell, dense hat weights
-// fp32 arithmetic for every type (reference kernels: K.cu:577-702, 836-999, 1285-1408).
+// fp32 arithmetic for every type (reference kernels: K.cu:577-702, 836-999, 1285-1408).  What the reference skips -- a tap
+// outside the image, off the stride's grid or outside the scope, a cell that a tap does not read -- takes nothing from a value
+// that is not finite.  Registers: 1024 threads leave 128 of them; scope 7 spills 96 bytes per lane, the others nothing.
 #include <algorithm>
 
 #include "dk_common.h"
@@ -54,6 +56,17 @@ struct WaveTable {
   }
 };
 
+// A tap's descriptor; one that contributes nothing (`in` false: not `ok`, or outside the scope) points at a block of zeros
+// behind the table.  (The table's own block (-1, -1), which make_lite_tap takes for it, holds cell (0, 0) in its last entry:
+// a weight that is not finite there would reach every such tap.)
+template <int S>
+__device__ __forceinline__ LiteTap small_tap(float h, float w, bool ok, bool& in) {
+  in = ok && h > -1.f && w > -1.f && h < float(S) && w < float(S);
+  LiteTap t = make_lite_tap<S, S>(h, w, in);
+  t.cell = in ? t.cell : WideTable<S, S>::SIZE;
+  return t;
+}
+
 template <typename T, int S>
 __global__ __launch_bounds__(64 * kSmWaves) void local_small_backward_kernel(Geo g, SmallStrides st, SmallRoles roles, const T* __restrict__ gout,
                                                                              const T* __restrict__ x, const T* __restrict__ rot,
@@ -61,7 +74,7 @@ __global__ __launch_bounds__(64 * kSmWaves) void local_small_backward_kernel(Geo
                                                                              T* __restrict__ grot, T* __restrict__ gfilter) {
   using Tb = WideTable<S, S>;
   constexpr int CELLS = S * S, PARTS = kSmTaps * 64 > CELLS ? kSmTaps * 64 : CELLS;
-  __shared__ __align__(16) float tables[kSmWaves][Tb::SIZE];
+  __shared__ __align__(16) float tables[kSmWaves][Tb::SIZE + 4];  // and the block of zeros
   __shared__ float part[kSmWaves][PARTS];
   constexpr const T* tag = nullptr;
   constexpr unsigned E = sizeof(T);
@@ -70,6 +83,7 @@ __global__ __launch_bounds__(64 * kSmWaves) void local_small_backward_kernel(Geo
   const rsrc_t rg = plane_rsrc(gout, g.batch * g.channel * out_plane), rx = plane_rsrc(x, g.batch * g.channel * in_plane);
   const rsrc_t rr = plane_rsrc(rot, g.batch * g.groups * 2 * kSmTaps * out_plane), rf = plane_rsrc(filter, g.channel * CELLS);
   int b = blockIdx.x;
+  if (lane < 4) tables[wave][Tb::SIZE + lane] = 0.f;
 
   if (b < roles.input_tiles * roles.input_splits) {
     const int split = b % roles.input_splits, tile = b / roles.input_splits;
@@ -89,7 +103,8 @@ __global__ __launch_bounds__(64 * kSmWaves) void local_small_backward_kernel(Geo
       const unsigned ro = hit ? (unsigned)(n * st.rn + (grp * 18 + 2 * t) * st.rc + p * st.rp) * E : kOutOfRange;
       const float h = scope_coord<float>(g, t / 3, buf_ld2(rr, ro, 0, tag), g.centre_h);
       const float w = scope_coord<float>(g, t % 3, buf_ld2(rr, ro, st.rc * (int)E, tag), g.centre_w);
-      tap[t] = make_lite_tap<S, S>(h, w, hit);
+      bool in;
+      tap[t] = small_tap<S>(h, w, hit, in);
       off[t] = hit ? (unsigned)(n * st.on + p * st.op) * E : kOutOfRange;
     }
     WaveTable<T, S> table;
@@ -128,17 +143,19 @@ __global__ __launch_bounds__(64 * kSmWaves) void local_small_backward_kernel(Geo
     const bool live = pix0 + lane < total;
     const int n = live ? (pix0 + lane) / out_plane : 0, p = live ? pix0 + lane - n * out_plane : 0, oh = p / g.out_w, ow = p - oh * g.out_w;
     LiteTap tap[kSmTaps];
-    unsigned off[kSmTaps], open = 0;  // bits 2 t + dir of `open`: the offset is not clamped
+    unsigned off[kSmTaps], open = 0;  // bits 2 t + dir of `open`: the tap reads image and scope, and the offset is not clamped
 #pragma unroll
     for (int t = 0; t < kSmTaps; ++t) {
       const unsigned ro = live ? (unsigned)(n * st.rn + (grp * 18 + 2 * t) * st.rc + p * st.rp) * E : kOutOfRange;
       bool oh_open, ow_open;
       const float h = scope_coord<float>(g, t / 3, buf_ld2(rr, ro, 0, tag), g.centre_h, &oh_open);
       const float w = scope_coord<float>(g, t % 3, buf_ld2(rr, ro, st.rc * (int)E, tag), g.centre_w, &ow_open);
-      tap[t] = make_lite_tap<S, S>(h, w, live);
-      open |= (oh_open ? 1u : 0u) << (2 * t) | (ow_open ? 2u : 0u) << (2 * t);
       const int iy = oh * g.stride_h - g.pad_h + t / 3 * g.dil_h, ix = ow * g.stride_w - g.pad_w + t % 3 * g.dil_w;
-      off[t] = live && iy >= 0 && iy < g.in_h && ix >= 0 && ix < g.in_w ? (unsigned)(n * st.xn + (iy * g.in_w + ix) * st.xp) * E : kOutOfRange;
+      const bool hit = live && iy >= 0 && iy < g.in_h && ix >= 0 && ix < g.in_w;
+      bool in;
+      tap[t] = small_tap<S>(h, w, hit, in);
+      open |= (in && oh_open ? 1u : 0u) << (2 * t) | (in && ow_open ? 2u : 0u) << (2 * t);
+      off[t] = hit ? (unsigned)(n * st.xn + (iy * g.in_w + ix) * st.xp) * E : kOutOfRange;
     }
     const unsigned goff = live ? (unsigned)(n * st.on + p * st.op) * E : kOutOfRange;
     WaveTable<T, S> table;
@@ -209,16 +226,41 @@ __global__ __launch_bounds__(64 * kSmWaves) void local_small_backward_kernel(Geo
       const unsigned ro = live ? (unsigned)(n * st.rn + (grp * 18 + 2 * t) * st.rc + p * st.rp) * E : kOutOfRange;
       rh[t] = buf_ld2(rr, ro, 0, tag), rw[t] = buf_ld2(rr, ro, st.rc * (int)E, tag);
     }
+    float v[kSmTaps], z = 0.f;  // z: NaN where a product is not finite
+#pragma unroll
+    for (int t = 0; t < kSmTaps; ++t) v[t] = xv[t] * gv, z = fmaf(v[t], 0.f, z);
+    if (__any(z != 0.f)) {
+      // such a product must not meet the zero hats of the cells that its tap does not read (K.cu:85-114), nor the zero read for a
+      // tap outside the image: a tap at a time, its operands read again
+#pragma unroll 1
+      for (int t = 0; t < kSmTaps; ++t) {
+        const int iy = oh * g.stride_h - g.pad_h + t / 3 * g.dil_h, ix = ow * g.stride_w - g.pad_w + t % 3 * g.dil_w;
+        const bool hit = live && iy >= 0 && iy < g.in_h && ix >= 0 && ix < g.in_w;
+        const float p1 = gv * buf_ld2(rx, hit ? (unsigned)(n * st.xn + (iy * g.in_w + ix) * st.xp) * E : kOutOfRange, c * st.xc * (int)E, tag);
+        const unsigned ro = live ? (unsigned)(n * st.rn + (grp * 18 + 2 * t) * st.rc + p * st.rp) * E : kOutOfRange;
+        const float h = scope_coord<float>(g, t / 3, buf_ld2(rr, ro, 0, tag), g.centre_h);
+        const float w = scope_coord<float>(g, t % 3, buf_ld2(rr, ro, st.rc * (int)E, tag), g.centre_w);
+        const bool in = hit && h > -1.f && w > -1.f && h < float(S) && w < float(S);
+        const int i0 = in ? (int)floorf(h) : 0, k0 = in ? (int)floorf(w) : 0;
+#pragma unroll
+        for (int i = 0; i < S; ++i) {
+          const float a = p1 * (1.f - fabsf(h - (float)i));
+#pragma unroll
+          for (int k = 0; k < S; ++k)
+            acc[i * S + k] += in && (unsigned)(i - i0) < 2u && (unsigned)(k - k0) < 2u ? a * (1.f - fabsf(w - (float)k)) : 0.f;
+        }
+      }
+      continue;
+    }
 #pragma unroll
     for (int t = 0; t < kSmTaps; ++t) {
       const float h = scope_coord<float>(g, t / 3, rh[t], g.centre_h), w = scope_coord<float>(g, t % 3, rw[t], g.centre_w);
-      const float v = xv[t] * gv;
       float hw[S];
 #pragma unroll
       for (int k = 0; k < S; ++k) hw[k] = fmaxf(0.f, 1.f - fabsf(w - (float)k));
 #pragma unroll
       for (int i = 0; i < S; ++i) {
-        const float a = v * fmaxf(0.f, 1.f - fabsf(h - (float)i));
+        const float a = v[t] * fmaxf(0.f, 1.f - fabsf(h - (float)i));
 #pragma unroll
         for (int k = 0; k < S; ++k) acc[i * S + k] = fmaf(a, hw[k], acc[i * S + k]);
       }

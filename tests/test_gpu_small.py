@@ -79,3 +79,37 @@ def test_clipped_offsets_and_single_gradients(clip):
     for a, b in zip(res, ref):
         assert rel_err(a.cpu(), b.cpu()) < 1e-5
     assert torch.equal(res[1] == 0, ref[1] == 0)   # where the clamp is active
+
+
+# ---- values that are not finite: the default dispatch against the oracle's own NaN and Inf ----
+
+NON_FINITE = {
+    "weight, first cell": lambda x, wt, rot, gout: wt[5, 0].__setitem__((0, 0), float("inf")),
+    "weight, inner cell": lambda x, wt, rot, gout: wt[5, 0].__setitem__((1, 2), float("nan")),
+    "output gradient": lambda x, wt, rot, gout: gout[1, 4].__setitem__((2, 3), float("inf")),
+    "input": lambda x, wt, rot, gout: x[1, 4].__setitem__((4, 5), float("inf")),
+    "output gradient of a corner pixel": lambda x, wt, rot, gout: gout[0, 4].__setitem__((0, 0), float("nan")),
+}
+
+
+@pytest.mark.parametrize("layout", ["planar", "channels_last"])
+@pytest.mark.parametrize("dtype_name", ["float32", "float16", "bfloat16"])
+@pytest.mark.parametrize("S, stride, G", [(3, 1, 1), (4, 1, 1), (4, 2, 1), (5, 1, 2), (7, 2, 1)])
+@pytest.mark.parametrize("what", NON_FINITE)
+def test_a_non_finite_value_reaches_what_the_reference_lets_it_reach(what, S, stride, G, dtype_name, layout):
+    """No test switch is set.  Taps outside the image or the scope and, at stride 2, off its grid read nothing of the channel
+    with the poisoned value, and a product reaches the four cells of its own sample."""
+    from deformable_kernels.ops.deform_kernel.functions import sample_depthwise
+    x, wt, rot, gout, cfg = make_local(2, 32, 11, 13, 3, (S, S), stride, 1, 1, G, 0.7, seed=8)
+    rot[0, :, 1, 1] = 50.0   # all taps of this pixel leave the scope
+    x, wt, rot, gout = [t.to(getattr(torch, dtype_name)) for t in (x, wt, rot, gout)]
+    NON_FINITE[what](x, wt, rot, gout)
+    fmt = torch.contiguous_format if layout == "planar" else torch.channels_last
+    leaves = [t.to(DEV).requires_grad_() for t in (x.contiguous(memory_format=fmt), rot.contiguous(memory_format=fmt), wt)]
+    out = sample_depthwise(*leaves, *(cfg[k] for k in ("kernel_size", "stride", "padding", "dilation", "groups")))
+    got = torch.autograd.grad(out, leaves, gout.to(DEV).contiguous(memory_format=fmt))
+    want = orc.sample_depthwise_backward(*[t.double().numpy() for t in (gout, x, rot, wt)], **cfg)
+    for name, a, b in zip(("input", "rotation", "filter"), got, want):
+        finite = torch.from_numpy(b).isfinite()
+        assert torch.equal(a.cpu().isfinite(), finite), name
+        assert rel_err(a.cpu().double()[finite], b[finite.numpy()]) < (1e-5 if dtype_name == "float32" else 1e-2), name
