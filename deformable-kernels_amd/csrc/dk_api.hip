@@ -409,11 +409,16 @@ int dk_sample_depthwise_backward(const dk_conv_desc* desc, const void* out_grad,
   if (!out_grad || !input || !rotation || !filter) return DK_ERR_NULL_POINTER;
   const size_t need = backward_need(g, desc, rotation_grad != nullptr, filter_grad != nullptr);
   if (need && (!workspace || workspace_bytes < need)) return DK_ERR_WORKSPACE;
-  if (backward_in_one_launch(g, desc))
-    return by_tensor_dtype(desc->dtype, [&]<typename T>() {
-      local_small_backward<T>(g, desc->layout == DK_LAYOUT_NHWC, in<T>(out_grad), in<T>(input), in<T>(rotation), in<T>(filter), out<T>(in_grad),
-                              out<T>(rotation_grad), out<T>(filter_grad), static_cast<hipStream_t>(stream));
+  if (backward_in_one_launch(g, desc)) {
+    // (float32 channels-last layers above stride 1: the input gradient, like that of larger layers of few channels or pixels, is the
+    // table kernel's to the bit, a launch of its own)
+    const bool apart = in_grad && desc->layout == DK_LAYOUT_NHWC && desc->dtype == DK_F32 && (g.stride_h > 1 || g.stride_w > 1);
+    const int st = by_tensor_dtype(desc->dtype, [&]<typename T>() {
+      local_small_backward<T>(g, desc->layout == DK_LAYOUT_NHWC, in<T>(out_grad), in<T>(input), in<T>(rotation), in<T>(filter),
+                              apart ? nullptr : out<T>(in_grad), out<T>(rotation_grad), out<T>(filter_grad), static_cast<hipStream_t>(stream));
     });
+    return apart && st == DK_OK ? dk_sample_depthwise_backward_data(desc, out_grad, rotation, filter, in_grad, stream) : st;
+  }
   // Filter gradient first, input gradient last: measured 4 % faster than the reference's order
   // (input, rotation, filter) on a 245 MB layer -- the two kernels that read out_grad, input and
   // rotation run back to back and the input gradient's 115 MB of writes do not push those
