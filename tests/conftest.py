@@ -48,17 +48,3 @@ def switch_off():
 
     yield off
     _lib.lib().dk_test_switches(before)
-
-
-@pytest.fixture(autouse=True)
-def _kernels_of_the_larger_layers(request):
-    """The suite's layers are small, so that the oracle is quick: without this the operator would compute most gradients
-    by its one-launch form, which any test switch takes away (tests/test_gpu_small.py tests that one)."""
-    if "gpu" not in request.keywords or not _have_gpu() or request.module.__name__ in ("test_gpu_small", "test_native_operators"):
-        yield
-        return
-    from deformable_kernels.ops.deform_kernel import _lib
-    before = _lib.lib().dk_test_switches(0)
-    _lib.lib().dk_test_switches(before | 1 << _lib.TEST_SWITCHES.index("DK_NO_SMALL_BACKWARD"))
-    yield
-    _lib.lib().dk_test_switches(before)
