@@ -51,6 +51,19 @@ __device__ __forceinline__ void st_stream(T* p, float v) { dk::st(p, v); }
 // put 36 samples on an element on average and about 65 on the fullest element of a large plane.)
 constexpr int kPairHead = 7;
 
+// Grad input with the lanes along the channels, in bands of rows (dk_deform_lanes.hip): 64 consecutive output pixels are walked
+// once for every band that their samples read, with wide offsets nearly all of them.  Whether that form takes a call is
+// therefore read off the offsets, on the device: it does while its units meet at most `most` bands in all; the form with a
+// pixel per lane is launched behind it and takes the others.  (Not per image: with a few images each the two would run one after
+// the other on a chip that is half empty, N=24 C=64 64 x 64 116 -> 216 us.)
+struct BandWalk {
+  int2* unit_rows;  // [image][ceil(output pixels / 64)]: least and largest image row that a unit's samples read
+  unsigned* met;    // bands that all units meet, written by deform_tile_rows_kernel; null: the bands, if there are any, take the call
+  unsigned most;
+  int rows;         // image rows of a band; 0: no bands
+};
+__device__ __forceinline__ bool bands_take(const BandWalk& walk) { return *walk.met <= walk.most; }
+
 // floor(v + 0.5) as a signed 32-bit integer, one instruction
 __device__ __forceinline__ int round_half_up(float v) {
   int r;

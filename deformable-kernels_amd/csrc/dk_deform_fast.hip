@@ -1002,9 +1002,11 @@ __global__ __launch_bounds__(kDWinCoordBlock, 1) void deform_grad_coord_chw_kern
 // float maximum would drop a NaN; the consumer takes the maximum of the kAbsParts words
 // (one atomic maximum per workgroup on a single word cost more than the reads: the atomics on one
 // address serialise).  16-byte loads, four in flight per thread; p must be 16-byte aligned (the
-// host checks).
+// host checks).  zero: a word cleared beside it, for the next kernel's count (BandWalk).
 template <typename T>
-__global__ __launch_bounds__(256) void absmax_kernel(const T* __restrict__ p, long n, unsigned* __restrict__ out) {
+__global__ __launch_bounds__(256) void absmax_kernel(const T* __restrict__ p, long n, unsigned* __restrict__ out,
+                                                     unsigned* __restrict__ zero) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) *zero = 0u;
   __shared__ unsigned wave_max[4];
   constexpr int V = 16 / (int)sizeof(T);
   struct alignas(16) Vec {
@@ -1035,7 +1037,7 @@ template <typename T, int SH, int SW>
 __global__ __launch_bounds__(1024) void deform_grad_input_kernel(
     Geo g, const T* __restrict__ gout, const T* __restrict__ off, const T* __restrict__ rot,
     const T* __restrict__ filter, T* __restrict__ gin, const unsigned* __restrict__ gmax_bits,
-    int ch_per_block, int shift) {
+    int ch_per_block, int shift, BandWalk walk) {
   using Tb = WideTable<SH, SW>;
   extern __shared__ __align__(16) float lds[];
   const int H = g.in_h, W = g.in_w, RS = W + 2;
@@ -1047,7 +1049,7 @@ __global__ __launch_bounds__(1024) void deform_grad_input_kernel(
   const int cpg = g.channel / g.groups;
   const int out_plane = g.out_h * g.out_w, in_plane = H * W;
   const BlockId b = decode_block(g, 1, ceil_div(cpg, ch_per_block));
-  if (!b.valid) return;
+  if (!b.valid || (walk.met && bands_take(walk))) return;
   const int j0 = b.chunk * ch_per_block;
   const int nch = min(ch_per_block, cpg - j0);
 
@@ -1215,12 +1217,17 @@ __global__ __launch_bounds__(1024) void deform_grad_input_kernel(
 // The input rows a tile of 1024 output pixels samples, for the band form of the tiled grad input below:
 // table[(image * tiles + tile) * 2] = least, [.. + 1] = largest padded row (image row + 1) of the top corners of
 // the tile's samples that hit the image (K.cu:486-500); a tile without such samples gets an empty range.
-// The offsets belong to the image, not to the rotation group.  grid = image * tiles
+// The offsets belong to the image, not to the rotation group.  walk.unit_rows, if not null: the same per 64 pixels, as image rows of the top
+// and bottom corners, and how many bands they meet (BandWalk; absmax_kernel has cleared the count).  grid = image * tiles
 // ---------------------------------------------------------------------------
 template <typename T>
 __global__ __launch_bounds__(1024) void deform_tile_rows_kernel(Geo g, const T* __restrict__ off, int* __restrict__ table,
-                                                                int ntiles, unsigned* __restrict__ most_img) {
+                                                                int ntiles, unsigned* __restrict__ most_img,
+                                                                BandWalk walk) {
   __shared__ int wave_lo[16], wave_hi[16];
+  __shared__ unsigned met;
+  if (threadIdx.x == 0) met = 0u;
+  __syncthreads();
   const int out_plane = g.out_h * g.out_w;
   const int tile = blockIdx.x % ntiles, n = blockIdx.x / ntiles;
   const int p = tile * 1024 + threadIdx.x;
@@ -1248,6 +1255,10 @@ __global__ __launch_bounds__(1024) void deform_tile_rows_kernel(Geo g, const T* 
   if ((threadIdx.x & 63) == 0) {
     wave_lo[threadIdx.x >> 6] = lo;
     wave_hi[threadIdx.x >> 6] = hi;
+    if (walk.unit_rows && p < out_plane) {
+      walk.unit_rows[(size_t)n * ceil_div(out_plane, 64) + p / 64] = make_int2(lo - 1, hi);
+      if (hi >= 0) atomicAdd(&met, (unsigned)(min(hi, g.in_h - 1) / walk.rows - max(lo - 1, 0) / walk.rows + 1));
+    }
   }
   __syncthreads();
   if (threadIdx.x == 0) {
@@ -1257,6 +1268,7 @@ __global__ __launch_bounds__(1024) void deform_tile_rows_kernel(Geo g, const T* 
     }
     table[(size_t)blockIdx.x * 2] = lo;
     table[(size_t)blockIdx.x * 2 + 1] = hi;
+    if (walk.met && met) atomicAdd(walk.met, met);
     if (tile == 0) most_img[n] = 0u;  // deform_sample_count_kernel, next on the stream, takes maxima into it
   }
 }
@@ -1272,7 +1284,7 @@ template <typename T>
 __global__ __launch_bounds__(1024) void deform_sample_count_kernel(Geo g, const T* __restrict__ off,
                                                                    const int* __restrict__ tile_rows,
                                                                    unsigned* __restrict__ most_img, int ntiles,
-                                                                   int band_rows) {
+                                                                   int band_rows, BandWalk walk) {
   extern __shared__ __align__(16) float lds[];
   unsigned* count = reinterpret_cast<unsigned*>(lds);
   __shared__ unsigned wave_most[16];
@@ -1280,6 +1292,7 @@ __global__ __launch_bounds__(1024) void deform_sample_count_kernel(Geo g, const 
   const int out_plane = g.out_h * g.out_w;
   const int nbands = ceil_div(H, band_rows);
   const int band = blockIdx.x % nbands, n = blockIdx.x / nbands;
+  if (walk.met && bands_take(walk)) return;
   const int r_lo = band * band_rows, r_hi = min(H, r_lo + band_rows);
   const int lo_idx = (r_lo + 1) * RS, hi_idx = (r_hi + 1) * RS;
   const int cells = band_rows * RS;
@@ -1348,7 +1361,7 @@ template <typename T, int SH, int SW, int NP, bool BAND = false>
 __global__ __launch_bounds__(1024) void deform_grad_input_tiled_kernel(
     Geo g, const T* __restrict__ gout, const T* __restrict__ off, const T* __restrict__ rot,
     const T* __restrict__ filter, T* __restrict__ gin, const unsigned* __restrict__ gmax_bits, int shift,
-    int band_rows, const int* __restrict__ tile_rows, const unsigned* __restrict__ most_img) {
+    int band_rows, const int* __restrict__ tile_rows, const unsigned* __restrict__ most_img, BandWalk walk) {
   using Tb = WideTable<SH, SW>;
   constexpr int NC = 2 * NP;  // channels per workgroup
   extern __shared__ __align__(16) float lds[];
@@ -1361,7 +1374,7 @@ __global__ __launch_bounds__(1024) void deform_grad_input_tiled_kernel(
   const int cpg = g.channel / g.groups;
   const int out_plane = g.out_h * g.out_w, in_plane = H * W;
   const BlockId b = decode_block(g, BAND ? ceil_div(H, band_rows) : 1, ceil_div(cpg, NC));
-  if (!b.valid) return;
+  if (!b.valid || (walk.met && bands_take(walk))) return;
   const int j0 = b.chunk * NC;
   const int nch = min(NC, cpg - j0);
   // BAND: the image rows r_lo .. r_hi - 1 are this workgroup's; row r sits in LDS row r - r_lo (no padding rows),
@@ -2789,51 +2802,68 @@ bool run_deform_grad_input(const Geo& g, const T* gout, const T* off, const T* r
                            void* ws, hipStream_t stream) {
   const DeformPlan d = grad_input_plan<SH, SW>(g);
   const bool tiled = !d.ok;  // output planes of more than 1024 pixels, input planes wider than 64 columns
-  size_t tiled_lds = 0;
-  int tiled_shift = 0, tiled_ch = 0;
+  // the tiled form's launch: channels / 2 per workgroup, bands of rows where not even one 64-bit plane fits, or only one (two
+  // channels per workgroup and walk), rows of the counting kernel's bands
+  int tiled_shift = 0, np = 0, brows = 0, crows = 0;
+  size_t lds = 0;
+  bool band = false;
+  auto count_kernel = deform_sample_count_kernel<T>;
   if (tiled) {
     // the basic limits of the tuned family (any width: the read-back loop walks the rows), then room for the 64-bit planes
     const DeformPlan basic = deform_plan(g, WideTable<SH, SW>::SIZE, 0, 1024, 2, 64 * 1024, 1 << 30, 1 << 30);
     if (!basic.ok) return false;
     tiled_shift = basic.shift;
-    tiled_ch = tiled_planes<SH, SW>(basic, &tiled_lds);
-  }
-  if (reinterpret_cast<uintptr_t>(gout) % 16 != 0) return false;  // absmax_kernel reads 16-byte vectors
-  unsigned* gmax = static_cast<unsigned*>(ws);
-  const long n = (long)g.batch * g.channel * g.out_h * g.out_w;
-  if (lanes_deform_grad_input_applies(g)) {
-    absmax_kernel<T><<<kAbsParts, 256, 0, stream>>>(gout, n, gmax);
-    if (lanes_deform_grad_input<T>(g, gout, off, rot, filter, gin, gmax, gmax + kAbsParts, stream)) return true;
-  }
-  if (tiled) {
-    // workspace: the maxima of |gout|, the images' sample counts, the tiles' rows
-    unsigned* most_img = gmax + kAbsParts;
-    int* table = reinterpret_cast<int*>(most_img + g.batch);
-    const int ntiles = ceil_div(g.out_h * g.out_w, 1024), cpg = g.channel / g.groups;
+    np = tiled_planes<SH, SW>(basic, &lds);
+    if (np <= 1 && !path_disabled(kNoDeformWindow)) {
+      size_t blds = 0;
+      const int bnp = band_planes<SH, SW>(g, &brows, &blds);
+      band = bnp >= 2 || (np == 0 && bnp == 1);
+      if (band) np = bnp, lds = blds;
+    }
     // the counting kernel's bands: about 512 workgroups, of at least 8 rows, of at most what fits as 32-bit counters
     const long cfit = (150L * 1024 / 4) / (g.in_w + 2) - 1;
     const int cbands = std::max(1, std::min(g.in_h / 8, ceil_div(512, std::max(1, g.batch))));
-    const int crows = (int)std::min<long>(cfit, ceil_div(g.in_h, cbands));
-    auto count_kernel = deform_sample_count_kernel<T>;
-    if (crows < 1 || !allow_max_dynamic_lds(reinterpret_cast<const void*>(count_kernel))) return false;
-    // not even one 64-bit plane fits, or only one (two channels per workgroup and walk): bands of rows
-    size_t blds = 0;
-    int brows = 0;
-    const int bnp = tiled_ch <= 1 && !path_disabled(kNoDeformWindow) ? band_planes<SH, SW>(g, &brows, &blds) : 0;
-    const bool band = bnp >= 2 || (tiled_ch == 0 && bnp == 1);
-    if (!band && tiled_ch == 0) return false;
-    const int np = band ? bnp : tiled_ch;
-    const size_t lds = band ? blds : tiled_lds;
+    crows = (int)std::min<long>(cfit, ceil_div(g.in_h, cbands));
+  }
+  if (reinterpret_cast<uintptr_t>(gout) % 16 != 0) return false;  // absmax_kernel reads 16-byte vectors
+  const bool pixel_lanes = !tiled || (np > 0 && crows >= 1 && allow_max_dynamic_lds(reinterpret_cast<const void*>(count_kernel)));
+  const bool channel_lanes = lanes_deform_grad_input_applies(g);
+  if (!pixel_lanes && !channel_lanes) return false;
+  // workspace: the maxima of |gout|, the units' rows, the images' sample counts, the tiles' rows, the count of a BandWalk
+  unsigned* gmax = static_cast<unsigned*>(ws);
+  int2* unit_rows = reinterpret_cast<int2*>(gmax + kAbsParts);
+  unsigned* most_img = reinterpret_cast<unsigned*>(unit_rows + (size_t)g.batch * ceil_div(g.out_h * g.out_w, 64));
+  int* table = reinterpret_cast<int*>(most_img + g.batch);
+  const int ntiles = ceil_div(g.out_h * g.out_w, 1024), cpg = g.channel / g.groups;
+  unsigned* met = reinterpret_cast<unsigned*>(table + (size_t)g.batch * ntiles * 2);
+  BandWalk walk{};
+  auto rows_kernel = [&] {
+    deform_tile_rows_kernel<T><<<(unsigned)(g.batch * ntiles), 1024, 0, stream>>>(g, off, table, ntiles, most_img, walk);
+  };
+  absmax_kernel<T><<<kAbsParts, 256, 0, stream>>>(gout, (long)g.batch * g.channel * g.out_h * g.out_w, gmax, met);
+  if (channel_lanes) {
+    walk = lanes_band_walk(g, rot != nullptr);
+    if (walk.rows) {
+      walk.unit_rows = unit_rows;
+      if (pixel_lanes && walk.most != ~0u) walk.met = met;
+      rows_kernel();
+    }
+    if (!lanes_deform_grad_input<T>(g, gout, off, rot, filter, gin, gmax, walk, stream))
+      walk = BandWalk{};
+    else if (!walk.met)
+      return true;
+  }
+  if (!pixel_lanes) return false;
+  if (tiled) {
     const unsigned tgrid = (unsigned)xcd_grid_size((long)(band ? ceil_div(g.in_h, brows) : 1) * ceil_div(cpg, 2 * np) * g.batch * g.groups);
 #define DK_LAUNCH(CH, BAND)                                                                                       \
   {                                                                                                               \
     auto kernel = deform_grad_input_tiled_kernel<T, SH, SW, CH, BAND>;                                            \
     if (!allow_max_dynamic_lds(reinterpret_cast<const void*>(kernel))) return false;                              \
-    absmax_kernel<T><<<kAbsParts, 256, 0, stream>>>(gout, n, gmax);                                               \
-    deform_tile_rows_kernel<T><<<(unsigned)(g.batch * ntiles), 1024, 0, stream>>>(g, off, table, ntiles, most_img); \
+    if (!walk.met) rows_kernel();                                                                                 \
     count_kernel<<<(unsigned)(g.batch * ceil_div(g.in_h, crows)), 1024, (size_t)crows * (g.in_w + 2) * 4, stream>>>( \
-        g, off, table, most_img, ntiles, crows);                                                                  \
-    kernel<<<tgrid, 1024, lds, stream>>>(g, gout, off, rot, filter, gin, gmax, tiled_shift, brows, table, most_img); \
+        g, off, table, most_img, ntiles, crows, walk);                                                            \
+    kernel<<<tgrid, 1024, lds, stream>>>(g, gout, off, rot, filter, gin, gmax, tiled_shift, brows, table, most_img, walk); \
   }
     if (band) {
       if (np == 4) DK_LAUNCH(4, true) else if (np == 2) DK_LAUNCH(2, true) else DK_LAUNCH(1, true)
@@ -2843,10 +2873,9 @@ bool run_deform_grad_input(const Geo& g, const T* gout, const T* off, const T* r
 #undef DK_LAUNCH
     return true;
   }
-  absmax_kernel<T><<<kAbsParts, 256, 0, stream>>>(gout, n, gmax);
   const unsigned grid = (unsigned)xcd_grid_size((long)d.chunks * g.batch * g.groups);
   deform_grad_input_kernel<T, SH, SW><<<grid, grad_input_block(g), d.lds, stream>>>(g, gout, off, rot, filter, gin, gmax,
-                                                                                   d.per, d.shift);
+                                                                                   d.per, d.shift, walk);
   return true;
 }
 
@@ -3091,10 +3120,10 @@ bool fast_deform_grad_input(const Geo& g, const T* gout, const T* off, const T* 
 }
 
 size_t fast_deform_grad_input_workspace(const Geo& g) {
-  // absmax_kernel's per-workgroup maxima of |gout|; then the tiled form's sample count per image and its table of two rows
-  // per (image, tile), or the lanes form's of two rows per image and 64 pixels
-  return (size_t)kAbsParts * sizeof(unsigned) + (size_t)g.batch * sizeof(unsigned) +
-         (size_t)g.batch * ceil_div(g.out_h * g.out_w, 64) * 2 * sizeof(int);
+  // absmax_kernel's per-workgroup maxima of |gout|, the least and largest row per image and 64 pixels (BandWalk), the tiled
+  // form's sample count per image and its table of two rows per (image, tile), one more count
+  return (size_t)kAbsParts * sizeof(unsigned) + (size_t)g.batch * ceil_div(g.out_h * g.out_w, 64) * sizeof(int2) +
+         (size_t)g.batch * sizeof(unsigned) + (size_t)g.batch * ceil_div(g.out_h * g.out_w, 1024) * 2 * sizeof(int) + sizeof(unsigned);
 }
 
 template <typename T>

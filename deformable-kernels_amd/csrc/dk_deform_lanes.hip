@@ -86,33 +86,6 @@ __host__ __device__ __forceinline__ int lanes_positions(int rows, int w, bool ba
   return band ? rows * (w + 1) + 3 : (rows + 2) * (w + 1) + 1;
 }
 
-// unit_rows of the band form: per 64 consecutive output pixels of an image the least and largest image row that their samples
-// read (K.cu:486-500); none: an empty range.  A wave per 64 pixels.
-template <typename T>
-__global__ __launch_bounds__(256) void deform_unit_rows_kernel(Geo g, const T* __restrict__ off, int2* __restrict__ unit_rows) {
-  const int out_plane = g.out_h * g.out_w, tiles = ceil_div(out_plane, 64);
-  const int id = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-  if (id >= g.batch * tiles) return;
-  const int n = id / tiles, p = (id - n * tiles) * 64 + lane;
-  const bool live = p < out_plane;
-  const int oh = live ? p / g.out_w : 0, ow = live ? p - oh * g.out_w : 0;
-  const rsrc_t ro = plane_rsrc(off + (size_t)n * 18 * out_plane, 18 * out_plane);
-  const unsigned step = (unsigned)out_plane * (unsigned)sizeof(T);
-  int lo = 1 << 29, hi = -(1 << 29);
-#pragma unroll
-  for (int t = 0; t < 9; ++t) {
-    const unsigned o = live ? (unsigned)(2 * t * out_plane + p) * (unsigned)sizeof(T) : kOutOfRange;
-    const float h = float(oh * g.stride_h - g.pad_h + t / 3 * g.dil_h) + buf_ld(ro, o, off);
-    const float w = float(ow * g.stride_w - g.pad_w + t % 3 * g.dil_w) + buf_ld(ro, o + step, off);
-    const bool hit = live && h > -1.f && w > -1.f && h < float(g.in_h) && w < float(g.in_w);
-    const int top = (int)floorf(h);
-    lo = hit ? min(lo, top) : lo;
-    hi = hit ? max(hi, top + 1) : hi;
-  }
-  lo = wave_min(lo), hi = wave_max(hi);
-  if (lane == 0) unit_rows[id] = make_int2(lo, hi);
-}
-
 // ---------------------------------------------------------------------------
 // One workgroup per (image, group, 32 channels); its LDS holds the whole zero-padded plane.  A unit of work is 16 output pixels x one row of
 // three taps: 12 samples for each of the wave's four rows of lanes, the waves take units in turn and load the next
@@ -124,8 +97,7 @@ __global__ __launch_bounds__(256) void deform_unit_rows_kernel(Geo g, const T* _
 // per channel, a lane's two of each tap of its unit in registers, instead of two table reads and six multiply-adds per
 // sample (N=64 C=192 28x28 float16: 99 -> 82 us).
 // BAND: planes whose sums do not fit LDS for 32 channels.  A workgroup owns `band_rows` image rows of its 32 channels and
-// walks the units whose samples touch them (unit_rows: per 64 output pixels the least and largest image row that their
-// samples read); a corner pair in another band's row is added to two spare positions instead, uncounted.  A band of 19
+// walks the units whose samples touch them (BandWalk, dk_deform.h, which also says in which calls); a corner pair in another band's row is added to two spare positions instead, uncounted.  A band of 19
 // rows of a 56 x 56 plane meets 61 % of the samples of the 31 - 36 rows it walks; N=64 C=144 56x56 float32, all kernels of
 // the gradient: 428 us with eight channels per workgroup and a pixel per lane (deform_grad_input_tiled_kernel, whose
 // descriptors alone take 100 vector instructions per sample and eight channels), 342 here; without a rotation tensor 417 and
@@ -134,10 +106,11 @@ template <typename T, int SH, int SW, bool PLAIN, bool BAND>
 __global__ __launch_bounds__(kLnBlock) void deform_grad_input_lanes_kernel(
     Geo g, const T* __restrict__ gout, const T* __restrict__ off, const T* __restrict__ rot,
     const T* __restrict__ filter, T* __restrict__ gin, const unsigned* __restrict__ gmax_bits, unsigned inv_out_w,
-    unsigned inv_in_w, int wide, int band_rows, const int2* __restrict__ unit_rows) {
+    unsigned inv_in_w, int wide, BandWalk by_bands, const int2* __restrict__ unit_rows) {
   constexpr int CELLS = (SH + 1) * (SW + 1);
   extern __shared__ __align__(16) unsigned long long sums[];  // [positions][kLnPitch], then the tables
   const int H = g.in_h, W = g.in_w, RS = W + 1;               // one padding column between two rows serves both
+  const int band_rows = by_bands.rows;
   const int npos = lanes_positions(BAND ? band_rows : H, W, BAND);
   float4* tbl = reinterpret_cast<float4*>(sums + ((npos * kLnPitch + 1) & ~1));  // [CELLS][2][kLnPairs]
   __shared__ float wmax[kLnCh];
@@ -156,6 +129,7 @@ __global__ __launch_bounds__(kLnBlock) void deform_grad_input_lanes_kernel(
   const int row0 = BAND ? -r_lo : 1;
   const int spare = BAND ? band_rows * RS + 1 : 0;  // position of what is no sample of these rows (not BAND: the padding row on top)
   const int n = z / g.groups, grp = z % g.groups;
+  if (BAND && by_bands.met && !bands_take(by_bands)) return;
   const int j0 = chunk * kLnCh, nch = min(kLnCh, cpg - j0);
 
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -464,8 +438,8 @@ LanesPlan lanes_plan(const Geo& g) {
   if (lanes_positions(g.in_h, g.in_w, false) > fit) {
     // bands of equal height.  Every band walks the rows its samples can come from: with fewer than kLnBandRows rows the
     // walk is mostly over samples of other bands (us here / with a pixel per lane, offsets ~ N(0, 2^2): N=64 C=96 40 x 40
-    // 130 / 149, N=24 C=64 64 x 64 101 / 113, N=16 80 x 80 (12 rows) 106 / 113; 75 x 101 float16 (10 rows) 135 / 118.  Offsets
-    // ~ N(0, 5^2) widen the walk: 56 x 56 402 / 387)
+    // 130 / 149, N=24 C=64 64 x 64 101 / 113, N=16 80 x 80 (12 rows) 106 / 113; 75 x 101 float16 (10 rows) 135 / 118).
+    // Wide offsets: band_limit
     const int most = (int)std::max(0L, (fit - 3) / (g.in_w + 1));
     if (most < 1) return m;
     m.rows = ceil_div(g.in_h, ceil_div(g.in_h, most));
@@ -481,9 +455,20 @@ LanesPlan lanes_plan(const Geo& g) {
   return m;
 }
 
+// Bands that a unit of 64 pixels meets on average, in sixteenths, up to which the bands are the faster form.  float32, us in
+// bands / with a pixel per lane at so many, offsets ~ N(0, 2^2 .. 10^2), with a rotation tensor: N=64 C=96 40 x 40 (two bands) 1.51: 136 / 143,
+// 1.78: 145 / 139; N=64 C=144 56 x 56 (three) 1.72: 360 / 403, 2.15: 405 / 390, 2.73: 468 / 373; N=24 C=64 64 x 64 (four) 1.95:
+// 113 / 116, 2.45: 130 / 114; N=16 C=64 80 x 80 (seven) 2.08: 108 / 115, 2.49: 121 / 119, 4.9: 187 / 127.  Without one: 56 x 56 2.73: 378 /
+// 376; 64 x 64 2.45: 108 / 116, 3.4: 127 / 111; 80 x 80 3.25: 118 / 121, 4.9: 152 / 127; two bands are never slower.  The launches of
+// the form that finds nothing to do take 5 - 9 us (56 x 56: 340 -> 343 in bands, 390 -> 396 beside them).
+int band_limit(bool plain, int bands) {
+  if (plain) return bands <= 4 ? 43 : 50;
+  return bands == 2 ? 25 : bands <= 4 ? 32 : 36;
+}
+
 template <typename T, int SH, int SW>
 bool run_lanes_grad_input(const Geo& g, const T* gout, const T* off, const T* rot, const T* filter, T* gin,
-                          const unsigned* gmax, void* table, hipStream_t stream) {
+                          const unsigned* gmax, BandWalk walk, hipStream_t stream) {
   const LanesPlan m = lanes_plan<SH, SW>(g);
   if (!m.ok) return false;
   const int wide = g.out_h * g.out_w % 4 == 0 && reinterpret_cast<uintptr_t>(gout) % (4 * sizeof(T)) == 0;
@@ -492,13 +477,9 @@ bool run_lanes_grad_input(const Geo& g, const T* gout, const T* off, const T* ro
   auto kernel = m.band ? plain ? deform_grad_input_lanes_kernel<T, SH, SW, true, true> : deform_grad_input_lanes_kernel<T, SH, SW, false, true>
                        : plain ? deform_grad_input_lanes_kernel<T, SH, SW, true, false> : deform_grad_input_lanes_kernel<T, SH, SW, false, false>;
   if (!allow_dynamic_lds(reinterpret_cast<const void*>(kernel), kLnLds)) return false;
-  int2* unit_rows = static_cast<int2*>(table);
-  if (m.band) {
-    const int tiles = g.batch * ceil_div(g.out_h * g.out_w, 64);
-    deform_unit_rows_kernel<T><<<ceil_div(tiles, 4), 256, 0, stream>>>(g, off, unit_rows);
-  }
+  walk.rows = m.rows;
   kernel<<<(unsigned)xcd_grid_size(m.blocks), kLnBlock, m.lds, stream>>>(g, gout, off, rot, filter, gin, gmax,
-                                                                         inverse(g.out_w), inverse(g.in_w), wide, m.rows, unit_rows);
+                                                                         inverse(g.out_w), inverse(g.in_w), wide, walk, walk.unit_rows);
   return true;
 }
 
@@ -517,10 +498,25 @@ bool lanes_deform_grad_input_applies(const Geo& g) {
   return false;
 }
 
+BandWalk lanes_band_walk(const Geo& g, bool rotation) {
+  auto walk = [&](const LanesPlan& m) {
+    BandWalk w{};
+    if (!m.ok || !m.band) return w;
+    const int bands = ceil_div(g.in_h, m.rows), limit = band_limit(!rotation && !path_disabled(kNoDeformPlain), bands);
+    w.rows = m.rows;
+    w.most = path_disabled(kForceDeformLanes) || 16 * bands <= limit ? ~0u : (unsigned)((long)g.batch * ceil_div(g.out_h * g.out_w, 64) * limit / 16);
+    return w;
+  };
+#define CALL(SH, SW) walk(lanes_plan<SH, SW>(g))
+  DK_LANES_SCOPE(g, CALL)
+#undef CALL
+  return BandWalk{};
+}
+
 template <typename T>
 bool lanes_deform_grad_input(const Geo& g, const T* gout, const T* off, const T* rot, const T* filter, T* gin,
-                             const unsigned* gmax, void* table, hipStream_t stream) {
-#define CALL(SH, SW) run_lanes_grad_input<T, SH, SW>(g, gout, off, rot, filter, gin, gmax, table, stream)
+                             const unsigned* gmax, const BandWalk& walk, hipStream_t stream) {
+#define CALL(SH, SW) run_lanes_grad_input<T, SH, SW>(g, gout, off, rot, filter, gin, gmax, walk, stream)
   DK_LANES_SCOPE(g, CALL)
 #undef CALL
   return false;
@@ -528,7 +524,7 @@ bool lanes_deform_grad_input(const Geo& g, const T* gout, const T* off, const T*
 
 #define DK_INSTANTIATE(T)                                                                                         \
   template bool lanes_deform_grad_input<T>(const Geo&, const T*, const T*, const T*, const T*, T*, const unsigned*, \
-                                           void*, hipStream_t);
+                                           const BandWalk&, hipStream_t);
 DK_INSTANTIATE(float)
 DK_INSTANTIATE(__half)
 DK_INSTANTIATE(bf16_t)

@@ -113,12 +113,14 @@ size_t fast_deform_grad_input_workspace(const Geo& g);
 template <typename T>
 bool fast_deform_grad_input(const Geo& g, const T* gout, const T* off, const T* rot, const T* filter, T* gin,
                             void* ws, hipStream_t stream);
-// its form with the lanes along the channels (dk_deform_lanes.hip), called behind absmax_kernel: gmax = its maxima;
-// table: 8-byte aligned, two words per image and 64 output pixels
+// its form with the lanes along the channels (dk_deform_lanes.hip), called behind absmax_kernel: gmax = its maxima.
+// lanes_band_walk: `rows` and `most` (~0: any) of the walk where it works in bands of rows; the caller adds the rest
+struct BandWalk;
 bool lanes_deform_grad_input_applies(const Geo& g);
+BandWalk lanes_band_walk(const Geo& g, bool rotation);
 template <typename T>
 bool lanes_deform_grad_input(const Geo& g, const T* gout, const T* off, const T* rot, const T* filter, T* gin,
-                             const unsigned* gmax, void* table, hipStream_t stream);
+                             const unsigned* gmax, const BandWalk& walk, hipStream_t stream);
 // rotation = false: gradient w.r.t. the image-space offsets
 size_t fast_deform_grad_coord_workspace(const Geo& g, bool rotation);
 template <typename T>

@@ -440,6 +440,55 @@ def test_grad_input_with_the_lanes_along_the_channels_in_bands(case, dtype, rota
     _grad_input_with_the_lanes_along_the_channels(case, dtype, rotation)
 
 
+@pytest.mark.parametrize("rotation", [True, False])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("N, C, H, W, bands_of", [
+    (5, 288, 56, 56, 3),    # beside the form that walks tiles of 1024 pixels
+    (5, 544, 128, 8, 2),    # beside the form of one workgroup per plane
+    (5, 224, 64, 64, 4),
+])
+def test_grad_input_in_bands_leaves_wide_offsets_to_the_form_with_a_pixel_per_lane(N, C, H, W, bands_of, dtype, rotation):
+    """The default dispatch on offsets of half a pixel, of most of the plane's height, of one such image among narrow ones, and beyond
+    the plane (no sample inside): the gradient is one form's to the bit -- the bands' for few rows per unit and for none -- and
+    that of the oracle.  The workspace starts as garbage each time."""
+    from deformable_kernels.ops.deform_kernel import _lib
+    x, wt, rot, off, gout, cfg = make_deform(N, C, H, W, 3, (4, 4), 1, 1, 1, 1, 0.7, 0.5, seed=6, dtype=torch.float32)
+    if not rotation:
+        rot.zero_()
+    x, wt, rot, gout = [t.to(dtype) for t in (x, wt, rot, gout)]
+    dev = torch.device("cuda:0")
+    wg, rg, gg = [t.to(dev) for t in (wt, rot, gout)]
+    L, P = _lib.lib(), _lib.ptr
+    desc = _lib.conv_desc(x, wg, cfg["kernel_size"], cfg["stride"], cfg["padding"], cfg["dilation"], 1)
+    ws, nbytes = _lib.workspace(L.dk_deformable_sample_depthwise_backward_data_workspace(desc), dev)
+
+    def grad_input(og, *switches):
+        gin = torch.full((N, C, H, W), float("nan"), device=dev, dtype=dtype)
+        ws.fill_(0xEE)
+        with _lib.test_switches(*switches):
+            _lib.check(L.dk_deformable_sample_depthwise_backward_data(
+                desc, P(gg), P(og), P(rg if rotation else None), P(wg), P(gin), P(ws), nbytes, _lib.stream_ptr(gin)), "grad input")
+        return gin.cpu()
+
+    # rows of offsets: per image; whether the bands take them
+    always = not rotation and bands_of == 2   # without a rotation tensor two bands are never the slower form
+    for rows, bands in ([1.0] * N, True), ([2.0 * H] * N, always), ([2.0 * H] + [1.0] * (N - 1), True), (None, True):
+        o = off.clone()
+        if rows is None:
+            o += 2.5 * H
+        else:
+            o[:, 0::2] *= torch.tensor(rows).view(N, 1, 1, 1)
+        o = o.to(dtype)
+        og = o.to(dev)
+        got = grad_input(og)
+        assert torch.equal(got, grad_input(og, "DK_FORCE_DEFORM_LANES" if bands else "DK_NO_DEFORM_LANES"))
+        want = _oracle((x, wt, rot, o, gout, cfg), np.float64)[1]
+        if dtype == torch.float32:
+            assert mixed_err(got, want) < 1e-5
+        else:
+            assert rel_err(got.float(), want) < 1e-2
+
+
 @pytest.mark.parametrize("clip", [(0.25, 0.75), (-1.5, -0.75)])
 def test_grad_input_with_the_lanes_along_the_channels_at_a_clipped_zero_rotation(clip):
     _grad_input_with_the_lanes_along_the_channels(LANES_CASES[2], torch.float32, rotation=False, clip=clip)
