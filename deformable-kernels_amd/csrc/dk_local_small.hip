@@ -10,7 +10,7 @@
 //   grad filter    one channel: 16 waves share the pixels; a lane keeps a sum per scope cell, dense hat weights
 // fp32 arithmetic for every type (reference kernels: K.cu:577-702, 836-999, 1285-1408).  What the reference skips -- a tap
 // outside the image, off the stride's grid or outside the scope, a cell that a tap does not read -- takes nothing from a value
-// that is not finite.  Registers: 1024 threads leave 128 of them; scope 7 spills 96 bytes per lane, the others nothing.
+// that is not finite.  Registers: 1024 threads leave 128 of them; nothing spills.
 #include <algorithm>
 
 #include "dk_common.h"
@@ -210,7 +210,7 @@ __global__ __launch_bounds__(64 * kSmWaves) void local_small_backward_kernel(Geo
   b -= roles.rotation_tiles;
 
   const int c = b, grp = c % g.groups, total = g.batch * out_plane;
-  float acc[CELLS];
+  float acc[CELLS], z = 0.f;  // z: NaN where a product is not finite
 #pragma unroll
   for (int i = 0; i < CELLS; ++i) acc[i] = 0.f;
   for (int base = wave * 64; base < total; base += kSmWaves * 64) {
@@ -226,43 +226,48 @@ __global__ __launch_bounds__(64 * kSmWaves) void local_small_backward_kernel(Geo
       const unsigned ro = live ? (unsigned)(n * st.rn + (grp * 18 + 2 * t) * st.rc + p * st.rp) * E : kOutOfRange;
       rh[t] = buf_ld2(rr, ro, 0, tag), rw[t] = buf_ld2(rr, ro, st.rc * (int)E, tag);
     }
-    float v[kSmTaps], z = 0.f;  // z: NaN where a product is not finite
-#pragma unroll
-    for (int t = 0; t < kSmTaps; ++t) v[t] = xv[t] * gv, z = fmaf(v[t], 0.f, z);
-    if (__any(z != 0.f)) {
-      // such a product must not meet the zero hats of the cells that its tap does not read (K.cu:85-114), nor the zero read for a
-      // tap outside the image: a tap at a time, its operands read again
-#pragma unroll 1
-      for (int t = 0; t < kSmTaps; ++t) {
-        const int iy = oh * g.stride_h - g.pad_h + t / 3 * g.dil_h, ix = ow * g.stride_w - g.pad_w + t % 3 * g.dil_w;
-        const bool hit = live && iy >= 0 && iy < g.in_h && ix >= 0 && ix < g.in_w;
-        const float p1 = gv * buf_ld2(rx, hit ? (unsigned)(n * st.xn + (iy * g.in_w + ix) * st.xp) * E : kOutOfRange, c * st.xc * (int)E, tag);
-        const unsigned ro = live ? (unsigned)(n * st.rn + (grp * 18 + 2 * t) * st.rc + p * st.rp) * E : kOutOfRange;
-        const float h = scope_coord<float>(g, t / 3, buf_ld2(rr, ro, 0, tag), g.centre_h);
-        const float w = scope_coord<float>(g, t % 3, buf_ld2(rr, ro, st.rc * (int)E, tag), g.centre_w);
-        const bool in = hit && h > -1.f && w > -1.f && h < float(S) && w < float(S);
-        const int i0 = in ? (int)floorf(h) : 0, k0 = in ? (int)floorf(w) : 0;
-#pragma unroll
-        for (int i = 0; i < S; ++i) {
-          const float a = p1 * (1.f - fabsf(h - (float)i));
-#pragma unroll
-          for (int k = 0; k < S; ++k)
-            acc[i * S + k] += in && (unsigned)(i - i0) < 2u && (unsigned)(k - k0) < 2u ? a * (1.f - fabsf(w - (float)k)) : 0.f;
-        }
-      }
-      continue;
-    }
 #pragma unroll
     for (int t = 0; t < kSmTaps; ++t) {
       const float h = scope_coord<float>(g, t / 3, rh[t], g.centre_h), w = scope_coord<float>(g, t % 3, rw[t], g.centre_w);
+      const float v = xv[t] * gv;
+      z = fmaf(v, 0.f, z);
       float hw[S];
 #pragma unroll
       for (int k = 0; k < S; ++k) hw[k] = fmaxf(0.f, 1.f - fabsf(w - (float)k));
 #pragma unroll
       for (int i = 0; i < S; ++i) {
-        const float a = v[t] * fmaxf(0.f, 1.f - fabsf(h - (float)i));
+        const float a = v * fmaxf(0.f, 1.f - fabsf(h - (float)i));
 #pragma unroll
         for (int k = 0; k < S; ++k) acc[i * S + k] = fmaf(a, hw[k], acc[i * S + k]);
+      }
+    }
+  }
+  if (__any(z != 0.f)) {
+    // a product that is not finite must not meet the zero hats of the cells that its tap does not read (K.cu:85-114), nor the zero
+    // read for a tap outside the image: the wave's pixels once more, a tap and its own cells at a time
+#pragma unroll
+    for (int i = 0; i < CELLS; ++i) acc[i] = 0.f;
+    for (int base = wave * 64; base < total; base += kSmWaves * 64)
+#pragma unroll 1
+    for (int t = 0; t < kSmTaps; ++t) {
+      const int q = base + lane;
+      const bool live = q < total;
+      const int n = live ? q / out_plane : 0, p = live ? q - n * out_plane : 0, oh = p / g.out_w, ow = p - oh * g.out_w;
+      const int iy = oh * g.stride_h - g.pad_h + t / 3 * g.dil_h, ix = ow * g.stride_w - g.pad_w + t % 3 * g.dil_w;
+      const bool hit = live && iy >= 0 && iy < g.in_h && ix >= 0 && ix < g.in_w;
+      const float v = buf_ld2(rg, live ? (unsigned)(n * st.on + p * st.op) * E : kOutOfRange, c * st.oc * (int)E, tag) *
+                      buf_ld2(rx, hit ? (unsigned)(n * st.xn + (iy * g.in_w + ix) * st.xp) * E : kOutOfRange, c * st.xc * (int)E, tag);
+      const unsigned ro = live ? (unsigned)(n * st.rn + (grp * 18 + 2 * t) * st.rc + p * st.rp) * E : kOutOfRange;
+      const float h = scope_coord<float>(g, t / 3, buf_ld2(rr, ro, 0, tag), g.centre_h);
+      const float w = scope_coord<float>(g, t % 3, buf_ld2(rr, ro, st.rc * (int)E, tag), g.centre_w);
+      const bool in = hit && h > -1.f && w > -1.f && h < float(S) && w < float(S);
+      const int i0 = in ? (int)floorf(h) : 0, k0 = in ? (int)floorf(w) : 0;
+#pragma unroll
+      for (int i = 0; i < S; ++i) {
+        const float a = v * (1.f - fabsf(h - (float)i));
+#pragma unroll
+        for (int k = 0; k < S; ++k)
+          acc[i * S + k] += in && (unsigned)(i - i0) < 2u && (unsigned)(k - k0) < 2u ? a * (1.f - fabsf(w - (float)k)) : 0.f;
       }
     }
   }
