@@ -384,7 +384,9 @@ int dk_sample_depthwise_backward_filter_static(const dk_conv_desc* desc, const v
 
 // Small layers: the gradients in one launch (dk_local_small.hip), which has no partial sums of its own
 static bool backward_in_one_launch(const Geo& g, const dk_conv_desc* desc) {
-  return desc->dtype != DK_F64 && (desc->layout != DK_LAYOUT_NHWC || nhwc_supported(g, desc->dtype)) && local_small_backward_supported(g);
+  const bool channels_last = desc->layout == DK_LAYOUT_NHWC;
+  return desc->dtype != DK_F64 && (!channels_last || nhwc_supported(g, desc->dtype)) &&
+         local_small_backward_supported(g, channels_last, desc->dtype == DK_F32);
 }
 
 static size_t backward_need(const Geo& g, const dk_conv_desc* desc, bool rotation, bool filter) {

@@ -206,7 +206,7 @@ bool offset_wgrad16(int batch, int cin, int cout, int h, int w, int stride, cons
 
 // dk_local_small.hip: the gradients of the local operator on small layers in one launch (not float64; never while a test
 // switch is set: the switches are about the kernels of the larger layers).  A null result is not computed.
-bool local_small_backward_supported(const Geo& g);
+bool local_small_backward_supported(const Geo& g, bool channels_last, bool float32);
 template <typename T>
 void local_small_backward(const Geo& g, bool channels_last, const T* gout, const T* x, const T* rot, const T* filter, T* gin,
                           T* grot, T* gfilter, hipStream_t stream);

@@ -285,18 +285,40 @@ __global__ __launch_bounds__(64 * kSmWaves) void local_small_backward_kernel(Geo
   }
 }
 
+SmallRoles small_roles(const Geo& g, bool input, bool rotation, bool filter) {
+  SmallRoles roles{};
+  if (input) {
+    roles.input_tiles = g.groups * ceil_div(g.batch * g.in_h * g.in_w, 64);
+    // two channels per wave at least, about a workgroup per CU
+    roles.input_splits = std::max(1, std::min(ceil_div(g.channel / g.groups, 2 * kSmWaves), 256 / roles.input_tiles));
+  }
+  if (rotation) roles.rotation_tiles = g.groups * ceil_div(g.batch * g.out_h * g.out_w, 64);
+  if (filter) roles.filter_channels = g.channel;
+  return roles;
+}
+int small_blocks(const SmallRoles& r) { return r.input_tiles * r.input_splits + r.rotation_tiles + r.filter_channels; }
 }  // namespace
 
 // At most 2048 output pixels and 256 channels per group: a wave of the grad filter then has two groups of pixels, one of the
-// grad rotation at most 16 channels in a row.  All gradients through the autograd operator on a box with slow host calls, us,
-// one launch / the larger layers' kernels: 2 x 32 x 28^2 float32 48.6 / 58.6, 1 x 16 x 7^2 46.6 / 55.0, 10 x 96 x 14^2 scope 5
-// float16 47.5 / 59.0, 1 x 17 x 56^2 stride 2 45.3 / 57.1; beyond: 3 x 912 x 14^2 (57 channels in a row) 87.5 / 57.2, 100 x
-// 200 x 7^2 (4900 pixels) 74.4 / 58.3, and 5 x 192 x 28^2 level.
-bool local_small_backward_supported(const Geo& g) {
-  return test_switches() == 0 && g.k_h == 3 && g.k_w == 3 && g.scope_h == g.scope_w &&
-         (g.scope_h == 3 || g.scope_h == 4 || g.scope_h == 5 || g.scope_h == 7) && g.batch > 0 &&
-         (long)g.batch * g.out_h * g.out_w <= 2048 && (long)g.batch * g.in_h * g.in_w <= 16384 && g.channel / g.groups <= 256 &&
-         g.groups <= 16;
+// grad rotation at most 16 channels in a row.  All gradients, us on the GPU alone, one launch / the larger layers' kernels, whose
+// four or five launches also take 14 - 20 us of host time more: 2 x 32 x 28^2 float32 12.1 / 33.3, 10 x 96 x 14^2 18.3 / 37.2, 2 x 256 x
+// 32^2 37.4 / 45.7, 2 x 128 x 56^2 stride 2 26.0 / 39.3; beyond: 3 x 912 x 14^2 (57 channels in a row) and 100 x 200 x 7^2 (4900 pixels)
+// a third slower.  Several groups multiply the input's and rotation's workgroups: up to 850 of all roles (a CU holds one at a
+// time) 2 x 512 x 32^2 in two groups 47 / 59, 28^2 in eight 30 / 36; more: 28^2 in sixteen (928) bfloat16 35 / 33, 2 x 512 x 32^2 in eight
+// (1024) 50 / 45, 2 x 256 x 32^2 in sixteen (1280) 48 / 31.
+// Channels-last: a channel's lanes read elements that are far apart, so where the larger layers' kernels run on the matrix
+// cores (one group, channels in eights) they are level at 32 channels: 2 x 16 x 32^2 18.7 / 19.1, 32 channels 22.8 / 21.0 (float32 at stride 2, whose
+// input gradient is a launch of its own, 16 channels 22.6 / 20.7, 32 channels 27.6 / 22.4), 64 channels 32.5 / 25.1, 128 channels 51 / 32; scope 7,
+// 128 channels, 51 / 55, 192 channels of 28^2 69 / 65.  Elsewhere: 2 x 33 x 32^2 20 / 48, 132 channels 39 / 57, 2 x 64 x 32^2 in two groups 26 / 378.
+bool local_small_backward_supported(const Geo& g, bool channels_last, bool float32) {
+  if (test_switches() != 0 || g.k_h != 3 || g.k_w != 3 || g.scope_h != g.scope_w || g.batch <= 0) return false;
+  if (g.scope_h != 3 && g.scope_h != 4 && g.scope_h != 5 && g.scope_h != 7) return false;
+  if ((long)g.batch * g.out_h * g.out_w > 2048 || (long)g.batch * g.in_h * g.in_w > 16384) return false;
+  if (g.channel / g.groups > 256 || g.groups > 16) return false;
+  if (!channels_last) return small_blocks(small_roles(g, true, true, true)) <= 850;
+  if (g.groups > 1 || g.channel % 8 != 0) return true;
+  const bool apart = float32 && (g.stride_h > 1 || g.stride_w > 1);
+  return g.channel <= (g.scope_h == 7 ? 128 : apart ? 16 : 32);
 }
 
 template <typename T>
@@ -305,16 +327,8 @@ void local_small_backward(const Geo& g, bool channels_last, const T* gout, const
   const int pi = g.in_h * g.in_w, po = g.out_h * g.out_w, cr = 18 * g.groups;
   const SmallStrides st = channels_last ? SmallStrides{pi * g.channel, 1, g.channel, po * g.channel, 1, g.channel, po * cr, 1, cr}
                                         : SmallStrides{pi * g.channel, pi, 1, po * g.channel, po, 1, po * cr, po, 1};
-  SmallRoles roles{};
-  const int cpg = g.channel / g.groups;
-  if (gin) {
-    roles.input_tiles = g.groups * ceil_div(g.batch * pi, 64);
-    // two channels per wave at least, about a workgroup per CU
-    roles.input_splits = std::max(1, std::min(ceil_div(cpg, 2 * kSmWaves), 256 / roles.input_tiles));
-  }
-  if (grot) roles.rotation_tiles = g.groups * ceil_div(g.batch * po, 64);
-  if (gfilter) roles.filter_channels = g.channel;
-  const int blocks = roles.input_tiles * std::max(1, roles.input_splits) + roles.rotation_tiles + roles.filter_channels;
+  const SmallRoles roles = small_roles(g, gin, grot, gfilter);
+  const int blocks = small_blocks(roles);
   if (blocks == 0) return;
 #define DK_LAUNCH(S) local_small_backward_kernel<T, S><<<blocks, 64 * kSmWaves, 0, stream>>>(g, st, roles, gout, x, rot, filter, gin, grot, gfilter)
   if (g.scope_h == 3) DK_LAUNCH(3);

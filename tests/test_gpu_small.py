@@ -100,7 +100,7 @@ def test_a_non_finite_value_reaches_what_the_reference_lets_it_reach(what, S, st
     """No test switch is set.  Taps outside the image or the scope and, at stride 2, off its grid read nothing of the channel
     with the poisoned value, and a product reaches the four cells of its own sample."""
     from deformable_kernels.ops.deform_kernel.functions import sample_depthwise
-    x, wt, rot, gout, cfg = make_local(2, 32, 11, 13, 3, (S, S), stride, 1, 1, G, 0.7, seed=8)
+    x, wt, rot, gout, cfg = make_local(2, 16, 11, 13, 3, (S, S), stride, 1, 1, G, 0.7, seed=8)
     rot[0, :, 1, 1] = 50.0   # all taps of this pixel leave the scope
     x, wt, rot, gout = [t.to(getattr(torch, dtype_name)) for t in (x, wt, rot, gout)]
     NON_FINITE[what](x, wt, rot, gout)
@@ -143,3 +143,21 @@ def test_float32_channels_last_grad_input_above_stride_1_is_the_table_kernels_to
     assert torch.equal(small[0], table[0]) and torch.equal(grads(leaves[:1])[0], table[0])
     for a, b in zip(small[1:], table[1:]):
         assert rel_err(a.cpu(), b.double().cpu().numpy()) < 1e-5
+
+
+@pytest.mark.parametrize("one_launch, shape, scope, stride, G, dtype_name, channels_last", [
+    (True, (2, 32, 28, 28), 4, 1, 1, "float32", False), (True, (2, 256, 32, 32), 7, 1, 1, "bfloat16", False),
+    (True, (2, 512, 32, 32), 4, 1, 2, "float32", False), (True, (1, 512, 28, 28), 4, 1, 8, "float32", False),
+    (False, (1, 512, 28, 28), 4, 1, 16, "bfloat16", False), (False, (2, 256, 32, 32), 4, 1, 16, "float32", False),
+    (False, (2, 1024, 32, 32), 4, 1, 4, "float32", False), (False, (1, 4096, 7, 7), 7, 1, 16, "float32", False),
+    (False, (2, 256, 32, 33), 4, 1, 1, "float32", False), (False, (1, 257, 7, 7), 4, 1, 1, "float32", False),
+    (True, (2, 32, 32, 32), 4, 1, 1, "float32", True), (False, (2, 40, 32, 32), 4, 1, 1, "bfloat16", True),
+    (True, (2, 16, 56, 56), 4, 2, 1, "float32", True), (False, (2, 24, 56, 56), 4, 2, 1, "float32", True),
+    (True, (2, 24, 56, 56), 4, 2, 1, "float16", True), (True, (2, 128, 32, 32), 7, 1, 1, "float32", True),
+    (False, (2, 136, 32, 32), 7, 1, 1, "float32", True), (True, (2, 132, 32, 32), 4, 1, 1, "float32", True),
+    (True, (2, 64, 32, 32), 4, 1, 2, "bfloat16", True),
+])
+def test_layers_that_take_the_one_launch(one_launch, shape, scope, stride, G, dtype_name, channels_last):
+    """Either side of the rule's lines (channels-last too, where the gradients' own tests cannot tell the route)."""
+    cfg = {"kernel_size": (3, 3), "stride": (stride,) * 2, "padding": (1, 1), "dilation": (1, 1), "groups": G}
+    assert _supported(cfg, shape, (scope, scope), dtype_name, int(channels_last)) == one_launch
