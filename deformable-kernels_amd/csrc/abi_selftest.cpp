@@ -130,6 +130,9 @@ int main() {
   oc.w = 57;
   EXPECT(dk_offset_conv_supported(&oc) == 0);
   EXPECT(dk_offset_conv_forward(&oc, one, one, one, one, one, 1 << 30, nullptr) == DK_ERR_UNSUPPORTED);
+  const dk_offset_conv_desc wide = {1, 2000000, 18, 1, 1, DK_F32};  // more rows of channels than a grid has
+  EXPECT(dk_offset_conv_direct_worthwhile(&wide) == 0 && dk_offset_conv_direct_backward_worthwhile(&wide) == 0);
+  EXPECT(dk_offset_conv_direct_backward_input(&wide, one, one, one, nullptr) == DK_ERR_UNSUPPORTED);
   EXPECT(dk_offset_conv_backward_bias(nullptr, one, one, one, 0, nullptr) == DK_ERR_NULL_POINTER);
   // the input gradient: planes 7 .. 112 wide; float32 tensors as bfloat16 pairs unless that is switched off
   oc.w = 56;

@@ -993,13 +993,40 @@ static int check_offset_conv_direct(const dk_offset_conv_desc* d) {
   return offset_conv_direct_supported(d->batch, d->in_channels, d->out_channels, d->h, d->w) ? DK_OK : DK_ERR_UNSUPPORTED;
 }
 
-// Measured through the autograd operator against the library convolution, us (forward, gradients), here / library:
-// 1 x 192 x 28^2 float32 13 / 31, 33 / 73; 15 x 192 x 28^2 stride 2 22 / 66, 67 / 93; 63 x 608 x 7^2 52 / 101, 94 / 96
-// (1.9 M pixel-channels); above that the vector unit falls behind: 30 x 384 x 14^2 bfloat16 (2.3 M) 55 / 49, 96 / 86.
-int dk_offset_conv_direct_worthwhile(const dk_offset_conv_desc* desc) {
+// Channels-times-pixels of the calls that these kernels are for, or 0: too few images for the matrix-instruction kernels.
+static long offset_conv_direct_work(const dk_offset_conv_desc* desc) {
   if (check_offset_conv_direct(desc) != DK_OK || !dk_offset_conv_supported(desc) || dk_offset_conv_worthwhile(desc)) return 0;
   const long stride = desc->stride == 2 ? 2 : 1, pixels = ((desc->h - 1) / stride + 1) * ((desc->w - 1) / stride + 1);
-  return pixels * desc->batch * desc->in_channels <= 2000000;
+  return pixels * desc->batch * desc->in_channels;
+}
+
+// Measured through the operator against the library convolution, us here / library: 1 x 192 x 28^2 float32 13 / 31; 15 x 192 x 28^2
+// stride 2 22 / 66; 63 x 608 x 7^2 52 / 101 (1.9 M pixel-channels); above that the vector unit falls behind: 30 x 384 x 14^2 bfloat16
+// (2.3 M) 55 / 49.  A wave's channels are a serial chain, so many of them lose to the library where it has a kernel that suits:
+//   stride 2 on planes from 56 on (the lanes' reads are far apart): 1 x 304 x 56^2 32 / 34, 1 x 336 x 56^2 37 / 33, 1 x 768 x 56^2 bfloat16 81 / 38
+//   multiples of 128 channels: 1 x 640 x 14^2 39 / 47, 4 x 768 x 7^2 51 / 37; stride 2 8 x 384 x 28^2 35 / 40, 8 x 640 x 14^2 58 / 49, 8 x 768 x
+//   14^2 69 / 38 (others: 8 x 736 x 14^2 67 / 163, 4 x 944 x 7^2 61 / 144)
+//   one image in 16 bits: 832 channels of 14^2 48 / 52, 864 channels 51 / 48, 960 channels at stride 2 57 / 48 (four images 61 / 87)
+//   two pixels per lane (more than 8192 pixels): float32 16 x 96 x 28^2 26 / 27, 144 channels 36 / 34; float16 64 channels 22 / 22, 96 channels
+//   30 / 23; bfloat16 144 channels 39 / 107
+int dk_offset_conv_direct_worthwhile(const dk_offset_conv_desc* desc) {
+  const long work = offset_conv_direct_work(desc);
+  if (work == 0 || work > 2000000) return 0;
+  const int c = desc->in_channels;
+  const bool half = desc->dtype != DK_F32, strided = desc->stride == 2;
+  if (strided && desc->w >= 56 && c > 304) return 0;
+  if (c % 128 == 0 && c > (strided ? 384 : 640)) return 0;
+  if (half && desc->batch == 1 && c > 840) return 0;
+  if (!strided && work / c > 8192 && desc->dtype != DK_BF16) return c <= (half ? 64 : 128);
+  return 1;
+}
+
+// The input and the weight gradient: 1 x 192 x 28^2 float32 33 / 73, 63 x 608 x 7^2 94 / 96; 30 x 384 x 14^2 bfloat16 (2.3 M) 96 / 86.  At stride 2
+// the input has four times the pixels: 15 x 192 x 28^2 (560 k) 67 / 93, 8 x 384 x 28^2 (600 k) 71 / 98; 16 x 960 x 14^2 (750 k) 103 / 98, 16 x
+// 384 x 28^2 (1.2 M) 98 / 97, 8 x 288 x 56^2 (1.8 M) 124 / 98.
+int dk_offset_conv_direct_backward_worthwhile(const dk_offset_conv_desc* desc) {
+  const long work = offset_conv_direct_work(desc);
+  return work > 0 && work <= (desc->stride == 2 ? 620000 : 2000000);
 }
 
 // pass 0: forward (a, b = input, weight), 1: input gradient (out_grad, weight), 2: weight gradient (out_grad, input)

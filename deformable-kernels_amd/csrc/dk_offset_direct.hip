@@ -187,8 +187,8 @@ __global__ __launch_bounds__(256) void direct_conv_backward_input_kernel(DirectC
 }
 
 // Weight gradient.  A workgroup owns one input channel and ROWS tap rows; its waves take every WAVES-th group of 64 output
-// pixels, a lane keeps the ROWS x 3 x 18 products' sums of its pixels.  The sums are added over the lanes by halving
-// exchanges through LDS and over the waves in order: no atomics, the same result every time.
+// pixels, a lane keeps the ROWS x 3 x 18 products' sums of its pixels.  The sums are added over the lanes by DPP steps
+// (wave_sum) and over the waves, through LDS, in order: no atomics, the same result every time.
 template <typename T, int ROWS, int WAVES>
 __global__ __launch_bounds__(64 * WAVES) void direct_conv_backward_weight_kernel(DirectConv g, const T* __restrict__ gout,
                                                                                  const T* __restrict__ x, T* __restrict__ gweight) {
@@ -246,9 +246,9 @@ DirectConv geometry(int batch, int cin, int cout, int h, int w, int stride) {
 
 }  // namespace
 
-// 32-bit byte offsets into the tensors, below the out-of-range marker
+// 32-bit byte offsets into the tensors, below the out-of-range marker; the input gradient's grid has 16 channels per row at least
 bool offset_conv_direct_supported(int batch, int cin, int cout, int h, int w) {
-  return cout <= kDcOut && batch >= 1 && (long)batch * std::max(cin, cout) * h * w * 4 < (1L << 30);
+  return cout <= kDcOut && batch >= 1 && cin <= 16 * 65535 && (long)batch * std::max(cin, cout) * h * w * 4 < (1L << 30);
 }
 
 template <typename T>

@@ -509,6 +509,7 @@ Tensor offset_conv(const Tensor& input, const Tensor& weight, const OptTensor& b
   const bool native = offset_conv_covered(input, weight, stride, padding, dilation, force ? dk_offset_conv_supported : dk_offset_conv_worthwhile);
   // few images: one launch per pass on the vector unit
   const bool direct = !native && offset_conv_covered(input, weight, stride, padding, dilation, dk_offset_conv_direct_worthwhile);
+  const bool direct_grads = !native && offset_conv_covered(input, weight, stride, padding, dilation, dk_offset_conv_direct_backward_worthwhile);
   Tensor x, w;
   return record<OffsetConvFunctionBackward>(
       {&input, &weight, &bias},
@@ -530,7 +531,7 @@ Tensor offset_conv(const Tensor& input, const Tensor& weight, const OptTensor& b
       [&](OffsetConvFunctionBackward& n) {
         n.input = SavedVariable(x, false), n.weight = SavedVariable(w, false);
         n.stride = stride, n.padding = padding, n.dilation = dilation;
-        n.native = native, n.direct = direct, n.forced = force, n.has_bias = bias.defined();
+        n.native = native, n.direct = direct_grads, n.forced = force, n.has_bias = bias.defined();
       });
 }
 

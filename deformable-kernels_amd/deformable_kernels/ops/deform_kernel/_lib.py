@@ -100,6 +100,7 @@ SIGNATURES = {
     "dk_image_depthwise_backward_weight": (ctypes.c_int, [_CD, _P, _P, _P, _I64P, _P]),
     "dk_offset_conv_supported": (ctypes.c_int, [_OC]),
     "dk_offset_conv_direct_worthwhile": (ctypes.c_int, [_OC]),
+    "dk_offset_conv_direct_backward_worthwhile": (ctypes.c_int, [_OC]),
     "dk_offset_conv_direct_forward": (ctypes.c_int, [_OC, _P, _P, _P, _P, _P]),
     "dk_offset_conv_direct_backward_input": (ctypes.c_int, [_OC, _P, _P, _P, _P]),
     "dk_offset_conv_direct_backward_weight": (ctypes.c_int, [_OC, _P, _P, _P, _P]),

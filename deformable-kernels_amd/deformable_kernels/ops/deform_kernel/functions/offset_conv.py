@@ -13,11 +13,12 @@ at most 16, on planes 7, 14, 28, 56 or 112 wide (stride 2: input planes 14 to 11
     outputs; float32 tensors again as bfloat16 pairs), per-workgroup partial sums added in a fixed order,
   * the bias gradient on the library's reduction kernel for every shape (the framework's
     reduction over (N, H, W) takes 60-230 us on the large planes),
-  * of these shapes, those with too few images to fill the GPU that way (up to 2 M output pixels times input
-    channels): one fp32 vector-unit kernel per pass (``csrc/dk_offset_direct.hip``),
+  * of these shapes, most of those with too few images to fill the GPU that way (up to 2 M output pixels times input
+    channels, at stride 2 0.6 M for the gradients; the queries ``dk_offset_conv_direct_worthwhile`` and
+    ``dk_offset_conv_direct_backward_worthwhile`` tell): one fp32 vector-unit kernel per pass (``csrc/dk_offset_direct.hip``),
   * everything else -- other shapes, and passes the library reports as covered
     but not worthwhile (the float32 input gradient with fewer than 64 channels or
-    on 7 x 7 planes) unless ``force=True`` -- on the framework's convolution routines.
+    on 7 x 7 planes; few images of many channels) unless ``force=True`` -- on the framework's convolution routines.
 
 float64, CPU tensors, mixed dtypes and autocast regions go to ``F.conv2d`` unchanged.  The autograd node is native code
 (``csrc/dk_torch.cpp``).

@@ -308,3 +308,70 @@ def test_few_images_run_on_the_vector_unit_kernels(case):
     assert rel_err(out.detach().double().cpu(), want) < tol, "forward"
     assert rel_err(x.grad.double().cpu(), gx) < tol, "input gradient"
     assert rel_err(w.grad.double().cpu(), gw) < tol, "weight gradient"
+
+
+@pytest.mark.parametrize("forward, backward, case", [
+    # either side of each line of the two rules: N, C, H, W, outputs, stride, dtype
+    (1, 1, (1, 192, 28, 28, 18, 1, "float32")), (1, 1, (63, 608, 7, 7, 18, 1, "float32")),
+    (0, 1, (3, 768, 7, 7, 18, 1, "float32")), (1, 1, (3, 736, 7, 7, 18, 1, "float32")), (1, 1, (1, 640, 14, 14, 18, 1, "bfloat16")),
+    (0, 1, (1, 640, 14, 14, 18, 2, "bfloat16")), (1, 1, (1, 384, 14, 14, 18, 2, "float16")),
+    (0, 1, (1, 320, 56, 56, 18, 2, "float32")), (1, 1, (1, 304, 56, 56, 18, 2, "float32")),
+    (0, 1, (1, 960, 14, 14, 18, 1, "float16")), (1, 1, (2, 960, 14, 14, 18, 1, "float16")), (1, 1, (1, 960, 14, 14, 18, 1, "float32")),
+    (0, 1, (11, 80, 28, 28, 18, 1, "float16")), (1, 1, (11, 64, 28, 28, 18, 1, "float16")), (1, 1, (11, 128, 28, 28, 18, 1, "float32")),
+    (0, 1, (11, 144, 28, 28, 18, 1, "float32")), (1, 1, (11, 144, 28, 28, 18, 1, "bfloat16")),
+    (1, 0, (17, 192, 28, 28, 18, 2, "float32")), (1, 1, (16, 192, 28, 28, 18, 2, "float32")),
+])
+def test_calls_that_take_the_vector_unit_kernels(forward, backward, case):
+    """The rules, and the operator's own way through each combination of them against the float64 convolution.  The framework's
+    kernels: 16-bit results up to two of whose roundings meet (2^-10, 2^-7); bounds of the vector-unit kernels as above with up to
+    9 * 960 terms, and float32 sums of the framework of up to 1e-5."""
+    from deformable_kernels.ops.deform_kernel import _lib
+    from deformable_kernels.ops.deform_kernel.functions import offset_conv
+    N, C, H, W, O, stride, dtype_name = case
+    desc = _lib.OffsetConvDesc(N, C, O, H, W, {"float32": 0, "float16": 1, "bfloat16": 2}[dtype_name], stride)
+    assert _lib.lib().dk_offset_conv_direct_worthwhile(desc) == forward
+    assert _lib.lib().dk_offset_conv_direct_backward_worthwhile(desc) == backward
+    if N * C * H * W > 1000000:
+        return
+    dtype = getattr(torch, dtype_name)
+    tol = {"float32": 1e-5, "float16": 1e-3 + 1e-5, "bfloat16": 8e-3 + 1e-5}[dtype_name]
+    g = torch.Generator().manual_seed(73)
+    x, w, b = [t.to(dtype).cuda().requires_grad_() for t in (torch.randn(N, C, H, W, generator=g), torch.randn(O, C, 3, 3, generator=g) * 0.05,
+                                                             torch.randn(O, generator=g))]
+    out = offset_conv(x, w, b, stride)
+    gout = torch.randn(out.shape, generator=g).to(dtype).cuda()
+    want = reference(x, w, b, gout, stride=stride)
+    out.backward(gout)
+    for name, got, ref in zip(("forward", "input", "weight", "bias"), (out.detach(), x.grad, w.grad, b.grad), want):
+        assert rel_err(got.double().cpu(), ref) < tol, name
+
+
+@pytest.mark.parametrize("dtype_name", ["float32", "float16", "bfloat16"])
+@pytest.mark.parametrize("case", [
+    (1, 10, 1, 1, 5, 1),      # one pixel: eight of nine taps in the padding; fewer channels than waves
+    (2, 7, 9, 13, 18, 1),     # a width no layer has
+    (3, 33, 13, 5, 1, 2),     # one output, odd sides at stride 2
+    (1, 300, 2, 65, 17, 1),   # the weight gradient's form for 256 channels and more; a row wider than a wave
+    (70, 3, 11, 13, 4, 1),    # more than 128 tiles of pixels
+    (2, 20, 3, 4, 18, 2),
+])
+def test_vector_unit_entry_points_on_sizes_that_the_operator_leaves_to_the_framework(case, dtype_name):
+    """The three C calls take any size: float32 sums of at most 9 * 300 terms (2e-6 of the largest element), one rounding of a 16-bit
+    result (2^-11, 2^-8)."""
+    from deformable_kernels.ops.deform_kernel import _lib
+    N, C, H, W, O, stride = case
+    dtype = getattr(torch, dtype_name)
+    tol = {"float32": 2e-6, "float16": 5e-4 + 2e-6, "bfloat16": 4e-3 + 2e-6}[dtype_name]
+    g = torch.Generator().manual_seed(79)
+    x, w, b, gout = [t.to(dtype).cuda() for t in (torch.randn(N, C, H, W, generator=g), torch.randn(O, C, 3, 3, generator=g) * 0.05,
+                                                 torch.randn(O, generator=g), torch.randn(N, O, (H - 1) // stride + 1, (W - 1) // stride + 1, generator=g))]
+    out, gx, gw = torch.full_like(gout, float("nan")), torch.full_like(x, float("nan")), torch.full_like(w, float("nan"))
+    L, P = _lib.lib(), _lib.ptr
+    desc = _lib.OffsetConvDesc(N, C, O, H, W, {"float32": 0, "float16": 1, "bfloat16": 2}[dtype_name], stride)
+    st = _lib.stream_ptr(x)
+    _lib.check(L.dk_offset_conv_direct_forward(desc, P(x), P(w), P(b), P(out), st), "forward")
+    _lib.check(L.dk_offset_conv_direct_backward_input(desc, P(gout), P(w), P(gx), st), "input gradient")
+    _lib.check(L.dk_offset_conv_direct_backward_weight(desc, P(gout), P(x), P(gw), st), "weight gradient")
+    want = reference(x, w, b, gout, stride=stride)
+    for name, got, ref in zip(("forward", "input", "weight"), (out, gx, gw), want):
+        assert rel_err(got.double().cpu(), ref) < tol, name
