@@ -120,6 +120,11 @@ int main() {
   }
   nd.batch = 4;
   EXPECT(dk_nd_linear_sample_backward(&nd, one, one, one, nullptr, one, nullptr, nullptr, 0, nullptr) == DK_ERR_NULL_POINTER);
+  // an empty batch: only in_grad is written, and the others may be null (the answer is the missing workspace's)
+  dk_nd_desc empty = nd;
+  empty.batch = 0, empty.dtype = DK_F16;
+  EXPECT(dk_nd_linear_sample_backward(&empty, nullptr, nullptr, nullptr, nullptr, one, nullptr, nullptr, 0, nullptr) == DK_ERR_WORKSPACE);
+  EXPECT(dk_nd_linear_sample_backward(&empty, one, one, one, nullptr, nullptr, one, one, 1 << 30, nullptr) == DK_ERR_NULL_POINTER);
   EXPECT(dk_nd_linear_sample_forward(&nd, nullptr, one, nullptr, one, nullptr, 0, nullptr) == DK_ERR_NULL_POINTER);
 
   // offset branch

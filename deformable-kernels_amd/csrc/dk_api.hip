@@ -1174,7 +1174,8 @@ int dk_nd_linear_sample_backward(const dk_nd_desc* desc, const void* out_grad, c
                                  void* stream) {
   const int rc = check_nd(desc);
   if (rc != DK_OK) return rc;
-  if (!out_grad || !data || !coord || !in_grad || !coord_grad) return DK_ERR_NULL_POINTER;
+  // (an empty batch: the data's gradient is zeros, and there is nothing else to read or write)
+  if (!in_grad || (desc->batch > 0 && (!out_grad || !data || !coord || !coord_grad))) return DK_ERR_NULL_POINTER;
   const size_t need = nd_backward_workspace(*desc);
   if (need && (!workspace || workspace_bytes < need)) return DK_ERR_WORKSPACE;
   hipStream_t s = static_cast<hipStream_t>(stream);

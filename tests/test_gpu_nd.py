@@ -216,3 +216,19 @@ def test_sort_on_either_side_of_the_most_tiles_that_the_scatter_sums_itself(B):
     want = torch.zeros_like(rows).index_add_(0, low, gout.double() * (1 - frac)[:, None])
     want.index_add_(0, low + 1, gout.double() * frac[:, None])
     assert rel_err(grad.cpu(), want.t().cpu().numpy()) < 1e-5
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.float64])
+def test_both_gradients_of_no_points_through_the_c_call(dtype):
+    """As dk_nd_linear_sample_backward_data: zeros in in_grad, and nothing else is looked at."""
+    from deformable_kernels.ops.deform_kernel import _lib
+    L, P = _lib.lib(), _lib.ptr
+    gdata = torch.full((64, 6, 5, 4), float("nan"), device="cuda:0", dtype=dtype)
+    desc = _lib.NdDesc()
+    desc.batch, desc.channel, desc.dims = 0, 64, 3
+    desc.dtype = {torch.float32: 0, torch.float16: 1, torch.float64: 3}[dtype]
+    for d, n in enumerate((6, 5, 4)):
+        desc.shape[d] = n
+    ws, n = _lib.workspace(L.dk_nd_linear_sample_backward_workspace(desc), gdata.device)
+    _lib.check(L.dk_nd_linear_sample_backward(desc, None, None, None, None, P(gdata), None, P(ws), n, _lib.stream_ptr(gdata)), "backward")
+    assert bool((gdata == 0).all())
