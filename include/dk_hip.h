@@ -162,9 +162,12 @@ int dk_sample_depthwise_backward_rotation(const dk_conv_desc *desc, const void *
 
 /* The three gradients of one backward pass in one call; any of in_grad / rotation_grad /
  * filter_grad may be NULL to skip it.  Stands in for the three consecutive pybind calls of
- * SampleDepthwiseFunction.backward (functions/filter_sample_depthwise.py:63-85): one call that
- * issues the launches of the three entry points above on `stream`.  Workspace as for
- * *_backward_filter (only needed when filter_grad is requested). */
+ * SampleDepthwiseFunction.backward (functions/filter_sample_depthwise.py:63-85).  Small layers (at most 2048 output
+ * pixels; float64 not) have one launch of their own for the gradients asked for, without a workspace -- float32
+ * channels-last layers above stride 1 a second one for in_grad; every other call issues the launches of the three entry
+ * points above on `stream`.  The two ways round differently.  dk_sample_depthwise_backward_workspace() is this call's
+ * alone: the most that any choice of gradients takes, 0 where the one launch serves them.  A buffer that the entry
+ * points above share with this call is as large as the largest of their own queries too. */
 size_t dk_sample_depthwise_backward_workspace(const dk_conv_desc *desc);
 int dk_sample_depthwise_backward(const dk_conv_desc *desc, const void *out_grad, const void *input,
                                  const void *rotation, const void *filter, void *in_grad,
