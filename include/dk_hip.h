@@ -458,6 +458,8 @@ const char *dk_status_string(int status);
  * started with DK_ENABLE_TEST_SWITCHES=1 in its environment also reads the environment variables of
  * those names, once, at the first call that consults the mask (a stray variable in a production
  * environment changes nothing).  This call replaces the mask and returns the previous one.
+ * While any bit is set, small layers' gradients take the kernels of the larger layers (as with DK_NO_SMALL_BACKWARD):
+ * the other switches are about those.
  * Workspace queries consult it too: query and call must see the same mask.  The one piece of
  * process-wide state in the library. */
 unsigned dk_test_switches(unsigned mask);
