@@ -1824,14 +1824,22 @@ void nhwc_grad_filter(const Geo& g, const T* gout, const T* x, const T* rot, T* 
     if (fast_local_grad_filter_cl<T>(g, gout, x, rot, gfilter, ws, stream)) return;
     const int nct = (cells + 15) / 16;
     const bool small = (long)g.batch * g.channel * std::max((long)g.in_h * g.in_w, (long)g.out_h * g.out_w) * (long)sizeof(T) < (1L << 31);
-    if (g.groups == 1 && nct <= 2 && taps <= kMfRows && small && !path_disabled(kNoNhwcMfma)) {
+    // up to 64 cells: the kernel below keeps more than 25 sums of a thread's channel in LDS, an LDS read, add and write per
+    // cell and sample (N=39 C=14 16 x 15 scope 7 x 7 float32: 2687 us, 56 here)
+    if (g.groups == 1 && nct <= 4 && taps <= kMfRows && small && !path_disabled(kNoNhwcMfma)) {
       const int ntiles = ceil_div(g.channel, 16), wpb = std::min(ntiles, 16);
       const dim3 mgrid((unsigned)parts, (unsigned)ceil_div(ntiles, wpb));
       if (nct == 1)
         hipLaunchKernelGGL((nhwc_grad_filter_mfma_kernel<T, 1>), mgrid, dim3(64 * wpb), 0, stream, g, gout, x, rot, partial,
                            kFilterPixPerBlock);
-      else
+      else if (nct == 2)
         hipLaunchKernelGGL((nhwc_grad_filter_mfma_kernel<T, 2>), mgrid, dim3(64 * wpb), 0, stream, g, gout, x, rot, partial,
+                           kFilterPixPerBlock);
+      else if (nct == 3)
+        hipLaunchKernelGGL((nhwc_grad_filter_mfma_kernel<T, 3>), mgrid, dim3(64 * wpb), 0, stream, g, gout, x, rot, partial,
+                           kFilterPixPerBlock);
+      else
+        hipLaunchKernelGGL((nhwc_grad_filter_mfma_kernel<T, 4>), mgrid, dim3(64 * wpb), 0, stream, g, gout, x, rot, partial,
                            kFilterPixPerBlock);
       launch_reduce_partials<CT, T>(partial, parts, (long)g.channel * cells, gfilter, stream);
       return;

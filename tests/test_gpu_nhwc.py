@@ -335,3 +335,18 @@ def test_fp32_quads_at_stride_2(case, switch_off):
     switch_off("DK_FORCE_NHWC_GATHER_MFMA")
     inputs, got = _run(case, torch.float32, seed=3)
     assert rel_err(got[1], _oracle(inputs, np.float32)[1]) < 1e-5
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("case", [
+    (3, 14, 16, 15, 3, (7, 7), 1, 1, 1, 1, 1.5),    # 49 cells, channels not in fours: four tiles of 16 cells
+    (2, 33, 11, 13, 3, (7, 7), 2, 1, 1, 1, 1.5),    # stride 2, three tiles of channels
+    (1, 16, 9, 10, 3, (6, 7), 1, 1, 1, 1, 1.5),     # 42 cells: three tiles
+    (1, 5, 7, 7, 3, (8, 8), 1, 1, 1, 1, 1.5),       # 64 cells, the most
+    (1, 6, 7, 7, 3, (9, 8), 1, 1, 1, 1, 1.5),       # 72 cells: the kernel with its sums in LDS columns
+])
+def test_grad_filter_of_more_than_32_cells(case, dtype):
+    inputs, got = _run(case, dtype, seed=9)
+    want = _oracle(inputs, np.float64)
+    for g, w, tol in zip(got, want, (1e-5, 1e-5, 1e-4, 1e-4)):
+        assert rel_err(g.float(), w) < (tol if dtype == torch.float32 else 1e-2)
