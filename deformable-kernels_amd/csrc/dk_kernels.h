@@ -44,6 +44,7 @@ enum TestSwitch : unsigned {
   kForceDeformLanes = 1u << 26, // DK_FORCE_DEFORM_LANES ... wherever they apply, not only where they are the faster ones
   kNoDeformPlain = 1u << 27,    // DK_NO_DEFORM_PLAIN    the deformable kernels for calls without a rotation tensor (those that take one run instead)
   kNoSmallBackward = 1u << 28,  // DK_NO_SMALL_BACKWARD  the one-launch gradients of small layers (dk_local_small.hip; every other switch takes them away as well)
+  kNoNdRows = 1u << 29,         // DK_NO_ND_ROWS         the N-d kernels of narrow rows and the grad data with its sums in LDS
   kNoOffsetPairs = 1u << 18,    // DK_NO_OFFSET_PAIRS    the offset branch's convolution on float32 tensors as bfloat16 pairs (the fp32 matrix-instruction forward runs instead, the other passes are not offered)
 };
 unsigned test_switches();  // dk_api.hip

@@ -4,7 +4,7 @@
 //   nd_linear ND.cu:45-88, nd_linear_backward_data ND.cu:90-131,
 //   nd_linear_backward_coord ND.cu:133-177; kernels ND.cu:183-287.
 //
-// Two paths.
+// Two main paths.
 //  * Channel-last path (1..3 sampling dimensions, enough work to pay for a transpose):
 //    `data` [C, P] is first copied to [P, C] in the caller's workspace, so the C values of
 //    one corner are contiguous.  A wave takes 64 points: with lane <-> point it derives each
@@ -570,6 +570,160 @@ __global__ __launch_bounds__(kBlock) void nd_small_grad_coord_kernel(NdGeo g, co
   if (lane == 0) {
 #pragma unroll
     for (int d = 0; d < NDIM; ++d) st(gcoord + b * NDIM + d, gd[d]);
+  }
+}
+
+// ---------------------------------------------------------------------------
+// channel-last path of narrow rows: a wave holds 64 >> lg points, 1 << lg lanes of each along the channels (the least power
+// of two that holds them, at most 64), and every lane derives its point's corners itself.
+// ---------------------------------------------------------------------------
+template <int ND>
+struct RowCorners {
+  static constexpr int N = 1 << ND;
+  int off[N];  // cells; 0 for an absent corner
+  float w[N];  // 0 for an absent corner
+  unsigned present;
+};
+
+template <typename T, int ND>
+__device__ __forceinline__ RowCorners<ND> row_corners(const NdGeo& g, const T* coord_b, bool valid, NdPoint<float>& p) {
+  p = small_point<T, ND>(g, coord_b);
+  RowCorners<ND> r;
+  r.present = 0u;
+#pragma unroll
+  for (int i = 0; i < RowCorners<ND>::N; ++i) {
+    long o = 0;
+    float w = 0.f;
+    const bool ok = valid && p.inside && corner<float>(g, p, (unsigned)i, -1, o, w);
+    r.off[i] = ok ? (int)o : 0;
+    r.w[i] = ok ? w : 0.f;
+    r.present |= ok ? 1u << i : 0u;
+  }
+  return r;
+}
+
+// Sum over aligned groups of 1 << lg lanes, for every lane
+__device__ __forceinline__ float group_sum(float v, int lg) {
+  auto add = [&](auto ctrl) {
+    v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), decltype(ctrl)::value, 0xf, 0xf, true));
+  };
+  if (lg > 0) add(std::integral_constant<int, 0xb1>{});   // quad_perm: the neighbour
+  if (lg > 1) add(std::integral_constant<int, 0x4e>{});   // quad_perm: the other pair
+  if (lg > 2) add(std::integral_constant<int, 0x141>{});  // row_half_mirror: the other four
+  if (lg > 3) add(std::integral_constant<int, 0x140>{});  // row_mirror: the other eight
+  if (lg > 4) v += __shfl_xor(v, 16, 64);
+  if (lg > 5) v += __shfl_xor(v, 32, 64);
+  return v;
+}
+
+template <typename T, int ND>
+__global__ __launch_bounds__(kBlock) void nd_forward_rows_kernel(NdGeo g, const T* __restrict__ data_cl,
+                                                                 const T* __restrict__ coord, T* __restrict__ out, int lg) {
+  g.dims = ND;
+  const long b = (long)blockIdx.x * (kBlock >> lg) + (threadIdx.x >> lg);
+  if (b >= g.batch) return;
+  NdPoint<float> p;
+  const RowCorners<ND> r = row_corners<T, ND>(g, coord + b * ND, true, p);
+  for (int c = threadIdx.x & ((1 << lg) - 1); c < g.channel; c += 1 << lg) {
+    T raw[RowCorners<ND>::N];
+#pragma unroll
+    for (int i = 0; i < RowCorners<ND>::N; ++i) raw[i] = data_cl[(size_t)r.off[i] * g.channel + c];
+    float acc = 0.f;
+#pragma unroll
+    for (int i = 0; i < RowCorners<ND>::N; ++i) acc += r.w[i] * (r.present >> i & 1u ? (float)ld(&raw[i]) : 0.f);
+    st(out + b * g.channel + c, acc);
+  }
+}
+
+template <typename T, int ND>
+__global__ __launch_bounds__(kBlock) void nd_grad_coord_rows_kernel(NdGeo g, const T* __restrict__ gout,
+                                                                    const T* __restrict__ data_cl,
+                                                                    const T* __restrict__ coord, T* __restrict__ gcoord, int lg) {
+  constexpr int N = RowCorners<ND>::N;
+  g.dims = ND;
+  const long at = (long)blockIdx.x * (kBlock >> lg) + (threadIdx.x >> lg);
+  const long b = min(at, g.batch - 1);  // (no lane leaves before the sum over its group)
+  NdPoint<float> p;
+  const RowCorners<ND> r = row_corners<T, ND>(g, coord + b * ND, true, p);
+  float s[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) s[i] = 0.f;
+  const int lane = threadIdx.x & ((1 << lg) - 1);
+  for (int c = lane; c < g.channel; c += 1 << lg) {
+    T raw[N];
+    const T graw = gout[b * g.channel + c];
+#pragma unroll
+    for (int i = 0; i < N; ++i) raw[i] = data_cl[(size_t)r.off[i] * g.channel + c];
+    const float go = ld(&graw);
+#pragma unroll
+    for (int i = 0; i < N; ++i) s[i] += r.present >> i & 1u ? go * ld(&raw[i]) : 0.f;
+  }
+  float gd[ND];
+#pragma unroll
+  for (int d = 0; d < ND; ++d) {
+    gd[d] = 0.f;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      long o;
+      float w;
+      if ((r.present >> i & 1u) && corner<float>(g, p, (unsigned)i, d, o, w)) gd[d] += s[i] * w;  // ND.cu:161,165
+    }
+    gd[d] = group_sum(gd[d], lg);
+  }
+  if (lane == 0 && at < g.batch)
+#pragma unroll
+    for (int d = 0; d < ND; ++d) st(gcoord + b * ND + d, gd[d]);
+}
+
+// grad data with the sums in LDS: a workgroup takes a share of the points, a slice of the channels and, of volumes that do
+// not fit for one channel, a range of the cells, and holds the sums [cell][pitch] of that; they leave planar, one copy per
+// share, and are added up in order.  Where points meet in cells, float atomics on memory take the additions one by one.  The
+// sums are doubles: an LDS add of a wave takes 5 - 9 ns of the CU in double, 81 in float (the same addresses, 16 waves).
+template <typename T, int ND>
+__global__ __launch_bounds__(1024) void nd_grad_data_lds_kernel(NdGeo g, const T* __restrict__ gout, const T* __restrict__ coord,
+                                                                float* __restrict__ partial, int lg, int slice_ch, int pitch,
+                                                                int slices, int range, int ranges, long share) {
+  constexpr int N = RowCorners<ND>::N, PU = 4;  // points of a lane in flight
+  extern __shared__ __align__(16) unsigned char nd_lds_sums[];
+  double* img = reinterpret_cast<double*>(nd_lds_sums);
+  g.dims = ND;
+  const int cells = (int)g.prod_shape;
+  const int slice = blockIdx.x % slices, from = blockIdx.x / slices % ranges * range, part = blockIdx.x / slices / ranges;
+  const int own = min(range, cells - from);
+  const int c0 = slice * slice_ch, nc = min(slice_ch, g.channel - c0);
+  for (int e = threadIdx.x; e < own * pitch; e += 1024) img[e] = 0.0;
+  __syncthreads();
+  const int lane = threadIdx.x & ((1 << lg) - 1), points = 1024 >> lg;
+  const long b1 = min(g.batch, (part + 1) * share);
+  for (long b0 = part * share + (threadIdx.x >> lg); b0 < b1; b0 += PU * points) {
+    T x[PU][ND], graw[PU];
+#pragma unroll
+    for (int u = 0; u < PU; ++u) {
+      const long b = min(b0 + u * points, b1 - 1);
+#pragma unroll
+      for (int d = 0; d < ND; ++d) x[u][d] = coord[b * ND + d];
+      graw[u] = gout[b * g.channel + c0 + min(lane, nc - 1)];
+    }
+#pragma unroll
+    for (int u = 0; u < PU; ++u) {
+      const long b = b0 + u * points;
+      if (b >= b1) break;
+      NdPoint<float> p;
+      const RowCorners<ND> r = row_corners<T, ND>(g, x[u], true, p);
+      for (int c = lane; c < nc; c += 1 << lg) {
+        const float go = c == lane ? ld(&graw[u]) : ld(gout + b * g.channel + c0 + c);
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+          const int at = r.off[i] - from;
+          if ((r.present >> i & 1u) && (unsigned)at < (unsigned)own) atomicAdd(img + at * pitch + c, (double)(r.w[i] * go));
+        }
+      }
+    }
+  }
+  __syncthreads();
+  for (int c = 0; c < nc; ++c) {
+    float* out = partial + ((size_t)part * g.channel + c0 + c) * cells + from;
+    for (int e = threadIdx.x; e < own; e += 1024) out[e] = (float)img[e * pitch + c];
   }
 }
 
@@ -1591,28 +1745,97 @@ void transpose(const A* in, B* out, long rows, long cols, hipStream_t stream, fl
 
 }  // namespace
 
-// The channel-last path pays for a transpose of `data`; it is taken for 1..3 dimensions in
-// fp32 / fp16 / bf16 when there are enough (point, channel) pairs to amortise it.
 // Few points on a tiny volume: the direct kernels and the one-launch grad data (nd_small_grad_data_kernel).
 bool nd_small(const dk_nd_desc& d) {
   if (d.dtype == DK_F64 || d.dims > kClMaxDims || path_disabled(kNoNdSmall)) return false;
   long prod = 1;
   for (int i = 0; i < d.dims; ++i) prod *= d.shape[i];
-  return prod <= kSmallMaxCells && d.batch > 0 && d.batch * d.channel <= (1L << 20);
+  // (a workgroup of the grad data walks over all points: 8000 points x 16 channels of 7 x 7 float32 88 us a pass, 40 with the
+  // sums of nd_grad_data_lds_kernel; 17000 x 4 of 50 160 / 39)
+  return prod <= kSmallMaxCells && d.batch > 0 && d.batch * d.channel <= (1L << 20) && (d.batch <= 4096 || path_disabled(kNoNdRows));
 }
 
+// The channel-last path pays for a transpose of `data`; it is taken for 1..3 dimensions in
+// fp32 / fp16 / bf16 when there are enough (point, channel) pairs to amortise it (5500 points x 12 channels of 30 x 20: 55 us a
+// pass on the planar volume, 42 here).
 bool nd_use_channel_last(const dk_nd_desc& d) {
   if (d.dtype == DK_F64 || d.dims > kClMaxDims || nd_small(d)) return false;
   long prod = 1;
   for (int i = 0; i < d.dims; ++i) prod *= d.shape[i];
   if (prod > 2147483647L / 4) return false;  // corner offsets are kept as 32-bit element counts
-  return d.batch * d.channel >= 65536 && d.channel >= 16;
+  return d.batch * d.channel >= 65536 && (d.channel >= 16 || !path_disabled(kNoNdRows));
 }
+
+namespace {
+
+// log2 of a point's lanes in the kernels of narrow rows, or -1 where a wave per point serves the call.  Up to 32 channels, us
+// a wave per point / narrow rows, forward and grad coord: 19023 points x 22 channels of 29 x 6 x 25 bfloat16 15.5 / 6.2 and
+// 12.0 / 8.8; but 60000 x 40 of 40 x 30 float32 13.9 / 13.0 and 12.6 / 21.4.  Below 16 channels, against a lane per (point,
+// channel) on the planar volume: 568761 x 14 of 70 x 78 float16 102 / 27 and 164 / 46, and 4.5 for the transposes.
+int row_lanes(const NdGeo& g) {
+  if (path_disabled(kNoNdRows) || g.channel > 32) return -1;
+  int lg = 0;
+  while (1 << lg < g.channel && lg < 6) ++lg;
+  return lg;
+}
+
+struct LdsSums {
+  int slices, channels, pitch, lg;  // slices == 0: not this way
+  int range, ranges;                // cells of a workgroup
+  long share;                       // points of a workgroup
+  int parts;
+  size_t lds;
+};
+
+LdsSums lds_sums(const dk_nd_desc& d) {
+  LdsSums m{};
+  if (!nd_use_channel_last(d) || path_disabled(kNoNdRows)) return m;
+  long cells = 1;
+  for (int i = 0; i < d.dims; ++i) cells *= d.shape[i];
+  const long adds = d.batch << d.dims;  // of a channel
+  // How many additions a sum must receive, and how often the points may be walked over.  Float atomics on memory take a row of 16
+  // channels and more at once, fewer mostly one by one.  us a pass with the atomics / the sums in LDS: 60000 points x 40
+  // channels of 40 x 30 float32 (200 additions, 8 slices) 76 / 58; 19023 x 22 of 29 x 6 x 25 (35) 51 / 66; 10^5 x 10 of 30^3 (30,
+  // 20 slices of cells and channels) 108 / 67; 2^20 x 3 of 40^3 (131, 12) 564 / 168; 568761 x 14 of 70 x 78 float16 (416, 5)
+  // 1842 / 129; 128941 x 11 of 6 x 12 bfloat16 (7164, 1) 1540 / 42.
+  const bool narrow = d.channel < 16;
+  if (adds < (narrow ? 4 : 64) * cells) return m;
+  auto pitch_of = [](long c) { return c | 1; };
+  const long all = kMaxDynamicLds / 8, half = 78 * 1024 / 8;  // sums of a workgroup that has its CU alone, and of one that shares it
+  long c = d.channel;
+  m.range = (int)cells;
+  if (cells * pitch_of(c) > half) {
+    c = std::min<long>(all / cells, d.channel);
+    if (c % 2 == 0) --c;
+    if (c < 1) {
+      c = 1;
+      m.range = (int)((cells + (cells + all - 1) / all - 1) / ((cells + all - 1) / all));
+    }
+  }
+  m.ranges = (int)((cells + m.range - 1) / m.range);
+  m.slices = (int)((d.channel + c - 1) / c);
+  if (m.slices * m.ranges > (narrow ? 32 : 16)) return LdsSums{};
+  m.channels = (d.channel + m.slices - 1) / m.slices;
+  m.pitch = (int)pitch_of(m.channels);
+  m.lds = (size_t)m.range * m.pitch * 8;
+  while (1 << m.lg < m.channels && m.lg < 6) ++m.lg;
+  const long room = (m.lds <= 78 * 1024 ? 512 : 256) / (m.slices * m.ranges);
+  const long parts = std::max(1L, std::min({room, adds / (2 * cells), (d.batch + 255) / 256}));
+  m.share = (d.batch + parts - 1) / parts;
+  m.parts = (int)((d.batch + m.share - 1) / m.share);
+  return m;
+}
+
+}  // namespace
 
 // Bins of the counting sort (cells of low corners plus the bin of outside points), or 0 when
 // the binned kernels do not apply: they pay off with several points per cell.
 int nd_bins(const dk_nd_desc& d) {
-  if (!nd_use_channel_last(d) || path_disabled(kNoNdBins)) return 0;
+  if (!nd_use_channel_last(d) || d.channel < 16 || path_disabled(kNoNdBins)) return 0;
+  // What the sort gives the kernels that do not run on the matrix cores is less than it costs where two slices of LDS hold
+  // the volume's sums: us a pass sorted / not: 400000 points x 16 channels of 8^3 float16 194 / 144, 262000 x 250 of 90 cells
+  // bfloat16 311 / 217, 200000 x 128 of 16 x 16 195 / 182; but 300000 x 100 of 30 x 20 float32 (four slices) 192 / 253.
+  if (const LdsSums m = lds_sums(d); m.slices && m.slices * m.ranges <= 2 && !(d.dtype == DK_F32 && d.channel % 64 == 0)) return 0;
   long bins = 1;
   for (int i = 0; i < d.dims; ++i) bins *= (long)d.shape[i] + 1;
   bins += 1;
@@ -1717,6 +1940,11 @@ void nd_forward(const dk_nd_desc& d, const T* data, const T* coord, T* out, void
         DK_ND_BY_DIMS(g.dims, nd_forward_binned_kernel<T, ND><<<(unsigned)xcd_grid_size((g.batch + 255) / 256), kBlock, 0, stream>>>(g, data_cl, coord, order, bins, out));
         return;
       }
+      if (const int lg = row_lanes(g); lg >= 0) {
+        const unsigned grid = (unsigned)((g.batch + (kBlock >> lg) - 1) / (kBlock >> lg));
+        DK_ND_BY_DIMS(g.dims, nd_forward_rows_kernel<T, ND><<<grid, kBlock, 0, stream>>>(g, data_cl, coord, out, lg));
+        return;
+      }
       const int ppw = points_per_wave(g);
       const long waves = (g.batch + ppw - 1) / ppw;
       DK_ND_BY_DIMS(g.dims, nd_forward_cl_kernel<T, ND><<<(unsigned)((waves + 3) / 4), kBlock, 0, stream>>>(g, data_cl, coord, out, ppw));
@@ -1731,7 +1959,11 @@ size_t nd_grad_data_workspace(const dk_nd_desc& d) {
   if (nd_small(d)) return 0;
   size_t n = (size_t)d.channel;
   for (int i = 0; i < d.dims; ++i) n *= (size_t)d.shape[i];
-  if (nd_use_channel_last(d)) return round256(n * sizeof(float)) + nd_sort_workspace(d);  // fp32 channel-last accumulation image
+  if (nd_use_channel_last(d)) {
+    const LdsSums m = lds_sums(d);
+    // fp32 channel-last accumulation image; or copies of the sums, without a sort
+    return std::max(round256(n * sizeof(float)) + nd_sort_workspace(d), (size_t)m.parts * n * sizeof(float));
+  }
   if (d.dtype == DK_F16 || d.dtype == DK_BF16) return n * sizeof(float);
   return 0;
 }
@@ -1766,6 +1998,19 @@ void nd_grad_data(const dk_nd_desc& d, const T* gout, const T* coord, T* gdata, 
 #undef DK_ND_SMALL_GD_NT
 #undef DK_ND_SMALL_GD
       return;
+    }
+    if (const LdsSums m = lds_sums(d); m.slices && !nd_bins(d)) {
+      float* partial = static_cast<float*>(ws);
+      bool ok = true;
+      DK_ND_BY_DIMS(g.dims, {
+        auto kernel = nd_grad_data_lds_kernel<T, ND>;
+        ok = m.lds <= 64 * 1024 || allow_dynamic_lds(reinterpret_cast<const void*>(kernel), kMaxDynamicLds);
+        if (ok) kernel<<<(unsigned)(m.slices * m.ranges * m.parts), 1024, m.lds, stream>>>(g, gout, coord, partial, m.lg, m.channels, m.pitch, m.slices, m.range, m.ranges, m.share);
+      });
+      if (ok) {
+        launch_reduce_partials<float, T>(partial, m.parts, n_data, gdata, stream);
+        return;
+      }
     }
     if (nd_use_channel_last(d)) {
       float* acc = static_cast<float*>(ws);
@@ -1826,6 +2071,11 @@ void nd_grad_coord(const dk_nd_desc& d, const T* gout, const T* data, const T* c
           }
         }
         DK_ND_BY_DIMS(g.dims, nd_grad_coord_binned_kernel<T, ND><<<(unsigned)xcd_grid_size((g.batch + 255) / 256), kBlock, 0, stream>>>(g, gout, data_cl, coord, order, bins, gcoord));
+        return;
+      }
+      if (const int lg = row_lanes(g); lg >= 0) {
+        const unsigned grid = (unsigned)((g.batch + (kBlock >> lg) - 1) / (kBlock >> lg));
+        DK_ND_BY_DIMS(g.dims, nd_grad_coord_rows_kernel<T, ND><<<grid, kBlock, 0, stream>>>(g, gout, data_cl, coord, gcoord, lg));
         return;
       }
       const int ppw = points_per_wave(g);

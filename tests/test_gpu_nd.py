@@ -232,3 +232,45 @@ def test_both_gradients_of_no_points_through_the_c_call(dtype):
     ws, n = _lib.workspace(L.dk_nd_linear_sample_backward_workspace(desc), gdata.device)
     _lib.check(L.dk_nd_linear_sample_backward(desc, None, None, None, None, P(gdata), None, P(ws), n, _lib.stream_ptr(gdata)), "backward")
     assert bool((gdata == 0).all())
+
+
+@pytest.mark.parametrize("shape,C,B,lo,hi", [
+    ((20, 31), 14, 9001, -1.5, 32.0),        # narrow rows, a lane group partly idle; the sums in LDS
+    ((90,), 1, 70000, -1.0, 90.0),           # one channel, a lane per point
+    ((13, 9, 8), 3, 30011, -1.5, 13.5),
+    ((6, 12), 11, 20000, 2.0, 2.9),          # every point in one cell
+    ((70, 78), 15, 30000, -1.0, 78.0),       # five slices of channels
+    ((40, 40, 40), 2, 70000, -1.0, 40.0),    # one channel in four ranges of cells, two slices
+    ((28, 28, 24), 4, 70000, -1.0, 28.0),    # 18816 cells: one channel per workgroup, one range
+    ((80, 80, 80), 5, 20000, -1.0, 80.0),    # fewer additions than the sums in LDS want: float atomics
+    ((40, 30), 17, 30000, -1.5, 41.0),       # 32 lanes per point
+    ((40, 30), 32, 20000, -1.5, 41.0),
+    ((40, 30), 33, 20000, -1.5, 41.0),       # a wave per point forward, the sums in LDS
+    ((8, 8, 8), 20, 66000, -1.5, 9.0),       # two slices: not sorted
+    ((7, 7), 16, 4097, -1.5, 8.0),           # a tiny volume, one point more than the few-points kernels take
+])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_narrow_rows_and_sums_in_lds(shape, C, B, lo, hi, dtype, switch_off):
+    """Against float64, and against the kernels that take the calls without these."""
+    g = torch.Generator().manual_seed(50)
+    data = torch.randn(C, *shape, generator=g).to(dtype)
+    coord = (torch.rand(B, len(shape), generator=g) * (hi - lo) + lo).to(dtype)
+    gout = torch.randn(B, C, generator=g).to(dtype)
+    got = _run(data, coord, gout)
+    switch_off("DK_NO_ND_ROWS")
+    general = _run(data, coord, gout)
+    want = _oracle(data, coord, gout, np.float64)
+    tol = (1e-5, 1e-5, 1e-5) if dtype == torch.float32 else (1e-3, 1e-3, 1e-3)  # 16-bit: the results' rounding, 2^-11
+    for a, b, w, t in zip(got, general, want, tol):
+        assert rel_err(a.float(), w) < t and rel_err(a.float(), b.double().numpy()) < t
+
+
+def test_non_finite_output_gradient_stays_with_its_point_and_channel():
+    """Sums in LDS: what is not finite reaches the corners of its point in its channel, and nothing else; a point outside the grid
+    adds nothing."""
+    data, coord, gout = _inputs((20, 31), 6, 20000, seed=51, dtype=torch.float32)
+    coord[0], coord[1] = torch.tensor([3.25, 4.5]), torch.tensor([-1.0, 4.0])
+    gout[0, 2], gout[1, 3] = float("inf"), float("nan")
+    got = _run(data, coord, gout)[1]
+    bad = ~torch.isfinite(got)
+    assert bad[2, 3:5, 4:6].all() and int(bad.sum()) == 4
