@@ -47,6 +47,8 @@ int main() {
   EXPECT(dk_deformable_sample_depthwise_backward_rotation(&ok, one, one, one, one, one, nullptr, one, 1 << 20, nullptr) == DK_ERR_NULL_POINTER);
   EXPECT(dk_deformable_sample_depthwise_backward_offset_rotation(&ok, one, one, one, nullptr, one, one, one, one, 1 << 20, nullptr) == DK_ERR_NULL_POINTER);
   EXPECT(dk_deformable_sample_depthwise_backward_offset_rotation(&ok, one, one, one, one, one, one, nullptr, one, 1 << 20, nullptr) == DK_ERR_NULL_POINTER);
+  EXPECT(dk_deformable_sample_depthwise_backward_parameters(&ok, one, one, one, nullptr, one, one, one, one, one, 1 << 20, nullptr) == DK_ERR_NULL_POINTER);
+  EXPECT(dk_deformable_sample_depthwise_backward_parameters(&ok, one, one, one, one, one, one, one, one, one, 1, nullptr) == DK_ERR_WORKSPACE);
   EXPECT(dk_deformable_sample_depthwise_backward_offset_filter(&ok, one, one, one, nullptr, one, one, nullptr, one, 1 << 20, nullptr) == DK_ERR_NULL_POINTER);
   EXPECT(dk_deformable_sample_depthwise_backward_offset_filter(&ok, one, one, one, nullptr, one, one, one, one, 1, nullptr) == DK_ERR_WORKSPACE);
 
@@ -98,7 +100,8 @@ int main() {
                        dk_deformable_sample_depthwise_backward_filter_workspace(&d) +
                        dk_deformable_sample_depthwise_backward_offset_workspace(&d) +
                        dk_deformable_sample_depthwise_backward_rotation_workspace(&d) +
-                       dk_deformable_sample_depthwise_backward_offset_rotation_workspace(&d);
+                       dk_deformable_sample_depthwise_backward_offset_rotation_workspace(&d) +
+                       dk_deformable_sample_depthwise_backward_parameters_workspace(&d);
             }
   EXPECT(total > 0);
 

@@ -611,7 +611,7 @@ int dk_deformable_sample_depthwise_backward_offset_rotation(const dk_conv_desc* 
 size_t dk_deformable_sample_depthwise_backward_offset_filter_workspace(const dk_conv_desc* desc) {
   Geo g;
   if (make_geo(desc, g) != DK_OK) return 0;
-  return std::max(plain_deform_grad_offset_filter_workspace(g),
+  return std::max(std::max(plain_deform_grad_offset_filter_workspace(g), tile_deform_grads_workspace(g, false)),
                   std::max(dk_deformable_sample_depthwise_backward_offset_workspace(desc),
                            dk_deformable_sample_depthwise_backward_filter_workspace(desc)));
 }
@@ -633,13 +633,51 @@ int dk_deformable_sample_depthwise_backward_offset_filter(const dk_conv_desc* de
     const int st = by_dtype(desc->dtype, [&]<typename T>() {
       if constexpr (kHasFast<T>)
         fused = plain_deform_grad_offset_filter<T>(g, in<T>(out_grad), in<T>(input), in<T>(offset), in<T>(filter),
-                                                   out<T>(offset_grad), out<T>(filter_grad), static_cast<float*>(workspace), s);
+                                                   out<T>(offset_grad), out<T>(filter_grad), static_cast<float*>(workspace), s) ||
+                tile_deform_grads<T>(g, in<T>(out_grad), in<T>(input), in<T>(offset), nullptr, in<T>(filter), out<T>(offset_grad),
+                                     nullptr, out<T>(filter_grad), static_cast<float*>(workspace), s);
     });
     if (st != DK_OK || fused) return st;
   }
   // one after the other, sharing the workspace (stream order)
   const int so = dk_deformable_sample_depthwise_backward_offset(desc, out_grad, input, offset, rotation, filter, offset_grad,
                                                                 workspace, workspace_bytes, stream);
+  if (so != DK_OK) return so;
+  return dk_deformable_sample_depthwise_backward_filter(desc, out_grad, input, offset, rotation, filter_grad, workspace,
+                                                        workspace_bytes, stream);
+}
+
+size_t dk_deformable_sample_depthwise_backward_parameters_workspace(const dk_conv_desc* desc) {
+  Geo g;
+  if (make_geo(desc, g) != DK_OK) return 0;
+  return std::max(tile_deform_grads_workspace(g, true), std::max(dk_deformable_sample_depthwise_backward_offset_rotation_workspace(desc),
+                                                           dk_deformable_sample_depthwise_backward_filter_workspace(desc)));
+}
+
+int dk_deformable_sample_depthwise_backward_parameters(const dk_conv_desc* desc, const void* out_grad, const void* input,
+                                                       const void* offset, const void* rotation, const void* filter,
+                                                       void* offset_grad, void* rotation_grad, void* filter_grad,
+                                                       void* workspace, size_t workspace_bytes, void* stream) {
+  Geo g;
+  const int rc = make_geo(desc, g);
+  if (rc != DK_OK) return rc;
+  if (desc->layout != DK_LAYOUT_NCHW) return DK_ERR_UNSUPPORTED;
+  if (!out_grad || !input || !offset || !rotation || !filter || !offset_grad || !rotation_grad || !filter_grad) return DK_ERR_NULL_POINTER;
+  const size_t need = dk_deformable_sample_depthwise_backward_parameters_workspace(desc);
+  if (need && (!workspace || workspace_bytes < need)) return DK_ERR_WORKSPACE;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  bool fused = false;
+  if (g.batch > 0) {
+    const int st = by_dtype(desc->dtype, [&]<typename T>() {
+      if constexpr (kHasFast<T>)
+        fused = tile_deform_grads<T>(g, in<T>(out_grad), in<T>(input), in<T>(offset), in<T>(rotation), in<T>(filter), out<T>(offset_grad),
+                                     out<T>(rotation_grad), out<T>(filter_grad), static_cast<float*>(workspace), s);
+    });
+    if (st != DK_OK || fused) return st;
+  }
+  // one after the other, sharing the workspace (stream order)
+  const int so = dk_deformable_sample_depthwise_backward_offset_rotation(desc, out_grad, input, offset, rotation, filter, offset_grad,
+                                                                         rotation_grad, workspace, workspace_bytes, stream);
   if (so != DK_OK) return so;
   return dk_deformable_sample_depthwise_backward_filter(desc, out_grad, input, offset, rotation, filter_grad, workspace,
                                                         workspace_bytes, stream);

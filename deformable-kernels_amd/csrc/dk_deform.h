@@ -64,6 +64,31 @@ struct BandWalk {
 };
 __device__ __forceinline__ bool bands_take(const BandWalk& walk) { return *walk.met <= walk.most; }
 
+// All gradients but the input's from one pass over the samples (dk_deform_tile.hip): a tile of 64 output pixels is walked once
+// for every window of the input that its samples read, with wide offsets four times and more.  As above the offsets
+// decide, on the device: deform_tile_boxes_kernel leaves the windows of all tiles in `words` words, and beyond `most` in all the
+// kernels of the separate gradients, launched behind, take the call.  (Those read one word, 1 where the call is theirs.)
+struct TileChoice {
+  const unsigned* windows;  // null: no choice
+  int words;
+  unsigned most;
+};
+__device__ __forceinline__ bool tiles_take(const TileChoice& c) {
+  unsigned sum = 0u;
+  for (int i = threadIdx.x & 63; i < c.words; i += 64) sum += c.windows[i];
+  for (int s = 32; s > 0; s >>= 1) sum += (unsigned)__shfl_xor((int)sum, s);
+  return (unsigned)__builtin_amdgcn_readfirstlane((int)sum) <= c.most;
+}
+
+// A reduction left to the caller: `parts` partial sums of `count` elements each, to be added up in order into `out`
+template <typename T>
+struct ReduceJob {
+  const float* partial;
+  int parts;
+  long count;
+  T* out;
+};
+
 // floor(v + 0.5) as a signed 32-bit integer, one instruction
 __device__ __forceinline__ int round_half_up(float v) {
   int r;

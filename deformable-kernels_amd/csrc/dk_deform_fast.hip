@@ -409,6 +409,25 @@ __global__ __launch_bounds__(BLOCK, BLOCK == kDBlock ? 2 : 1) void deform_forwar
 }
 
 
+// Value and slopes of a sample from its corners; the slopes are differences of corners, the value a corner and the slopes.
+struct Sample {
+  float val, h, w;
+};
+__device__ __forceinline__ Sample sample_slopes(float a, float b, float c, float d, float lh, float lw) {
+  const float ba = b - a, down = c - a, cross = (d - c) - ba;
+  Sample s;
+  s.h = fmaf(lw, cross, down), s.w = fmaf(lh, cross, ba);
+  s.val = fmaf(lh, s.h, fmaf(lw, ba, a));
+  return s;
+}
+// ... of the scope read, from the entry of the difference-form table (val = lite_weight)
+__device__ __forceinline__ Sample scope_slopes(const LiteTap& t, const float4& q) {
+  Sample s;
+  s.h = fmaf(t.lw, q.w, q.z), s.w = fmaf(t.lh, q.w, q.y);
+  s.val = fmaf(t.lh, s.h, fmaf(t.lw, q.y, q.x));
+  return s;
+}
+
 // ---------------------------------------------------------------------------
 // grad offset / grad rotation: the lane owns output pixel p and sums over the channels of its
 // chunk; one fp32 partial per chunk goes to the workspace and reduce_partials_kernel adds the
@@ -534,7 +553,8 @@ template <typename T, int SH, int SW, int NPASS, int MODE, int CH, int BLOCK = k
 __global__ __launch_bounds__(BLOCK, BLOCK == kDBlock ? 2 : 1) void deform_grad_coord_ch_kernel(
     Geo g, const T* __restrict__ gout, const T* __restrict__ x, const T* __restrict__ off,
     const T* __restrict__ rot, const T* __restrict__ filter, float* __restrict__ partial,
-    int ch_per_block, int shift, int tile_pix, float* __restrict__ partial_off) {
+    int ch_per_block, int shift, int tile_pix, float* __restrict__ partial_off, TileChoice choice) {
+  if (choice.windows && tiles_take(choice)) return;
   constexpr bool ROTATION = MODE != 0, OFFSET = MODE != 1;
   using Tb = WideTable<SH, SW>;
   extern __shared__ __align__(16) float lds[];
@@ -571,10 +591,10 @@ __global__ __launch_bounds__(BLOCK, BLOCK == kDBlock ? 2 : 1) void deform_grad_c
   const size_t x_step = (size_t)g.groups * in_plane, g_step = (size_t)g.groups * out_plane;
   const unsigned goff = live ? (unsigned)p * (unsigned)sizeof(T) : kOutOfRange;
 
-  float s0[K9], s1[K9], s2[K9];                    // rotation: sums of sample * gout * {b, c, d}
+  float s0[K9], s1[K9];                            // rotation: sums of sample * gout * d B / d{h, w}
   float o0[OFFSET ? K9 : 1], o1[OFFSET ? K9 : 1];  // offset: sums of d sample / d{h, w} * gout * B
 #pragma unroll
-  for (int t = 0; t < K9; ++t) s0[t] = s1[t] = s2[t] = 0.f;
+  for (int t = 0; t < K9; ++t) s0[t] = s1[t] = 0.f;
 #pragma unroll
   for (int t = 0; t < (OFFSET ? K9 : 1); ++t) o0[t] = o1[t] = 0.f;
 
@@ -605,26 +625,22 @@ __global__ __launch_bounds__(BLOCK, BLOCK == kDBlock ? 2 : 1) void deform_grad_c
       for (int c = 0; c < CH; ++c) {
         const float4 q = MODE == 1 ? lds_read4(tb + c * Tb::SIZE + st[t].cell)
                                    : *reinterpret_cast<const float4*>(tb + c * Tb::SIZE + st[t].cell);
+        const Sample sm = sample_slopes(cq.a[c], cq.b[c], cq.c[c], cq.d[c], it[t].lh, it[t].lw), sw = scope_slopes(st[t], q);
         if constexpr (ROTATION) {
-          const float top = fmaf(it[t].lw, cq.b[c] - cq.a[c], cq.a[c]), bot = fmaf(it[t].lw, cq.d[c] - cq.c[c], cq.c[c]);
-          const float ps = fmaf(it[t].lh, bot - top, top) * gv[c];
-          s0[t] = fmaf(ps, q.y, s0[t]);
-          s1[t] = fmaf(ps, q.z, s1[t]);
-          s2[t] = fmaf(ps, q.w, s2[t]);
+          const float ps = sm.val * gv[c];
+          s0[t] = fmaf(ps, sw.h, s0[t]);
+          s1[t] = fmaf(ps, sw.w, s1[t]);
         }
         if constexpr (OFFSET) {
-          const float gw = gv[c] * lite_weight(st[t], q);
-          const float ca = cq.c[c] - cq.a[c], ba = cq.b[c] - cq.a[c];
-          const float dh = fmaf(it[t].lw, (cq.d[c] - cq.b[c]) - ca, ca);
-          const float dw = fmaf(it[t].lh, (cq.d[c] - cq.c[c]) - ba, ba);
-          o0[t] = fmaf(dh, gw, o0[t]);
-          o1[t] = fmaf(dw, gw, o1[t]);
+          const float gw = gv[c] * sw.val;
+          o0[t] = fmaf(sm.h, gw, o0[t]);
+          o1[t] = fmaf(sm.w, gw, o1[t]);
         }
       }
       // keeps the compiler from issuing every tap's reads first (8 x 16 bytes per tap: registers)
       // the tap's sums are complete here: without this the compiler sinks the arithmetic of all nine
       // taps below the plane store and keeps their 9 x 32 loaded values in registers meanwhile
-      if constexpr (ROTATION) asm volatile("" : "+v"(s0[t]), "+v"(s1[t]), "+v"(s2[t])::"memory");
+      if constexpr (ROTATION) asm volatile("" : "+v"(s0[t]), "+v"(s1[t])::"memory");
       if constexpr (OFFSET) asm volatile("" : "+v"(o0[t]), "+v"(o1[t])::"memory");
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -640,8 +656,7 @@ __global__ __launch_bounds__(BLOCK, BLOCK == kDBlock ? 2 : 1) void deform_grad_c
       const T* rp = rot + (size_t)(b.n * g.groups + b.grp) * (K9 * 2) * out_plane + p;
 #pragma unroll
       for (int t = 0; t < K9; ++t) {
-        float dh = fmaf(st[t].lw, s2[t], s1[t]);
-        float dw = fmaf(st[t].lh, s2[t], s0[t]);
+        float dh = s0[t], dw = s1[t];
         if (g.clip_mode != kClipNone) {  // a clamped offset has no gradient
           bool open_h, open_w;
           scope_coord<float>(g, t / 3, ld(rp + (size_t)(2 * t) * out_plane), g.centre_h, &open_h);
@@ -840,7 +855,8 @@ template <typename T, int SH, int SW, int MODE>
 __global__ __launch_bounds__(kDWinCoordBlock, 1) void deform_grad_coord_chw_kernel(
     Geo g, const T* __restrict__ gout, const T* __restrict__ x, const T* __restrict__ off,
     const T* __restrict__ rot, const T* __restrict__ filter, float* __restrict__ partial,
-    int ch_per_block, int shift, int wr, float* __restrict__ partial_off) {
+    int ch_per_block, int shift, int wr, float* __restrict__ partial_off, TileChoice choice) {
+  if (choice.windows && tiles_take(choice)) return;
   constexpr bool ROTATION = MODE != 0, OFFSET = MODE != 1;
   constexpr int CH = kDWinCh, BLOCK = kDWinCoordBlock;
   using Tb = WideTable<SH, SW>;
@@ -880,10 +896,10 @@ __global__ __launch_bounds__(kDWinCoordBlock, 1) void deform_grad_coord_chw_kern
   const size_t x_step = (size_t)g.groups * in_plane, g_step = (size_t)g.groups * out_plane;
   const unsigned goff = live ? (unsigned)p * (unsigned)sizeof(T) : kOutOfRange;
 
-  float s0[K9], s1[K9], s2[K9];                    // rotation: sums of sample * gout * {b, c, d}
+  float s0[K9], s1[K9];                            // rotation: sums of sample * gout * d B / d{h, w}
   float o0[OFFSET ? K9 : 1], o1[OFFSET ? K9 : 1];  // offset: sums of d sample / d{h, w} * gout * B
 #pragma unroll
-  for (int t = 0; t < K9; ++t) s0[t] = s1[t] = s2[t] = 0.f;
+  for (int t = 0; t < K9; ++t) s0[t] = s1[t] = 0.f;
 #pragma unroll
   for (int t = 0; t < (OFFSET ? K9 : 1); ++t) o0[t] = o1[t] = 0.f;
 
@@ -917,24 +933,20 @@ __global__ __launch_bounds__(kDWinCoordBlock, 1) void deform_grad_coord_chw_kern
 #pragma unroll
         for (int c = 0; c < CH; ++c) {
           const float4 q = *reinterpret_cast<const float4*>(tb + c * Tb::SIZE + st[t].cell);
+          const Sample sm = sample_slopes(cq.a[c], cq.b[c], cq.c[c], cq.d[c], it[t].lh, it[t].lw), sw = scope_slopes(st[t], q);
           if constexpr (ROTATION) {
-            const float top = fmaf(it[t].lw, cq.b[c] - cq.a[c], cq.a[c]), bot = fmaf(it[t].lw, cq.d[c] - cq.c[c], cq.c[c]);
-            const float ps = fmaf(it[t].lh, bot - top, top) * gv[c];
-            s0[t] = fmaf(ps, q.y, s0[t]);
-            s1[t] = fmaf(ps, q.z, s1[t]);
-            s2[t] = fmaf(ps, q.w, s2[t]);
+            const float ps = sm.val * gv[c];
+            s0[t] = fmaf(ps, sw.h, s0[t]);
+            s1[t] = fmaf(ps, sw.w, s1[t]);
           }
           if constexpr (OFFSET) {
-            const float gw = gv[c] * lite_weight(st[t], q);
-            const float ca = cq.c[c] - cq.a[c], ba = cq.b[c] - cq.a[c];
-            const float dh = fmaf(it[t].lw, (cq.d[c] - cq.b[c]) - ca, ca);
-            const float dw = fmaf(it[t].lh, (cq.d[c] - cq.c[c]) - ba, ba);
-            o0[t] = fmaf(dh, gw, o0[t]);
-            o1[t] = fmaf(dw, gw, o1[t]);
+            const float gw = gv[c] * sw.val;
+            o0[t] = fmaf(sm.h, gw, o0[t]);
+            o1[t] = fmaf(sm.w, gw, o1[t]);
           }
         }
         // the tap's sums are complete here: keeps the arithmetic of all nine taps from sinking below the plane store
-        if constexpr (ROTATION) asm volatile("" : "+v"(s0[t]), "+v"(s1[t]), "+v"(s2[t])::"memory");
+        if constexpr (ROTATION) asm volatile("" : "+v"(s0[t]), "+v"(s1[t])::"memory");
         if constexpr (OFFSET) asm volatile("" : "+v"(o0[t]), "+v"(o1[t])::"memory");
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -951,8 +963,7 @@ __global__ __launch_bounds__(kDWinCoordBlock, 1) void deform_grad_coord_chw_kern
       const T* rp = rot + (size_t)(b.n * g.groups + b.grp) * (K9 * 2) * out_plane + p;
 #pragma unroll
       for (int t = 0; t < K9; ++t) {
-        float dh = fmaf(st[t].lw, s2[t], s1[t]);
-        float dw = fmaf(st[t].lh, s2[t], s0[t]);
+        float dh = s0[t], dw = s1[t];
         if (g.clip_mode != kClipNone) {  // a clamped offset has no gradient
           bool open_h, open_w;
           scope_coord<float>(g, t / 3, ld(rp + (size_t)(2 * t) * out_plane), g.centre_h, &open_h);
@@ -1928,7 +1939,8 @@ constexpr int kGwGrid = 256; // resident workgroups: one per CU (the window take
 template <typename T, int SH, int SW, int CELL0>
 __global__ __launch_bounds__(kGwBlock, 1) void deform_grad_filter_win_kernel(
     Geo g, const T* __restrict__ gout, const T* __restrict__ x, const T* __restrict__ off,
-    const T* __restrict__ rot, float* __restrict__ partial, int tiles, int nwg, int shift, int wr) {
+    const T* __restrict__ rot, float* __restrict__ partial, int tiles, int nwg, int shift, int wr, TileChoice choice) {
+  if (choice.windows && tiles_take(choice)) return;
   constexpr int CELLS = SH * SW;
   constexpr int kWaves = kGwBlock / 64;
   static_assert(CELL0 % 16 == 0 && CELL0 < CELLS, "the cells come in slices of 16, the rows of one MFMA block");
@@ -2204,7 +2216,8 @@ constexpr int kG2Wc = 32;                         // window columns (a power of 
 template <typename T, int SH, int SW, int CELL0>
 __global__ __launch_bounds__(kGwBlock, 1) void deform_grad_filter_win2_kernel(
     Geo g, const T* __restrict__ gout, const T* __restrict__ x, const T* __restrict__ off,
-    const T* __restrict__ rot, float* __restrict__ partial, int tiles_x, int tiles, int nwg, int wr) {
+    const T* __restrict__ rot, float* __restrict__ partial, int tiles_x, int tiles, int nwg, int wr, TileChoice choice) {
+  if (choice.windows && tiles_take(choice)) return;
   constexpr int CELLS = SH * SW;
   constexpr int kWaves = kGwBlock / 64;
   constexpr int WC = kG2Wc;
@@ -2645,9 +2658,11 @@ bool run_deform_forward(const Geo& g, const T* x, const T* off, const T* rot, co
 }
 
 
+// jobs != null: the reduction is not launched but noted there (wide_deform_grads)
 template <typename T, int SH, int SW>
 bool run_deform_grad_coord(const Geo& g, bool rotation, const T* gout, const T* x, const T* off, const T* rot,
-                           const T* filter, T* result, float* ws, hipStream_t stream) {
+                           const T* filter, T* result, float* ws, hipStream_t stream, const TileChoice& choice = TileChoice{},
+                           ReduceJob<T>* jobs = nullptr) {
   const DeformPlan d4 = deform_plan_ch(g, WideTable<SH, SW>::SIZE, 3);
   DeformPlan d = d4.ok ? d4 : deform_plan(g, WideTable<SH, SW>::SIZE, 2, kDBlock, rotation ? 2 : 3);
   const bool wide = !d.ok;
@@ -2662,7 +2677,7 @@ bool run_deform_grad_coord(const Geo& g, bool rotation, const T* gout, const T* 
   if (window) {
     auto kernel = rotation ? deform_grad_coord_chw_kernel<T, SH, SW, 1> : deform_grad_coord_chw_kernel<T, SH, SW, 0>;
     if (!allow_max_dynamic_lds(reinterpret_cast<const void*>(kernel))) return false;
-    kernel<<<grid, kDWinCoordBlock, d.lds, stream>>>(g, gout, x, off, rot, filter, ws, d.per, d.shift, d.wr, nullptr);
+    kernel<<<grid, kDWinCoordBlock, d.lds, stream>>>(g, gout, x, off, rot, filter, ws, d.per, d.shift, d.wr, nullptr, choice);
   } else if (wide) {
     auto kernel = rotation ? deform_grad_coord_kernel<T, SH, SW, kDWidePasses, true, kDWideBlock>
                            : deform_grad_coord_kernel<T, SH, SW, kDWidePasses, false, kDWideBlock>;
@@ -2673,12 +2688,12 @@ bool run_deform_grad_coord(const Geo& g, bool rotation, const T* gout, const T* 
                            : deform_grad_coord_ch_kernel<T, SH, SW, 4, 0, kDeformCh, kDBigBlock>;
     if (!allow_max_dynamic_lds(reinterpret_cast<const void*>(kernel)))
       return false;
-    kernel<<<grid, kDBigBlock, d.lds, stream>>>(g, gout, x, off, rot, filter, ws, d.per, d.shift, d.tile_pix, nullptr);
+    kernel<<<grid, kDBigBlock, d.lds, stream>>>(g, gout, x, off, rot, filter, ws, d.per, d.shift, d.tile_pix, nullptr, TileChoice{});
   } else if (d4.ok) {
     if (rotation)
-      deform_grad_coord_ch_kernel<T, SH, SW, 4, 1, kDeformCh><<<grid, kDBlock, d.lds, stream>>>(g, gout, x, off, rot, filter, ws, d.per, d.shift, d.tile_pix, nullptr);
+      deform_grad_coord_ch_kernel<T, SH, SW, 4, 1, kDeformCh><<<grid, kDBlock, d.lds, stream>>>(g, gout, x, off, rot, filter, ws, d.per, d.shift, d.tile_pix, nullptr, TileChoice{});
     else
-      deform_grad_coord_ch_kernel<T, SH, SW, 4, 0, kDeformCh><<<grid, kDBlock, d.lds, stream>>>(g, gout, x, off, rot, filter, ws, d.per, d.shift, d.tile_pix, nullptr);
+      deform_grad_coord_ch_kernel<T, SH, SW, 4, 0, kDeformCh><<<grid, kDBlock, d.lds, stream>>>(g, gout, x, off, rot, filter, ws, d.per, d.shift, d.tile_pix, nullptr, TileChoice{});
   } else {
 #define DK_LAUNCH(NP, ROT)                                                                          \
   deform_grad_coord_kernel<T, SH, SW, NP, ROT><<<grid, kDBlock, d.lds, stream>>>(g, gout, x, off, rot, filter, ws, \
@@ -2695,6 +2710,10 @@ bool run_deform_grad_coord(const Geo& g, bool rotation, const T* gout, const T* 
 #undef DK_LAUNCH
   }
   const int plane18 = 18 * g.out_h * g.out_w;
+  if (jobs) {
+    jobs[0] = {ws, d.chunks * (rotation ? 1 : g.groups), (long)g.batch * plane18 * (rotation ? g.groups : 1), result};
+    return true;
+  }
   if (rotation)
     launch_reduce_partials<float, T>(ws, d.chunks, g.batch * g.groups * plane18, result, stream);
   else
@@ -2732,7 +2751,8 @@ bool coords_window(const Geo& g, int table_floats, DeformPlan* d) {
 // Workspace: the rotation partials, then the offset partials (the same number of floats).
 template <typename T, int SH, int SW>
 bool run_deform_grad_coords(const Geo& g, const T* gout, const T* x, const T* off, const T* rot, const T* filter,
-                            T* goff, T* grot, float* ws, hipStream_t stream) {
+                            T* goff, T* grot, float* ws, hipStream_t stream, const TileChoice& choice = TileChoice{},
+                            ReduceJob<T>* jobs = nullptr) {
   DeformPlan d = coords_plan(g, WideTable<SH, SW>::SIZE);
   const bool window = !d.ok && coords_window(g, WideTable<SH, SW>::SIZE, &d);
   if (!d.ok) return false;
@@ -2742,13 +2762,18 @@ bool run_deform_grad_coords(const Geo& g, const T* gout, const T* x, const T* of
   if (window) {
     auto kernel = deform_grad_coord_chw_kernel<T, SH, SW, 2>;
     if (!allow_max_dynamic_lds(reinterpret_cast<const void*>(kernel))) return false;
-    kernel<<<grid, kDWinCoordBlock, d.lds, stream>>>(g, gout, x, off, rot, filter, ws, d.per, d.shift, d.wr, ws_off);
+    kernel<<<grid, kDWinCoordBlock, d.lds, stream>>>(g, gout, x, off, rot, filter, ws, d.per, d.shift, d.wr, ws_off, choice);
   } else if (d.block == kDBlock) {
-    deform_grad_coord_ch_kernel<T, SH, SW, 4, 2, kDeformCh><<<grid, kDBlock, d.lds, stream>>>(g, gout, x, off, rot, filter, ws, d.per, d.shift, d.tile_pix, ws_off);
+    deform_grad_coord_ch_kernel<T, SH, SW, 4, 2, kDeformCh><<<grid, kDBlock, d.lds, stream>>>(g, gout, x, off, rot, filter, ws, d.per, d.shift, d.tile_pix, ws_off, choice);
   } else {
     auto kernel = deform_grad_coord_ch_kernel<T, SH, SW, 8, 2, kDeformCh, kDCoordsBlock>;
     if (!allow_max_dynamic_lds(reinterpret_cast<const void*>(kernel))) return false;
-    kernel<<<grid, kDCoordsBlock, d.lds, stream>>>(g, gout, x, off, rot, filter, ws, d.per, d.shift, d.tile_pix, ws_off);
+    kernel<<<grid, kDCoordsBlock, d.lds, stream>>>(g, gout, x, off, rot, filter, ws, d.per, d.shift, d.tile_pix, ws_off, choice);
+  }
+  if (jobs) {
+    jobs[0] = {ws, d.chunks, (long)g.batch * g.groups * plane18, grot};
+    jobs[1] = {ws_off, d.chunks * g.groups, (long)g.batch * plane18, goff};
+    return true;
   }
   launch_reduce_partials<float, T>(ws, d.chunks, g.batch * g.groups * plane18, grot, stream);
   launch_reduce_partials<float, T>(ws_off, d.chunks * g.groups, g.batch * plane18, goff, stream);
@@ -2971,21 +2996,21 @@ GradFilterWin2 grad_filter_win2_plan(const Geo& g) {
 
 template <typename T, int SH, int SW, int CELL0>
 bool launch_deform_grad_filter_win2(const Geo& g, const GradFilterWin2& m, const T* gout, const T* x, const T* off,
-                                    const T* rot, float* ws, hipStream_t stream) {
+                                    const T* rot, float* ws, hipStream_t stream, const TileChoice& choice = TileChoice{}) {
   auto kernel = deform_grad_filter_win2_kernel<T, SH, SW, CELL0>;
   if (!allow_max_dynamic_lds(reinterpret_cast<const void*>(kernel))) return false;
   const unsigned grid = (unsigned)xcd_grid_size(m.nwg);
-  kernel<<<grid, kGwBlock, m.lds, stream>>>(g, gout, x, off, rot, ws, m.tiles_x, m.tiles, m.nwg, m.wr);
+  kernel<<<grid, kGwBlock, m.lds, stream>>>(g, gout, x, off, rot, ws, m.tiles_x, m.tiles, m.nwg, m.wr, choice);
   return true;
 }
 
 template <typename T, int SH, int SW, int CELL0>
 bool launch_deform_grad_filter_win(const Geo& g, const GradFilterWin& m, const T* gout, const T* x, const T* off,
-                                   const T* rot, float* ws, hipStream_t stream) {
+                                   const T* rot, float* ws, hipStream_t stream, const TileChoice& choice = TileChoice{}) {
   const unsigned grid = (unsigned)xcd_grid_size(m.nwg);
   auto kernel = deform_grad_filter_win_kernel<T, SH, SW, CELL0>;
   if (!allow_max_dynamic_lds(reinterpret_cast<const void*>(kernel))) return false;
-  kernel<<<grid, kGwBlock, m.lds, stream>>>(g, gout, x, off, rot, ws, m.tiles, m.nwg, m.shift, m.wr);
+  kernel<<<grid, kGwBlock, m.lds, stream>>>(g, gout, x, off, rot, ws, m.tiles, m.nwg, m.shift, m.wr, choice);
   return true;
 }
 
@@ -3054,6 +3079,51 @@ bool run_deform_grad_filter(const Geo& g, const T* gout, const T* x, const T* of
   }
 }
 
+// The kernels that wide_deform_grads launches: both coordinate gradients from one pass (with a rotation tensor) or the offset
+// gradient's row-window form, and a window form of the filter gradient.  Floats of their workspaces, 0: they do not apply.
+struct WidePlan {
+  size_t coords, filter;
+};
+template <int SH, int SW>
+WidePlan wide_plan(const Geo& g, bool rotation) {
+  constexpr int SIZE = WideTable<SH, SW>::SIZE;
+  WidePlan w{0, 0};
+  if (path_disabled(kNoDeformFast) || !block_planes_fit<float>(g) || grad_filter_mfma_plan(g).ok) return w;
+  const GradFilterWin wn = grad_filter_win_plan(g);
+  const GradFilterWin2 w2 = grad_filter_win2_plan(g);
+  if (!wn.ok && !w2.ok) return w;
+  DeformPlan d{};
+  d.ok = false;
+  if (rotation) {
+    d = coords_plan(g, SIZE);
+    if (!d.ok) coords_window(g, SIZE, &d);
+  } else if (!deform_plan_ch(g, SIZE, 3).ok && !deform_plan(g, SIZE, 2, kDBlock, 3).ok) {
+    d = deform_plan_chw(g, SIZE, kDWinCoordBlock, kDWinCoordPass);
+  }
+  if (!d.ok) return w;
+  w.coords = (size_t)(rotation ? 2 : 1) * d.chunks * g.groups * g.batch * 18 * g.out_h * g.out_w;
+  w.filter = (size_t)g.batch * (wn.ok && !path_disabled(kForceWin2) ? wn.tiles : w2.ok ? w2.tiles : wn.tiles) * g.channel * SH * SW;
+  return w;
+}
+
+template <typename T, int SH, int SW>
+bool run_wide_grads(const Geo& g, const T* gout, const T* x, const T* off, const T* rot, const T* filter, T* goff, T* grot,
+                    T* gfilter, float* ws, const TileChoice& choice, ReduceJob<T>* jobs, hipStream_t stream) {
+  const WidePlan w = wide_plan<SH, SW>(g, rot != nullptr);
+  const bool coords = rot ? run_deform_grad_coords<T, SH, SW>(g, gout, x, off, rot, filter, goff, grot, ws, stream, choice, jobs)
+                          : run_deform_grad_coord<T, SH, SW>(g, false, gout, x, off, rot, filter, goff, ws, stream, choice, jobs);
+  if (!coords) return false;
+  float* ws_filter = ws + w.coords;
+  const GradFilterWin2 w2 = grad_filter_win2_plan(g);
+  const GradFilterWin wn = grad_filter_win_plan(g);
+  const bool second = w2.ok && (!wn.ok || path_disabled(kForceWin2));
+  if (!(second ? launch_deform_grad_filter_win2<T, SH, SW, 0>(g, w2, gout, x, off, rot, ws_filter, stream, choice)
+               : launch_deform_grad_filter_win<T, SH, SW, 0>(g, wn, gout, x, off, rot, ws_filter, stream, choice)))
+    return false;
+  jobs[2] = {ws_filter, g.batch * (second ? w2.tiles : wn.tiles), (long)g.channel * SH * SW, gfilter};
+  return true;
+}
+
 }  // namespace
 
 #define DK_DISPATCH_SCOPE(g, CALL)    \
@@ -3111,6 +3181,24 @@ bool fast_deform_grad_coords(const Geo& g, const T* gout, const T* x, const T* o
 #undef CALL
 }
 
+bool deform_small_plane(const Geo& g) {
+  const int table = g.scope_h == 3 ? WideTable<3, 3>::SIZE : g.scope_h == 4 ? WideTable<4, 4>::SIZE : WideTable<5, 5>::SIZE;
+  const DeformPlan d = deform_plan_ch(g, table, 3);
+  return d.ok && d.block == kDBlock;
+}
+
+size_t wide_deform_grads_workspace(const Geo& g, bool rotation) {
+  const WidePlan w = g.scope_h == 3 ? wide_plan<3, 3>(g, rotation) : wide_plan<4, 4>(g, rotation);
+  return (w.coords + w.filter) * sizeof(float);
+}
+
+template <typename T>
+bool wide_deform_grads(const Geo& g, const T* gout, const T* x, const T* off, const T* rot, const T* filter, T* goff, T* grot,
+                       T* gfilter, float* ws, const TileChoice& choice, ReduceJob<T>* jobs, hipStream_t stream) {
+  if (g.scope_h == 3) return run_wide_grads<T, 3, 3>(g, gout, x, off, rot, filter, goff, grot, gfilter, ws, choice, jobs, stream);
+  return run_wide_grads<T, 4, 4>(g, gout, x, off, rot, filter, goff, grot, gfilter, ws, choice, jobs, stream);
+}
+
 template <typename T>
 bool fast_deform_grad_input(const Geo& g, const T* gout, const T* off, const T* rot, const T* filter, T* gin,
                             void* ws, hipStream_t stream) {
@@ -3145,6 +3233,8 @@ size_t fast_deform_grad_filter_workspace(const Geo& g) {  // one partial per (im
   template bool fast_deform_forward<T>(const Geo&, const T*, const T*, const T*, const T*, T*, hipStream_t);      \
   template bool fast_deform_grad_coord<T>(const Geo&, bool, const T*, const T*, const T*, const T*, const T*, T*,  \
                                           void*, hipStream_t);                                                     \
+  template bool wide_deform_grads<T>(const Geo&, const T*, const T*, const T*, const T*, const T*, T*, T*, T*, float*,  \
+                                     const TileChoice&, ReduceJob<T>*, hipStream_t);                                 \
   template bool fast_deform_grad_coords<T>(const Geo&, const T*, const T*, const T*, const T*, const T*, T*, T*,    \
                                            void*, hipStream_t);                                                    \
   template bool fast_deform_grad_input<T>(const Geo&, const T*, const T*, const T*, const T*, T*, void*,           \

@@ -122,6 +122,21 @@ BandWalk lanes_band_walk(const Geo& g, bool rotation);
 template <typename T>
 bool lanes_deform_grad_input(const Geo& g, const T* gout, const T* off, const T* rot, const T* filter, T* gin,
                              const unsigned* gmax, const BandWalk& walk, hipStream_t stream);
+// offset, rotation (null with rot) and filter gradient from one pass (dk_deform_tile.hip); workspace 0: not this way
+size_t tile_deform_grads_workspace(const Geo& g, bool rotation);
+template <typename T>
+bool tile_deform_grads(const Geo& g, const T* gout, const T* x, const T* off, const T* rot, const T* filter, T* goff, T* grot,
+                       T* gfilter, float* ws, hipStream_t stream);
+// ... by the separate kernels of planes that no 256-thread form takes, if the choice falls on them (dk_deform.h), up to the
+// reductions of their partial sums, which are noted in jobs[0 .. 2]; workspace 0: they do not apply
+struct TileChoice;
+template <typename T>
+struct ReduceJob;
+size_t wide_deform_grads_workspace(const Geo& g, bool rotation);
+template <typename T>
+bool wide_deform_grads(const Geo& g, const T* gout, const T* x, const T* off, const T* rot, const T* filter, T* goff, T* grot,
+                       T* gfilter, float* ws, const TileChoice& choice, ReduceJob<T>* jobs, hipStream_t stream);
+bool deform_small_plane(const Geo& g);  // served by the channel-interleaved kernels in 256-thread workgroups
 // rotation = false: gradient w.r.t. the image-space offsets
 size_t fast_deform_grad_coord_workspace(const Geo& g, bool rotation);
 template <typename T>

@@ -294,6 +294,13 @@ struct DeformableSampleDepthwiseFunctionBackward : OpNode {
             "deform_sample_depthwise backward_offset_filter");
       return res;
     }
+    if (need_offset && need_rotation && need_filter) {
+      const Workspace ws(dk_deformable_sample_depthwise_backward_parameters_workspace(&desc), x);
+      check(dk_deformable_sample_depthwise_backward_parameters(&desc, in(g), in(x), in(f), in(r), in(w), out(res[1]), out(res[2]),
+                                                               out(res[3]), ws.ptr(), ws.bytes, s),
+            "deform_sample_depthwise backward_parameters");
+      return res;
+    }
     if (need_offset && need_rotation) {
       // one call for both coordinate gradients (one pass over the input where the library has that kernel)
       const Workspace ws(dk_deformable_sample_depthwise_backward_offset_rotation_workspace(&desc), x);

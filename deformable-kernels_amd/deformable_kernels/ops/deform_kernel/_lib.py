@@ -76,6 +76,8 @@ SIGNATURES = {
     "dk_deformable_sample_depthwise_backward_rotation": (ctypes.c_int, [_CD, _P, _P, _P, _P, _P, _P, _P, _SZ, _P]),
     "dk_deformable_sample_depthwise_backward_offset_rotation_workspace": (_SZ, [_CD]),
     "dk_deformable_sample_depthwise_backward_offset_rotation": (ctypes.c_int, [_CD, _P, _P, _P, _P, _P, _P, _P, _P, _SZ, _P]),
+    "dk_deformable_sample_depthwise_backward_parameters_workspace": (_SZ, [_CD]),
+    "dk_deformable_sample_depthwise_backward_parameters": (ctypes.c_int, [_CD, _P, _P, _P, _P, _P, _P, _P, _P, _P, _SZ, _P]),
     "dk_deformable_sample_depthwise_backward_offset_filter_workspace": (_SZ, [_CD]),
     "dk_deformable_sample_depthwise_backward_offset_filter": (ctypes.c_int, [_CD, _P, _P, _P, _P, _P, _P, _P, _P, _SZ, _P]),
     "dk_nd_linear_sample_forward_workspace": (_SZ, [_ND]),

@@ -249,6 +249,16 @@ int dk_deformable_sample_depthwise_backward_offset_filter(const dk_conv_desc *de
                                                           void *workspace, size_t workspace_bytes,
                                                           void *stream);
 
+/* Offset, rotation and filter gradient in one call, where one pass over the samples gives all three; otherwise the call of both
+ * coordinate gradients and the filter gradient's run one after the other on the stream.  `rotation` must not be NULL here. */
+size_t dk_deformable_sample_depthwise_backward_parameters_workspace(const dk_conv_desc *desc);
+int dk_deformable_sample_depthwise_backward_parameters(const dk_conv_desc *desc, const void *out_grad,
+                                                       const void *input, const void *offset,
+                                                       const void *rotation, const void *filter,
+                                                       void *offset_grad, void *rotation_grad, void *filter_grad,
+                                                       void *workspace, size_t workspace_bytes,
+                                                       void *stream);
+
 /* ---- N-d linear sample -------------------------------------------------------
  * data [channel, shape[0..dims-1]], coord [batch, dims] in absolute index units,
  * output [batch, channel].  The reference passes `shape` as a device tensor of the

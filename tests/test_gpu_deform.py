@@ -641,3 +641,70 @@ def test_an_infinite_output_gradient_of_taps_outside_the_image_reaches_no_filter
     og, wg = off.cuda().requires_grad_(), wt.cuda().requires_grad_()
     got = torch.autograd.grad(deform_sample_depthwise(x.cuda(), og, None, wg, *args), [wg], gout.cuda())[0]
     assert bool(got[4].isnan().any()) and bool(got[:4].isfinite().all()) and bool(got[5:].isfinite().all())
+
+
+# one pass for the coordinates' and the filter's gradient: N, C, H, W, scope, groups, rotation std, offset std
+ONE_PASS = [
+    (2, 16, 7, 7, 4, 1, 0.7, 2.0),      # one tile, one block; the plane fits the window
+    (5, 35, 25, 25, 4, 1, 0.7, 9.0),    # the largest such plane, ragged tiles, a block of three channels; offsets beyond it
+    (3, 40, 26, 31, 3, 1, 0.7, 2.0),    # windows from the offsets; scope 3
+    (2, 24, 9, 70, 4, 2, 0.7, 2.0),     # two groups of twelve channels: the offsets' gradient adds up over them
+    (1, 200, 40, 36, 4, 1, 0.7, 1.0),   # thirteen blocks in shares of one: partial sums of both coordinate gradients
+    (6, 176, 56, 56, 4, 1, 0.7, 2.0),   # more tiles than workgroups, eleven blocks: two shares
+    (2, 20, 60, 66, 4, 1, 0.7, 6.0),    # samples spread over several windows: the separate kernels take the call
+    (1, 9, 33, 35, 3, 1, 0.7, 14.0),
+]
+
+
+@pytest.mark.parametrize("wide_too", [False, True])
+@pytest.mark.parametrize("clip", [None, (-0.5, 0.75)])
+@pytest.mark.parametrize("case", ONE_PASS)
+def test_coordinate_and_filter_gradients_from_one_pass(case, clip, wide_too, switch_off):
+    """wide_too: without the separate kernels' channel-interleaved forms there is no choice, and calls with wide offsets walk
+    their tiles in several windows."""
+    from deformable_kernels.ops.deform_kernel.functions import deform_sample_depthwise
+    N, C, H, W, S, G, rs, os_ = case
+    x, wt, rot, off, gout, cfg = make_deform(N, C, H, W, 3, (S, S), 1, 1, 1, G, rs, os_, seed=21)
+    if wide_too:
+        switch_off("DK_NO_DEFORM_CH")
+    dev = torch.device("cuda:0")
+    leaves = [t.to(dev).requires_grad_() for t in (x, off, rot, wt)]
+    args = (cfg["kernel_size"], cfg["stride"], cfg["padding"], cfg["dilation"], G)
+    out = deform_sample_depthwise(*leaves, *args, clip)
+    got = torch.autograd.grad(out, leaves, gout.to(dev))
+    used, open_ = (rot, torch.ones_like(rot)) if clip is None else clipped_rotation(rot, clip, cfg["kernel_size"], (S, S), G)
+    want = orc.deform_sample_depthwise_backward(*[t.double().numpy() for t in (gout, x, off, used, wt)], **cfg)
+    # sums of at most 9 * N * H * W products of three factors in float32, in blocks
+    assert rel_err(got[1].cpu(), want[1]) < 2e-5
+    assert rel_err(got[2].cpu(), torch.as_tensor(want[2]) * open_) < 2e-5
+    assert rel_err(got[3].cpu(), want[3]) < 2e-5
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("plain", [False, True])
+def test_one_pass_in_16_bits_and_without_a_rotation_tensor(dtype, plain):
+    from deformable_kernels.ops.deform_kernel.functions import deform_sample_depthwise
+    x, wt, rot, off, gout, cfg = make_deform(2, 36, 70, 90, 3, (4, 4), 1, 1, 1, 1, 0.0 if plain else 0.7, 2.0, seed=22, dtype=dtype)
+    dev = torch.device("cuda:0")
+    leaves = [t.to(dev).requires_grad_() for t in ((x, off, wt) if plain else (x, off, rot, wt))]
+    xs, offs, rots, wts = (leaves[0], leaves[1], None, leaves[2]) if plain else leaves
+    out = deform_sample_depthwise(xs, offs, rots, wts, cfg["kernel_size"], cfg["stride"], cfg["padding"], cfg["dilation"], 1)
+    got = torch.autograd.grad(out, leaves, gout.to(dev))
+    want = orc.deform_sample_depthwise_backward(*[t.double().numpy() for t in (gout, x, off, rot, wt)], **cfg)
+    want = (want[0], want[1], want[3]) if plain else want
+    for g, w in list(zip(got, want))[1:]:
+        assert g.dtype == dtype and rel_err(g.float().cpu(), w) < (2e-3 if dtype == torch.float16 else 1e-2)  # the result's rounding
+
+
+def test_one_pass_non_finite_output_gradient_reaches_its_pixel_and_channel_only():
+    from deformable_kernels.ops.deform_kernel.functions import deform_sample_depthwise
+    x, wt, rot, off, gout, cfg = make_deform(2, 24, 40, 40, 3, (4, 4), 1, 1, 1, 1, 0.5, 1.0, seed=23)
+    gout[1, 17, 20, 21] = float("nan")
+    leaves = [t.to("cuda:0").requires_grad_() for t in (x, off, rot, wt)]
+    out = deform_sample_depthwise(*leaves, cfg["kernel_size"], cfg["stride"], cfg["padding"], cfg["dilation"], 1)
+    _, goff, grot, gw = torch.autograd.grad(out, leaves, gout.to("cuda:0"))
+    for g in (goff, grot):
+        bad = ~torch.isfinite(g)
+        assert bad[1, :, 20, 21].all() and int(bad.sum()) == 18
+    bad = ~torch.isfinite(gw)
+    assert bad[17].any() and int(bad.sum()) == int(bad[17].sum())
