@@ -823,6 +823,13 @@ int dk_global_kernels_backward(const dk_conv_desc* desc, const void* kernels_gra
   });
 }
 
+// Tensors on planes the 16-bit matrix-instruction kernels cover: 16-bit elements as they are, float32 ones as
+// bfloat16 (hi, lo) pairs
+static bool offset_conv_on_16_bit_matrix(const dk_offset_conv_desc* d) {
+  if (d->dtype == DK_F32 && path_disabled(kNoOffsetPairs)) return false;
+  return offset_conv16_supported(d->in_channels, d->out_channels, d->h, d->w);
+}
+
 // forward: the call is (or asks about) the forward, the one pass that has a stride-2 kernel
 static int check_offset_conv(const dk_offset_conv_desc* d, bool forward = false) {
   if (!d) return DK_ERR_NULL_POINTER;
@@ -831,22 +838,19 @@ static int check_offset_conv(const dk_offset_conv_desc* d, bool forward = false)
   if (d->dtype != DK_F32 && d->dtype != DK_F16 && d->dtype != DK_BF16) return d->dtype == DK_F64 ? DK_ERR_UNSUPPORTED : DK_ERR_BAD_DTYPE;
   if ((long)d->batch * d->in_channels * d->h * d->w > kMaxElems) return DK_ERR_TOO_LARGE;
   if (d->stride == 2)
-    return forward && (d->dtype != DK_F32 || !path_disabled(kNoOffsetPairs)) && d->in_channels % 16 == 0 &&
+    return forward && (d->dtype != DK_F32 || (!path_disabled(kNoOffsetPairs) && d->in_channels % 16 == 0)) &&
                    offset_conv16_s2_supported(d->in_channels, d->out_channels, d->h, d->w)
                ? DK_OK
                : DK_ERR_UNSUPPORTED;
-  if (!offset_conv_supported(d->in_channels, d->out_channels, d->h, d->w)) return DK_ERR_UNSUPPORTED;
-  return DK_OK;
+  // 16-bit tensors: any number of channels.  (float32 ones in sixteens only: as bfloat16 pairs they are further from the float64
+  // convolution than the framework's kernels, which serve the others.)  us forward and both gradients, library / here: 80 x
+  // 577 x 7^2 float16 66 and 55 / 25 and 40, 76 x 61 x 28^2 bfloat16 67 and 81 / 18 and 55, 11 x 41 x 112^2 float16 43 and 96 / 21 and 62, 64 x 250 x
+  // 28^2 bfloat16 stride 2 207 and 111 / 33 and 51.
+  if (!offset_conv_supported(ceil_div(d->in_channels, 16) * 16, d->out_channels, d->h, d->w)) return DK_ERR_UNSUPPORTED;
+  return d->in_channels % 16 == 0 || (d->dtype != DK_F32 && offset_conv_on_16_bit_matrix(d)) ? DK_OK : DK_ERR_UNSUPPORTED;
 }
 
 int dk_offset_conv_supported(const dk_offset_conv_desc* desc) { return check_offset_conv(desc, true) == DK_OK; }
-
-// Tensors on planes the 16-bit matrix-instruction kernels cover: 16-bit elements as they are, float32 ones as
-// bfloat16 (hi, lo) pairs
-static bool offset_conv_on_16_bit_matrix(const dk_offset_conv_desc* d) {
-  if (d->dtype == DK_F32 && path_disabled(kNoOffsetPairs)) return false;
-  return offset_conv16_supported(d->in_channels, d->out_channels, d->h, d->w);
-}
 
 int dk_offset_conv_worthwhile(const dk_offset_conv_desc* desc) {
   if (check_offset_conv(desc, true) != DK_OK) return 0;
@@ -962,6 +966,7 @@ static int check_offset_conv_backward_weight(const dk_offset_conv_desc* d) {
     if (rc != DK_OK) return rc;
     return offset_wgrad_on_16_bit_matrix(d) ? DK_OK : DK_ERR_UNSUPPORTED;
   }
+  if (d->in_channels % 16 != 0 && !offset_wgrad_on_16_bit_matrix(d)) return DK_ERR_UNSUPPORTED;
   return check_offset_conv(d);
 }
 
@@ -1031,9 +1036,13 @@ static int check_offset_conv_direct(const dk_offset_conv_desc* d) {
   return offset_conv_direct_supported(d->batch, d->in_channels, d->out_channels, d->h, d->w) ? DK_OK : DK_ERR_UNSUPPORTED;
 }
 
-// Channels-times-pixels of the calls that these kernels are for, or 0: too few images for the matrix-instruction kernels.
-static long offset_conv_direct_work(const dk_offset_conv_desc* desc) {
-  if (check_offset_conv_direct(desc) != DK_OK || !dk_offset_conv_supported(desc) || dk_offset_conv_worthwhile(desc)) return 0;
+// Channels-times-pixels of the calls that these kernels are for, or 0: too few images for the matrix-instruction kernels, or
+// (`general`) 16-bit tensors on a plane that those have no kernel for (float32 ones keep the library's results there), or whose
+// channels are no multiple of sixteen.
+static long offset_conv_direct_work(const dk_offset_conv_desc* desc, bool* general) {
+  if (check_offset_conv_direct(desc) != DK_OK || dk_offset_conv_worthwhile(desc)) return 0;
+  *general = !dk_offset_conv_supported(desc) || desc->in_channels % 16 != 0;
+  if (*general && desc->dtype == DK_F32) return 0;
   const long stride = desc->stride == 2 ? 2 : 1, pixels = ((desc->h - 1) / stride + 1) * ((desc->w - 1) / stride + 1);
   return pixels * desc->batch * desc->in_channels;
 }
@@ -1048,8 +1057,13 @@ static long offset_conv_direct_work(const dk_offset_conv_desc* desc) {
 //   two pixels per lane (more than 8192 pixels): float32 16 x 96 x 28^2 26 / 27, 144 channels 36 / 34; float16 64 channels 22 / 22, 96 channels
 //   30 / 23; bfloat16 144 channels 39 / 107
 int dk_offset_conv_direct_worthwhile(const dk_offset_conv_desc* desc) {
-  const long work = offset_conv_direct_work(desc);
+  bool general;
+  const long work = offset_conv_direct_work(desc, &general);
   if (work == 0 || work > 2000000) return 0;
+  // other planes, us here / library: 9 x 240 x 12 x 13 float16 18 / 35, 10 x 60 x 10 x 11 bfloat16 7 / 38, stride 2 7 x 37 x 57 x 55 bfloat16
+  // 11 / 36, 13 x 32 x 103 x 30 float16 14 / 27, 2 x 300 x 33 x 35 24 / 68; but 2 x 80 x 55 x 90 (0.8 M) 26 / 22, 30 x 128 x 17 x 17 (1.1 M) 39 / 26,
+  // 10 x 547 x 14^2 (1.1 M) 62 / 61
+  if (general) return work <= 600000;
   const int c = desc->in_channels;
   const bool half = desc->dtype != DK_F32, strided = desc->stride == 2;
   if (strided && desc->w >= 56 && c > 304) return 0;
@@ -1063,7 +1077,12 @@ int dk_offset_conv_direct_worthwhile(const dk_offset_conv_desc* desc) {
 // the input has four times the pixels: 15 x 192 x 28^2 (560 k) 67 / 93, 8 x 384 x 28^2 (600 k) 71 / 98; 16 x 960 x 14^2 (750 k) 103 / 98, 16 x
 // 384 x 28^2 (1.2 M) 98 / 97, 8 x 288 x 56^2 (1.8 M) 124 / 98.
 int dk_offset_conv_direct_backward_worthwhile(const dk_offset_conv_desc* desc) {
-  const long work = offset_conv_direct_work(desc);
+  bool general;
+  const long work = offset_conv_direct_work(desc, &general);
+  // other planes: 9 x 240 x 12 x 13 float16 40 / 48, 10 x 60 x 10 x 11 bfloat16 21 / 62, stride 2 7 x 37 x 57 x 55 bfloat16 37 / 66, 13 x 32 x 103 x 30
+  // float16 (324 k) 47 / 49; 60 x 16 x 40 x 20 (48000 pixels, a channel's walk over which is serial) 78 / 49, 10 x 547 x 14^2 (1.1 M)
+  // 82 / 51
+  if (work > 0 && general) return work <= (desc->stride == 2 ? 370000 : 600000) && work / desc->in_channels <= 16384;
   return work > 0 && work <= (desc->stride == 2 ? 620000 : 2000000);
 }
 

@@ -104,8 +104,9 @@ __global__ __launch_bounds__(kW16Block, 2) void offset_wgrad16_kernel(int batch,
   unsigned short* gs = lds16 + P * kW16Chunk * XPL * XP;     // [part][cout + 1][GP]; plane `cout` stays zero
   const int gplanes = cout + 1;
 
-  const int nchunks = cin / kW16Chunk;
+  const int nchunks = (cin + kW16Chunk - 1) / kW16Chunk;
   const int chunk = blockIdx.x % nchunks, part = blockIdx.x / nchunks;
+  const int live = min(kW16Chunk, cin - chunk * kW16Chunk);  // channels of the chunk; the others stay zero
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int m = lane & 15, kg = lane >> 4;
   const int plane_in = h * WIN, plane_out = ho * W, items = batch * tiles;
@@ -138,15 +139,15 @@ __global__ __launch_bounds__(kW16Block, 2) void offset_wgrad16_kernel(int batch,
 #define DK_LOAD_ITEM(ITEM)                                                                                          \
   {                                                                                                                 \
     const int n_ = (ITEM) / tiles, r0_ = (ITEM) % tiles * TH;                                                       \
-    const rsrc_t rx = plane_rsrc(x + ((size_t)n_ * cin + (size_t)chunk * kW16Chunk) * plane_in, kW16Chunk * plane_in); \
+    const rsrc_t rx = plane_rsrc(x + ((size_t)n_ * cin + (size_t)chunk * kW16Chunk) * plane_in, live * plane_in); \
     const rsrc_t rg = plane_rsrc(gout + (size_t)n_ * cout * plane_out, cout * plane_out);                           \
     const int xrow0 = S == 1 ? r0_ - 1 : 2 * (r0_ - 1);                                                             \
     _Pragma("unroll") for (int i = 0; i < kXStage; ++i) {                                                           \
       const int chq = i / kXLoads, e = i % kXLoads * 64 + lane;                                                     \
-      const int row = xrow0 + e / WIN;                                                                              \
-      const bool ok = e < kInRows * WIN && row >= 0 && row < h;                                                     \
+      const int row = xrow0 + e / WIN, c = wave + kW16Waves * chq;                                                  \
+      const bool ok = e < kInRows * WIN && row >= 0 && row < h && c < live;                                         \
       xst[i] = w16_load<T>(rx, ok ? (unsigned)((xrow0 * WIN + e) * (int)sizeof(T)) : kOutOfRange,                   \
-                           (wave + kW16Waves * chq) * plane_in * (int)sizeof(T));                                   \
+                           c < live ? c * plane_in * (int)sizeof(T) : 0);                                           \
     }                                                                                                               \
     _Pragma("unroll") for (int i = 0; i < kGStage; ++i) {                                                           \
       const int o = wave + kW16Waves * (i / kGLoads), e = i % kGLoads * 64 + lane;                                  \
@@ -297,15 +298,15 @@ size_t w16_lds_bytes(int parts_per_tensor, int cout) {
 
 // parts of the (image, row tile) items a chunk's workgroups split: about two workgroups per CU
 int w16_parts(int batch, int cin, int ho, int wo, int stride, bool pairs) {
-  const int items = batch * ceil_div(ho, w16_rows(wo, stride, pairs)), nchunks = cin / kW16Chunk;
-  return std::max(1, std::min(items, 512 / nchunks));
+  const int items = batch * ceil_div(ho, w16_rows(wo, stride, pairs)), nchunks = ceil_div(cin, kW16Chunk);
+  return std::max(1, std::min(items, 512 / std::min(nchunks, 512)));
 }
 
 }  // namespace
 
 // stride 1: planes 7 .. 112 wide; stride 2: input planes 14 .. 112 wide (output planes 7 .. 56)
 bool offset_wgrad16_supported(int cin, int cout, int h, int w, int stride) {
-  if (cin < kW16Chunk || cin % kW16Chunk != 0 || cout < 1 || cout > 20 || h < 1) return false;  // (20: the output planes a wave stages)
+  if (cin < 1 || cout < 1 || cout > 20 || h < 1) return false;  // (20: the output planes a wave stages)
   if ((long)cin * h * w >= (1L << 31) / 4 || (long)cout * h * w >= (1L << 31) / 4) return false;
   if (stride == 2) return w == 14 || w == 28 || w == 56 || w == 112;
   return w == 7 || w == 14 || w == 28 || w == 56 || w == 112;
@@ -314,7 +315,7 @@ bool offset_wgrad16_supported(int cin, int cout, int h, int w, int stride) {
 size_t offset_wgrad16_workspace(int batch, int cin, int cout, int h, int w, int stride, bool pairs) {
   if (!offset_wgrad16_supported(cin, cout, h, w, stride)) return 0;
   const int ho = stride == 2 ? (h - 1) / 2 + 1 : h, wo = stride == 2 ? w / 2 : w;
-  return (size_t)w16_parts(batch, cin, ho, wo, stride, pairs) * (cin / kW16Chunk) * kW16Tiles * 256 * sizeof(float);
+  return (size_t)w16_parts(batch, cin, ho, wo, stride, pairs) * ceil_div(cin, kW16Chunk) * kW16Tiles * 256 * sizeof(float);
 }
 
 template <typename T>
@@ -323,7 +324,7 @@ bool offset_wgrad16(int batch, int cin, int cout, int h, int w, int stride, cons
   if (!offset_wgrad16_supported(cin, cout, h, w, stride)) return false;
   constexpr bool pairs = sizeof(T) == 4;
   const int ho = stride == 2 ? (h - 1) / 2 + 1 : h, wo = stride == 2 ? w / 2 : w;
-  const int nchunks = cin / kW16Chunk;
+  const int nchunks = ceil_div(cin, kW16Chunk);
   const int parts = w16_parts(batch, cin, ho, wo, stride, pairs);
   float* partial = static_cast<float*>(ws);
   bool ok = true;

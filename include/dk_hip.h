@@ -325,7 +325,7 @@ int dk_nd_linear_sample_backward(const dk_nd_desc *desc, const void *out_grad, c
  * (modules/deform_kernel.py:165-168: nn.Conv2d(in_planes, rotation_groups*k*k*2, k, stride,
  * padding, dilation, bias=True), applied at :214).  The reference calls the framework's
  * convolution there; this entry point is a faster kernel for that one shape family: padding 1,
- * dilation 1, float32 / float16 / bfloat16 tensors, in_channels a multiple of 16, out_channels <= 16
+ * dilation 1, float32 (in_channels a multiple of 16) / float16 / bfloat16 tensors, out_channels <= 16
  * or 18 or 20, width 7, 14, 28, 56 or 112.  Arithmetic: fp32 sums throughout, results rounded once;
  * float16 / bfloat16 elements are multiplied as they are (exact products) on the 16-bit matrix
  * instructions; float32 elements go to the same instructions as bfloat16 (hi, lo) pairs, hi = bf16(v),
@@ -386,8 +386,8 @@ int dk_offset_conv_backward_input(const dk_offset_conv_desc *desc, const void *o
 /* The same convolution and its input and weight gradients on few images: up to 18 output channels, any other size whose
  * tensors hold less than 2^28 elements, stride 1 or 2 (output ((h - 1) / s + 1) x ((w - 1) / s + 1)), fp32 products and
  * sums for every dtype, no workspace, one launch each.  dk_offset_conv_direct_worthwhile(): 1 where the forward is
- * expected to beat both the kernels above and the library convolution (covered by dk_offset_conv_supported(), too few
- * images for dk_offset_conv_worthwhile()); dk_offset_conv_direct_backward_worthwhile(): the two gradients. */
+ * expected to beat both the kernels above and the library convolution (too few images for dk_offset_conv_worthwhile(), or a
+ * plane that the kernels above do not cover, 16-bit tensors of up to 600000 channels times pixels); dk_offset_conv_direct_backward_worthwhile(): the two gradients. */
 int dk_offset_conv_direct_backward_worthwhile(const dk_offset_conv_desc *desc);
 int dk_offset_conv_direct_worthwhile(const dk_offset_conv_desc *desc);
 int dk_offset_conv_direct_forward(const dk_offset_conv_desc *desc, const void *input, const void *weight,

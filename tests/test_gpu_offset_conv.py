@@ -375,3 +375,51 @@ def test_vector_unit_entry_points_on_sizes_that_the_operator_leaves_to_the_frame
     want = reference(x, w, b, gout, stride=stride)
     for name, got, ref in zip(("forward", "input", "weight"), (out, gx, gw), want):
         assert rel_err(got.double().cpu(), ref) < tol, name
+
+
+@pytest.mark.parametrize("dtype,tol", [(torch.float16, 2e-3), (torch.bfloat16, 1e-2)])
+@pytest.mark.parametrize("shape", [
+    (2, 1, 5, 7, 1),         # N, C, H, W, stride: one channel
+    (3, 17, 14, 14, 1),      # a chunk of sixteen and one of one
+    (2, 33, 28, 28, 1),      # two of the forward's chunks, the second of one channel
+    (2, 61, 9, 56, 1),
+    (1, 41, 6, 112, 1),
+    (2, 15, 13, 28, 2),
+    (2, 50, 14, 14, 2),
+    (1, 37, 10, 112, 2),
+])
+def test_any_number_of_channels_in_16_bits(shape, dtype, tol):
+    """Forward and both gradients on the 16-bit matrix instructions: the last chunk's missing channels read as zeros, whatever lies
+    behind the tensor."""
+    from deformable_kernels.ops.deform_kernel.functions import offset_conv, offset_conv_supported
+    N, C, H, W, s = shape
+    g = torch.Generator().manual_seed(41)
+    behind = torch.full((N * C * H * W + 64 * H * W,), float("nan"), device="cuda:0", dtype=dtype)
+    x = behind[:N * C * H * W].view(N, C, H, W).copy_(torch.randn(N, C, H, W, generator=g))
+    w = (torch.randn(18, C, 3, 3, generator=g) / (9 * C) ** 0.5).to(dtype).cuda()
+    b = torch.randn(18, generator=g).to(dtype).cuda()
+    leaves = [t.requires_grad_() for t in (x, w, b)]
+    assert offset_conv_supported(x, w, b, s, 1, 1)
+    out = offset_conv(x, w, b, s, force=True)
+    gout = torch.randn(out.shape, generator=g).to(dtype).cuda()
+    got = (out.detach(),) + torch.autograd.grad(out, leaves, gout)
+    for a, want in zip(got, reference(x, w, b, gout, s)):
+        assert a.dtype == dtype and rel_err(a.float().cpu(), want) < tol
+
+
+@pytest.mark.parametrize("shape,dtype", [
+    ((35, 15, 17, 19, 1), torch.float16), ((2, 300, 33, 35, 2), torch.float16), ((10, 60, 10, 11, 1), torch.bfloat16),
+])
+def test_few_images_on_any_plane(shape, dtype):
+    from deformable_kernels.ops.deform_kernel.functions import offset_conv
+    N, C, H, W, s = shape
+    g = torch.Generator().manual_seed(42)
+    leaves = [(torch.randn(N, C, H, W, generator=g)).to(dtype).cuda().requires_grad_(),
+              (torch.randn(18, C, 3, 3, generator=g) / (9 * C) ** 0.5).to(dtype).cuda().requires_grad_(),
+              torch.randn(18, generator=g).to(dtype).cuda().requires_grad_()]
+    out = offset_conv(*leaves, s)
+    gout = torch.randn(out.shape, generator=g).to(dtype).cuda()
+    got = (out.detach(),) + torch.autograd.grad(out, leaves, gout)
+    tol = 2e-3 if dtype == torch.float16 else 1e-2
+    for a, want in zip(got, reference(*leaves, gout, s)):
+        assert rel_err(a.float().cpu(), want) < tol
