@@ -843,9 +843,8 @@ static int check_offset_conv(const dk_offset_conv_desc* d, bool forward = false)
                ? DK_OK
                : DK_ERR_UNSUPPORTED;
   // 16-bit tensors: any number of channels.  (float32 ones in sixteens only: as bfloat16 pairs they are further from the float64
-  // convolution than the framework's kernels, which serve the others.)  us forward and both gradients, library / here: 80 x
-  // 577 x 7^2 float16 66 and 55 / 25 and 40, 76 x 61 x 28^2 bfloat16 67 and 81 / 18 and 55, 11 x 41 x 112^2 float16 43 and 96 / 21 and 62, 64 x 250 x
-  // 28^2 bfloat16 stride 2 207 and 111 / 33 and 51.
+  // convolution than the framework's kernels, which serve the others.)  us both gradients, library / here: 80 x 577 x 7^2 float16
+  // 55 / 40, 76 x 61 x 28^2 bfloat16 81 / 55, 11 x 41 x 112^2 float16 96 / 62, 64 x 250 x 28^2 bfloat16 stride 2 111 / 51.
   if (!offset_conv_supported(ceil_div(d->in_channels, 16) * 16, d->out_channels, d->h, d->w)) return DK_ERR_UNSUPPORTED;
   return d->in_channels % 16 == 0 || (d->dtype != DK_F32 && offset_conv_on_16_bit_matrix(d)) ? DK_OK : DK_ERR_UNSUPPORTED;
 }
@@ -1060,10 +1059,7 @@ int dk_offset_conv_direct_worthwhile(const dk_offset_conv_desc* desc) {
   bool general;
   const long work = offset_conv_direct_work(desc, &general);
   if (work == 0 || work > 2000000) return 0;
-  // other planes, us here / library: 9 x 240 x 12 x 13 float16 18 / 35, 10 x 60 x 10 x 11 bfloat16 7 / 38, stride 2 7 x 37 x 57 x 55 bfloat16
-  // 11 / 36, 13 x 32 x 103 x 30 float16 14 / 27, 2 x 300 x 33 x 35 24 / 68; but 2 x 80 x 55 x 90 (0.8 M) 26 / 22, 30 x 128 x 17 x 17 (1.1 M) 39 / 26,
-  // 10 x 547 x 14^2 (1.1 M) 62 / 61
-  if (general) return work <= 600000;
+  if (general) return 0;  // (the framework's: see offset_conv in dk_torch.cpp)
   const int c = desc->in_channels;
   const bool half = desc->dtype != DK_F32, strided = desc->stride == 2;
   if (strided && desc->w >= 56 && c > 304) return 0;

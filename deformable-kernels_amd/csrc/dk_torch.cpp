@@ -516,13 +516,17 @@ Tensor offset_conv(const Tensor& input, const Tensor& weight, const OptTensor& b
   const bool native = offset_conv_covered(input, weight, stride, padding, dilation, force ? dk_offset_conv_supported : dk_offset_conv_worthwhile);
   // few images: one launch per pass on the vector unit
   const bool direct = !native && offset_conv_covered(input, weight, stride, padding, dilation, dk_offset_conv_direct_worthwhile);
+  // Channels in sixteens; layers of others have the framework's forward.  A 16-bit offset that rounds the other way moves its
+  // sample by its last bit, and where it crosses a cell's border the slope jumps: the offsets of a trained layer stay what
+  // they were, the gradients of the convolution itself are the library's.
+  const bool own_forward = native && (force || input.size(1) % 16 == 0);
   const bool direct_grads = !native && offset_conv_covered(input, weight, stride, padding, dilation, dk_offset_conv_direct_backward_worthwhile);
   Tensor x, w;
   return record<OffsetConvFunctionBackward>(
       {&input, &weight, &bias},
       [&] {
         x = input.contiguous(), w = weight.contiguous();
-        if (!native && !direct) return at::conv2d(x, w, bias_arg, stride, padding, dilation);
+        if (!own_forward && !direct) return at::conv2d(x, w, bias_arg, stride, padding, dilation);
         const Tensor b = bias.defined() ? bias.contiguous() : at::zeros({w.size(0)}, x.options());
         const int64_t st = stride[0];
         Tensor res = at::empty({x.size(0), w.size(0), (x.size(2) - 1) / st + 1, (x.size(3) - 1) / st + 1}, x.options());

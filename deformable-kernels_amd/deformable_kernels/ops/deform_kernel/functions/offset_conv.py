@@ -3,8 +3,8 @@
 
 ``offset_conv(input, weight, bias, stride, padding, dilation)`` returns what
 ``torch.nn.functional.conv2d`` returns.  For float32, float16 and bfloat16 GPU tensors (all of one dtype; fp32
-sums, results rounded once) with padding 1, dilation 1, input channels a multiple of 16 (16-bit tensors: any number),
-18 output channels or at most 16, on planes 7, 14, 28, 56 or 112 wide (stride 2: input planes 14 to 112 wide) it runs
+sums, results rounded once) with padding 1, dilation 1, input channels a multiple of 16 (16-bit tensors: any number,
+with the forward on the framework's routine unless ``force=True``), 18 output channels or at most 16, on planes 7, 14, 28, 56 or 112 wide (stride 2: input planes 14 to 112 wide) it runs
 
   * the forward and the input gradient on the library's shift-GEMM kernels on the 16-bit matrix instructions:
     float16 / bfloat16 elements as they are (exact products), float32 elements as bfloat16 (hi, lo) pairs
@@ -15,8 +15,8 @@ sums, results rounded once) with padding 1, dilation 1, input channels a multipl
     reduction over (N, H, W) takes 60-230 us on the large planes),
   * of these shapes, most of those with too few images to fill the GPU that way (up to 2 M output pixels times input
     channels, at stride 2 0.6 M for the gradients; the queries ``dk_offset_conv_direct_worthwhile`` and
-    ``dk_offset_conv_direct_backward_worthwhile`` tell), and 16-bit tensors on any other plane up to 0.6 M (the gradients at
-    stride 2 0.37 M): one fp32 vector-unit kernel per pass (``csrc/dk_offset_direct.hip``),
+    ``dk_offset_conv_direct_backward_worthwhile`` tell), and the gradients of 16-bit tensors with other channel counts and on other
+    planes up to 0.6 M (stride 2 0.37 M): one fp32 vector-unit kernel per pass (``csrc/dk_offset_direct.hip``),
   * everything else -- other shapes, and passes the library reports as covered
     but not worthwhile (the float32 input gradient with fewer than 64 channels or
     on 7 x 7 planes; few images of many channels) unless ``force=True`` -- on the framework's convolution routines.

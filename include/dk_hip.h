@@ -386,8 +386,9 @@ int dk_offset_conv_backward_input(const dk_offset_conv_desc *desc, const void *o
 /* The same convolution and its input and weight gradients on few images: up to 18 output channels, any other size whose
  * tensors hold less than 2^28 elements, stride 1 or 2 (output ((h - 1) / s + 1) x ((w - 1) / s + 1)), fp32 products and
  * sums for every dtype, no workspace, one launch each.  dk_offset_conv_direct_worthwhile(): 1 where the forward is
- * expected to beat both the kernels above and the library convolution (too few images for dk_offset_conv_worthwhile(), or a
- * plane that the kernels above do not cover, 16-bit tensors of up to 600000 channels times pixels); dk_offset_conv_direct_backward_worthwhile(): the two gradients. */
+ * expected to beat both the kernels above and the library convolution (covered by dk_offset_conv_supported(), channels in
+ * sixteens, too few images for dk_offset_conv_worthwhile()); dk_offset_conv_direct_backward_worthwhile(): the two gradients, also
+ * of 16-bit tensors with other channel counts and on other planes, up to 600000 channels times pixels. */
 int dk_offset_conv_direct_backward_worthwhile(const dk_offset_conv_desc *desc);
 int dk_offset_conv_direct_worthwhile(const dk_offset_conv_desc *desc);
 int dk_offset_conv_direct_forward(const dk_offset_conv_desc *desc, const void *input, const void *weight,
