@@ -261,7 +261,8 @@ __global__ __launch_bounds__(kW16Block, 2) void offset_wgrad16_kernel(int batch,
 // gW[o][c][t] = sum over parts of partial[part][chunk(c)][t][block(o)][...].
 // D[row 4 (l / 16) + r][column l % 16] of a block sits at entry 4 l + r: row = o % 16, column = c % 16.
 // A wave takes every sixteenth part of 64 elements, the waves' sums are added in order.  (One thread per element: with few
-// channels some twenty workgroups, each a chain of up to 256 loads, 27 channels of 69 x 80 x 14 26 us.)
+// channels some twenty workgroups, each a chain of up to 256 loads, 27 channels of 69 x 80 x 14 26 us, 11 here;
+// 192 channels of 28 x 28 7.3 and 6.9.)
 constexpr int kW16RedWaves = 16;
 template <typename T>
 __global__ __launch_bounds__(64 * kW16RedWaves) void offset_wgrad16_reduce_kernel(const float* __restrict__ partial, int parts,
