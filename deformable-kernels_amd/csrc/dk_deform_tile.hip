@@ -486,7 +486,7 @@ __global__ __launch_bounds__(1024) void deform_reduce_jobs_kernel(ReduceJobs<T> 
   const int e = threadIdx.x & 15, row = threadIdx.x >> 4;
   for (int k = 0; k < 3; ++k) {
     const ReduceJob<T> j = wide ? jobs.wide[k] : jobs.tile[k];
-    if (j.count >= kTlManyElements && j.count % 4 == 0) {
+    if (j.count >= kTlManyElements && j.count % 4 == 0 && reinterpret_cast<size_t>(j.partial) % 16 == 0) {
       for (long at = ((long)blockIdx.x * 1024 + threadIdx.x) * 4; at < j.count; at += (long)gridDim.x * 4096) {
         tl_f4 s = {0.f, 0.f, 0.f, 0.f};
         for (int p0 = 0; p0 < j.parts; p0 += PU / 2) {
@@ -574,8 +574,8 @@ TilePlan tile_plan(const Geo& g, bool rotation) {
   return m;
 }
 
-// Workspace: the tiles' boxes, the windows of the workgroups that made them and the word that says whose the call is; then the partial sums, of the offset, rotation and
-// filter gradient or, if the choice falls on the separate kernels, theirs.
+// Workspace: the tiles' boxes, the windows of the workgroups that made them and the word that says whose the call is; then the
+// partial sums, of the offset, rotation and filter gradient or, if the choice falls on the separate kernels, theirs.
 constexpr int kTlBoxGrid = 256;
 struct TileWorkspace {
   size_t boxes, off, rot, filter;  // bytes; floats
