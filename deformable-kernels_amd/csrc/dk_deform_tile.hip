@@ -541,6 +541,7 @@ TilePlan tile_plan(const Geo& g, bool rotation) {
   if (!(g.scope_h == 4 && g.scope_w == 4) && !(g.scope_h == 3 && g.scope_w == 3)) return m;
   const long out_plane = (long)g.out_h * g.out_w, in_plane = (long)g.in_h * g.in_w;
   // 32-bit byte offsets in the 18 offset planes, and in a block's planes of 16 channels
+  if (g.in_h >= 1 << 15 || g.in_w >= 1 << 16) return m;  // Tap::at: row and column of a corner, up to the sides, in one word
   if (18 * out_plane * 4 >= (1L << 31) || 16L * g.groups * std::max(out_plane, in_plane) * 4 >= (1L << 31)) return m;
   if ((long)g.channel * g.scope_h * g.scope_w * 4 >= (1L << 31)) return m;
   const int cpg = g.channel / g.groups, nblk = ceil_div(cpg, kTlCh);

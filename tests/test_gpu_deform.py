@@ -708,3 +708,21 @@ def test_one_pass_non_finite_output_gradient_reaches_its_pixel_and_channel_only(
         assert bad[1, :, 20, 21].all() and int(bad.sum()) == 18
     bad = ~torch.isfinite(gw)
     assert bad[17].any() and int(bad.sum()) == int(bad[17].sum())
+
+
+@pytest.mark.parametrize("plain", [False, True])
+@pytest.mark.parametrize("plane", [(3, 65534), (3, 65535), (3, 65536), (3, 66000), (32766, 3), (32767, 3), (32768, 3), (33100, 3)])
+def test_coordinate_and_filter_gradients_of_planes_with_a_long_side(plane, plain):
+    """Around the sides up to which the one-pass form holds a corner's row and column in one word."""
+    from deformable_kernels.ops.deform_kernel.functions import deform_sample_depthwise
+    x, wt, rot, off, gout, cfg = make_deform(1, 9, *plane, 3, (4, 4), 1, 1, 1, 1, 0.0 if plain else 0.5, 1.0, seed=24)
+    # coordinates that float32 holds to the last bit, 2^-7 above 2^16: none of the 10^6 samples rounds over a cell's border
+    off, rot = (off * 64).round() / 64, (rot * 64).round() / 64
+    leaves = [t.to("cuda:0").requires_grad_() for t in ((off, wt) if plain else (off, rot, wt))]
+    offs, rots, wts = (leaves[0], None, leaves[1]) if plain else leaves
+    out = deform_sample_depthwise(x.to("cuda:0"), offs, rots, wts, cfg["kernel_size"], cfg["stride"], cfg["padding"], cfg["dilation"], 1)
+    got = torch.autograd.grad(out, leaves, gout.to("cuda:0"))
+    want = orc.deform_sample_depthwise_backward(*[t.double().numpy() for t in (gout, x, off, rot, wt)], **cfg)
+    # sums of at most 2 * 10^6 products of three factors in float32, in blocks
+    for g, w in zip(got, (want[1], want[3]) if plain else want[1:]):
+        assert rel_err(g.cpu(), w) < 2e-5
