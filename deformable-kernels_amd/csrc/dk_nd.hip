@@ -195,12 +195,13 @@ __global__ __launch_bounds__(kBlock) void nd_grad_coord_kernel(NdGeo g, const T*
 // ---------------------------------------------------------------------------
 
 // in [rows][cols] -> out [cols][rows], converting A -> B; 32 x 32 tiles through LDS.  zero != nullptr: as many floats, cleared
-// beside it (a launch less)
+// beside it (a launch less).  One workgroup per tile, numbered along the columns first: in a two-dimensional grid a volume of more
+// than 2.1 million cells passes the 65535 workgroups of its second dimension.
 template <typename A, typename B>
 __global__ __launch_bounds__(256) void nd_transpose_kernel(const A* __restrict__ in, B* __restrict__ out, float* __restrict__ zero,
-                                                           long rows, long cols) {
+                                                           long rows, long cols, unsigned col_tiles) {
   __shared__ float tile[32][33];
-  const long r0 = (long)blockIdx.y * 32, c0 = (long)blockIdx.x * 32;
+  const long r0 = (long)(blockIdx.x / col_tiles) * 32, c0 = (long)(blockIdx.x % col_tiles) * 32;
   const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
 #pragma unroll
   for (int k = 0; k < 32; k += 8) {
@@ -1739,8 +1740,8 @@ int chunks_per_wave(const NdGeo& g) {
 
 template <typename A, typename B>
 void transpose(const A* in, B* out, long rows, long cols, hipStream_t stream, float* zero = nullptr) {
-  const dim3 grid((unsigned)((cols + 31) / 32), (unsigned)((rows + 31) / 32));
-  nd_transpose_kernel<A, B><<<grid, 256, 0, stream>>>(in, out, zero, rows, cols);
+  const unsigned col_tiles = (unsigned)((cols + 31) / 32);
+  nd_transpose_kernel<A, B><<<col_tiles * (unsigned)((rows + 31) / 32), 256, 0, stream>>>(in, out, zero, rows, cols, col_tiles);
 }
 
 }  // namespace

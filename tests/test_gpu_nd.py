@@ -274,3 +274,11 @@ def test_non_finite_output_gradient_stays_with_its_point_and_channel():
     got = _run(data, coord, gout)[1]
     bad = ~torch.isfinite(got)
     assert bad[2, 3:5, 4:6].all() and int(bad.sum()) == 4
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_volume_of_more_cells_than_32_times_65535(dtype):
+    """Both transposes: their tiles along the cells outnumber the second dimension of a grid."""
+    data, coord, gout = _inputs((130, 130, 130), 16, 4500, seed=52, dtype=dtype)
+    for a, w in zip(_run(data, coord, gout), _oracle(data, coord, gout, np.float64)):
+        assert rel_err(a.float(), w) < (1e-5 if dtype == torch.float32 else 8e-3)  # bfloat16: the results' rounding, 2^-8
