@@ -576,7 +576,7 @@ __global__ __launch_bounds__(kBlock) void nd_small_grad_coord_kernel(NdGeo g, co
 
 // ---------------------------------------------------------------------------
 // channel-last path of narrow rows: a wave holds 64 >> lg points, 1 << lg lanes of each along the channels (the least power
-// of two that holds them, at most 64), and every lane derives its point's corners itself.
+// of two that holds them, at most 64), and every lane derives its point's corners itself.  (One channel: the volume as it lies.)
 // ---------------------------------------------------------------------------
 template <int ND>
 struct RowCorners {
@@ -1746,26 +1746,46 @@ void transpose(const A* in, B* out, long rows, long cols, hipStream_t stream, fl
 
 }  // namespace
 
+static long nd_cells(const dk_nd_desc& d) {
+  long cells = 1;
+  for (int i = 0; i < d.dims; ++i) cells *= d.shape[i];
+  return cells;
+}
+
 // Few points on a tiny volume: the direct kernels and the one-launch grad data (nd_small_grad_data_kernel).
 bool nd_small(const dk_nd_desc& d) {
   if (d.dtype == DK_F64 || d.dims > kClMaxDims || path_disabled(kNoNdSmall)) return false;
-  long prod = 1;
-  for (int i = 0; i < d.dims; ++i) prod *= d.shape[i];
   // (a workgroup of the grad data walks over all points: 8000 points x 16 channels of 7 x 7 float32 88 us a pass, 40 with the
   // sums of nd_grad_data_lds_kernel; 17000 x 4 of 50 160 / 39)
-  return prod <= kSmallMaxCells && d.batch > 0 && d.batch * d.channel <= (1L << 20) && (d.batch <= 4096 || path_disabled(kNoNdRows));
+  return nd_cells(d) <= kSmallMaxCells && d.batch > 0 && d.batch * d.channel <= (1L << 20) && (d.batch <= 4096 || path_disabled(kNoNdRows));
 }
 
 // The channel-last path pays for a transpose of `data`; it is taken for 1..3 dimensions in
-// fp32 / fp16 / bf16 when there are enough (point, channel) pairs to amortise it (5500 points x 12 channels of 30 x 20: 55 us a
-// pass on the planar volume, 42 here).
+// fp32 / fp16 / bf16 when there are enough (point, channel) pairs to amortise it.
+//
+// Below 16 channels the planar volume serves many calls faster: its cost goes with the corners that the points read and add to
+// (corners x channels), the copies' with the volume.  us a pass, planar / here, float32, by channels:
+//   copies of a volume larger than what is read of it: 61250 points x 3 of 1400 x 1400 83 / 154, 122500 x 3 148 / 173, 245000 x 3
+//   278 / 213, 31250 x 3 of 100^3 78 / 102, 62500 x 3 138 / 122; 122500 x 2 of 1400 x 1400 115 / 161, 245000 x 2 212 / 196; 61250 x 8 177 / 172,
+//   61250 x 12 258 / 235: corners x channels from 1.5 times the cells on;
+//   little work, where the launches count (six instead of four): 8000 x 15 of 60 x 60 (480 k) 56 / 63, 8000 x 15 of 8^3 (960 k) 57 / 62,
+//   65000 x 2 of 60 x 60 (520 k) 57 / 63, 16000 x 15 of 60 x 60 (960 k) 66 / 62, 65000 x 4 (1.0 M) 82 / 63;
+//   additions of many points to the same cells, one by one: 16000 x 8 of 400 (80 corners a cell) 55 / 62, 32000 x 4 (160) 62 / 62,
+//   32000 x 8 (160) 69 / 63, 16000 x 8 of 100 (320) 88 / 62, 130000 x 4 of 30 x 20 (870) 217 / 62.
+// One channel is in this layout as it is and is never copied.
 bool nd_use_channel_last(const dk_nd_desc& d) {
   if (d.dtype == DK_F64 || d.dims > kClMaxDims || nd_small(d)) return false;
-  long prod = 1;
-  for (int i = 0; i < d.dims; ++i) prod *= d.shape[i];
-  if (prod > 2147483647L / 4) return false;  // corner offsets are kept as 32-bit element counts
-  return d.batch * d.channel >= 65536 && (d.channel >= 16 || !path_disabled(kNoNdRows));
+  const long cells = nd_cells(d);
+  if (cells > 2147483647L / 4) return false;  // corner offsets are kept as 32-bit element counts
+  if (d.batch * d.channel < 65536) return false;
+  if (d.channel >= 16) return true;
+  if (path_disabled(kNoNdRows)) return false;
+  const long corners = d.batch << d.dims, all = corners * d.channel;
+  return d.channel == 1 || corners >= 200 * cells || (all >= 900000 && 2 * all >= 3 * cells);
 }
+
+// ... by way of copies of the volume
+static bool nd_copies(const dk_nd_desc& d) { return d.channel > 1 && nd_use_channel_last(d); }
 
 namespace {
 
@@ -1791,8 +1811,7 @@ struct LdsSums {
 LdsSums lds_sums(const dk_nd_desc& d) {
   LdsSums m{};
   if (!nd_use_channel_last(d) || path_disabled(kNoNdRows)) return m;
-  long cells = 1;
-  for (int i = 0; i < d.dims; ++i) cells *= d.shape[i];
+  const long cells = nd_cells(d);
   const long adds = d.batch << d.dims;  // of a channel
   // How many additions a sum must receive, and how often the points may be walked over.  Float atomics on memory take a row of 16
   // channels and more at once, fewer mostly one by one.  us a pass with the atomics / the sums in LDS: 60000 points x 40
@@ -1867,7 +1886,7 @@ size_t nd_sort_workspace(const dk_nd_desc& d) {
 }
 
 size_t nd_data_cl_workspace(const dk_nd_desc& d) {
-  if (!nd_use_channel_last(d)) return 0;
+  if (!nd_copies(d)) return 0;
   size_t n = (size_t)d.channel;
   for (int i = 0; i < d.dims; ++i) n *= (size_t)d.shape[i];
   return round256(n * elem_size(d.dtype)) + nd_sort_workspace(d);
@@ -1927,8 +1946,11 @@ void nd_forward(const dk_nd_desc& d, const T* data, const T* coord, T* out, void
   const NdGeo g = make_geo(d);
   if constexpr (!std::is_same<T, double>::value) {
     if (nd_use_channel_last(d)) {
-      T* data_cl = static_cast<T*>(ws);
-      transpose<T, T>(data, data_cl, g.channel, g.prod_shape, stream);
+      const T* data_cl = data;
+      if (nd_copies(d)) {
+        data_cl = static_cast<T*>(ws);
+        transpose<T, T>(data, static_cast<T*>(ws), g.channel, g.prod_shape, stream);
+      }
       if (const int bins = nd_bins(d)) {
         if (!order) order = sort_points<T>(g, coord, bins, static_cast<char*>(ws) + round256(data_bytes(d) * sizeof(T)), stream);
         if constexpr (std::is_same<T, float>::value) {
@@ -1960,13 +1982,10 @@ size_t nd_grad_data_workspace(const dk_nd_desc& d) {
   if (nd_small(d)) return 0;
   size_t n = (size_t)d.channel;
   for (int i = 0; i < d.dims; ++i) n *= (size_t)d.shape[i];
-  if (nd_use_channel_last(d)) {
-    const LdsSums m = lds_sums(d);
-    // fp32 channel-last accumulation image; or copies of the sums, without a sort
-    return std::max(round256(n * sizeof(float)) + nd_sort_workspace(d), (size_t)m.parts * n * sizeof(float));
-  }
-  if (d.dtype == DK_F16 || d.dtype == DK_BF16) return n * sizeof(float);
-  return 0;
+  const size_t sums = (size_t)lds_sums(d).parts * n * sizeof(float);
+  // fp32 channel-last accumulation image; or copies of the sums, without a sort
+  if (nd_copies(d)) return std::max(round256(n * sizeof(float)) + nd_sort_workspace(d), sums);
+  return std::max(d.dtype == DK_F16 || d.dtype == DK_BF16 ? n * sizeof(float) : 0, sums);
 }
 
 template <typename T>
@@ -2013,7 +2032,7 @@ void nd_grad_data(const dk_nd_desc& d, const T* gout, const T* coord, T* gdata, 
         return;
       }
     }
-    if (nd_use_channel_last(d)) {
+    if (nd_copies(d)) {
       float* acc = static_cast<float*>(ws);
       nd_fill_zero_kernel<float><<<grid_for(n_data), kBlock, 0, stream>>>(acc, n_data);
       if (const int bins = nd_bins(d)) {
@@ -2060,8 +2079,11 @@ void nd_grad_coord(const dk_nd_desc& d, const T* gout, const T* data, const T* c
       return;
     }
     if (nd_use_channel_last(d)) {
-      T* data_cl = static_cast<T*>(ws);
-      transpose<T, T>(data, data_cl, g.channel, g.prod_shape, stream);
+      const T* data_cl = data;
+      if (nd_copies(d)) {
+        data_cl = static_cast<T*>(ws);
+        transpose<T, T>(data, static_cast<T*>(ws), g.channel, g.prod_shape, stream);
+      }
       if (const int bins = nd_bins(d)) {
         if (!order) order = sort_points<T>(g, coord, bins, static_cast<char*>(ws) + round256(data_bytes(d) * sizeof(T)), stream);
         if constexpr (std::is_same<T, float>::value) {

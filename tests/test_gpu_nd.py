@@ -282,3 +282,46 @@ def test_volume_of_more_cells_than_32_times_65535(dtype):
     data, coord, gout = _inputs((130, 130, 130), 16, 4500, seed=52, dtype=dtype)
     for a, w in zip(_run(data, coord, gout), _oracle(data, coord, gout, np.float64)):
         assert rel_err(a.float(), w) < (1e-5 if dtype == torch.float32 else 8e-3)  # bfloat16: the results' rounding, 2^-8
+
+
+def _workspaces(dtype, C, shape, B):
+    import ctypes
+    from deformable_kernels.ops.deform_kernel import _lib
+    L = _lib.lib()
+    desc = _lib.NdDesc(B, C, len(shape), (ctypes.c_int32 * 8)(*shape, *([1] * (8 - len(shape)))), dtype)
+    return [getattr(L, f"dk_nd_linear_sample_{k}_workspace")(ctypes.byref(desc)) for k in ("forward", "backward_data", "backward_coord")]
+
+
+@pytest.mark.parametrize("shape,C,B,lo,hi,route", [
+    ((20, 31), 14, 36000, -1.5, 32.0, "copied"),      # 1.5 * 10^5 corners of 620 cells
+    ((2000, 1500), 3, 30000, -1.0, 1500.0, "planar"),  # a volume that the points hardly read
+    ((80, 80, 80), 5, 30000, -1.0, 80.0, "copied"),   # 1.2 * 10^6 corners and channels, 512000 cells; float atomics
+    ((80, 80, 80), 5, 20000, -1.0, 80.0, "planar"),   # 0.8 * 10^6
+    ((100, 100, 100), 2, 90000, -1.0, 100.0, "planar"),   # 1.44 * 10^6 of 10^6 cells
+    ((100, 100, 100), 2, 94000, -1.0, 100.0, "copied"),   # 1.504 * 10^6
+    ((64, 64, 64), 1, 65536, -1.0, 64.0, "in place"),  # one channel: no sums in LDS
+    ((64, 64, 64), 1, 140000, -1.0, 64.0, "in place"),  # ... with them
+    ((1, 70000), 1, 66000, -1.0, 70000.0, "in place"),
+])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_few_channels_of_volumes_larger_than_what_is_read(shape, C, B, lo, hi, route, dtype):
+    from deformable_kernels.ops.deform_kernel import _lib
+    ws = _workspaces(_lib.DK_F32 if dtype == torch.float32 else _lib.DK_F16, C, shape, B)
+    assert (ws[0] > 0) == (ws[2] > 0) == (route == "copied")
+    if dtype == torch.float16 and max(shape) > 2000:
+        pytest.skip("coordinates that float16 does not hold")
+    g = torch.Generator().manual_seed(53)
+    data = torch.randn(C, *shape, generator=g).to(dtype)
+    coord = (torch.rand(B, len(shape), generator=g) * (hi - lo) + lo).to(dtype)
+    gout = torch.randn(B, C, generator=g).to(dtype)
+    for a, w in zip(_run(data, coord, gout), _oracle(data, coord, gout, np.float64)):
+        assert rel_err(a.float(), w) < (1e-5 if dtype == torch.float32 else 1e-3)  # 16-bit: the results' rounding, 2^-11
+
+
+def test_non_finite_output_gradient_stays_with_its_point_and_channel_in_sums_of_many_points():
+    data, coord, gout = _inputs((20, 31), 6, 40000, seed=51, dtype=torch.float32)
+    coord[0], coord[1] = torch.tensor([3.25, 4.5]), torch.tensor([-1.0, 4.0])
+    gout[0, 2], gout[1, 3] = float("inf"), float("nan")
+    got = _run(data, coord, gout)[1]
+    bad = ~torch.isfinite(got)
+    assert bad[2, 3:5, 4:6].all() and int(bad.sum()) == 4

@@ -149,6 +149,22 @@ def test_c_abi_rejects_bad_arguments_before_any_launch():
     assert b"workspace" in L.dk_status_string(-5)
 
 
+def test_workspaces_of_few_channels_on_large_volumes():
+    """30000 points read corners of 3 x 256^3 cells and copy no volume; one channel lies as the kernels want it."""
+    import ctypes
+    from deformable_kernels.ops.deform_kernel import _lib
+    L = _lib.lib()
+
+    def sizes(points, channels, *shape):
+        desc = _lib.NdDesc(points, channels, len(shape), (ctypes.c_int32 * 8)(*shape, *([1] * (8 - len(shape)))), _lib.DK_F32)
+        return [getattr(L, f"dk_nd_linear_sample_{k}_workspace")(ctypes.byref(desc)) for k in ("forward", "backward_data", "backward_coord")]
+
+    assert sizes(30000, 3, 256, 256, 256) == [0, 0, 0]
+    assert sizes(100000, 1, 256, 256, 256) == [0, 0, 0]
+    assert sizes(1000000, 1, 64, 64)[::2] == [0, 0]
+    assert all(n >= 3 * 64 * 64 * 4 for n in sizes(1000000, 3, 64, 64))
+
+
 def test_native_self_tests_of_the_c_abi_and_the_oracle():
     """The C driver of the C ABI's argument handling (every rejection path and the workspace arithmetic
     over a sweep of geometries; all answered on the host) against the library as built, and the oracle's
