@@ -1135,7 +1135,7 @@ static int check_nd(const dk_nd_desc* d) {
 
 size_t dk_nd_linear_sample_forward_workspace(const dk_nd_desc* desc) {
   if (check_nd(desc) != DK_OK) return 0;
-  return nd_data_cl_workspace(*desc);
+  return nd_forward_workspace(*desc);
 }
 
 size_t dk_nd_linear_sample_order_bytes(const dk_nd_desc* desc) {
@@ -1168,7 +1168,7 @@ int dk_nd_linear_sample_forward(const dk_nd_desc* desc, const void* data, const 
   const int rc = check_nd(desc);
   if (rc != DK_OK) return rc;
   if (!data || !coord || !output) return DK_ERR_NULL_POINTER;
-  const size_t need = nd_data_cl_workspace(*desc);
+  const size_t need = nd_forward_workspace(*desc);
   if (need && (!workspace || workspace_bytes < need)) return DK_ERR_WORKSPACE;
   if (desc->batch == 0) return DK_OK;
   hipStream_t s = static_cast<hipStream_t>(stream);

@@ -6,6 +6,7 @@
 namespace dk {
 
 // bytes of workspace for the channel-last copy of `data` (0 when the direct path is used)
+size_t nd_forward_workspace(const dk_nd_desc& d);
 size_t nd_data_cl_workspace(const dk_nd_desc& d);
 template <typename T>
 void nd_forward(const dk_nd_desc& d, const T* data, const T* coord, T* out, void* ws, const int* order,

@@ -1787,6 +1787,15 @@ bool nd_use_channel_last(const dk_nd_desc& d) {
 // ... by way of copies of the volume
 static bool nd_copies(const dk_nd_desc& d) { return d.channel > 1 && nd_use_channel_last(d); }
 
+// The forward reads a corner where the gradients also add to it, so its copy needs more of them below 16 channels.  us, planar / copied:
+// 61250 points x 3 of 1400 x 1400 14 / 41, 245000 x 3 (2.9 M corners times channels, 1.5 per cell) 49 / 51, 490000 x 3 89 / 60, 125000 x 3 of 100^3 (3.0 M,
+// 3 per cell) 40 / 37; 250000 x 2 (4 per cell) 39 / 42, 500000 x 2 73 / 53; 31250 x 8 of 50^3 (2.0 M) 16 / 18, 62500 x 8 24 / 18.
+static bool nd_forward_channel_last(const dk_nd_desc& d) {
+  if (!nd_use_channel_last(d) || !nd_copies(d) || d.channel >= 16) return nd_use_channel_last(d);
+  const long all = (d.batch << d.dims) * d.channel;
+  return all >= 2500000 && 2 * all >= 5 * nd_cells(d);
+}
+
 namespace {
 
 // log2 of a point's lanes in the kernels of narrow rows, or -1 where a wave per point serves the call.  Up to 32 channels, us
@@ -1885,6 +1894,8 @@ size_t nd_sort_workspace(const dk_nd_desc& d) {
   return 4 * n4 + round256((table + table / kScanTile + 1) * sizeof(unsigned));
 }
 
+size_t nd_forward_workspace(const dk_nd_desc& d) { return nd_forward_channel_last(d) ? nd_data_cl_workspace(d) : 0; }
+
 size_t nd_data_cl_workspace(const dk_nd_desc& d) {
   if (!nd_copies(d)) return 0;
   size_t n = (size_t)d.channel;
@@ -1945,7 +1956,7 @@ void nd_forward(const dk_nd_desc& d, const T* data, const T* coord, T* out, void
                 hipStream_t stream) {
   const NdGeo g = make_geo(d);
   if constexpr (!std::is_same<T, double>::value) {
-    if (nd_use_channel_last(d)) {
+    if (nd_forward_channel_last(d)) {
       const T* data_cl = data;
       if (nd_copies(d)) {
         data_cl = static_cast<T*>(ws);

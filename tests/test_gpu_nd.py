@@ -293,12 +293,15 @@ def _workspaces(dtype, C, shape, B):
 
 
 @pytest.mark.parametrize("shape,C,B,lo,hi,route", [
-    ((20, 31), 14, 36000, -1.5, 32.0, "copied"),      # 1.5 * 10^5 corners of 620 cells
+    ((20, 31), 14, 36000, -1.5, 32.0, "gradients"),   # 2.0 * 10^6 corners times channels of 620 cells
+    ((20, 31), 14, 45000, -1.5, 32.0, "copied"),      # 2.52 * 10^6: the forward as well
     ((2000, 1500), 3, 30000, -1.0, 1500.0, "planar"),  # a volume that the points hardly read
-    ((80, 80, 80), 5, 30000, -1.0, 80.0, "copied"),   # 1.2 * 10^6 corners and channels, 512000 cells; float atomics
+    ((80, 80, 80), 5, 30000, -1.0, 80.0, "gradients"),  # 1.2 * 10^6, 512000 cells; float atomics
+    ((80, 80, 80), 5, 62500, -1.0, 80.0, "copied"),   # 2.5 * 10^6
     ((80, 80, 80), 5, 20000, -1.0, 80.0, "planar"),   # 0.8 * 10^6
     ((100, 100, 100), 2, 90000, -1.0, 100.0, "planar"),   # 1.44 * 10^6 of 10^6 cells
-    ((100, 100, 100), 2, 94000, -1.0, 100.0, "copied"),   # 1.504 * 10^6
+    ((100, 100, 100), 2, 94000, -1.0, 100.0, "gradients"),   # 1.504 * 10^6
+    ((100, 100, 100), 2, 157000, -1.0, 100.0, "copied"),   # 2.512 * 10^6, 2.5 per cell
     ((64, 64, 64), 1, 65536, -1.0, 64.0, "in place"),  # one channel: no sums in LDS
     ((64, 64, 64), 1, 140000, -1.0, 64.0, "in place"),  # ... with them
     ((1, 70000), 1, 66000, -1.0, 70000.0, "in place"),
@@ -307,7 +310,7 @@ def _workspaces(dtype, C, shape, B):
 def test_few_channels_of_volumes_larger_than_what_is_read(shape, C, B, lo, hi, route, dtype):
     from deformable_kernels.ops.deform_kernel import _lib
     ws = _workspaces(_lib.DK_F32 if dtype == torch.float32 else _lib.DK_F16, C, shape, B)
-    assert (ws[0] > 0) == (ws[2] > 0) == (route == "copied")
+    assert (ws[2] > 0) == (route in ("copied", "gradients")) and (ws[0] > 0) == (route == "copied")
     if dtype == torch.float16 and max(shape) > 2000:
         pytest.skip("coordinates that float16 does not hold")
     g = torch.Generator().manual_seed(53)

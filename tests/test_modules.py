@@ -162,6 +162,8 @@ def test_workspaces_of_few_channels_on_large_volumes():
     assert sizes(30000, 3, 256, 256, 256) == [0, 0, 0]
     assert sizes(100000, 1, 256, 256, 256) == [0, 0, 0]
     assert sizes(1000000, 1, 64, 64)[::2] == [0, 0]
+    # the gradients' copies are worth it before the forward's
+    assert sizes(245000, 3, 1400, 1400)[0] == 0 < sizes(245000, 3, 1400, 1400)[2]
     assert all(n >= 3 * 64 * 64 * 4 for n in sizes(1000000, 3, 64, 64))
 
 
