@@ -328,3 +328,31 @@ def test_non_finite_output_gradient_stays_with_its_point_and_channel_in_sums_of_
     got = _run(data, coord, gout)[1]
     bad = ~torch.isfinite(got)
     assert bad[2, 3:5, 4:6].all() and int(bad.sum()) == 4
+
+
+def test_more_points_than_threads_of_a_launch():
+    """One channel, 2^32 + 77 points: the rows' kernels walk over them.  Every 2^16 points repeat, so the results do."""
+    from deformable_kernels.ops.deform_kernel.functions import nd_linear_sample
+    if torch.cuda.mem_get_info()[0] < 64 << 30:
+        pytest.skip("needs 35 GB of GPU memory")
+    n, period, dev = (1 << 32) + 77, 1 << 16, torch.device("cuda:0")
+    g = torch.Generator().manual_seed(54)
+    data, one = torch.randn(1, 90, generator=g).half().to(dev), (torch.rand(period, 1, generator=g) * 91 - 1).half().to(dev)
+    gone = torch.randn(period, 1, generator=g).half().to(dev)
+
+    def spread(t):
+        full = torch.empty(n, 1, dtype=t.dtype, device=dev)
+        full[:1 << 32].view(-1, period).copy_(t.view(1, period).expand(1 << 16, period))
+        full[1 << 32:] = t[:77]
+        return full
+
+    want_c = one.clone().requires_grad_()
+    want = nd_linear_sample(data, want_c)
+    want_g, = torch.autograd.grad(want, want_c, gone)
+    coord = spread(one).requires_grad_()
+    out = nd_linear_sample(data, coord)
+    for full, part in ((out, want), (torch.autograd.grad(out, coord, spread(gone))[0], want_g)):
+        full, part = full.detach(), part.detach()
+        assert torch.equal(full[1 << 32:], part[:77])
+        for rows in full[:1 << 32].view(-1, period).split(1 << 13):
+            assert bool((rows == part.view(1, period)).all())
