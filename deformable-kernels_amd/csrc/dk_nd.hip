@@ -1756,9 +1756,13 @@ static long nd_cells(const dk_nd_desc& d) {
 // Few points on a tiny volume: the direct kernels and the one-launch grad data (nd_small_grad_data_kernel).
 bool nd_small(const dk_nd_desc& d) {
   if (d.dtype == DK_F64 || d.dims > kClMaxDims || path_disabled(kNoNdSmall)) return false;
-  // (a workgroup of the grad data walks over all points: 8000 points x 16 channels of 7 x 7 float32 88 us a pass, 40 with the
-  // sums of nd_grad_data_lds_kernel; 17000 x 4 of 50 160 / 39)
-  return nd_cells(d) <= kSmallMaxCells && d.batch > 0 && d.batch * d.channel <= (1L << 20) && (d.batch <= 4096 || path_disabled(kNoNdRows));
+  const long cells = nd_cells(d);
+  if (cells > kSmallMaxCells || d.batch <= 0 || d.batch * d.channel > 1L << 20) return false;
+  // A workgroup of the grad data walks over all points, in rows of 16 cells per tile: up to about 50 us of that, and 4096 points at
+  // least; beyond, however few the channels, the sums of nd_grad_data_lds_kernel.  us a pass, here / there: 16 channels of 60
+  // cells 5000 points 54 / 62 (six launches instead of three), 20000 188 / 62; 15 of 30 cells 8000 54 / 62, 16000 97 / 62; 15 of 7 x 7 4097 54 / 62, 8000
+  // 88 / 63; 15 of 4^3 4097 63 / 62, 8000 109 / 63; 1 of 4^3 30000 377 / 64.
+  return d.batch * (7 * ((cells + 15) / 16) + 5 * d.dims + 3) <= 200000 || path_disabled(kNoNdRows);
 }
 
 // The channel-last path pays for a transpose of `data`; it is taken for 1..3 dimensions in
@@ -1778,9 +1782,11 @@ bool nd_use_channel_last(const dk_nd_desc& d) {
   if (d.dtype == DK_F64 || d.dims > kClMaxDims || nd_small(d)) return false;
   const long cells = nd_cells(d);
   if (cells > 2147483647L / 4) return false;  // corner offsets are kept as 32-bit element counts
+  const bool rows = !path_disabled(kNoNdRows);
+  if (rows && cells <= kSmallMaxCells && d.batch > 4096) return true;  // too many points for nd_small()
   if (d.batch * d.channel < 65536) return false;
   if (d.channel >= 16) return true;
-  if (path_disabled(kNoNdRows)) return false;
+  if (!rows) return false;
   const long corners = d.batch << d.dims, all = corners * d.channel;
   return d.channel == 1 || corners >= 200 * cells || (all >= 900000 && 2 * all >= 3 * cells);
 }

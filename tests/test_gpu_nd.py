@@ -356,3 +356,12 @@ def test_more_points_than_threads_of_a_launch():
         assert torch.equal(full[1 << 32:], part[:77])
         for rows in full[:1 << 32].view(-1, period).split(1 << 13):
             assert bool((rows == part.view(1, period)).all())
+
+
+@pytest.mark.parametrize("C", [1, 3, 15, 16])
+@pytest.mark.parametrize("shape,most", [((64,), 5555), ((7, 7), 4878), ((4, 4, 4), 4347), ((30,), 9090), ((2, 3, 2), 8000)])
+def test_tiny_volumes_around_the_most_points_of_the_one_launch_gradients(shape, most, C):
+    for B in (most, most + 1):
+        data, coord, gout = _inputs(shape, C, B, seed=55, dtype=torch.float32)
+        for a, w in zip(_run(data, coord, gout), _oracle(data, coord, gout, np.float64)):
+            assert rel_err(a, w) < 1e-5

@@ -167,6 +167,25 @@ def test_workspaces_of_few_channels_on_large_volumes():
     assert all(n >= 3 * 64 * 64 * 4 for n in sizes(1000000, 3, 64, 64))
 
 
+def test_no_calls_between_the_kernels_of_few_points_and_the_sums_in_lds():
+    """Volumes of up to 64 cells: every call of more points than the one-launch gradients take has partial sums to add up."""
+    import ctypes
+    from deformable_kernels.ops.deform_kernel import _lib
+    L = _lib.lib()
+    for shape in ((1,), (30,), (64,), (5, 5), (7, 7), (8, 8), (2, 2, 2), (4, 4, 4)):
+        cells = 1
+        for s in shape:
+            cells *= s
+        for channels in (1, 3, 8, 15, 16, 100):
+            need = {}
+            for points in (1, 4096, 4500, 6000, 9000, 14000, 30000, 65536 // channels + 1, 200000):
+                desc = _lib.NdDesc(points, channels, len(shape), (ctypes.c_int32 * 8)(*shape, *([1] * (8 - len(shape)))), _lib.DK_F32)
+                need[points] = L.dk_nd_linear_sample_backward_data_workspace(ctypes.byref(desc))
+            assert need[1] == need[4096] == 0
+            assert need[14000] >= 4 * channels * cells and need[200000] >= 4 * channels * cells
+            assert [n > 0 for _, n in sorted(need.items())] == sorted(n > 0 for n in need.values()), (shape, channels, need)
+
+
 def test_native_self_tests_of_the_c_abi_and_the_oracle():
     """The C driver of the C ABI's argument handling (every rejection path and the workspace arithmetic
     over a sweep of geometries; all answered on the host) against the library as built, and the oracle's
