@@ -1878,10 +1878,25 @@ LdsSums lds_sums(const dk_nd_desc& d) {
 // the binned kernels do not apply: they pay off with several points per cell.
 int nd_bins(const dk_nd_desc& d) {
   if (!nd_use_channel_last(d) || d.channel < 16 || path_disabled(kNoNdBins)) return 0;
-  // What the sort gives the kernels that do not run on the matrix cores is less than it costs where two slices of LDS hold
-  // the volume's sums: us a pass sorted / not: 400000 points x 16 channels of 8^3 float16 194 / 144, 262000 x 250 of 90 cells
-  // bfloat16 311 / 217, 200000 x 128 of 16 x 16 195 / 182; but 300000 x 100 of 30 x 20 float32 (four slices) 192 / 253.
-  if (const LdsSums m = lds_sums(d); m.slices && m.slices * m.ranges <= 2 && !(d.dtype == DK_F32 && d.channel % 64 == 0)) return 0;
+  // Where two slices of LDS hold the volume's sums, calls that do not run on the matrix cores go unsorted up to some number of
+  // points: the sort costs 30 - 60 us, and the sorted kernels take less for each point.  us on the device, sorted / not:
+  //   16 channels, a lane each: 10^3 float32 1.2 M points 437 / 348, 20 x 30 float16 352 / 199: never sorted;
+  //   17 - 32 and more than 64, float32: 300 cells x 24 300 k 94 / 87, 600 k 138 / 141; 16 x 16 x 20 300 k 116 / 112, 600 k 176 / 194; 90 cells x 100 150 k
+  //   111 / 104, 300 k 143 / 159; 8 x 7 x 160 150 k 186 / 157, 300 k 257 / 273; in three dimensions 7^3 x 24 150 k 134 / 118, 300 k 167 / 197, 4 x 4 x 5 x 100
+  //   150 k 209 / 204, 300 k 265 / 354 (float16 the same); float16, whose sorted kernels convert more: 90 cells x 100 600 k 313 / 267, 70 x 250 300 k
+  //   343 / 256, 16 x 16 x 28 600 k 212 / 206, 1.2 M 347 / 377, 5 x 5 x 100 600 k 367 / 369;
+  //   33 - 64, a wave per point with lanes idle or one channel each: float32 200 x 40 150 k 78 / 80, 12 x 14 x 40 70 k 77 / 76, 5^3 x 40 70 k 103 / 116, 1.2 M
+  //   478 / 985; float16 200 x 40 150 k 100 / 80, 300 k 116 / 118, 7 x 9 x 48 150 k 111 / 102, 300 k 136 / 166, 5^3 x 48 70 k 99 / 119.
+  if (const LdsSums m = lds_sums(d); m.slices && m.slices * m.ranges <= 2 && !(d.dtype == DK_F32 && d.channel % 64 == 0)) {
+    const bool half = d.dtype != DK_F32, idle = d.channel > 32 && d.channel <= 64;
+    long most;
+    if (d.channel == 16) most = std::numeric_limits<long>::max();
+    else if (idle) most = half && d.dims < 3 ? 150000 : 0;
+    else if (d.dims == 3) most = 160000;
+    else if (half) most = d.dims == 1 ? std::numeric_limits<long>::max() : 520000;
+    else most = 260000;
+    if (d.batch <= most) return 0;
+  }
   long bins = 1;
   for (int i = 0; i < d.dims; ++i) bins *= (long)d.shape[i] + 1;
   bins += 1;

@@ -186,6 +186,23 @@ def test_no_calls_between_the_kernels_of_few_points_and_the_sums_in_lds():
             assert [n > 0 for _, n in sorted(need.items())] == sorted(n > 0 for n in need.values()), (shape, channels, need)
 
 
+def test_many_points_on_small_volumes_are_sorted():
+    """Calls whose points the sorted kernels serve faster have an order to keep, those below the line have none."""
+    import ctypes
+    from deformable_kernels.ops.deform_kernel import _lib
+    L = _lib.lib()
+
+    def sorted_(points, channels, shape, dtype):
+        desc = _lib.NdDesc(points, channels, len(shape), (ctypes.c_int32 * 8)(*shape, *([1] * (8 - len(shape)))), dtype)
+        return L.dk_nd_linear_sample_order_bytes(ctypes.byref(desc)) > 0
+
+    for channels, shape, dtype, most in ((16, (8, 8, 8), _lib.DK_F32, None), (24, (300,), _lib.DK_F32, 260000), (24, (7, 7, 7), _lib.DK_F16, 160000),
+                                         (100, (5, 5), _lib.DK_BF16, 520000), (100, (90,), _lib.DK_BF16, None), (48, (7, 9), _lib.DK_F32, 0),
+                                         (48, (7, 9), _lib.DK_F16, 150000), (48, (5, 5, 5), _lib.DK_F16, 0), (64, (150,), _lib.DK_F32, 0)):
+        for points in (70000, 150000, 150001, 160001, 260001, 520001, 1200000):
+            assert sorted_(points, channels, shape, dtype) == (most is not None and points > most), (channels, shape, dtype, points)
+
+
 def test_native_self_tests_of_the_c_abi_and_the_oracle():
     """The C driver of the C ABI's argument handling (every rejection path and the workspace arithmetic
     over a sweep of geometries; all answered on the host) against the library as built, and the oracle's
