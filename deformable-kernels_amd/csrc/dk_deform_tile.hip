@@ -56,12 +56,32 @@ template <int K>
 __device__ __forceinline__ float row_lane(float v) {
   return __builtin_bit_cast(float, row_lane<K>(__builtin_bit_cast(int, v)));
 }
-// c + (the value of a that lane K of the row holds) * b in one instruction.  (A DPP operand must not have been written by the
-// two vector instructions in front: a is written once per block of channels, ahead of its LDS reads.)
-template <int K>
-__device__ __forceinline__ float fma_row(float a, float b, float c) {
-  asm("v_fmac_f32_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(c) : "v"(a), "v"(b), "n"(K));
-  return c;
+// A sample and the scope's weight at it.  In: the corners (a, b; c, d); {wgt, w_w, w_h, wc}, the table's entry {value, difference along
+// the columns, along the rows, difference of these}; the four fractions, in lane K of the row, as DPP operands.  Out: the slopes, from
+// differences of the corners, and the values, a corner and the slopes.
+// A DPP operand must not have been written by the two vector instructions in front, and the compiler, which does not look into the
+// asm, may place a register's copy or reload there.  The block's own first instructions, subtractions of corners, keep that distance,
+// and it writes none of the four.  (s_nop 1 in front in their place: 2 % of the kernel's time.)
+template <int K, bool ROT>
+__device__ __forceinline__ void lerp_row(float lh, float lw, float fh, float fw, float a, float b, float c, float d, float wc, float& s_h,
+                                         float& s_w, float& val, float& w_h, float& w_w, float& wgt) {
+#define DK_SUB(D, A, B) "v_sub_f32 %[" D "], %[" A "], %[" B "]\n\t"
+#define DK_FMAC_ROW(D, A, B) "v_fmac_f32_dpp %[" D "], %[" A "], %[" B "] row_newbcast:%[k] row_mask:0xf bank_mask:0xf\n\t"
+#define DK_LERP_ROW(W_W)                                                                                                         \
+  asm(DK_SUB("s_w", "b", "a") DK_SUB("s_h", "c", "a") DK_SUB("c", "d", "c") DK_SUB("c", "c", "s_w")                              \
+      DK_FMAC_ROW("a", "lw", "s_w") DK_FMAC_ROW("wgt", "fw", "w_w") DK_FMAC_ROW("s_h", "lw", "c") DK_FMAC_ROW("w_h", "fw", "wc") \
+      DK_FMAC_ROW("s_w", "lh", "c") W_W DK_FMAC_ROW("a", "lh", "s_h") DK_FMAC_ROW("wgt", "fh", "w_h")                            \
+      : [s_h] "=&v"(s_h), [s_w] "=&v"(s_w), [a] "+&v"(a), [c] "+&v"(c), [w_h] "+&v"(w_h), [w_w] "+&v"(w_w),                      \
+        [wgt] "+&v"(wgt)                                                                                                         \
+      : [lh] "v"(lh), [lw] "v"(lw), [fh] "v"(fh), [fw] "v"(fw), [b] "v"(b), [d] "v"(d), [wc] "v"(wc), [k] "n"(K))
+  if constexpr (ROT)
+    DK_LERP_ROW(DK_FMAC_ROW("w_w", "fh", "wc"));
+  else  // (w_w stays)
+    DK_LERP_ROW("");
+#undef DK_LERP_ROW
+#undef DK_FMAC_ROW
+#undef DK_SUB
+  val = a;
 }
 template <int CTRL>
 __device__ __forceinline__ float dpp(float v) {
@@ -396,18 +416,14 @@ __global__ __launch_bounds__(kTlBlock, 1) void deform_grad_tile_kernel(
           __builtin_amdgcn_sched_barrier(0);
           const float ca = cr[t & 1][0], cb = cr[t & 1][1], cc = cr[t & 1][2], cd = cr[t & 1][3];
           const float4 f = wt[t & 1];
-          // slopes from differences of the corners, value from a corner and the slopes
-          const float ba = cb - ca, down = cc - ca, cross = (cd - cc) - ba;
-          const float s_h = fma_row<t>(lw_, cross, down), s_w = fma_row<t>(lh_, cross, ba);
-          const float val = fma_row<t>(lh_, s_h, fma_row<t>(lw_, ba, ca));
-          const float w_h = fma_row<t>(fw_, f.w, f.z);
-          const float wgt = fma_row<t>(fh_, w_h, fma_row<t>(fw_, f.y, f.x));
+          float s_h, s_w, val, w_h = f.z, w_w = f.y, wgt = f.x;
+          lerp_row<t, ROT>(lh_, lw_, fh_, fw_, ca, cb, cc, cd, f.w, s_h, s_w, val, w_h, w_w, wgt);
           const float ps = gv * val, gw = gv * wgt;
           o_h[t] = fmaf(gw, s_h, o_h[t]);
           o_w[t] = fmaf(gw, s_w, o_w[t]);
           if constexpr (ROT) {
             r_h[t] = fmaf(ps, w_h, r_h[t]);
-            r_w[t] = fmaf(ps, fma_row<t>(fh_, f.w, f.y), r_w[t]);
+            r_w[t] = fmaf(ps, w_w, r_w[t]);
           }
           if (t & 1)
             acc1 = __builtin_amdgcn_mfma_f32_16x16x4f32(A[t], ps, acc1, 0, 0, 0);
