@@ -95,6 +95,15 @@ __device__ __forceinline__ float row_sums(float a, float b, float c, float d, in
   v += dpp<0x124>(v);                                      // row_ror:4, row_ror:8
   return v + dpp<0x128>(v);
 }
+// v[0] + ... + v[N - 1] in pairs: the rounding error of a chain grows with its length
+template <int N>
+__device__ __forceinline__ float tree_sum(float (&v)[N]) {
+#pragma unroll
+  for (int n = N / 2; n > 0; n /= 2)
+#pragma unroll
+    for (int i = 0; i < n; ++i) v[i] += v[i + n];
+  return v[0];
+}
 template <int... I, typename F>
 __device__ __forceinline__ void static_for(std::integer_sequence<int, I...>, F&& f) {
   (f(std::integral_constant<int, I>{}), ...);
@@ -312,14 +321,14 @@ __global__ __launch_bounds__(kTlBlock, 1) void deform_grad_tile_kernel(
     r_g = buf_ld(rg, p.at >= 0 ? (unsigned)(q * g_cs) + (unsigned)p.at * (unsigned)sizeof(T) : kOutOfRange, gout);
   };
 
-  // the waves' products of a block, added in wave order by the threads that own them
+  // the waves' products of a block, added up in pairs by the threads that own them
   auto flush = [&](int b, int par) {
     if (threadIdx.x >= kTlBlock - 256) {  // (the first waves make the table)
       const int e = threadIdx.x - (kTlBlock - 256);
-      float s = 0.f;
+      float s[kTlWaves];
 #pragma unroll
-      for (int w = 0; w < kTlWaves; ++w) s += red[par * kTlWaves * 256 + w * 256 + e];
-      fsum[b * 256 + e] += s;
+      for (int w = 0; w < kTlWaves; ++w) s[w] = red[par * kTlWaves * 256 + w * 256 + e];
+      fsum[b * 256 + e] += tree_sum(s);
     }
   };
 
@@ -497,7 +506,7 @@ constexpr long kTlManyElements = 32768;
 template <typename T>
 __global__ __launch_bounds__(1024) void deform_reduce_jobs_kernel(ReduceJobs<T> jobs, TileChoice choice) {
   constexpr int PU = 8;
-  __shared__ float rows[64][16];
+  __shared__ float rows[16][16];
   const bool wide = choice.windows && !tiles_take(choice);
   const int e = threadIdx.x & 15, row = threadIdx.x >> 4;
   for (int k = 0; k < 3; ++k) {
@@ -539,12 +548,17 @@ __global__ __launch_bounds__(1024) void deform_reduce_jobs_kernel(ReduceJobs<T> 
 #pragma unroll 4
         for (int p = row; p < j.parts; p += 64) s += j.partial[(size_t)p * j.count + at];
       }
+      // 64 rows in pairs: the four of a wave, then the waves'
+      s += __shfl_xor(s, 16);
+      s += __shfl_xor(s, 32);
       __syncthreads();
-      rows[row][e] = s;
+      if (row % 4 == 0) rows[row / 4][e] = s;
       __syncthreads();
       if (row == 0 && at < j.count) {
-        for (int r = 1; r < 64; ++r) s += rows[r][e];
-        st(j.out + at, s);
+        float v[16];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) v[r] = rows[r][e];
+        st(j.out + at, tree_sum(v));
       }
     }
   }

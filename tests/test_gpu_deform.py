@@ -726,3 +726,21 @@ def test_coordinate_and_filter_gradients_of_planes_with_a_long_side(plane, plain
     # sums of at most 2 * 10^6 products of three factors in float32, in blocks
     for g, w in zip(got, (want[1], want[3]) if plain else want[1:]):
         assert rel_err(g.cpu(), w) < 2e-5
+
+
+@pytest.mark.parametrize("shape, gradient, bound", [
+    # the filter's sums in pairs: 1.2 and 1.3 * 10^-7 measured, 1.9 and 2.0 with 64 partial sums in a chain
+    ((16, 192, 14, 14), 2, 1.6e-7), ((8, 144, 56, 56), 2, 1.6e-7),
+])
+def test_rounding_error_of_the_gradients(shape, gradient, bound):
+    """Against the operator in float64, on coordinates that float32 holds to the last bit: what the kernels' own arithmetic rounds."""
+    from deformable_kernels.ops.deform_kernel.functions import deform_sample_depthwise
+    x, wt, rot, off, gout, cfg = make_deform(*shape, 3, (4, 4), 1, 1, 1, 1, 0.5, 1.0, seed=25)
+    off, rot = (off * 4096).round() / 4096, (rot * 4096).round() / 4096
+
+    def grads(dtype):
+        leaves = [t.to("cuda:0", dtype).requires_grad_() for t in (off, rot, wt)]
+        out = deform_sample_depthwise(x.to("cuda:0", dtype), *leaves, cfg["kernel_size"], cfg["stride"], cfg["padding"], cfg["dilation"], 1)
+        return torch.autograd.grad(out, leaves, gout.to("cuda:0", dtype))[gradient].double()
+    got, want = grads(torch.float32), grads(torch.float64)
+    assert float((got - want).norm() / want.norm()) < bound
