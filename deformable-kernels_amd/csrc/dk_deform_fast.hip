@@ -409,14 +409,16 @@ __global__ __launch_bounds__(BLOCK, BLOCK == kDBlock ? 2 : 1) void deform_forwar
 }
 
 
-// Value and slopes of a sample from its corners; the slopes are differences of corners, the value a corner and the slopes.
+// Value and slopes of a sample from its corners.  A slope is a difference of corners and its change across the cell, from the
+// differences on either side: with one change for both slopes, down - across as it comes from the columns' differences, the row slope's
+// rounding error is a quarter larger (5.7 against 4.6 * 10^-8 on normally distributed corners).
 struct Sample {
   float val, h, w;
 };
 __device__ __forceinline__ Sample sample_slopes(float a, float b, float c, float d, float lh, float lw) {
-  const float ba = b - a, down = c - a, cross = (d - c) - ba;
+  const float ba = b - a, ca = c - a;
   Sample s;
-  s.h = fmaf(lw, cross, down), s.w = fmaf(lh, cross, ba);
+  s.h = fmaf(lw, (d - b) - ca, ca), s.w = fmaf(lh, (d - c) - ba, ba);
   s.val = fmaf(lh, s.h, fmaf(lw, ba, a));
   return s;
 }

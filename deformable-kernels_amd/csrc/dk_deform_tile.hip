@@ -57,8 +57,9 @@ __device__ __forceinline__ float row_lane(float v) {
   return __builtin_bit_cast(float, row_lane<K>(__builtin_bit_cast(int, v)));
 }
 // A sample and the scope's weight at it.  In: the corners (a, b; c, d); {wgt, w_w, w_h, wc}, the table's entry {value, difference along
-// the columns, along the rows, difference of these}; the four fractions, in lane K of the row, as DPP operands.  Out: the slopes, from
-// differences of the corners, and the values, a corner and the slopes.
+// the columns, along the rows, difference of these}; the four fractions, in lane K of the row, as DPP operands.  Out: the slopes, each
+// a difference of corners and its change across the cell, from the differences on either side (sample_slopes has why), and the values, a
+// corner and the slopes.
 // A DPP operand must not have been written by the two vector instructions in front, and the compiler, which does not look into the
 // asm, may place a register's copy or reload there.  The block's own first instructions, subtractions of corners, keep that distance,
 // and it writes none of the four.  (s_nop 1 in front in their place: 2 % of the kernel's time.)
@@ -67,13 +68,13 @@ __device__ __forceinline__ void lerp_row(float lh, float lw, float fh, float fw,
                                          float& s_w, float& val, float& w_h, float& w_w, float& wgt) {
 #define DK_SUB(D, A, B) "v_sub_f32 %[" D "], %[" A "], %[" B "]\n\t"
 #define DK_FMAC_ROW(D, A, B) "v_fmac_f32_dpp %[" D "], %[" A "], %[" B "] row_newbcast:%[k] row_mask:0xf bank_mask:0xf\n\t"
-#define DK_LERP_ROW(W_W)                                                                                                         \
-  asm(DK_SUB("s_w", "b", "a") DK_SUB("s_h", "c", "a") DK_SUB("c", "d", "c") DK_SUB("c", "c", "s_w")                              \
-      DK_FMAC_ROW("a", "lw", "s_w") DK_FMAC_ROW("wgt", "fw", "w_w") DK_FMAC_ROW("s_h", "lw", "c") DK_FMAC_ROW("w_h", "fw", "wc") \
-      DK_FMAC_ROW("s_w", "lh", "c") W_W DK_FMAC_ROW("a", "lh", "s_h") DK_FMAC_ROW("wgt", "fh", "w_h")                            \
-      : [s_h] "=&v"(s_h), [s_w] "=&v"(s_w), [a] "+&v"(a), [c] "+&v"(c), [w_h] "+&v"(w_h), [w_w] "+&v"(w_w),                      \
-        [wgt] "+&v"(wgt)                                                                                                         \
-      : [lh] "v"(lh), [lw] "v"(lw), [fh] "v"(fh), [fw] "v"(fw), [b] "v"(b), [d] "v"(d), [wc] "v"(wc), [k] "n"(K))
+#define DK_LERP_ROW(W_W)                                                                                                                          \
+  asm(DK_SUB("s_w", "b", "a") DK_SUB("s_h", "c", "a") DK_SUB("b", "d", "b") DK_SUB("c", "d", "c") DK_SUB("b", "b", "s_h") DK_SUB("c", "c", "s_w") \
+      DK_FMAC_ROW("a", "lw", "s_w") DK_FMAC_ROW("wgt", "fw", "w_w") DK_FMAC_ROW("s_h", "lw", "b") DK_FMAC_ROW("w_h", "fw", "wc")                  \
+      DK_FMAC_ROW("s_w", "lh", "c") W_W DK_FMAC_ROW("a", "lh", "s_h") DK_FMAC_ROW("wgt", "fh", "w_h")                                             \
+      : [s_h] "=&v"(s_h), [s_w] "=&v"(s_w), [a] "+&v"(a), [b] "+&v"(b), [c] "+&v"(c), [w_h] "+&v"(w_h), [w_w] "+&v"(w_w),                         \
+        [wgt] "+&v"(wgt)                                                                                                                          \
+      : [lh] "v"(lh), [lw] "v"(lw), [fh] "v"(fh), [fw] "v"(fw), [d] "v"(d), [wc] "v"(wc), [k] "n"(K))
   if constexpr (ROT)
     DK_LERP_ROW(DK_FMAC_ROW("w_w", "fh", "wc"));
   else  // (w_w stays)

@@ -731,6 +731,8 @@ def test_coordinate_and_filter_gradients_of_planes_with_a_long_side(plane, plain
 @pytest.mark.parametrize("shape, gradient, bound", [
     # the filter's sums in pairs: 1.2 and 1.3 * 10^-7 measured, 1.9 and 2.0 with 64 partial sums in a chain
     ((16, 192, 14, 14), 2, 1.6e-7), ((8, 144, 56, 56), 2, 1.6e-7),
+    # the slopes' changes across a cell from the differences on either side: 1.311 and 1.086 measured, 1.330 and 1.109 with one change for both
+    ((16, 192, 28, 28), 0, 1.32e-7), ((64, 16, 20, 20), 0, 1.097e-7),
 ])
 def test_rounding_error_of_the_gradients(shape, gradient, bound):
     """Against the operator in float64, on coordinates that float32 holds to the last bit: what the kernels' own arithmetic rounds."""
