@@ -58,28 +58,31 @@ __device__ __forceinline__ float row_lane(float v) {
 }
 // A sample and the scope's weight at it.  In: the corners (a, b; c, d); {wgt, w_w, w_h, wc}, the table's entry {value, difference along
 // the columns, along the rows, difference of these}; the four fractions, in lane K of the row, as DPP operands.  Out: the slopes, each
-// a difference of corners and its change across the cell, from the differences on either side (sample_slopes has why), and the values, a
-// corner and the slopes.
+// a difference of corners and its change across the cell (OWN: from the differences on either side, as sample_slopes; else one change
+// for both), and the values, a corner and the slopes.
 // A DPP operand must not have been written by the two vector instructions in front, and the compiler, which does not look into the
 // asm, may place a register's copy or reload there.  The block's own first instructions, subtractions of corners, keep that distance,
 // and it writes none of the four.  (s_nop 1 in front in their place: 2 % of the kernel's time.)
-template <int K, bool ROT>
+template <int K, bool ROT, bool OWN>
 __device__ __forceinline__ void lerp_row(float lh, float lw, float fh, float fw, float a, float b, float c, float d, float wc, float& s_h,
                                          float& s_w, float& val, float& w_h, float& w_w, float& wgt) {
 #define DK_SUB(D, A, B) "v_sub_f32 %[" D "], %[" A "], %[" B "]\n\t"
 #define DK_FMAC_ROW(D, A, B) "v_fmac_f32_dpp %[" D "], %[" A "], %[" B "] row_newbcast:%[k] row_mask:0xf bank_mask:0xf\n\t"
-#define DK_LERP_ROW(W_W)                                                                                                                          \
-  asm(DK_SUB("s_w", "b", "a") DK_SUB("s_h", "c", "a") DK_SUB("b", "d", "b") DK_SUB("c", "d", "c") DK_SUB("b", "b", "s_h") DK_SUB("c", "c", "s_w") \
-      DK_FMAC_ROW("a", "lw", "s_w") DK_FMAC_ROW("wgt", "fw", "w_w") DK_FMAC_ROW("s_h", "lw", "b") DK_FMAC_ROW("w_h", "fw", "wc")                  \
-      DK_FMAC_ROW("s_w", "lh", "c") W_W DK_FMAC_ROW("a", "lh", "s_h") DK_FMAC_ROW("wgt", "fh", "w_h")                                             \
-      : [s_h] "=&v"(s_h), [s_w] "=&v"(s_w), [a] "+&v"(a), [b] "+&v"(b), [c] "+&v"(c), [w_h] "+&v"(w_h), [w_w] "+&v"(w_w),                         \
-        [wgt] "+&v"(wgt)                                                                                                                          \
+#define DK_OWN DK_SUB("b", "d", "b") DK_SUB("c", "d", "c") DK_SUB("b", "b", "s_h")
+#define DK_LERP_ROW(CHANGES, ACROSS, W_W)                                                                                           \
+  asm(DK_SUB("s_w", "b", "a") DK_SUB("s_h", "c", "a") CHANGES DK_SUB("c", "c", "s_w")                                               \
+      DK_FMAC_ROW("a", "lw", "s_w") DK_FMAC_ROW("wgt", "fw", "w_w") DK_FMAC_ROW("s_h", "lw", ACROSS) DK_FMAC_ROW("w_h", "fw", "wc") \
+      DK_FMAC_ROW("s_w", "lh", "c") W_W DK_FMAC_ROW("a", "lh", "s_h") DK_FMAC_ROW("wgt", "fh", "w_h")                               \
+      : [s_h] "=&v"(s_h), [s_w] "=&v"(s_w), [a] "+&v"(a), [b] "+&v"(b), [c] "+&v"(c), [w_h] "+&v"(w_h), [w_w] "+&v"(w_w),           \
+        [wgt] "+&v"(wgt)                                                                                                            \
       : [lh] "v"(lh), [lw] "v"(lw), [fh] "v"(fh), [fw] "v"(fw), [d] "v"(d), [wc] "v"(wc), [k] "n"(K))
-  if constexpr (ROT)
-    DK_LERP_ROW(DK_FMAC_ROW("w_w", "fh", "wc"));
-  else  // (w_w stays)
-    DK_LERP_ROW("");
+  // (without ROT w_w stays)
+  if constexpr (ROT && OWN) DK_LERP_ROW(DK_OWN, "b", DK_FMAC_ROW("w_w", "fh", "wc"));
+  else if constexpr (ROT) DK_LERP_ROW(DK_SUB("c", "d", "c"), "c", DK_FMAC_ROW("w_w", "fh", "wc"));
+  else if constexpr (OWN) DK_LERP_ROW(DK_OWN, "b", "");
+  else DK_LERP_ROW(DK_SUB("c", "d", "c"), "c", "");
 #undef DK_LERP_ROW
+#undef DK_OWN
 #undef DK_FMAC_ROW
 #undef DK_SUB
   val = a;
@@ -166,8 +169,8 @@ __global__ __launch_bounds__(256) void deform_tile_boxes_kernel(Geo g, const T* 
   if (threadIdx.x == 0) windows[blockIdx.x] = (unsigned)(wave_sum_[0] + wave_sum_[1] + wave_sum_[2] + wave_sum_[3]);
 }
 
-// ROT: false: rotation is null (all zeros), and there is no gradient for it.
-template <typename T, int SH, int SW, bool ROT>
+// ROT: false: rotation is null (all zeros), and there is no gradient for it.  OWN: lerp_row.
+template <typename T, int SH, int SW, bool ROT, bool OWN>
 __global__ __launch_bounds__(kTlBlock, 1) void deform_grad_tile_kernel(
     Geo g, const T* __restrict__ gout, const T* __restrict__ x, const T* __restrict__ off, const T* __restrict__ rot,
     const T* __restrict__ filter, T* __restrict__ goff, T* __restrict__ grot, float* __restrict__ part_off,
@@ -427,7 +430,7 @@ __global__ __launch_bounds__(kTlBlock, 1) void deform_grad_tile_kernel(
           const float ca = cr[t & 1][0], cb = cr[t & 1][1], cc = cr[t & 1][2], cd = cr[t & 1][3];
           const float4 f = wt[t & 1];
           float s_h, s_w, val, w_h = f.z, w_w = f.y, wgt = f.x;
-          lerp_row<t, ROT>(lh_, lw_, fh_, fw_, ca, cb, cc, cd, f.w, s_h, s_w, val, w_h, w_w, wgt);
+          lerp_row<t, ROT, OWN>(lh_, lw_, fh_, fw_, ca, cb, cc, cd, f.w, s_h, s_w, val, w_h, w_w, wgt);
           const float ps = gv * val, gw = gv * wgt;
           o_h[t] = fmaf(gw, s_h, o_h[t]);
           o_w[t] = fmaf(gw, s_w, o_w[t]);
@@ -629,7 +632,12 @@ bool run_tile(const Geo& g, const TilePlan& m, const T* gout, const T* x, const 
   int4* boxes = m.boxed ? reinterpret_cast<int4*>(ws0) : nullptr;
   float* ws = ws0 + w.boxes / sizeof(float);
   float *p_off = w.off ? ws : nullptr, *p_rot = w.rot && rot ? ws + w.off : nullptr, *p_filter = ws + w.off + w.rot;
-  auto kernel = rot ? deform_grad_tile_kernel<T, SH, SW, true> : deform_grad_tile_kernel<T, SH, SW, false>;
+  // One change for both slopes is 3 % of the kernel's time; with few channels the longer sums of the separate kernels do not make up for its
+  // rounding: offset gradient's error against float64 in 10^-8, separate kernels / one change / each its own: 16 channels 10.4 / 10.6 / 10.4,
+  // 48 11.02 / 11.06 / 10.81, 64 11.3 / 11.0, 144 17.7 / 11.8.
+  const bool own = g.channel / g.groups < 64;
+  auto kernel = rot ? (own ? deform_grad_tile_kernel<T, SH, SW, true, true> : deform_grad_tile_kernel<T, SH, SW, true, false>)
+                    : (own ? deform_grad_tile_kernel<T, SH, SW, false, true> : deform_grad_tile_kernel<T, SH, SW, false, false>);
   if (!allow_dynamic_lds(reinterpret_cast<const void*>(kernel), kTlLds)) return false;
   TileChoice choice{}, behind{};
   unsigned* left = nullptr;

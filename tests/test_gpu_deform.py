@@ -696,6 +696,23 @@ def test_one_pass_in_16_bits_and_without_a_rotation_tensor(dtype, plain):
         assert g.dtype == dtype and rel_err(g.float().cpu(), w) < (2e-3 if dtype == torch.float16 else 1e-2)  # the result's rounding
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("plain", [False, True])
+@pytest.mark.parametrize("channels, scope", [(63, 4), (64, 4), (63, 3), (64, 3)])
+def test_one_pass_on_either_side_of_64_channels(channels, scope, plain, dtype):
+    """From 64 channels on one change across the cell serves both slopes."""
+    from deformable_kernels.ops.deform_kernel.functions import deform_sample_depthwise
+    x, wt, rot, off, gout, cfg = make_deform(1, channels, 70, 90, 3, (scope, scope), 1, 1, 1, 1, 0.0 if plain else 0.7, 1.0, seed=26, dtype=dtype)
+    leaves = [t.to("cuda:0").requires_grad_() for t in ((off, wt) if plain else (off, rot, wt))]
+    offs, rots, wts = (leaves[0], None, leaves[1]) if plain else leaves
+    out = deform_sample_depthwise(x.to("cuda:0"), offs, rots, wts, cfg["kernel_size"], cfg["stride"], cfg["padding"], cfg["dilation"], 1)
+    got = torch.autograd.grad(out, leaves, gout.to("cuda:0"))
+    want = orc.deform_sample_depthwise_backward(*[t.double().numpy() for t in (gout, x, off, rot, wt)], **cfg)
+    tol = {torch.float32: 2e-5, torch.float16: 2e-3, torch.bfloat16: 1e-2}[dtype]  # sums in float32; the result's rounding
+    for g, w in zip(got, (want[1], want[3]) if plain else want[1:]):
+        assert g.dtype == dtype and rel_err(g.float().cpu(), w) < tol
+
+
 def test_one_pass_non_finite_output_gradient_reaches_its_pixel_and_channel_only():
     from deformable_kernels.ops.deform_kernel.functions import deform_sample_depthwise
     x, wt, rot, off, gout, cfg = make_deform(2, 24, 40, 40, 3, (4, 4), 1, 1, 1, 1, 0.5, 1.0, seed=23)
