@@ -20,11 +20,12 @@
 // window take several passes over neighbouring windows, each sample counted in the pass that holds its corners.
 //
 // N=64 C=144 56 x 56 float32: both coordinate gradients 323 us and the filter gradient 320 with a pixel per lane, 20 of reductions;
-// 453 here and 5.  What bounds it is vector issue (24 instructions per tap and four pixels x 16 channels, and half as many again
+// 450 here and 6.  What bounds it is vector issue (24 instructions per tap and four pixels x 16 channels, and half as many again
 // per block and tile): 62 % of the cycles; without the loads of the window it takes 49 us less, without the matrix
 // instructions 22.  The DPP operands inside the multiply-adds (27 instructions per tap with moves: 563 -> 513 us) and the
-// tiles' windows from a kernel in front (513 -> 453: two barriers and a round trip to memory less per tile) carry it; a register
-// more per lane spills into the loop over the blocks and costs more than either.
+// tiles' windows from a kernel in front (513 -> 453: two barriers and a round trip to memory less per tile) carry it.  With a rotation
+// tensor the kernels take all 128 registers and keep 13 or 15 more in scratch, which are read once per tile; where a spill
+// falls into the loop over the blocks it costs more than either.
 #include <algorithm>
 #include <type_traits>
 
