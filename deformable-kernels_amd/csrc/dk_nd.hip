@@ -1780,7 +1780,8 @@ bool nd_small(const dk_nd_desc& d) {
 bool nd_use_channel_last(const dk_nd_desc& d) {
   if (d.dtype == DK_F64 || d.dims > kClMaxDims || nd_small(d)) return false;
   const long cells = nd_cells(d);
-  if (cells > 2147483647L / 4) return false;  // corner offsets are kept as 32-bit element counts
+  // corner offsets are kept as 32-bit element counts, and a launch holds fewer than 2^32 threads: 2^24 tiles of the transposes
+  if (cells > (1L << 29) - 32) return false;
   const bool rows = !path_disabled(kNoNdRows);
   if (rows && cells <= kSmallMaxCells && d.batch > 4096) return true;  // too many points for nd_small()
   if (d.batch * d.channel < 65536) return false;

@@ -165,6 +165,8 @@ def test_workspaces_of_few_channels_on_large_volumes():
     # the gradients' copies are worth it before the forward's
     assert sizes(245000, 3, 1400, 1400)[0] == 0 < sizes(245000, 3, 1400, 1400)[2]
     assert all(n >= 3 * 64 * 64 * 4 for n in sizes(1000000, 3, 64, 64))
+    # 2^24 tiles of 32 cells and 256 threads are more than a launch holds
+    assert sizes(1 << 30, 3, (1 << 29) - 32)[0] > 0 and sizes(1 << 30, 3, (1 << 29) - 31)[::2] == [0, 0]
 
 
 def test_no_calls_between_the_kernels_of_few_points_and_the_sums_in_lds():
