@@ -336,6 +336,8 @@ int dk_nd_linear_sample_backward(const dk_nd_desc *desc, const void *out_grad, c
  * whether a shape is covered, dk_offset_conv_worthwhile() whether it is also expected to beat the
  * library convolution (every covered plane with at least 64 (image, 448-pixel tile) items); the
  * caller keeps its library convolution otherwise.
+ * (16-bit tensors whose channels are no multiple of 16: the query speaks for the kernels' time alone.  The Python operator
+ * leaves the forward of such layers to the framework all the same, so that their offsets keep their bits, and takes the gradients.)
  *   input [batch, in_channels, h, w], weight [out_channels, in_channels, 3, 3],
  *   bias [out_channels], output [batch, out_channels, h, w]; workspace: packed weights. */
 typedef struct dk_offset_conv_desc {
