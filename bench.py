@@ -125,7 +125,7 @@ def summarise_traffic(a):
     out = {"workload": a.workload, "dtype": a.dtype, "kernel_source_sha256": kernel_source_hash(),
            "unit": "KiB per call of the entry point, as rocprofv3 reports the counter",
            "commands": ["rocprofv3 --pmc %s -d <dir> -o pmc -- python3 bench.py --workload %s --dtype %s --steps 3 "
-                        "--warmup 1 --no-cpu-baseline" % (c, a.workload, a.dtype) for c in ("FETCH_SIZE", "WRITE_SIZE")],
+                        "--warmup 1 --no-cpu-baseline --no-network-pass" % (c, a.workload, a.dtype) for c in ("FETCH_SIZE", "WRITE_SIZE")],
            "entries": {}, "kernels": {}}
     try:
         head = subprocess.run(["git", "-C", ROOT, "rev-parse", "HEAD"], capture_output=True, text=True).stdout.strip()
